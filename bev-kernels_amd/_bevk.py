@@ -38,6 +38,8 @@ _SIGNATURES = {
     + [_vp, _vp, _vp, _vp],
     "bevk_modulated_deformable_col2im_nhwc": [_i, _vp, _vp, _vp, _i, _vp] + [_i] * 15
     + [_vp, _vp, _vp, _vp],
+    "bevk_dcn_layer_im2col_nhwc": [_i, _vp, _vp, _vp] + [_i] * 15 + [_vp, _vp],
+    "bevk_dcn_layer_col2im_nhwc": [_i, _vp, _vp, _vp, _vp] + [_i] * 15 + [_vp, _vp, _vp, _vp],
     "bevk_dcn_fused_im2col_nhwc_workspace_bytes": [_i] * 7,
     "bevk_modulated_deformable_fused_im2col_nhwc": [_i, _vp, _vp, _vp] + [_i] * 15
     + [_vp, ctypes.c_int64, _vp, _vp],

@@ -40,6 +40,8 @@ __all__ = [
     "modulated_deformable_col2im_fused_smem_nhwc_cuda",
     "modulated_deformable_col2im_perelem_nhwc_cuda",
     "modulated_deformable_col2im_perelem_smem_nhwc_cuda",
+    "dcn_layer_im2col_nhwc",
+    "dcn_layer_col2im_nhwc",
     "dcn_packed_weight_numel",
     "dcn_pack_weight",
     "dcn_fused_fwd_nhwc",
@@ -406,6 +408,48 @@ def _col2im_nhwc(fn, dcol, data_im, data_offset, data_mask, batch_size, channels
             channels, height_im, width_im, height_col, width_col, kernel_h, kernel_w, pad_h,
             pad_w, stride_h, stride_w, dilation_h, dilation_w, deformable_group,
             _b.ptr(grad_im), _b.ptr(grad_offset), _b.ptr(grad_mask), _b.stream_of(dcol))
+
+
+def _layer_nhwc(fn, col, data_im, data_offset, data_mask, sizes, grads=()):
+    """Checks of the two layer steps below; sizes = (B, C, H, W, Ho, Wo, kh, kw, ph, pw, sh,
+    sw, dh, dw, dg)."""
+    batch, channels, height, width, height_col, width_col, kernel_h, kernel_w = sizes[:8]
+    dg = sizes[14]
+    _b.require_device(fn, col, data_im, data_offset, data_mask, *grads)
+    _b.require_contiguous(fn, col=col, data_im=data_im, data_offset=data_offset,
+                          data_mask=data_mask)
+    _b.require_dtype(fn, data_im, col=col, data_offset=data_offset, data_mask=data_mask)
+    taps, m = kernel_h * kernel_w, batch * height_col * width_col
+    _b.require_numel(fn, "columns", col, m * taps * channels)
+    _b.require_numel(fn, "data_im", data_im, batch * height * width * channels)
+    _b.require_numel(fn, "data_offset", data_offset, m * dg * 2 * taps)
+    _b.require_numel(fn, "data_mask", data_mask, m * dg * taps)
+    for name, t, n in zip(("grad_im", "grad_offset", "grad_mask"), grads,
+                          (batch * height * width * channels, m * dg * 2 * taps, m * dg * taps)):
+        if t.dtype != torch.float32 or not t.is_contiguous():
+            raise RuntimeError(f"{fn}: {name} must be contiguous float32")
+        _b.require_numel(fn, name, t, n)
+
+
+def dcn_layer_im2col_nhwc(data_im, data_offset, data_mask, *sizes_and_col):
+    """Columns [M, T*C] of NHWC data_im with offsets [M, dg, 2T] and mask [M, dg, T];
+    arguments as modulated_deformable_im2col_nhwc_cuda."""
+    *sizes, col = sizes_and_col
+    _layer_nhwc("dcn_layer_im2col_nhwc", col, data_im, data_offset, data_mask, sizes)
+    _b.call("bevk_dcn_layer_im2col_nhwc", _b.dtype_code(data_im), _b.ptr(data_im),
+            _b.ptr(data_offset), _b.ptr(data_mask), *sizes, _b.ptr(col), _b.stream_of(col))
+
+
+def dcn_layer_col2im_nhwc(dcol, data_im, data_offset, data_mask, *sizes_and_grads):
+    """Column-to-image with the NCHW layer's gate and deformable groups: grad_im [B,H,W,C]
+    fp32 accumulated (zero it first), grad_offset [M,dg,2T] / grad_mask [M,dg,T] fp32
+    written; arguments as modulated_deformable_col2im_nhwc_cuda."""
+    *sizes, grad_im, grad_offset, grad_mask = sizes_and_grads
+    _layer_nhwc("dcn_layer_col2im_nhwc", dcol, data_im, data_offset, data_mask, sizes,
+                (grad_im, grad_offset, grad_mask))
+    _b.call("bevk_dcn_layer_col2im_nhwc", _b.dtype_code(dcol), _b.ptr(dcol), _b.ptr(data_im),
+            _b.ptr(data_offset), _b.ptr(data_mask), *sizes, _b.ptr(grad_im),
+            _b.ptr(grad_offset), _b.ptr(grad_mask), _b.stream_of(dcol))
 
 
 def modulated_deformable_col2im_nhwc_cuda(dcol, data_im, data_offset, data_mask, batch_size,

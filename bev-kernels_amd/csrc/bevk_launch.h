@@ -52,6 +52,8 @@ struct DcnGeom {
   int batch, channels, height, width, height_col, width_col;
   int kernel_h, kernel_w, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w;
   int deformable_group;
+  int gate = 0;  // NHWC column-to-image: whole samples with h <= -1, w <= -1, h >= H or w >= W
+                 // contribute nothing (the NCHW layer's rule)
 };
 
 // NCHW modulated im2col; `tiled` picks the geometry-reuse kernel (im2col_opt).
@@ -59,7 +61,7 @@ hipError_t launch_im2col_nchw(int dtype, const DcnGeom &g, const void *data_im,
                               const void *data_offset, const void *data_mask,
                               void *data_col, bool tiled, hipStream_t stream);
 
-// NHWC gather (dg == 1). fused_y: data_offset is the raw [.., 3T] offset-conv output.
+// NHWC gather (offsets [M][dg][2T], mask [M][dg][T]). fused_y (dg == 1): data_offset is the raw [.., 3T] offset-conv output.
 hipError_t launch_im2col_nhwc(int dtype, const DcnGeom &g, const void *data_im,
                               const void *data_offset, bool fused_y, const void *data_mask,
                               void *data_col, hipStream_t stream);
@@ -119,10 +121,10 @@ hipError_t launch_col2im_nchw(int dtype, const DcnGeom &g, const void *col, cons
                               const void *off, const void *msk, void *grad_im,
                               void *grad_offset, void *grad_mask, hipStream_t stream);
 
-// NHWC column-to-image backward (dg == 1): grad_im [B,H,W,C] fp32 accumulated with atomics
-// (caller zeroes it; skipped when null), grad_offset [M][2T] and grad_mask [M][T] fp32
-// written (skipped when grad_offset is null). fused_y: offsets / pre-sigmoid mask from
-// y [M][3T] and grad_mask is the gradient of the pre-sigmoid value.
+// NHWC column-to-image backward (offsets [M][dg][2T], mask [M][dg][T]): grad_im [B,H,W,C] fp32 accumulated with atomics
+// (caller zeroes it; skipped when null), grad_offset [M][dg][2T] and grad_mask [M][dg][T] fp32
+// written (skipped when grad_offset is null). fused_y (dg == 1): offsets / pre-sigmoid mask
+// from y [M][3T] and grad_mask is the gradient of the pre-sigmoid value.
 hipError_t launch_col2im_nhwc(int dtype, const DcnGeom &g, const void *dcol, const void *im,
                               const void *off, bool fused_y, const void *msk, float *grad_im,
                               float *grad_offset, float *grad_mask, hipStream_t stream);

@@ -250,6 +250,64 @@ int bevk_modulated_deformable_col2im_nhwc(
                     fn);
 }
 
+int bevk_dcn_layer_im2col_nhwc(int dtype, const void *data_im, const void *data_offset,
+                               const void *data_mask, int batch_size, int channels, int height_im,
+                               int width_im, int height_col, int width_col, int kernel_h,
+                               int kernel_w, int pad_h, int pad_w, int stride_h, int stride_w,
+                               int dilation_h, int dilation_w, int deformable_group,
+                               void *data_col, void *stream) {
+  const char *fn = "dcn_layer_im2col_nhwc";
+  g_last_error.clear();
+  if (dtype != BEVK_F32 && dtype != BEVK_F16 && dtype != BEVK_BF16)
+    return fail(BEVK_ERR_UNSUPPORTED, "\"%s\" not implemented for '%s'", fn, dtype_name(dtype));
+  const bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w,
+                deformable_group);
+  if (int rc = check_geom(fn, g)) return rc;
+  const long long taps = (long long)kernel_h * kernel_w;
+  const long long m = (long long)batch_size * height_col * width_col;
+  if (m * taps * channels >= 2147483647LL || m * taps * deformable_group >= 2147483647LL)
+    return fail(BEVK_ERR_INVALID, "NHWC gather: Col element count exceeds int32 range");
+  if (m * taps * channels == 0) return ok();
+  if ((long long)channels * height_im * width_im * dtype_size(dtype) > kMaxBufferBytes)
+    return fail(BEVK_ERR_INVALID, "%s: one input image exceeds 2 GiB", fn);
+  if (!data_im || !data_offset || !data_mask || !data_col)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(bevk::launch_im2col_nhwc(dtype, g, data_im, data_offset, false, data_mask,
+                                             data_col, (hipStream_t)stream),
+                    fn);
+}
+
+int bevk_dcn_layer_col2im_nhwc(
+    int dtype, const void *dcol, const void *data_im, const void *data_offset,
+    const void *data_mask, int batch_size, int channels, int height_im, int width_im,
+    int height_col, int width_col, int kernel_h, int kernel_w, int pad_h, int pad_w, int stride_h,
+    int stride_w, int dilation_h, int dilation_w, int deformable_group, float *grad_im,
+    float *grad_offset, float *grad_mask, void *stream) {
+  const char *fn = "dcn_layer_col2im_nhwc";
+  g_last_error.clear();
+  if (dtype != BEVK_F32 && dtype != BEVK_F16 && dtype != BEVK_BF16)
+    return fail(BEVK_ERR_UNSUPPORTED, "\"%s\" not implemented for '%s'", fn, dtype_name(dtype));
+  bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w,
+                deformable_group);
+  if (int rc = check_geom(fn, g)) return rc;
+  g.gate = 1;
+  const long long taps = (long long)kernel_h * kernel_w;
+  const long long m = (long long)batch_size * height_col * width_col;
+  if (m * taps * channels >= 2147483647LL || m * taps * deformable_group >= 2147483647LL)
+    return fail(BEVK_ERR_INVALID, "NHWC col2im: Col element count exceeds int32 range");
+  if (m * taps == 0) return ok();
+  if (!dcol || !data_im || !data_offset || !data_mask || !grad_im || !grad_offset || !grad_mask)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(bevk::launch_col2im_nhwc(dtype, g, dcol, data_im, data_offset, false,
+                                             data_mask, grad_im, grad_offset, grad_mask,
+                                             (hipStream_t)stream),
+                    fn);
+}
+
 // Static scratch of the allocation-free front end
 // (bevk_modulated_deformable_fused_im2col_nhwc_noalloc): the packed offset-conv weight and
 // the fp32 offset-conv output y [M][3T] of one call. Every GPU the library runs on holds

@@ -13,6 +13,11 @@
 // A corner outside the image contributes nothing (the reference checks each corner; there
 // is no separate -1 / H gate in the backward).
 //
+// Two options serve the NCHW layer's backward (modulated_deform_conv_cuda_kernel.cuh:62-131,
+// :509-620), which runs these kernels on NHWC copies: deformable groups (channel c of group
+// c / (C / dg) takes offsets [M][dg][2T] and mask [M][dg][T]) and its gate (a sample with
+// h <= -1, w <= -1, h >= H or w >= W contributes nothing and gets zero gradients).
+//
 // Mapping: LPP = min(64, next power of two >= C) lanes own one (m, t) pair; lane li takes
 // channels li, li + LPP, ..., so each gX atomic instruction adds LPP consecutive floats
 // (fp32 atomics are issued per cache line: one lane holding 4 or 8 consecutive channels
@@ -35,14 +40,14 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
     const T *__restrict__ dcol, const T *__restrict__ im, const T *__restrict__ offset,
     const T *__restrict__ mask, const DcnGeom g, int lpp_log2, float *__restrict__ gx,
     float *__restrict__ goff, float *__restrict__ gmask) {
-  const int T_ = g.kernel_h * g.kernel_w;
+  const int T_ = g.kernel_h * g.kernel_w, dg = g.deformable_group;
   const int HoWo = g.height_col * g.width_col;
   const int b = blockIdx.y;
   const int pair = (blockIdx.x * kBlock + threadIdx.x) >> lpp_log2;
   const int LPP = 1 << lpp_log2;
   const int li = threadIdx.x & (LPP - 1);
   // Lanes past the last pair still take part in the butterfly below; they do no work.
-  const bool live = pair < HoWo * T_;
+  const bool live = pair < HoWo * T_ * dg;  // (pixel, tap, group)
   const int pc = live ? pair : 0;
   // Quotients by the runtime sizes from a float reciprocal, corrected by one step (the
   // launch keeps every quotient below 2^22, where the estimate is off by at most one).
@@ -51,10 +56,12 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
     const int r = a - q * d;
     return q + (r >= d) - (r < 0);
   };
-  const int sp = qdiv(pc, T_), t = pc - sp * T_;
+  const int pt = dg == 1 ? pc : pc / dg, grp = pc - pt * dg;
+  const int sp = qdiv(pt, T_), t = pt - sp * T_;
   const int oh = qdiv(sp, g.width_col), ow = sp - oh * g.width_col;
   const int i = qdiv(t, g.kernel_w), j = t - i * g.kernel_w;
-  const int m = b * HoWo + sp;  // 32-bit indices: the launch checks the tensor sizes
+  const int m = b * HoWo + sp;
+  const int64_t mg = (int64_t)m * dg + grp;  // row of offset / mask and their gradients
 
   float dy, dx, mk;
   if constexpr (FUSED_Y) {
@@ -63,9 +70,9 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
     dx = (float)yp[2 * t + 1];
     mk = sigmoid_f32((float)yp[2 * T_ + t]);
   } else {
-    dy = (float)offset[m * 2 * T_ + 2 * t];
-    dx = (float)offset[m * 2 * T_ + 2 * t + 1];
-    mk = (float)mask[m * T_ + t];
+    dy = (float)offset[mg * 2 * T_ + 2 * t];
+    dx = (float)offset[mg * 2 * T_ + 2 * t + 1];
+    mk = (float)mask[mg * T_ + t];
   }
   const float h = (float)(oh * g.stride_h - g.pad_h + i * g.dil_h) + dy;
   const float w = (float)(ow * g.stride_w - g.pad_w + j * g.dil_w) + dx;
@@ -79,16 +86,17 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
   const bool in_h0 = hl >= 0 && hl < g.height, in_h1 = hl + 1 >= 0 && hl + 1 < g.height;
   const bool in_w0 = wl >= 0 && wl < g.width, in_w1 = wl + 1 >= 0 && wl + 1 < g.width;
   // finite coordinates only: NaN / inf offsets touch nothing
-  const bool fin = live && fh == fhc && fw == fwc;
+  const bool fin = live && fh == fhc && fw == fwc &&
+                   (!g.gate || (h > -1.f && w > -1.f && h < (float)g.height && w < (float)g.width));
   const bool c1 = fin && in_h0 && in_w0, c2 = fin && in_h0 && in_w1;
   const bool c3 = fin && in_h1 && in_w0, c4 = fin && in_h1 && in_w1;
   const float w1 = hh * hw, w2 = hh * lw, w3 = lh * hw, w4 = lh * lw;
 
-  const int C = g.channels;
+  const int C = g.channels, cpg = C / dg;
   const int64_t img = (int64_t)b * g.height * g.width;
-  const int64_t p1 = (img + (int64_t)hl * g.width + wl) * C;
+  const int64_t p1 = (img + (int64_t)hl * g.width + wl) * C + grp * cpg;
   const int64_t p2 = p1 + C, p3 = p1 + (int64_t)g.width * C, p4 = p3 + C;
-  const T *drow = dcol + (m * T_ + t) * C;
+  const T *drow = dcol + ((int64_t)m * T_ + t) * C + grp * cpg;
   const bool coord = goff != nullptr;  // gX alone needs no image reads
   float ah = 0.f, aw = 0.f, am = 0.f;
   if (live) {
@@ -96,7 +104,7 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
     // LPP consecutive elements (fp32 atomics run several times slower when the lanes of
     // one instruction are spread over more cache lines)
 #pragma unroll 4
-    for (int c = li; c < C; c += LPP) {
+    for (int c = li; c < cpg; c += LPP) {
       const float dc = (float)drow[c], ds = dc * mk;
       float x1 = 0.f, x2 = 0.f, x3 = 0.f, x4 = 0.f;
       if (coord) {
@@ -122,9 +130,10 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
     am += __shfl_xor(am, s);
   }
   if (live && li == 0 && goff != nullptr) {
-    goff[m * 2 * T_ + 2 * t] = ah;
-    goff[m * 2 * T_ + 2 * t + 1] = aw;
-    gmask[m * T_ + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
+    if (g.gate && !fin) ah = aw = am = 0.f;  // also where the column gradient is not finite
+    goff[mg * 2 * T_ + 2 * t] = ah;
+    goff[mg * 2 * T_ + 2 * t + 1] = aw;
+    gmask[mg * T_ + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
   }
 }
 
@@ -261,13 +270,13 @@ __global__ void __launch_bounds__(kBlock) col2im_coord_nhwc_vec_kernel(
     float *__restrict__ goff, float *__restrict__ gmask) {
   constexpr int VEC = 16 / sizeof(T);
   constexpr uint32_t kPast = 0x80000000u;  // >= im_bytes: loads there return zeros
-  const int T_ = g.kernel_h * g.kernel_w;
+  const int T_ = g.kernel_h * g.kernel_w, dg = g.deformable_group;
   const int HoWo = g.height_col * g.width_col;
   const int b = blockIdx.y;
   const int pair = (blockIdx.x * kBlock + threadIdx.x) >> lpp_log2;
   const int LPP = 1 << lpp_log2;
   const int li = threadIdx.x & (LPP - 1);
-  const bool live = pair < HoWo * T_;
+  const bool live = pair < HoWo * T_ * dg;  // (pixel, tap, group)
   const int pc = live ? pair : 0;
   // Quotients by the runtime sizes from a float reciprocal, corrected by one step (the
   // launch keeps every quotient below 2^22, where the estimate is off by at most one).
@@ -276,10 +285,12 @@ __global__ void __launch_bounds__(kBlock) col2im_coord_nhwc_vec_kernel(
     const int r = a - q * d;
     return q + (r >= d) - (r < 0);
   };
-  const int sp = qdiv(pc, T_), t = pc - sp * T_;
+  const int pt = dg == 1 ? pc : pc / dg, grp = pc - pt * dg;
+  const int sp = qdiv(pt, T_), t = pt - sp * T_;
   const int oh = qdiv(sp, g.width_col), ow = sp - oh * g.width_col;
   const int i = qdiv(t, g.kernel_w), j = t - i * g.kernel_w;
   const int m = b * HoWo + sp;  // 32-bit indices: the launch checks the tensor sizes
+  const int mg = m * dg + grp;  // row of offset / mask and their gradients
 
   float dy, dx, mk;
   if constexpr (FUSED_Y) {
@@ -288,9 +299,9 @@ __global__ void __launch_bounds__(kBlock) col2im_coord_nhwc_vec_kernel(
     dx = (float)yp[2 * t + 1];
     mk = sigmoid_f32((float)yp[2 * T_ + t]);
   } else {
-    dy = (float)offset[m * 2 * T_ + 2 * t];
-    dx = (float)offset[m * 2 * T_ + 2 * t + 1];
-    mk = (float)mask[m * T_ + t];
+    dy = (float)offset[mg * 2 * T_ + 2 * t];
+    dx = (float)offset[mg * 2 * T_ + 2 * t + 1];
+    mk = (float)mask[mg * T_ + t];
   }
   const float h = (float)(oh * g.stride_h - g.pad_h + i * g.dil_h) + dy;
   const float w = (float)(ow * g.stride_w - g.pad_w + j * g.dil_w) + dx;
@@ -301,11 +312,12 @@ __global__ void __launch_bounds__(kBlock) col2im_coord_nhwc_vec_kernel(
   const int hl = (int)fhc, wl = (int)fwc;
   const bool in_h0 = hl >= 0 && hl < g.height, in_h1 = hl + 1 >= 0 && hl + 1 < g.height;
   const bool in_w0 = wl >= 0 && wl < g.width, in_w1 = wl + 1 >= 0 && wl + 1 < g.width;
-  const bool fin = live && fh == fhc && fw == fwc;
-  const int C = g.channels;
+  const bool fin = live && fh == fhc && fw == fwc &&
+                   (!g.gate || (h > -1.f && w > -1.f && h < (float)g.height && w < (float)g.width));
+  const int C = g.channels, cpg = C / dg;
   const int img = b * g.height * g.width;
   const uint32_t eb = (uint32_t)sizeof(T);
-  const uint32_t e1 = (uint32_t)((img + hl * g.width + wl) * C) * eb;  // corner 1, bytes
+  const uint32_t e1 = (uint32_t)((img + hl * g.width + wl) * C + grp * cpg) * eb;  // corner 1, bytes
   const uint32_t rowb = (uint32_t)(g.width * C) * eb, colb = (uint32_t)C * eb;
   const uint32_t o1 = (fin && in_h0 && in_w0) ? e1 : kPast;
   const uint32_t o2 = (fin && in_h0 && in_w1) ? e1 + colb : kPast;
@@ -313,13 +325,13 @@ __global__ void __launch_bounds__(kBlock) col2im_coord_nhwc_vec_kernel(
   const uint32_t o4 = (fin && in_h1 && in_w1) ? e1 + rowb + colb : kPast;
   const float w1 = hh * hw, w2 = hh * lw, w3 = lh * hw, w4 = lh * lw;
   const __amdgpu_buffer_rsrc_t rim = make_rsrc(im, im_bytes);
-  const T *drow = dcol + (m * T_ + t) * C;
+  const T *drow = dcol + (m * T_ + t) * C + grp * cpg;
   // The three gradients are fixed combinations of the corner dot products
   // S_k = sum_c dcol[c] * x_k[c]; the lanes accumulate S_1..S_4 (two channels per
   // v_dot2 for the 16-bit types: exact products, fp32 sums) and lane 0 combines them.
   float s1 = 0.f, s2 = 0.f, s3 = 0.f, s4 = 0.f;
   if (live) {
-    for (int c = li * VEC; c < C; c += LPP * VEC) {
+    for (int c = li * VEC; c < cpg; c += LPP * VEC) {
       const Vec<T, VEC> dv = load_vec_nt<T, VEC>(drow + c);  // read once: keep x in L2
       const uint32_t cb = (uint32_t)c * eb;
       const Vec<T, VEC> v1 = buffer_load_vec<T, VEC>(rim, o1 + cb);
@@ -385,16 +397,20 @@ __global__ void __launch_bounds__(kBlock) col2im_coord_nhwc_vec_kernel(
     }
   }
   if (live && li == 0) {
-    goff[m * 2 * T_ + 2 * t] = mk * (hw * (s3 - s1) + lw * (s4 - s2));
-    goff[m * 2 * T_ + 2 * t + 1] = mk * (hh * (s2 - s1) + lh * (s4 - s3));
-    const float am = w1 * s1 + w2 * s2 + w3 * s3 + w4 * s4;
-    gmask[m * T_ + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
+    float gy = mk * (hw * (s3 - s1) + lw * (s4 - s2));
+    float gx = mk * (hh * (s2 - s1) + lh * (s4 - s3));
+    float am = w1 * s1 + w2 * s2 + w3 * s3 + w4 * s4;
+    if (g.gate && !fin) gy = gx = am = 0.f;  // also where the column gradient is not finite
+    goff[mg * 2 * T_ + 2 * t] = gy;
+    goff[mg * 2 * T_ + 2 * t + 1] = gx;
+    gmask[mg * T_ + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
   }
 }
 
 // ---------------------------------------------------------------------------
-// NHWC grad_x by output tile (dg == 1), without float atomics in LDS. A workgroup takes a
-// TH x TW tile of output pixels of one image and 64*CPL channels:
+// NHWC grad_x by output tile, without float atomics in LDS. A workgroup takes a TH x TW tile
+// of output pixels of one image and up to 64*CPL channels of one deformable group (lanes
+// past the group's channels add nothing):
 //   1. every (pixel, tap) sample's valid bilinear corners become (dcol row, weight * mask)
 //      pairs, binned by target input position: one bin per position of the tile's input
 //      footprint (the rows / columns its taps reach, grown by kGbMargin pixels for the
@@ -425,7 +441,8 @@ struct GbPair {
 struct GxBin {
   int th, tw;        // output tile
   int rh, rw;        // footprint rows / columns
-  int tiles_x, ntile, chunks;
+  int tiles_x, ntile;
+  int chunks, cpgc;  // channel chunks in all, and per deformable group
   int per_xcd;       // items per XCD (XCD-contiguous item ranges)
   uint32_t dcol_bytes;  // bytes of dcol (the buffer range of the pair loads)
 };
@@ -467,6 +484,10 @@ __global__ void __launch_bounds__(kGbThreads) col2im_nhwc_gx_bin_kernel(
   const int b = item / (tl.chunks * tl.ntile);
   const int ty = tile / tl.tiles_x, tx = tile - ty * tl.tiles_x;
   const int oh0 = ty * tl.th, ow0 = tx * tl.tw;
+  const int dg = g.deformable_group, cpg = C / dg;
+  const int grp = chunk / tl.cpgc, c_in = (chunk - grp * tl.cpgc) * (kWave * CPL);
+  const int cbase = grp * cpg + c_in;                 // first channel of the chunk
+  const int cn = min(kWave * CPL, cpg - c_in);        // its channels
   const int fy0 = oh0 * g.stride_h - g.pad_h - kGbMargin;
   const int fx0 = ow0 * g.stride_w - g.pad_w - kGbMargin;
   // Footprint position p goes to bin (p % 8) * P8 + p / 8, so that wave w's bins (the
@@ -502,9 +523,10 @@ __global__ void __launch_bounds__(kGbThreads) col2im_nhwc_gx_bin_kernel(
         dx = (float)o[2 * tt + 1];
         mk = sigmoid_f32((float)o[2 * T_ + tt]);
       } else {
-        dy = (float)offset[(int64_t)m * 2 * T_ + 2 * tt];
-        dx = (float)offset[(int64_t)m * 2 * T_ + 2 * tt + 1];
-        mk = (float)mask[(int64_t)m * T_ + tt];
+        const int64_t mg = (int64_t)m * dg + grp;
+        dy = (float)offset[mg * 2 * T_ + 2 * tt];
+        dx = (float)offset[mg * 2 * T_ + 2 * tt + 1];
+        mk = (float)mask[mg * T_ + tt];
       }
     }
     prow[k] = (uint32_t)m * (uint32_t)T_ + (uint32_t)tt;
@@ -516,7 +538,8 @@ __global__ void __launch_bounds__(kGbThreads) col2im_nhwc_gx_bin_kernel(
     const float fhc = fminf(fmaxf(fh, -2.f), (float)g.height);
     const float fwc = fminf(fmaxf(fw, -2.f), (float)g.width);
     const int hl = (int)fhc, wl = (int)fwc;
-    const bool fin = live && fh == fhc && fw == fwc;
+    const bool fin = live && fh == fhc && fw == fwc &&
+                     (!g.gate || (h > -1.f && w > -1.f && h < (float)g.height && w < (float)g.width));
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int yy = hl + (q >> 1), xx = wl + (q & 1);
@@ -580,7 +603,6 @@ __global__ void __launch_bounds__(kGbThreads) col2im_nhwc_gx_bin_kernel(
   // atomics are issued per cache line).
   const int lane = tid & (kWave - 1), wave = tid / kWave;
   const int64_t img = (int64_t)b * g.height * g.width;
-  const int cbase = chunk * (kWave * CPL);
   float *gxc = gx + cbase + lane;
   float *xp = xpose[wave];
   const int lo = bin_at[wave * P8], hi = bin_at[(wave + 1) * P8];
@@ -598,10 +620,12 @@ __global__ void __launch_bounds__(kGbThreads) col2im_nhwc_gx_bin_kernel(
       const int y = fy0 + pos / tl.rw, x = fx0 + pos % tl.rw;
       float *dst = gxc + (img + (int64_t)y * g.width + x) * C;
 #pragma unroll
-      for (int c = 0; c < CPL; ++c) unsafeAtomicAdd(dst + c * kWave, xp[c * kWave + lane]);
+      for (int c = 0; c < CPL; ++c)
+        if (c * kWave + lane < cn) unsafeAtomicAdd(dst + c * kWave, xp[c * kWave + lane]);
     };
     const __amdgpu_buffer_rsrc_t rdc = make_rsrc(dcol + cbase, tl.dcol_bytes - (uint32_t)(cbase * sizeof(T)));
-    const uint32_t vlane = (uint32_t)(lane * CPL * sizeof(T));
+    // lanes past the chunk's channels read its first ones and add nothing
+    const uint32_t vlane = (uint32_t)((lane * CPL < cn ? lane * CPL : 0) * sizeof(T));
     const uint32_t row_bytes = (uint32_t)(C * sizeof(T));
     constexpr int kG = sizeof(T) * CPL <= 8 ? 16 : 8;  // pairs per group
     // Lanes u < kG (and their copies every kG lanes) hold the entries of the group at k0.
@@ -656,15 +680,28 @@ __global__ void __launch_bounds__(kGbThreads) col2im_nhwc_gx_bin_kernel(
     float *dst = gxc + (img + e.tgt) * C;
 #pragma unroll
     for (int c = 0; c < CPL; ++c)
-      unsafeAtomicAdd(dst + c * kWave, e.w * (float)dcs[(int64_t)e.row * C + c * kWave]);
+      if (c * kWave + lane < cn)
+        unsafeAtomicAdd(dst + c * kWave, e.w * (float)dcs[(int64_t)e.row * C + c * kWave]);
   }
 }
 
-// Tile plan for the binned grad_x kernel; false when C is not a multiple of 64 or a tile
-// of the smallest size does not fit the LDS bins / pair list.
+// Channels per lane of the binned grad_x kernel: whole 64-lane chunks where the group's
+// channels divide into them, else the fewest chunks (a group of 96 channels is one chunk of
+// 48 lanes with 2 each, not two chunks that sort the same pairs twice).
+int gx_bin_cpl(int cpg) {
+  if (cpg % kWave == 0) return cpg % (4 * kWave) == 0 ? 4 : (cpg % (2 * kWave) == 0 ? 2 : 1);
+  if (cpg > 2 * kWave && cpg % 4 == 0) return 4;
+  return cpg > kWave && cpg % 2 == 0 ? 2 : 1;
+}
+
+// Tile plan for the binned grad_x kernel; false for groups of fewer than kGbMinCpg channels
+// (most lanes of a pair's load would be idle) or when a tile of the smallest size does not
+// fit the LDS bins / pair list.
+constexpr int kGbMinCpg = 16;
 bool gx_bin_plan(const DcnGeom &g, int cpl, int elem_bytes, GxBin &tl) {
   const int T_ = g.kernel_h * g.kernel_w;
-  if (g.deformable_group != 1 || g.channels <= 0 || g.channels % (kWave * cpl) != 0) return false;
+  const int cpg = g.channels / g.deformable_group;
+  if (cpg < kGbMinCpg || cpg % cpl != 0) return false;
   const int64_t dcol_bytes = (int64_t)g.batch * g.height_col * g.width_col * T_ * g.channels * elem_bytes;
   if (dcol_bytes >= ((int64_t)1 << 32)) return false;  // 32-bit buffer offsets
   tl.dcol_bytes = (uint32_t)dcol_bytes;
@@ -688,7 +725,8 @@ bool gx_bin_plan(const DcnGeom &g, int cpl, int elem_bytes, GxBin &tl) {
   tl.rw = extent(tw, g.stride_w, g.kernel_w, g.dil_w);
   tl.tiles_x = (g.width_col + tw - 1) / tw;
   tl.ntile = tl.tiles_x * ((g.height_col + th - 1) / th);
-  tl.chunks = g.channels / (kWave * cpl);
+  tl.cpgc = (cpg + kWave * cpl - 1) / (kWave * cpl);
+  tl.chunks = tl.cpgc * g.deformable_group;
   const int64_t nitems = (int64_t)g.batch * tl.ntile * tl.chunks;
   if (nitems > (1 << 28)) return false;
   tl.per_xcd = (int)((nitems + 7) / 8);
@@ -699,8 +737,9 @@ template <typename T, bool FY>
 hipError_t launch_t(const DcnGeom &g, const void *dcol, const void *im, const void *off,
                     const void *msk, float *gx, float *goff, float *gmask, hipStream_t stream) {
   int lpp_log2 = 0;
-  while (lpp_log2 < 6 && (1 << lpp_log2) < g.channels) ++lpp_log2;
-  const int64_t pairs = (int64_t)g.height_col * g.width_col * g.kernel_h * g.kernel_w;
+  const int dg = g.deformable_group, cpg = g.channels / dg;
+  while (lpp_log2 < 6 && (1 << lpp_log2) < cpg) ++lpp_log2;
+  const int64_t pairs = (int64_t)g.height_col * g.width_col * g.kernel_h * g.kernel_w * dg;
   const int64_t threads = pairs << lpp_log2;
   const dim3 grid((unsigned)((threads + kBlock - 1) / kBlock), g.batch);
   const T *dc = static_cast<const T *>(dcol), *of = static_cast<const T *>(off);
@@ -711,19 +750,19 @@ hipError_t launch_t(const DcnGeom &g, const void *dcol, const void *im, const vo
   const int64_t im_bytes = (int64_t)g.batch * g.height * g.width * g.channels * sizeof(T);
   const int64_t col_elems = (int64_t)g.batch * g.height_col * g.width_col *
                             g.kernel_h * g.kernel_w * g.channels;
-  const bool vec = goff != nullptr && (sizeof(T) == 2 || sizeof(T) == 4) && g.channels % VEC == 0 &&
+  const bool vec = goff != nullptr && (sizeof(T) == 2 || sizeof(T) == 4) && cpg % VEC == 0 &&
                    im_bytes < ((int64_t)1 << 31) && col_elems < ((int64_t)1 << 31) &&
-                   (int64_t)g.batch * g.height_col * g.width_col * 3 * g.kernel_h * g.kernel_w <
+                   (int64_t)g.batch * g.height_col * g.width_col * 3 * g.kernel_h * g.kernel_w * dg <
                        ((int64_t)1 << 31) &&
-                   (int64_t)g.height_col * g.width_col < ((int64_t)1 << 22) &&
+                   pairs / (g.kernel_h * g.kernel_w) < ((int64_t)1 << 22) &&
                    reinterpret_cast<uintptr_t>(dcol) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(im) % 16 == 0;
   if (gx != nullptr) {
     // grad_x through the binned kernel where it applies, else through the per-sample
     // kernel (alone when the 16-byte kernel takes the coordinates).
     GxBin tl;
-    const int cpl = g.channels % (4 * kWave) == 0 ? 4 : (g.channels % (2 * kWave) == 0 ? 2 : 1);
-    if (g.channels % kWave == 0 && reinterpret_cast<uintptr_t>(dcol) % 16 == 0 &&
+    const int cpl = gx_bin_cpl(cpg);
+    if (reinterpret_cast<uintptr_t>(dcol) % 16 == 0 &&
         gx_bin_plan(g, cpl, (int)sizeof(T), tl)) {
       const dim3 bgrid((unsigned)(tl.per_xcd * 8));
       if (cpl == 4)
@@ -743,7 +782,7 @@ hipError_t launch_t(const DcnGeom &g, const void *dcol, const void *im, const vo
   }
   if (vec) {
     int vl2 = 0;
-    while (vl2 < 3 && (1 << vl2) * VEC < g.channels) ++vl2;  // at most 8 lanes per pair
+    while (vl2 < 3 && (1 << vl2) * VEC < cpg) ++vl2;  // at most 8 lanes per pair
     const dim3 vgrid((unsigned)(((pairs << vl2) + kBlock - 1) / kBlock), g.batch);
     hipLaunchKernelGGL((col2im_coord_nhwc_vec_kernel<T, FY>), vgrid, dim3(kBlock), 0, stream, dc,
                        xim, of, mk, g, vl2, (uint32_t)im_bytes, goff, gmask);

@@ -101,8 +101,9 @@ __global__ void __launch_bounds__(kBlock) im2col_nchw_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// NHWC (dg == 1): col[m, t*C + c], m = (b, oh, ow). A wave owns kPPW consecutive (m, t)
-// pairs of one image. Lane i < kPPW first computes the geometry of pair i (offsets and
+// NHWC: col[m, t*C + c], m = (b, oh, ow). A wave owns kPPW consecutive pairs (m, t) of one
+// image; with deformable groups a pair is (m, t, group) and covers the group's C / dg
+// channels. Lane i < kPPW first computes the geometry of pair i (offsets and
 // mask read once, bilinear weights, corner byte offsets) into LDS; then groups of LPP
 // lanes take the wave's pairs in turn and sweep the channels with 16-byte loads of the
 // four corner rows, so each pair costs four gathers and one store per channel chunk and
@@ -123,7 +124,7 @@ __global__ void __launch_bounds__(kBlock) im2col_nhwc_kernel(
     T *__restrict__ col, const DcnGeom g, int lpp_log2, uint32_t img_bytes,
     const float *__restrict__ y_bias, int chunks) {
   __shared__ PairGeo geo[kBlock / kWave * kPPW];
-  const int T_ = g.kernel_h * g.kernel_w;
+  const int T_ = g.kernel_h * g.kernel_w, dg = g.deformable_group;
   const int HoWo = g.height_col * g.width_col;
   // Block l runs on XCD l % 8 and takes chunk (l % 8) * (n / 8) + l / 8 of the n =
   // batch * chunks chunks (n a multiple of 8), so each XCD gathers from one contiguous
@@ -135,10 +136,10 @@ __global__ void __launch_bounds__(kBlock) im2col_nhwc_kernel(
   const int chunk = cid - b * chunks;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  const int npairs = HoWo * T_;
+  const int npairs = HoWo * T_ * dg;
   const int pbase = (chunk * (kBlock / kWave) + wave) * kPPW;  // first pair of the wave
   if (pbase >= npairs) return;                           // uniform over the wave
-  const int C = g.channels;
+  const int C = g.channels, cpg = C / dg;
   const uint32_t oob = img_bytes;
   const uint32_t row = (uint32_t)C * (uint32_t)sizeof(T);
 
@@ -150,7 +151,8 @@ __global__ void __launch_bounds__(kBlock) im2col_nhwc_kernel(
     G.mk = 0.f;
     G.o[0] = G.o[1] = G.o[2] = G.o[3] = oob;
     if (pair < npairs) {
-      const int sp = pair / T_, t = pair - (pair / T_) * T_;
+      const int pt = dg == 1 ? pair : pair / dg, grp = pair - pt * dg;
+      const int sp = pt / T_, t = pt - (pt / T_) * T_;
       const int oh = sp / g.width_col, ow = sp - oh * g.width_col;
       const int i = t / g.kernel_w, j = t - i * g.kernel_w;
       const int64_t m = (int64_t)b * HoWo + sp;
@@ -167,19 +169,21 @@ __global__ void __launch_bounds__(kBlock) im2col_nhwc_kernel(
         }
         mk = sigmoid_f32(ym);
       } else {
-        dy = (float)offset[m * 2 * T_ + 2 * t];
-        dx = (float)offset[m * 2 * T_ + 2 * t + 1];
-        mk = (float)mask[m * T_ + t];
+        const int64_t mg = m * dg + grp;
+        dy = (float)offset[mg * 2 * T_ + 2 * t];
+        dx = (float)offset[mg * 2 * T_ + 2 * t + 1];
+        mk = (float)mask[mg * T_ + t];
       }
       const float h = (float)(oh * g.stride_h - g.pad_h + i * g.dil_h) + dy;
       const float w = (float)(ow * g.stride_w - g.pad_w + j * g.dil_w) + dx;
       const Tap<float> tp = make_tap<float>(h, w, g.height, g.width);
       G.w[0] = tp.w1; G.w[1] = tp.w2; G.w[2] = tp.w3; G.w[3] = tp.w4;
       G.mk = mk;
-      G.o[0] = tp.i1 < 0 ? oob : (uint32_t)tp.i1 * row;
-      G.o[1] = tp.i2 < 0 ? oob : (uint32_t)tp.i2 * row;
-      G.o[2] = tp.i3 < 0 ? oob : (uint32_t)tp.i3 * row;
-      G.o[3] = tp.i4 < 0 ? oob : (uint32_t)tp.i4 * row;
+      const uint32_t gb = (uint32_t)(grp * cpg) * (uint32_t)sizeof(T);
+      G.o[0] = tp.i1 < 0 ? oob : (uint32_t)tp.i1 * row + gb;
+      G.o[1] = tp.i2 < 0 ? oob : (uint32_t)tp.i2 * row + gb;
+      G.o[2] = tp.i3 < 0 ? oob : (uint32_t)tp.i3 * row + gb;
+      G.o[3] = tp.i4 < 0 ? oob : (uint32_t)tp.i4 * row + gb;
     }
     geo[wave * kPPW + lane] = G;
   }
@@ -201,9 +205,9 @@ __global__ void __launch_bounds__(kBlock) im2col_nhwc_kernel(
   for (int k = gi; k < nk; k += PPI) {
     const PairGeo G = geo[wave * kPPW + k];
     const int pair = pbase + k;
-    const int sp = pair / T_, t = pair - (pair / T_) * T_;
-    T *out = col + ((int64_t)b * HoWo + sp) * T_ * C + (int64_t)t * C;
-    for (int c = li * VEC; c < C; c += LPP * VEC) {
+    // pairs are in column order: pair = (sp * T + t) * dg + group
+    T *out = col + ((int64_t)b * npairs + pair) * cpg;
+    for (int c = li * VEC; c < cpg; c += LPP * VEC) {
       const uint32_t cb = (uint32_t)c * (uint32_t)sizeof(T);
       V v1, v2, v3, v4;
       if constexpr (VEC > 1) {
@@ -261,15 +265,15 @@ template <typename T, bool FY, typename Y = T>
 hipError_t launch_nhwc_t(const DcnGeom &g, const void *im, const void *off, const void *msk,
                          void *col, hipStream_t stream, const float *y_bias = nullptr) {
   constexpr int VEC = 16 / sizeof(T);
-  const int C = g.channels;
-  const bool vec = (C % VEC) == 0;
+  const int C = g.channels, cpg = C / g.deformable_group;
+  const bool vec = (cpg % VEC) == 0;
   const int per_lane = vec ? VEC : 1;
   int lpp = 1;
-  while (lpp < 64 && lpp * per_lane < C) lpp *= 2;
+  while (lpp < 64 && lpp * per_lane < cpg) lpp *= 2;
   int lpp_log2 = 0;
   while ((1 << lpp_log2) < lpp) ++lpp_log2;
   const int T_ = g.kernel_h * g.kernel_w;
-  const int64_t pairs = (int64_t)g.height_col * g.width_col * T_;
+  const int64_t pairs = (int64_t)g.height_col * g.width_col * T_ * g.deformable_group;
   constexpr int kPairsPerBlock = kBlock / kWave * kPPW;
   const int chunks = (int)((pairs + kPairsPerBlock - 1) / kPairsPerBlock);
   const int64_t nblk = ((int64_t)chunks * g.batch + 7) / 8 * 8;

@@ -137,6 +137,27 @@ int bevk_modulated_deformable_col2im_nhwc(
     int stride_h, int stride_w, int dilation_h, int dilation_w, int deformable_group,
     float *grad_im, float *grad_offset, float *grad_mask, void *stream);
 
+/* The two column steps of a whole layer's backward on NHWC copies of an NCHW layer's
+ * tensors, with deformable groups (channel c belongs to group c / (C / dg)):
+ *   data_im      [B, H, W, C], data_offset [B*Ho*Wo, dg, 2T], data_mask [B*Ho*Wo, dg, T], dtype
+ *   data_col     [B*Ho*Wo, T*C] columns, written; dcol: the gradient of the columns
+ *   grad_im      [B, H, W, C] fp32, ACCUMULATED with atomics (zero it first)
+ *   grad_offset  [B*Ho*Wo, dg, 2T] and grad_mask [B*Ho*Wo, dg, T] fp32, written
+ * A sample outside (-1, H) x (-1, W) contributes nothing and gets zero gradients, as in
+ * bevk_modulated_deformable_col2im_nchw. dtypes F32, F16, BF16. */
+int bevk_dcn_layer_im2col_nhwc(int dtype, const void *data_im, const void *data_offset,
+                               const void *data_mask, int batch_size, int channels, int height_im,
+                               int width_im, int height_col, int width_col, int kernel_h,
+                               int kernel_w, int pad_h, int pad_w, int stride_h, int stride_w,
+                               int dilation_h, int dilation_w, int deformable_group,
+                               void *data_col, void *stream);
+int bevk_dcn_layer_col2im_nhwc(
+    int dtype, const void *dcol, const void *data_im, const void *data_offset,
+    const void *data_mask, int batch_size, int channels, int height_im, int width_im,
+    int height_col, int width_col, int kernel_h, int kernel_w, int pad_h, int pad_w, int stride_h,
+    int stride_w, int dilation_h, int dilation_w, int deformable_group, float *grad_im,
+    float *grad_offset, float *grad_mask, void *stream);
+
 /* Workspace bytes bevk_modulated_deformable_fused_im2col_nhwc needs (-1 on bad
  * arguments): the packed offset-conv weight and the fp32 offset-conv output [M][3T]. */
 int64_t bevk_dcn_fused_im2col_nhwc_workspace_bytes(int dtype, int batch_size, int channels,

@@ -201,6 +201,45 @@ def test_col2im_nchw(dtype, geom):
     check(gmask.cpu(), gr[2], dtype, "grad_mask")
 
 
+@pytest.mark.parametrize("dg,cpg", [(1, 64), (1, 96), (1, 160), (1, 7), (2, 24), (4, 16),
+                                    (4, 64), (3, 130)])
+def test_layer_column_steps(dg, cpg):
+    """The NHWC column steps of a whole layer's backward (deformable groups, the NCHW gate)
+    against the NCHW kernels (fp32 sums of the same terms in another order: the fp32 bound),
+    with samples on the gate's boundary (h == -1 gets zero gradients) and far outside, and a
+    NaN column gradient at a gated sample, which must not come through."""
+    import _modulated_deform_conv_ext as ext
+    g = torch.Generator().manual_seed(dg * 100 + cpg)
+    b, c, h, w, ho, wo = 2, dg * cpg, 11, 13, 6, 7  # 3 x 3, stride 2
+    args = (b, c, h, w, ho, wo, 3, 3, 1, 1, 2, 2, 1, 1, dg)
+    x = torch.randn(b, c, h, w, generator=g)
+    off = 2.0 * torch.randn(b, dg, 9, 2, ho, wo, generator=g)
+    off[:, :, 0, 0, 0, :] = 0.0    # tap 0 of the first output row at h == -1
+    off[:, :, 4, 1, 3, 2] = 40.0   # far right of the image
+    off = off.view(b, dg * 18, ho, wo)
+    mask = torch.rand(b, dg * 9, ho, wo, generator=g)
+    col = torch.randn(c, 9, b, ho, wo, generator=g)
+    col[:, 0, 0, 0, 1] = float("nan")
+    x, off, mask, col = (t.to(DEV) for t in (x, off, mask, col))
+    gi = torch.zeros_like(x)
+    go, gm = torch.empty_like(off), torch.empty_like(mask)
+    ext.modulated_deformable_col2im_cuda(col, off, mask, *args, gi)
+    ext.modulated_deformable_col2im_coord_cuda(col, x, off, mask, *args, go, gm)
+    cols = torch.empty(c * 9, b, ho, wo, device=DEV)
+    ext.modulated_deformable_im2col_cuda(x, off, mask, *args, cols)
+    xn, on, mn = (ext.nchw_to_nhwc(t) for t in (x, off, mask))
+    dcol = col.permute(2, 3, 4, 1, 0).reshape(b * ho * wo, 9 * c).contiguous()
+    gxn, gon, gmn = torch.zeros_like(xn), torch.empty_like(on), torch.empty_like(mn)
+    ext.dcn_layer_col2im_nhwc(dcol, xn, on, mn, *args, gxn, gon, gmn)
+    coln = torch.empty_like(dcol)
+    ext.dcn_layer_im2col_nhwc(xn, on, mn, *args, coln)
+    check(ext.nhwc_to_nchw(gxn).cpu(), gi.cpu(), torch.float32, "grad_im")
+    check(ext.nhwc_to_nchw(gon).cpu(), go.cpu(), torch.float32, "grad_offset")
+    check(ext.nhwc_to_nchw(gmn).cpu(), gm.cpu(), torch.float32, "grad_mask")
+    want = cols.view(c, 9, b, ho, wo).permute(2, 3, 4, 1, 0).reshape_as(coln)
+    check(coln.cpu(), want.cpu(), torch.float32, "columns")
+
+
 # ---------------------------------------------------------------------------------------
 # Autograd functions
 # ---------------------------------------------------------------------------------------
