@@ -45,6 +45,9 @@ __all__ = [
     "dcn_packed_weight_numel",
     "dcn_pack_weight",
     "dcn_fused_fwd_nhwc",
+    "dcn_split_weight",
+    "dcn_fused_fwd_nhwc_f32",
+    "gemm_f32",
     "dcn_offset_conv_nhwc",
     "dcn_mega_fwd_nhwc",
     "transpose",
@@ -230,6 +233,76 @@ def dcn_fused_fwd_nhwc(data_im, data_offset, data_mask, weight_packed, bias, bat
             _b.ptr(bias), batch_size, channels, height_im, width_im, height_col, width_col,
             channels_out, kernel_h, kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h,
             dilation_w, _b.ptr(out), _b.stream_of(data_im))
+
+
+def dcn_split_weight(weight, transposed=False):
+    """fp32 module weight [Cout, C, kh, kw] -> its split form (uint8) for dcn_fused_fwd_nhwc_f32
+    or, transposed, for gemm_f32 with columns (tap, C) and terms Cout."""
+    fn = "dcn_split_weight"
+    _b.require_device(fn, weight)
+    _b.require_contiguous(fn, weight=weight)
+    if weight.dtype != torch.float32 or weight.dim() != 4:
+        raise RuntimeError(f"{fn}: weight must be float32 [Cout, C, kh, kw]")
+    cout, c, kh, kw = weight.shape
+    n, k = (c * kh * kw, cout) if transposed else (cout, c * kh * kw)
+    split = torch.empty(max(0, _b.lib().bevk_f32_split_weight_bytes(n, k)), dtype=torch.uint8,
+                        device=weight.device)
+    _b.call("bevk_dcn_split_weight", _b.ptr(weight), cout, kh, kw, c, int(transposed),
+            _b.ptr(split), _b.stream_of(weight))
+    return split
+
+
+def _require_split(fn, split, n, k):
+    if split.dtype != torch.uint8:
+        raise RuntimeError(f"{fn}: weight_split must come from dcn_split_weight")
+    _b.require_numel(fn, "weight_split", split, _b.lib().bevk_f32_split_weight_bytes(n, k))
+
+
+def dcn_fused_fwd_nhwc_f32(data_im, data_offset, data_mask, weight_split, bias, batch_size,
+                           channels, height_im, width_im, height_col, width_col, channels_out,
+                           kernel_h, kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h,
+                           dilation_w, out, act_relu=False):
+    """dcn_fused_fwd_nhwc for float32 on the bf16 matrix cores (weight_split from
+    dcn_split_weight; C % 32 == 0, at most 9 taps), with an optional ReLU."""
+    fn = "dcn_fused_fwd_nhwc_f32"
+    _b.require_device(fn, data_im, data_offset, data_mask, weight_split, bias, out)
+    _b.require_contiguous(fn, data_im=data_im, data_offset=data_offset, data_mask=data_mask,
+                          weight_split=weight_split, bias=bias, out=out)
+    taps = kernel_h * kernel_w
+    last = data_offset.size(-1)
+    fused_y = last == 3 * taps
+    if data_im.dtype != torch.float32:
+        raise RuntimeError(f"{fn}: data_im must be float32, got {data_im.dtype}")
+    _b.require_dtype(fn, data_im, data_offset=data_offset, bias=bias, out=out,
+                     data_mask=None if fused_y else data_mask)
+    m = batch_size * height_col * width_col
+    _b.require_numel(fn, "data_im", data_im, batch_size * height_im * width_im * channels)
+    _b.require_numel(fn, "data_offset", data_offset, m * last)
+    if not fused_y:
+        _b.require_numel(fn, "data_mask", data_mask, m * taps)
+    _require_split(fn, weight_split, channels_out, taps * channels)
+    if bias is not None:
+        _b.require_numel(fn, "bias", bias, channels_out)
+    _b.require_numel(fn, "out", out, m * channels_out)
+    _b.call("bevk_dcn_fused_fwd_nhwc_f32", _b.ptr(data_im), _b.ptr(data_offset), last,
+            _b.ptr(data_mask), _b.ptr(weight_split), _b.ptr(bias), batch_size, channels,
+            height_im, width_im, height_col, width_col, channels_out, kernel_h, kernel_w, pad_h,
+            pad_w, stride_h, stride_w, dilation_h, dilation_w, int(act_relu), _b.ptr(out),
+            _b.stream_of(data_im))
+
+
+def gemm_f32(a, weight_split, n, out):
+    """out [m, n] = a [m, k] times the split weight's n columns of k terms (float32)."""
+    fn = "gemm_f32"
+    _b.require_device(fn, a, weight_split, out)
+    _b.require_contiguous(fn, a=a, weight_split=weight_split, out=out)
+    if a.dim() != 2 or a.dtype != torch.float32 or out.dtype != torch.float32:
+        raise RuntimeError(f"{fn}: a must be a float32 matrix and out float32")
+    m, k = a.shape
+    _require_split(fn, weight_split, n, k)
+    _b.require_numel(fn, "out", out, m * n)
+    _b.call("bevk_gemm_f32", _b.ptr(a), _b.ptr(weight_split), m, k, n, _b.ptr(out),
+            _b.stream_of(a))
 
 
 def _offset_conv_checks(fn, data_im, w_off_packed, b_off, batch_size, channels, height_im,

@@ -104,6 +104,20 @@ int64_t dcn_packed_weight_elems(int dtype, int cout, int K);
 hipError_t launch_dcn_pack_weight(int dtype, const void *weight, int cout, int C, int T,
                                   void *packed, hipStream_t stream, bool src_tc = false);
 
+// fp32 products on the bf16 matrix cores (three exact bf16 pieces per operand, dcn_f32.hip).
+// Split weight of n columns and k reduction elements (with its flags), from the module weight
+// [Cout][C][T]: n = Cout, k = t*C + c (C % 32 == 0), or transposed n = t*C + c, k = Cout
+// (C % 16 == 0, Cout % 32 == 0); T <= 9, 16-byte aligned buffers.
+int64_t f32_split_weight_bytes(int64_t n, int64_t k);
+hipError_t launch_f32_split_weight(const float *weight, int cout, int C, int T, bool transposed,
+                                   void *packed, hipStream_t stream);
+// out[m, n] = sum_k A[m, k] W[n, k] (+ bias): A the deformable columns of geometry g (dg == 1,
+// <= 9 taps, geo kGeoMask / kGeoY / kGeoYF32; M and K must match it), or with g == nullptr the
+// matrix x [M][K]. K % 32 == 0, x under 2 GiB, 16-byte aligned x.
+hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, const void *x,
+                            const void *off, int geo, const void *msk, const void *w_split,
+                            const float *bias, float *out, hipStream_t stream, bool relu);
+
 // dst[b][c][r] = src[b][r][c] for 2- or 4-byte elements (NCHW <-> NHWC).
 hipError_t launch_transpose(int elem_bytes, const void *src, void *dst, int batch, int rows,
                             int cols, hipStream_t stream);

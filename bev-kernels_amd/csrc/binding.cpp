@@ -552,6 +552,86 @@ int bevk_dcn_fused_fwd_nhwc(int dtype, const void *data_im, const void *data_off
                     fn);
 }
 
+int64_t bevk_f32_split_weight_bytes(int n, int k) {
+  return n < 0 || k < 0 ? -1 : bevk::f32_split_weight_bytes(n, k);
+}
+
+int bevk_dcn_split_weight(const void *weight, int channels_out, int kernel_h, int kernel_w,
+                          int channels, int transposed, void *split, void *stream) {
+  const char *fn = "dcn_split_weight";
+  g_last_error.clear();
+  if (channels_out <= 0 || kernel_h <= 0 || kernel_w <= 0 || channels <= 0)
+    return fail(BEVK_ERR_INVALID, "%s: invalid weight shape", fn);
+  const int taps = kernel_h * kernel_w;
+  if (taps > 9 || channels % (transposed ? 16 : 32) != 0 || (transposed && channels_out % 32 != 0))
+    return fail(BEVK_ERR_UNSUPPORTED,
+                "%s: at most 9 taps, and channels in whole blocks of the split layout", fn);
+  const long long n = transposed ? (long long)channels * taps : channels_out;
+  const long long k = transposed ? channels_out : (long long)channels * taps;
+  if (bevk::f32_split_weight_bytes(n, k) > kMaxBufferBytes)
+    return fail(BEVK_ERR_INVALID, "%s: weight too large for 32-bit buffer offsets", fn);
+  if (!weight || !split) return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(bevk::launch_f32_split_weight(static_cast<const float *>(weight), channels_out,
+                                                  channels, taps, transposed != 0, split,
+                                                  (hipStream_t)stream),
+                    fn);
+}
+
+int bevk_dcn_fused_fwd_nhwc_f32(const void *data_im, const void *data_offset, int offset_last_dim,
+                                const void *data_mask, const void *weight_split, const void *bias,
+                                int batch_size, int channels, int height_im, int width_im,
+                                int height_col, int width_col, int channels_out, int kernel_h,
+                                int kernel_w, int pad_h, int pad_w, int stride_h, int stride_w,
+                                int dilation_h, int dilation_w, int act_relu, void *out,
+                                void *stream) {
+  const char *fn = "dcn_fused_fwd_nhwc_f32";
+  g_last_error.clear();
+  const bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w, 1);
+  if (int rc = check_geom(fn, g)) return rc;
+  if (channels_out < 0) return fail(BEVK_ERR_INVALID, "%s: negative channels_out", fn);
+  const int taps = kernel_h * kernel_w;
+  if (offset_last_dim != 2 * taps && offset_last_dim != 3 * taps)
+    return fail(BEVK_ERR_INVALID, "%s: offset last dim must be 2T (%d) or 3T (%d), got %d", fn,
+                2 * taps, 3 * taps, offset_last_dim);
+  const bool fused_y = offset_last_dim == 3 * taps;
+  const long long m = (long long)batch_size * height_col * width_col;
+  if (m * channels_out == 0) return ok();
+  if (channels <= 0 || channels % 32 != 0 || taps > 9)
+    return fail(BEVK_ERR_UNSUPPORTED, "%s: channels (%d) must be a multiple of 32, at most 9 taps",
+                fn, channels);
+  if ((long long)batch_size * height_im * width_im * channels * 4 > kMaxBufferBytes ||
+      bevk::f32_split_weight_bytes(channels_out, (long long)taps * channels) > kMaxBufferBytes ||
+      m >= (1LL << 30))
+    return fail(BEVK_ERR_INVALID, "%s: problem too large for 32-bit buffer offsets", fn);
+  if (!data_im || !data_offset || (!fused_y && !data_mask) || !weight_split || !out)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(
+      bevk::launch_f32_split(&g, channels_out, (int)m, taps * channels, data_im, data_offset,
+                             fused_y ? bevk::kGeoY : bevk::kGeoMask, data_mask, weight_split,
+                             static_cast<const float *>(bias), static_cast<float *>(out),
+                             (hipStream_t)stream, act_relu != 0),
+      fn);
+}
+
+int bevk_gemm_f32(const void *a, const void *weight_split, int m, int k, int n, void *out,
+                  void *stream) {
+  const char *fn = "gemm_f32";
+  g_last_error.clear();
+  if (m < 0 || n < 0 || k <= 0 || k % 32 != 0)
+    return fail(BEVK_ERR_INVALID, "%s: sizes must not be negative and k a multiple of 32", fn);
+  if (m == 0 || n == 0) return ok();
+  if ((long long)m * k * 4 > kMaxBufferBytes ||
+      bevk::f32_split_weight_bytes(n, k) > kMaxBufferBytes || m >= (1 << 30))
+    return fail(BEVK_ERR_INVALID, "%s: problem too large for 32-bit buffer offsets", fn);
+  if (!a || !weight_split || !out) return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(bevk::launch_f32_split(nullptr, n, m, k, a, nullptr, bevk::kGeoMask, nullptr,
+                                           weight_split, nullptr, static_cast<float *>(out),
+                                           (hipStream_t)stream, false),
+                    fn);
+}
+
 // Shared checks of the offset-conv entry points (dg == 1, fused-kernel dtypes, channel
 // vectors, 32-bit buffer offsets). Returns 0 or the failure code.
 static int check_offset_conv(const char *fn, int dtype, const bevk::DcnGeom &g) {

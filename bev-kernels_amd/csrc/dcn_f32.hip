@@ -1,0 +1,654 @@
+// fp32 implicit GEMM on the bf16 matrix cores (gfx950): the fp32 DCNv2 forward and the plain
+// fp32 products of its backward.
+//
+//   out[m, n] = sum_k A[m, k] * W[n, k] (+ bias[n])
+//
+// with A either the deformable columns of an NHWC input, built on the fly (m = (b, oh, ow),
+// k = t*C + c), or the rows of a matrix. Every fp32 operand is cut into three bf16 pieces that
+// add up to it exactly (8 + 8 + 8 significant bits, each piece the next 16 high bits of what
+// is left), x = h + m + l, and a product is taken as
+//   h*h' + (h*m' + m*h') + (m*m' + h*l' + l*h'),
+// six v_mfma_f32_16x16x32_bf16 with fp32 accumulation. What is left out (m*l' + l*m' + l*l')
+// is below 2^-23 of the product and 4e-8 of it on average, and the large sum is rounded twice
+// per 32 terms instead of once per two terms as with v_mfma_f32_32x32x2_f32, so the sums come
+// out closer to the exact ones: 2-norm errors against 64 bits at 64 / 512 / 2,304 / 4,608 terms
+// 0.8e-7 / 1.6e-7 / 3.3e-7 / 4.8e-7, where a library fp32 product has 1.4e-7 / 4.0e-7 / 8.6e-7
+// / 12e-7 and this layer's fp32 matrix kernel had 5.9e-7 at 2,304 (all six products in one
+// accumulator: 7.3e-7).
+//
+// Bound: the matrix cores. Six cameras at 256 channels of 58 x 100 to 256 (41 GFLOP): 500 us
+// on the fp32 matrix cores (82 TFLOP/s of 157), 220-245 us here (1.0-1.1 PFLOP/s of bf16
+// products, where a large bf16 library product reaches 1.2 on the same card); with the module's
+// layout changes 253 us, of which four of the six products take 100, the gathers 64, the
+// weight loads 12 and the blend and cut 10 (each left out in turn).
+// Pairs of row blocks with four independent MFMA chains, or two chains for the small products,
+// measured the same or slower: their dependent chain is not what limits.
+//
+// Non-finite operands do not survive the cut (inf - inf, 0 * inf): a workgroup that meets one
+// (in its columns, or flagged when the weight was split) computes its tile again in plain
+// fp32 (slow_tile), which has the reference's NaN / Inf behaviour.
+#include "bevk_common.h"
+#include "bevk_launch.h"
+
+#include <hip/amd_detail/amd_hip_unsafe_atomics.h>
+
+#include <algorithm>
+
+namespace bevk {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef int int2v __attribute__((ext_vector_type(2)));
+
+constexpr int kMaxTaps = 9;
+constexpr int kThreads = 512;   // 8 waves
+constexpr int kBK = 32;         // K step: 128 bytes of an fp32 row
+constexpr int kRows = -1;       // GEO: A is a matrix, not deformable columns
+constexpr int kBlkBytes = 3072; // split weight block: 16 columns x 32 k, three planes
+
+struct TapGeo {
+  float w[4];
+  uint32_t o[4];
+};
+
+struct Params {
+  const void *x, *off, *msk;  // kRows: x is the matrix [M][K]
+  const float *yb;
+  const void *w;              // split weight, then its flags
+  const uint32_t *flags;
+  const float *bias;
+  float *out;
+  int relu;
+  int C, H, W, Ho, Wo, Cout, kw, ph, pw, sh, sw, dh, dw, M, taps;
+  int nb_total, kb_total;     // 16-column blocks, 32-k blocks
+  int rb_total, mch, nt, kparts, ksteps;  // 16-row blocks, row chunks, column tiles, K parts
+  int per_xcd;
+  uint32_t x_bytes, w_bytes;
+};
+
+// The three pieces as fp32 values (the low 16 bits of each are zero).
+struct Pieces {
+  float h, m, l;
+};
+__device__ __forceinline__ float high_part(float v) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xffff0000u);
+}
+__device__ __forceinline__ Pieces cut(float v) {
+  Pieces p;
+  p.h = high_part(v);
+  const float r = v - p.h;
+  p.m = high_part(r);
+  p.l = r - p.m;
+  return p;
+}
+// Two pieces' high halves in one word (the first in the low half).
+__device__ __forceinline__ int pack2(float a, float b) {
+  return (int)__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a),
+                                    0x07060302u);
+}
+
+__device__ __forceinline__ floatx4 mfma(int4v a, int4v b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Tap geometry of output row m, tap t: corner byte offsets (out of range when the corner is
+// outside the image) and mask-folded bilinear weights; the sample is zero unless -1 < h < H
+// and -1 < w < W (modulated_deform_conv.py:256-258, fused_tl.py:146-174).
+template <int GEO>
+__device__ __forceinline__ TapGeo tap_geo(const Params &p, int m, int t) {
+  TapGeo G;
+  G.w[0] = G.w[1] = G.w[2] = G.w[3] = 0.f;
+  G.o[0] = G.o[1] = G.o[2] = G.o[3] = p.x_bytes;
+  const int HoWo = p.Ho * p.Wo;
+  const int b = m / HoWo, r = m - b * HoWo, oh = r / p.Wo, ow = r - oh * p.Wo;
+  const int ki = t / p.kw, kj = t - ki * p.kw;
+  float dy, dx, mk;
+  tap_offsets<float, GEO>(p.off, p.msk, p.yb, m, t, p.taps, dy, dx, mk);
+  const float h = (float)(oh * p.sh - p.ph + ki * p.dh) + dy;
+  const float w = (float)(ow * p.sw - p.pw + kj * p.dw) + dx;
+  if (h > -1.f && w > -1.f && h < (float)p.H && w < (float)p.W) {
+    const float fh = floorf(h), fw = floorf(w);
+    const int hl = (int)fh, wl = (int)fw;
+    const float lh = h - fh, lw = w - fw, hh = 1.f - lh, hw = 1.f - lw;
+    const uint32_t rowb = (uint32_t)p.C * 4u;
+    const uint32_t base = (uint32_t)(b * p.H * p.W + hl * p.W + wl) * rowb;
+    const bool y0 = hl >= 0, y1 = hl + 1 <= p.H - 1, x0 = wl >= 0, x1 = wl + 1 <= p.W - 1;
+    if (y0 && x0) { G.w[0] = hh * hw * mk; G.o[0] = base; }
+    if (y0 && x1) { G.w[1] = hh * lw * mk; G.o[1] = base + rowb; }
+    if (y1 && x0) { G.w[2] = lh * hw * mk; G.o[2] = base + (uint32_t)p.W * rowb; }
+    if (y1 && x1) { G.w[3] = lh * lw * mk; G.o[3] = base + (uint32_t)(p.W + 1) * rowb; }
+  }
+  return G;
+}
+
+// LDS address (bytes) of the A tile's 16-byte fragment piece (row, chunk of 8 k) inside one
+// plane: rows in 16-row blocks of 1 KB, stored in the order the MFMA fragments are read, so a
+// fragment read is 1 KB of consecutive addresses. The row is rotated by 4 per chunk: the
+// gather's 8-byte stores (4 rows x 8 half chunks per 32 lanes) then touch every bank once.
+__device__ __forceinline__ int a_off(int row, int chunk) {
+  return (row >> 4) * 1024 + chunk * 256 + (((row & 15) + 4 * chunk) & 15) * 16;
+}
+
+template <int NRB, int GEO>
+struct Shape {
+  static constexpr int kRowsN = NRB * 16;
+  static constexpr int kPlane = NRB * 1024;              // bytes of one A plane
+  static constexpr int kSlots = kRowsN * (kBK / 4);      // (row, 4 channels) slots per step
+  static constexpr int kNS = (kSlots + kThreads - 1) / kThreads;
+  static constexpr int kFullWaves = (kSlots - (kNS - 1) * kThreads) / kWave;
+  static constexpr int kNQ = GEO == kRows ? 1 : 4;       // loads per slot
+};
+
+// The K loop of one wave. Per step: the MFMAs of A buffer `buf`; meanwhile the next step's
+// corners (in registers since the last step) are blended, cut and stored into the other
+// buffer, and the loads of the step after are issued (as dcn_fused_h.hip's symmetric kernel:
+// about one step of gathers in flight per wave, weight fragments two steps ahead).
+template <int NRB, int WN, int GEO, int NS>
+__device__ __forceinline__ float k_loop(const Params &p, const TapGeo *geo, char *ring, int n0,
+                                        int m0, int k0, int nk, floatx4 (&acc)[NRB * WN / 8][2]) {
+  using S = Shape<NRB, GEO>;
+  constexpr int R = NRB * WN / 8;   // row blocks of the wave
+  constexpr int NP = NS * 4;        // blend pieces per step (slot x element)
+  constexpr int NA = NS > 0 ? NS : 1;
+  constexpr int NQ = S::kNQ;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % WN, wm = wave / WN;
+  const int kv = tid & 7;
+  const int spt = GEO == kRows ? p.kb_total : p.C / kBK;  // K steps per tap
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, p.x_bytes);
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(p.w, p.w_bytes);
+
+  uint32_t bo[2];
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb) {
+    const int nb = (n0 >> 4) + wn * 2 + cb;
+    bo[cb] = nb < p.nb_total ? (uint32_t)nb * (uint32_t)p.kb_total * kBlkBytes + (uint32_t)lane * 16u
+                             : p.w_bytes;
+  }
+  auto issue_b = [&](int ks, int4v (&br)[2][3]) __attribute__((always_inline)) {
+    const uint32_t so = (uint32_t)min(ks, p.kb_total - 1) * kBlkBytes;
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        br[cb][q] = __builtin_amdgcn_raw_buffer_load_b128(wr, bo[cb] + q * 1024, so, 0);
+  };
+
+  auto slot_row = [&](int i) __attribute__((always_inline)) { return (tid >> 3) + i * (kThreads / 8); };
+  floatx4 ra[NA][NQ];
+  int it = k0 / spt, ics = k0 - it * spt;  // tap and step in the tap of the next loads
+  int bt = it, bcs = ics;                  // the same for the next blend
+  // Corner offsets (for the next loads) and weights (for the next blend) of one slot, read
+  // from the table a slot ahead of their use.
+  uint32_t go[NQ];
+  floatx4 w4;
+  auto load_go = [&](int i) __attribute__((always_inline)) {
+    if constexpr (GEO == kRows) {
+      const int m = m0 + slot_row(i);
+      go[0] = m < p.M ? ((uint32_t)m * (uint32_t)p.kb_total * kBK + (uint32_t)kv * 4u) * 4u : p.x_bytes;
+    } else {
+      const int4v o = *reinterpret_cast<const int4v *>(geo[slot_row(i) * p.taps + min(it, p.taps - 1)].o);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        go[q] = (uint32_t)o[q] == p.x_bytes ? p.x_bytes : (uint32_t)o[q] + (uint32_t)kv * 16u;
+    }
+  };
+  auto load_w = [&](int i) __attribute__((always_inline)) {
+    if constexpr (GEO != kRows)
+      w4 = *reinterpret_cast<const floatx4 *>(geo[slot_row(i) * p.taps + bt].w);
+  };
+  auto issue_slot = [&](int i) __attribute__((always_inline)) {
+    // past the last K step: a step read before, not used
+    const uint32_t so = (uint32_t)(GEO == kRows ? min(ics, spt - 1) : ics) * (kBK * 4u);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      ra[i][q] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, go[q], so, 0));
+  };
+  auto next_issue = [&]() __attribute__((always_inline)) {
+    if (++ics == spt && GEO != kRows) {
+      ics = 0;
+      ++it;
+    }
+  };
+  auto next_blend = [&]() __attribute__((always_inline)) {
+    if (++bcs == spt) {
+      bcs = 0;
+      bt = min(bt + 1, p.taps - 1);
+    }
+  };
+  float nf = 0.f;  // NaN once a non-finite value was cut
+  Pieces pc[4];
+  auto blend_one = [&](int i, int e) __attribute__((always_inline)) {
+    float v;
+    if constexpr (GEO == kRows) {
+      v = ra[i][0][e];
+    } else {
+      v = w4[0] * ra[i][0][e];
+      v = __builtin_fmaf(w4[1], ra[i][1][e], v);
+      v = __builtin_fmaf(w4[2], ra[i][2][e], v);
+      v = __builtin_fmaf(w4[3], ra[i][3][e], v);
+    }
+    pc[e] = cut(v);
+    nf += pc[e].l;
+  };
+  auto store_slot = [&](int i, char *buf) __attribute__((always_inline)) {
+    char *d = buf + a_off(slot_row(i), kv >> 1) + (kv & 1) * 8;
+    *reinterpret_cast<int2v *>(d) = int2v{pack2(pc[0].h, pc[1].h), pack2(pc[2].h, pc[3].h)};
+    *reinterpret_cast<int2v *>(d + S::kPlane) = int2v{pack2(pc[0].m, pc[1].m), pack2(pc[2].m, pc[3].m)};
+    *reinterpret_cast<int2v *>(d + 2 * S::kPlane) = int2v{pack2(pc[0].l, pc[1].l), pack2(pc[2].l, pc[3].l)};
+  };
+
+  const int fa = a_off(lane & 15, lane >> 4) + wm * R * 1024;  // the wave's first fragment
+  auto step = [&](int ks, int4v (&br)[2][3]) __attribute__((always_inline)) {
+    const char *tile = ring + (ks & 1) * 3 * S::kPlane;
+    char *next = ring + ((ks + 1) & 1) * 3 * S::kPlane;
+    int4v af[2][3];
+    auto read_frag = [&](int rb) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        af[rb & 1][q] = *reinterpret_cast<const int4v *>(tile + q * S::kPlane + rb * 1024 + fa);
+    };
+    read_frag(0);
+    next_issue();
+    if constexpr (NS > 0) {
+      load_w(0);
+      load_go(0);
+    }
+#pragma unroll
+    for (int rb = 0; rb < R; ++rb) {
+      if (rb + 1 < R) read_frag(rb + 1);
+      const int4v(&a)[3] = af[rb & 1];
+      // The five small products are summed by themselves and added once, so the large sum is
+      // rounded twice per K step instead of six times.
+      floatx4 lo[2];
+      constexpr int kTa[5] = {2, 0, 1, 1, 0}, kTb[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+      for (int q = 0; q < 5; ++q)
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+          lo[cb] = mfma(a[kTa[q]], br[cb][kTb[q]],
+                                q == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : lo[cb]);
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = mfma(a[0], br[cb][0], acc[rb][cb]);
+#pragma unroll
+      for (int pp = 0; pp < NP; ++pp) {
+        if (pp * R / (NA * 4) != rb) continue;
+        blend_one(pp / 4, pp % 4);
+        if (pp % 4 == 3) {
+          store_slot(pp / 4, next);
+          issue_slot(pp / 4);
+          if (pp / 4 + 1 < NS) {
+            load_w(pp / 4 + 1);
+            load_go(pp / 4 + 1);
+          }
+        }
+      }
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) acc[rb][cb] += lo[cb];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    next_blend();
+    issue_b(k0 + ks + 2, br);
+    __syncthreads();
+  };
+
+  int4v b0[2][3], b1[2][3];
+  issue_b(k0, b0);
+  issue_b(k0 + 1, b1);
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    load_go(i);
+    issue_slot(i);
+  }
+  next_issue();
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    load_w(i);
+    load_go(i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) blend_one(i, e);
+    store_slot(i, ring);
+    issue_slot(i);
+  }
+  next_blend();
+  __syncthreads();
+  int ks = 0;
+  for (; ks + 2 <= nk; ks += 2) {
+    step(ks, b0);
+    step(ks + 1, b1);
+  }
+  if (ks < nk) step(ks, b0);
+  return nf;
+}
+
+// The tile in plain fp32, one output column per thread and 16 rows at a time: only for tiles
+// that meet a non-finite operand.
+template <int NRB, int WN, int GEO>
+__device__ __forceinline__ void slow_tile(const Params &p, const TapGeo *geo, float *At, int n0, int m0,
+                                       int rows, int k0, int nk, bool add_bias) {
+  constexpr int BN = WN * 32, RT = 16 * BN / kThreads;
+  const int tid = threadIdx.x, n = n0 + tid % BN, r0 = (tid / BN) * RT;
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, p.x_bytes);
+  const int spt = GEO == kRows ? p.kb_total : p.C / kBK;
+  const unsigned short *w = static_cast<const unsigned short *>(p.w);
+  for (int rb = 0; rb * 16 < rows; ++rb) {
+    float s[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) s[r] = 0.f;
+    for (int ks = k0; ks < k0 + nk; ++ks) {
+      __syncthreads();
+      {
+        const int row = tid >> 5, c = tid & 31;
+        float v = 0.f;
+        if constexpr (GEO == kRows) {
+          const int m = m0 + rb * 16 + row;
+          if (m < p.M) v = buffer_load_one<float>(xr, ((uint32_t)m * (uint32_t)p.kb_total + ks) * (kBK * 4u) + c * 4u);
+        } else {
+          const int t = ks / spt;
+          const TapGeo G = geo[(rb * 16 + row) * p.taps + t];
+          const uint32_t cb = (uint32_t)((ks - t * spt) * kBK + c) * 4u;
+          for (int q = 0; q < 4; ++q) {
+            const float xv = G.o[q] == p.x_bytes ? 0.f : buffer_load_one<float>(xr, G.o[q] + cb);
+            v = q == 0 ? G.w[0] * xv : __builtin_fmaf(G.w[q], xv, v);
+          }
+        }
+        At[row * kBK + c] = v;
+      }
+      __syncthreads();
+      if (n < p.Cout) {
+        const unsigned short *blk = w + ((int64_t)(n >> 4) * p.kb_total + ks) * (kBlkBytes / 2);
+        for (int kk = 0; kk < kBK; ++kk) {
+          const int e = ((n & 15) + 16 * (kk >> 3)) * 8 + (kk & 7);
+          float wv = 0.f;
+          for (int q = 2; q >= 0; --q)
+            wv += __builtin_bit_cast(float, (uint32_t)blk[q * 512 + e] << 16);
+#pragma unroll
+          for (int r = 0; r < RT; ++r) s[r] = __builtin_fmaf(At[(r0 + r) * kBK + kk], wv, s[r]);
+        }
+      }
+    }
+    const float bv = (add_bias && p.bias != nullptr && n < p.Cout) ? p.bias[n] : 0.f;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int m = m0 + rb * 16 + r0 + r;
+      float v = s[r] + bv;
+      if (p.relu) v = v < 0.f ? 0.f : v;
+      if (m < p.M && rb * 16 + r0 + r < rows && n < p.Cout) {
+        if (p.kparts > 1) unsafeAtomicAdd(p.out + (int64_t)m * p.Cout + n, v);
+        else p.out[(int64_t)m * p.Cout + n] = v;
+      }
+    }
+  }
+}
+
+// One workgroup: up to NRB 16-row blocks x 32 WN columns, the whole K or one of two parts.
+template <int NRB, int WN, int GEO>
+__global__ void __launch_bounds__(kThreads) f32_gemm_kernel(const Params p) {
+  using S = Shape<NRB, GEO>;
+  constexpr int R = NRB * WN / 8;
+  __shared__ __attribute__((aligned(16))) char ring[2 * 3 * S::kPlane];
+  __shared__ __attribute__((aligned(16))) TapGeo geo[GEO == kRows ? 1 : S::kRowsN * kMaxTaps];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Workgroup b runs on XCD b % 8 and each XCD takes a contiguous range of (column tile,
+  // K part, row chunk), rows fastest: its L2 keeps the weight of few column tiles and the
+  // image rows of neighbouring chunks.
+  const int L = (int)(blockIdx.x & 7) * p.per_xcd + (int)(blockIdx.x >> 3);
+  if (L >= p.mch * p.nt * p.kparts) return;  // uniform
+  const int mc = L % p.mch, nk_id = L / p.mch;
+  const int kz = nk_id % p.kparts, n0 = (nk_id / p.kparts) * (WN * 32);
+  const int rb0 = (int)((int64_t)p.rb_total * mc / p.mch);
+  const int nrb = (int)((int64_t)p.rb_total * (mc + 1) / p.mch) - rb0;  // at most NRB
+  const int m0 = rb0 * 16, rows = nrb * 16;
+  const int k0 = kz * p.ksteps, nk = min(p.ksteps, p.kb_total - k0);
+
+  bool bad = false;  // a non-finite weight in this tile's columns and K part
+  for (int nb = n0 >> 4; nb < min((n0 >> 4) + 2 * WN, p.nb_total); ++nb)
+    for (int kb = tid; kb < nk; kb += kThreads) bad |= p.flags[(int64_t)nb * p.kb_total + k0 + kb] != 0;
+  if constexpr (GEO != kRows) {
+    for (int g = tid; g < S::kRowsN * p.taps; g += kThreads) {
+      const int row = g / p.taps, t = g - row * p.taps, m = m0 + row;
+      if (row < rows && m < p.M) {
+        geo[g] = tap_geo<GEO>(p, m, t);
+      } else {
+        TapGeo G;
+        G.w[0] = G.w[1] = G.w[2] = G.w[3] = 0.f;
+        G.o[0] = G.o[1] = G.o[2] = G.o[3] = p.x_bytes;
+        geo[g] = G;
+      }
+    }
+    __syncthreads();
+  }
+  floatx4 acc[R][2];
+#pragma unroll
+  for (int i = 0; i < R; ++i) acc[i][0] = acc[i][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float nf = 0.f;
+  if (wave < S::kFullWaves)
+    nf = k_loop<NRB, WN, GEO, S::kNS>(p, geo, ring, n0, m0, k0, nk, acc);
+  else if constexpr (S::kFullWaves < 8)
+    nf = k_loop<NRB, WN, GEO, S::kNS - 1>(p, geo, ring, n0, m0, k0, nk, acc);
+  bad |= !(nf == nf);
+  if (__syncthreads_or(bad)) {
+    slow_tile<NRB, WN, GEO>(p, geo, reinterpret_cast<float *>(ring), n0, m0, rows, k0, nk, kz == 0);
+    return;
+  }
+  const int wn = wave % WN, wm = wave / WN;
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb) {
+    const int n = n0 + wn * 32 + cb * 16 + (lane & 15);
+    const float bv = (kz == 0 && p.bias != nullptr && n < p.Cout) ? p.bias[n] : 0.f;
+#pragma unroll
+    for (int rb = 0; rb < R; ++rb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = (wm * R + rb) * 16 + 4 * (lane >> 4) + e, m = m0 + row;
+        float v = acc[rb][cb][e] + bv;
+        if (p.relu) v = v < 0.f ? 0.f : v;  // NaN stays NaN, as torch.relu
+        if (row < rows && m < p.M && n < p.Cout) {
+          if (p.kparts > 1) unsafeAtomicAdd(p.out + (int64_t)m * p.Cout + n, v);
+          else p.out[(int64_t)m * p.Cout + n] = v;
+        }
+      }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Split weight: blocks [N / 16][K / 32] of 3 KB, planes h, m, l of 64 lanes x 8 bf16 in the
+// MFMA fragment order (lane l: column l % 16, k = 8 (l / 16) .. + 8), then one flag word per
+// block (a non-finite value in it). From the module weight w [Cout][C][T]:
+//   TRANS false: n = Cout, k = t*C + c (the forward);
+//   TRANS true:  n = t*C + c, k = Cout (columns' gradient dO @ W).
+// A workgroup stages a 16 x 32 (n x c, or c x Cout) group of all taps through LDS, where each
+// source row's span is contiguous.
+// ---------------------------------------------------------------------------------------
+template <bool TRANS>
+__global__ void __launch_bounds__(256) split_weight_kernel(const float *__restrict__ w, char *packed,
+                                                           uint32_t *__restrict__ flags, int cout,
+                                                           int C, int T, int kb_total) {
+  constexpr int RO = TRANS ? 32 : 16, CO = TRANS ? 16 : 32;  // source rows (Cout), channels
+  __shared__ float s[RO * (CO * kMaxTaps + 1)];
+  const int r0 = (int)blockIdx.x * RO, c0 = (int)blockIdx.y * CO;
+  const int span = CO * T, pitch = span + 1;
+  const int vspan = span / 4;  // CO is a multiple of 16
+  const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+  for (int i = threadIdx.x; i < RO * vspan; i += 256) {
+    const int r = i / vspan, v = (i - r * vspan) * 4;
+    const float *src = w + ((int64_t)(r0 + r) * C + c0) * T + v;
+    floatx4 x = {0.f, 0.f, 0.f, 0.f};
+    if (r0 + r < cout) {
+      if (aligned) x = *reinterpret_cast<const floatx4 *>(src);
+      else x = floatx4{src[0], src[1], src[2], src[3]};
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[r * pitch + v + e] = x[e];
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  for (int t = threadIdx.x >> 6; t < T; t += 4) {  // a wave takes whole blocks (one per tap)
+    const int64_t blk = TRANS ? (int64_t)((t * C + c0) >> 4) * kb_total + (int)blockIdx.x
+                              : (int64_t)blockIdx.x * kb_total + ((t * C + c0) >> 5);
+    float h[8], m[8], l[8];
+    bool bad = false;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int n = lane & 15, k = (lane >> 4) * 8 + e;
+      const float v = TRANS ? s[k * pitch + n * T + t] : s[n * pitch + k * T + t];
+      Pieces p = cut(v);
+      if (!(p.l == p.l)) {  // non-finite: kept whole in h
+        bad = true;
+        p.h = v == v ? v : __builtin_nanf("");
+        p.m = p.l = 0.f;
+      }
+      h[e] = p.h; m[e] = p.m; l[e] = p.l;
+    }
+    char *d = packed + blk * kBlkBytes + lane * 16;
+    *reinterpret_cast<int4v *>(d) = int4v{pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
+    *reinterpret_cast<int4v *>(d + 1024) = int4v{pack2(m[0], m[1]), pack2(m[2], m[3]), pack2(m[4], m[5]), pack2(m[6], m[7])};
+    *reinterpret_cast<int4v *>(d + 2048) = int4v{pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7])};
+    const bool any = __any(bad);
+    if (lane == 0) flags[blk] = any ? 1u : 0u;
+  }
+}
+
+__global__ void __launch_bounds__(256) clear_f32x4(float *__restrict__ p, int64_t n4) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256)
+    reinterpret_cast<float4 *>(p)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// Tile height and K parts. A K step of a workgroup moves NRB * 8 KB of corner lines (a
+// quarter of that from a matrix) and 48 KB of weight per 256 columns through the CU's vector
+// memory path, about 38 cycles per KB, under NRB * BN * 1.5 cycles of matrix-core work per
+// SIMD; the plan with the least (rounds over the CUs) x (steps) x (the larger of the two)
+// runs. Two K parts add into a cleared output (two addends: the same result in any order).
+struct Plan {
+  int nrb, kparts, mch;
+};
+Plan plan(const Params &p, int bn, bool rows_mode, bool can_split) {
+  const int cus = std::max(1, device_cus());
+  Plan best{0, 1, 0};
+  double best_t = 0;
+  for (int kparts = 1; kparts <= (can_split ? 2 : 1); ++kparts) {
+    for (int nrb = 9; nrb >= 2; --nrb) {
+      if (bn == 128 && nrb % 2) continue;
+      if (bn == 64 && nrb % 4) continue;
+      const int64_t mch = (p.rb_total + nrb - 1) / nrb;
+      const int64_t wgs = mch * p.nt * kparts;
+      const int64_t rounds = (wgs + cus - 1) / cus;
+      const int steps = (p.kb_total + kparts - 1) / kparts;
+      const double kb = (rows_mode ? 2.0 : 8.0) * nrb + 48.0 * bn / 256;
+      double t = (double)rounds * (steps * (std::max(38.0 * kb, 1.5 * nrb * bn) + 250.0) + 6000.0);
+      if (kparts == 2) t += 8000.0 + (double)p.M * p.Cout * 8.0 / 1600.0;  // clear and add
+      if (best.nrb == 0 || t < best_t) {
+        best_t = t;
+        best = Plan{nrb, kparts, (int)mch};
+      }
+    }
+  }
+  return best;
+}
+
+template <int NRB, int WN, int GEO>
+void launch_one(const Params &p, hipStream_t stream) {
+  hipLaunchKernelGGL((f32_gemm_kernel<NRB, WN, GEO>), dim3(8 * p.per_xcd), dim3(kThreads), 0, stream, p);
+}
+
+template <int GEO>
+hipError_t launch_geo(Params p, hipStream_t stream) {
+  const int bn = p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64);
+  p.nt = (p.Cout + bn - 1) / bn;
+  p.rb_total = (p.M + 15) / 16;
+  const int64_t n_out = (int64_t)p.M * p.Cout;
+  const bool can_split = GEO != kRows && !p.relu && p.kb_total >= 16 && n_out % 4 == 0 &&
+                         reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
+  const Plan pl = plan(p, bn, GEO == kRows, can_split);
+  p.mch = pl.mch;
+  p.kparts = pl.kparts;
+  p.ksteps = (p.kb_total + pl.kparts - 1) / pl.kparts;
+  const int64_t wgs = (int64_t)p.mch * p.nt * p.kparts;
+  if (wgs > (1 << 28)) return hipErrorInvalidValue;
+  p.per_xcd = (int)((wgs + 7) / 8);
+  if (p.kparts == 2) {
+    const int64_t n4 = n_out / 4;
+    hipLaunchKernelGGL(clear_f32x4, dim3((unsigned)std::min<int64_t>((n4 + 255) / 256, 4096)),
+                       dim3(256), 0, stream, p.out, n4);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (bn == 256) {
+    switch (pl.nrb) {
+      case 2: launch_one<2, 8, GEO>(p, stream); break;
+      case 3: launch_one<3, 8, GEO>(p, stream); break;
+      case 4: launch_one<4, 8, GEO>(p, stream); break;
+      case 5: launch_one<5, 8, GEO>(p, stream); break;
+      case 6: launch_one<6, 8, GEO>(p, stream); break;
+      case 7: launch_one<7, 8, GEO>(p, stream); break;
+      case 8: launch_one<8, 8, GEO>(p, stream); break;
+      default: launch_one<9, 8, GEO>(p, stream); break;
+    }
+  } else if (bn == 128) {
+    switch (pl.nrb) {
+      case 2: launch_one<2, 4, GEO>(p, stream); break;
+      case 4: launch_one<4, 4, GEO>(p, stream); break;
+      case 6: launch_one<6, 4, GEO>(p, stream); break;
+      default: launch_one<8, 4, GEO>(p, stream); break;
+    }
+  } else {
+    if (pl.nrb == 4) launch_one<4, 2, GEO>(p, stream);
+    else launch_one<8, 2, GEO>(p, stream);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace
+
+int64_t f32_split_weight_bytes(int64_t n, int64_t k) {
+  return ((n + 15) / 16) * ((k + 31) / 32) * (kBlkBytes + 4);
+}
+
+hipError_t launch_f32_split_weight(const float *w, int cout, int C, int T, bool transposed,
+                                   void *packed, hipStream_t stream) {
+  const int n = transposed ? C * T : cout, k = transposed ? cout : C * T;
+  const int kb = (k + 31) / 32;
+  char *d = static_cast<char *>(packed);
+  uint32_t *flags = reinterpret_cast<uint32_t *>(d + (int64_t)((n + 15) / 16) * kb * kBlkBytes);
+  if (transposed)
+    hipLaunchKernelGGL((split_weight_kernel<true>), dim3((cout + 31) / 32, C / 16), dim3(256), 0,
+                       stream, w, d, flags, cout, C, T, kb);
+  else
+    hipLaunchKernelGGL((split_weight_kernel<false>), dim3((cout + 15) / 16, C / 32), dim3(256), 0,
+                       stream, w, d, flags, cout, C, T, kb);
+  return hipGetLastError();
+}
+
+hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, const void *x,
+                            const void *off, int geo, const void *msk, const void *w_split,
+                            const float *bias, float *out, hipStream_t stream, bool relu) {
+  Params p{};
+  p.x = x; p.off = off; p.msk = msk; p.w = w_split; p.bias = bias; p.out = out;
+  p.relu = relu ? 1 : 0;
+  p.Cout = channels_out;
+  p.nb_total = (channels_out + 15) / 16;
+  p.M = M;
+  p.kb_total = K / kBK;
+  p.taps = 1;
+  if (g != nullptr) {
+    p.C = g->channels; p.H = g->height; p.W = g->width; p.Ho = g->height_col; p.Wo = g->width_col;
+    p.kw = g->kernel_w; p.ph = g->pad_h; p.pw = g->pad_w; p.sh = g->stride_h; p.sw = g->stride_w;
+    p.dh = g->dil_h; p.dw = g->dil_w;
+    p.taps = g->kernel_h * g->kernel_w;
+    p.x_bytes = (uint32_t)((int64_t)g->batch * g->height * g->width * g->channels * 4);
+  } else {
+    p.x_bytes = (uint32_t)((int64_t)M * K * 4);
+  }
+  p.w_bytes = (uint32_t)((int64_t)p.nb_total * p.kb_total * kBlkBytes);
+  p.flags = reinterpret_cast<const uint32_t *>(static_cast<const char *>(w_split) + p.w_bytes);
+  if (g == nullptr) return launch_geo<kRows>(p, stream);
+  if (geo == kGeoMask) return launch_geo<kGeoMask>(p, stream);
+  return launch_geo<kGeoYF32>(p, stream);  // fp32 y: kGeoY and kGeoYF32 (no bias) are the same
+}
+
+}  // namespace bevk

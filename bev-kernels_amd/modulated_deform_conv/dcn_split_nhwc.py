@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from ._packing import pack_weight
+from ._packing import fused_conv, pack_weight, split_applies
 
 
 def out_size(H, pad, dil, k, stride):
@@ -101,11 +101,10 @@ def _fused_forward(x_nhwc, offset, mask, weight, bias, stride, padding, dilation
     out = torch.empty(B, Ho, Wo, Cout, device=x_nhwc.device, dtype=dt)
     vec = 16 // x_nhwc.element_size()
     if Cin % vec == 0 and dt != torch.float64:
-        _ext().dcn_fused_fwd_nhwc(
-            x_nhwc.contiguous(), offset.contiguous(),
-            (mask if mask is not None else offset).contiguous(), pack_weight(w, dt), b, B, Cin,
-            H, W, Ho, Wo, Cout, kH, kW, padding, padding, stride, stride, dilation, dilation,
-            out)
+        fused_conv(x_nhwc.contiguous(), offset.contiguous(),
+                   (mask if mask is not None else offset).contiguous(), w, b,
+                   (B, Cin, H, W, Ho, Wo, Cout, kH, kW, padding, padding, stride, stride,
+                    dilation, dilation), out)
     else:
         col = gather_cols_nhwc(x_nhwc, offset, mask, kH, kW, stride, padding, dilation)
         w_flat = w.permute(0, 2, 3, 1).to(dt).contiguous().view(Cout, kH * kW * Cin).t()
@@ -161,8 +160,15 @@ def mega_forward(x_nhwc, w_off, b_off, weight, bias=None, stride=1, padding=1, d
     Cout, _, kH, kW = weight.shape
     Ho, Wo = out_size(H, ph, dh, kH, sh), out_size(W, pw, dw, kW, sw)
     dt = x_nhwc.dtype
-    y = torch.empty(B, Ho, Wo, 3 * kH * kW, device=x_nhwc.device, dtype=torch.float32)
     out = torch.empty(B, Ho, Wo, Cout, device=x_nhwc.device, dtype=dt)
+    if split_applies(x_nhwc, Cin, Cout, kH * kW):
+        # two launches either way in fp32: the offset conv, then the split kernel reading y
+        x = x_nhwc.contiguous()
+        y = offset_conv_y(x, w_off, b_off, stride, padding, dilation)
+        fused_conv(x, y, None, weight, bias.to(dt).contiguous() if bias is not None else None,
+                   (B, Cin, H, W, Ho, Wo, Cout, kH, kW, ph, pw, sh, sw, dh, dw), out, act_relu)
+        return out, y
+    y = torch.empty(B, Ho, Wo, 3 * kH * kW, device=x_nhwc.device, dtype=torch.float32)
     _ext().dcn_mega_fwd_nhwc(
         x_nhwc.contiguous(), pack_weight(w_off, dt),
         b_off.float().contiguous() if b_off is not None else None, pack_weight(weight, dt),

@@ -22,7 +22,7 @@ import torch
 import torch.nn.functional as F
 
 from . import dcn_split_nhwc as _split
-from ._packing import pack_weight
+from ._packing import fused_conv
 
 
 def out_size(H, pad, dil, k, stride):
@@ -140,9 +140,8 @@ def fused_dcn_forward_nhwc(data_im, offset, mask, weight, bias=None, stride=1, p
     b = bias.to(dt).contiguous() if bias is not None else None
     vec = 16 // data_im.element_size()
     if Cin % vec == 0 and dt != torch.float64:
-        _ext().dcn_fused_fwd_nhwc(data_im.contiguous(), offset.contiguous(), mask.contiguous(),
-                                  pack_weight(weight, dt), b, B, Cin, H, W, Ho, Wo, Cout, kH, kW, ph, pw, sh, sw,
-                                  dh, dw, out)
+        fused_conv(data_im.contiguous(), offset.contiguous(), mask.contiguous(), weight, b,
+                   (B, Cin, H, W, Ho, Wo, Cout, kH, kW, ph, pw, sh, sw, dh, dw), out)
     else:
         cols = dcn_gather_cols_nhwc(data_im, offset, mask, kH, kW, (sh, sw), (ph, pw), (dh, dw))
         w_kc = weight.permute(0, 2, 3, 1).to(dt).contiguous()

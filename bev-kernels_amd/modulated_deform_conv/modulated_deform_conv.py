@@ -16,7 +16,7 @@ import torch.nn as nn
 from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _pair, _single
-from ._packing import pack_weight
+from ._packing import fused_conv
 
 _ext = None
 
@@ -376,12 +376,11 @@ def _modulated_deform_conv2d_forward(input, offset, mask, weight, bias, stride, 
         x_nhwc = ext.nchw_to_nhwc(input)
         off_nhwc = ext.nchw_to_nhwc(offset)
         msk_nhwc = ext.nchw_to_nhwc(mask)
-        w_packed = pack_weight(weight, input.dtype)
         b = bias.to(input.dtype).contiguous() if bias is not None else None
         out = input.new_empty(batch, ho, wo, channels_out)
-        ext.dcn_fused_fwd_nhwc(x_nhwc, off_nhwc, msk_nhwc, w_packed, b, batch, channels, height,
-                               width, ho, wo, channels_out, kernel_h, kernel_w, pad_h, pad_w,
-                               stride_h, stride_w, dil_h, dil_w, out)
+        fused_conv(x_nhwc, off_nhwc, msk_nhwc, weight, b,
+                   (batch, channels, height, width, ho, wo, channels_out, kernel_h, kernel_w,
+                    pad_h, pad_w, stride_h, stride_w, dil_h, dil_w), out)
         return ext.nhwc_to_nchw(out)
     # Columns [C*kh*kw, B*Ho*Wo] then one GEMM per group (modulated_deform_conv.py:369-401).
     bhw = batch * ho * wo

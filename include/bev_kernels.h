@@ -158,6 +158,30 @@ int bevk_dcn_layer_col2im_nhwc(
     int stride_w, int dilation_h, int dilation_w, int deformable_group, float *grad_im,
     float *grad_offset, float *grad_mask, void *stream);
 
+/* fp32 on the bf16 matrix cores: operands cut into three bf16 pieces that add up to them
+ * exactly, six products of pieces per product, fp32 sums (errors no larger than fp32 matrix
+ * instructions'; NaN / Inf as in plain fp32).
+ *   bevk_f32_split_weight_bytes  bytes of the split weight of n columns x k terms
+ *   bevk_dcn_split_weight        weight [Cout, C, kh, kw] fp32 -> split (16-byte aligned):
+ *                                columns Cout, terms (tap, C) with C % 32 == 0; transposed:
+ *                                columns (tap, C), terms Cout with C % 16 == 0, Cout % 32 == 0;
+ *                                at most 9 taps
+ *   bevk_dcn_fused_fwd_nhwc_f32  bevk_dcn_fused_fwd_nhwc for F32 with the split weight
+ *                                (C % 32 == 0, at most 9 taps) and an optional ReLU
+ *   bevk_gemm_f32                out [m, n] = a [m, k] times the split weight's columns */
+int64_t bevk_f32_split_weight_bytes(int n, int k);
+int bevk_dcn_split_weight(const void *weight, int channels_out, int kernel_h, int kernel_w,
+                          int channels, int transposed, void *split, void *stream);
+int bevk_dcn_fused_fwd_nhwc_f32(const void *data_im, const void *data_offset, int offset_last_dim,
+                                const void *data_mask, const void *weight_split, const void *bias,
+                                int batch_size, int channels, int height_im, int width_im,
+                                int height_col, int width_col, int channels_out, int kernel_h,
+                                int kernel_w, int pad_h, int pad_w, int stride_h, int stride_w,
+                                int dilation_h, int dilation_w, int act_relu, void *out,
+                                void *stream);
+int bevk_gemm_f32(const void *a, const void *weight_split, int m, int k, int n, void *out,
+                  void *stream);
+
 /* Workspace bytes bevk_modulated_deformable_fused_im2col_nhwc needs (-1 on bad
  * arguments): the packed offset-conv weight and the fp32 offset-conv output [M][3T]. */
 int64_t bevk_dcn_fused_im2col_nhwc_workspace_bytes(int dtype, int batch_size, int channels,
