@@ -46,3 +46,17 @@ def fused_conv(x, offset, mask, weight, bias, sizes, out, relu=False):
         return relu
     ext.dcn_fused_fwd_nhwc(x, offset, mask, pack_weight(weight, x.dtype), bias, *sizes, out)
     return False
+
+
+def columns_grad_f32(dout, weight):
+    """The columns' gradient [M, T*C] = dout [M, Cout] @ W, fp32, W [Cout, C, kh, kw] with its
+    columns in (tap, C) order."""
+    ext = _ext()
+    cout, c, kh, kw = weight.shape
+    lim = 2 ** 31 - 256
+    if (c % 16 == 0 and cout % 32 == 0 and kh * kw <= 9 and 4 * dout.numel() <= lim
+            and 6.5 * weight.numel() <= lim):
+        dcol = dout.new_empty(dout.size(0), kh * kw * c)
+        ext.gemm_f32(dout, ext.dcn_split_weight(weight.contiguous(), True), kh * kw * c, dcol)
+        return dcol
+    return torch.mm(dout, weight.permute(0, 2, 3, 1).reshape(cout, kh * kw * c))

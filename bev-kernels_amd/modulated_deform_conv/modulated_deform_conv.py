@@ -16,7 +16,7 @@ import torch.nn as nn
 from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _pair, _single
-from ._packing import fused_conv
+from ._packing import columns_grad_f32, fused_conv
 
 _ext = None
 
@@ -346,9 +346,8 @@ def _layer_backward_nhwc(ext, grad_output, input, offset, mask, weight, args):
     taps, channels_out = kernel_h * kernel_w, weight.size(0)
     m = batch * height_out * width_out
     x, off, msk, dout = (ext.nchw_to_nhwc(t) for t in (input, offset, mask, grad_output))
-    w_flat = weight.permute(0, 2, 3, 1).reshape(channels_out, taps * channels)
     dout = dout.view(m, channels_out)
-    cols = torch.mm(dout, w_flat)
+    cols = columns_grad_f32(dout, weight)
     grad_x = torch.zeros_like(x)
     grad_off, grad_msk = torch.empty_like(off), torch.empty_like(msk)
     ext.dcn_layer_col2im_nhwc(cols, x, off, msk, *args, grad_x, grad_off, grad_msk)
