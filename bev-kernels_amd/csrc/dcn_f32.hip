@@ -519,35 +519,41 @@ __global__ void __launch_bounds__(256) clear_f32x4(float *__restrict__ p, int64_
     reinterpret_cast<float4 *>(p)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Tile height and K parts. A K step of a workgroup moves NRB * 8 KB of corner lines (a
-// quarter of that from a matrix) and 48 KB of weight per 256 columns through the CU's vector
-// memory path, about 38 cycles per KB, under NRB * BN * 1.5 cycles of matrix-core work per
-// SIMD; the plan with the least (rounds over the CUs) x (steps) x (the larger of the two)
-// runs. Two K parts add into a cleared output (two addends: the same result in any order).
+// Tile height, tile width and K parts. A K step of a workgroup moves NRB * 8 KB of corner
+// lines (a quarter of that from a matrix) and 48 KB of weight per 256 columns through the CU's
+// vector memory path, about 38 cycles per KB, under NRB * BN * 1.5 cycles of matrix-core work
+// per SIMD; the plan with the least (rounds over the CUs) x (steps) x (the larger of the two)
+// runs. Tiles of up to 3 row blocks of a matrix leave room for two workgroups on a CU, whose
+// steps overlap (8,700 x 512 x 4,608: 220 us with 3 row blocks, 254 with 8; 34,800 x 256 x
+// 2,304: 281 and 297). Two K parts add into a cleared output (two addends: the same result in
+// any order). Swept over 8 layers and 6 products from 9 to 300 us, the choice was the fastest
+// or within 7% of it, one layer 10% off.
 struct Plan {
-  int nrb, kparts, mch;
+  int nrb, kparts, mch, bn;
 };
-Plan plan(const Params &p, int bn, bool rows_mode, bool can_split) {
+Plan plan(const Params &p, int bn_max, bool rows_mode, bool can_split) {
   const int cus = std::max(1, device_cus());
-  Plan best{0, 1, 0};
+  Plan best{0, 1, 0, bn_max};
   double best_t = 0;
-  for (int kparts = 1; kparts <= (can_split ? 2 : 1); ++kparts) {
-    for (int nrb = 9; nrb >= 2; --nrb) {
-      if (bn == 128 && nrb % 2) continue;
-      if (bn == 64 && nrb % 4) continue;
-      const int64_t mch = (p.rb_total + nrb - 1) / nrb;
-      const int64_t wgs = mch * p.nt * kparts;
-      const int64_t rounds = (wgs + cus - 1) / cus;
-      const int steps = (p.kb_total + kparts - 1) / kparts;
-      const double kb = (rows_mode ? 2.0 : 8.0) * nrb + 48.0 * bn / 256;
-      double t = (double)rounds * (steps * (std::max(38.0 * kb, 1.5 * nrb * bn) + 250.0) + 6000.0);
-      if (kparts == 2) t += 8000.0 + (double)p.M * p.Cout * 8.0 / 1600.0;  // clear and add
-      if (best.nrb == 0 || t < best_t) {
-        best_t = t;
-        best = Plan{nrb, kparts, (int)mch};
+  for (int bn = bn_max; bn >= 64; bn /= 2)
+    for (int kparts = 1; kparts <= (can_split ? 2 : 1); ++kparts)
+      for (int nrb = 9; nrb >= 2; --nrb) {
+        if ((bn == 128 && nrb % 2) || (bn == 64 && nrb % 4)) continue;
+        const int64_t mch = (p.rb_total + nrb - 1) / nrb;
+        const int64_t wgs = mch * ((p.Cout + bn - 1) / bn) * kparts;
+        const int64_t rounds = (wgs + cus - 1) / cus;
+        const int steps = (p.kb_total + kparts - 1) / kparts;
+        const double kb = (rows_mode ? 2.0 : 8.0) * nrb + 48.0 * bn / 256, mm = 1.5 * nrb * bn;
+        const bool two = rows_mode && nrb <= 3 && wgs > cus;
+        double t = two ? steps * std::max(20.0 * kb, mm) + 1200.0
+                       : steps * (std::max(38.0 * kb, mm) + 250.0) + 6000.0;
+        t *= (double)rounds;
+        if (kparts == 2) t += 8000.0 + (double)p.M * p.Cout * 8.0 / 1600.0;  // clear and add
+        if (best.nrb == 0 || t < best_t) {
+          best_t = t;
+          best = Plan{nrb, kparts, (int)mch, bn};
+        }
       }
-    }
-  }
   return best;
 }
 
@@ -558,13 +564,13 @@ void launch_one(const Params &p, hipStream_t stream) {
 
 template <int GEO>
 hipError_t launch_geo(Params p, hipStream_t stream) {
-  const int bn = p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64);
-  p.nt = (p.Cout + bn - 1) / bn;
   p.rb_total = (p.M + 15) / 16;
   const int64_t n_out = (int64_t)p.M * p.Cout;
   const bool can_split = GEO != kRows && !p.relu && p.kb_total >= 16 && n_out % 4 == 0 &&
                          reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
-  const Plan pl = plan(p, bn, GEO == kRows, can_split);
+  const Plan pl = plan(p, p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64), GEO == kRows, can_split);
+  const int bn = pl.bn;
+  p.nt = (p.Cout + bn - 1) / bn;
   p.mch = pl.mch;
   p.kparts = pl.kparts;
   p.ksteps = (p.kb_total + pl.kparts - 1) / pl.kparts;
