@@ -48,6 +48,7 @@ __all__ = [
     "dcn_split_weight",
     "dcn_fused_fwd_nhwc_f32",
     "gemm_f32",
+    "dcn_weight_grad",
     "dcn_offset_conv_nhwc",
     "dcn_mega_fwd_nhwc",
     "transpose",
@@ -303,6 +304,30 @@ def gemm_f32(a, weight_split, n, out):
     _b.require_numel(fn, "out", out, m * n)
     _b.call("bevk_gemm_f32", _b.ptr(a), _b.ptr(weight_split), m, k, n, _b.ptr(out),
             _b.stream_of(a))
+
+
+def dcn_weight_grad(cols, dout, kernel_h, kernel_w, out_dtype=None):
+    """grad_weight [Cout, C, kh, kw] (out_dtype, default cols') = sum over the rows of dout
+    [M, Cout] times cols [M, kh*kw*C], fp32 sums; None where the kernel does not take the
+    shape (channel counts that are not multiples of 16 bytes, more than 25 taps, float64)."""
+    fn = "dcn_weight_grad"
+    m, k = cols.shape
+    cout, taps = dout.shape[1], kernel_h * kernel_w
+    code = _b._DTYPE_CODES.get(cols.dtype, -1)
+    ws = _b.lib().bevk_dcn_weight_grad_workspace_bytes(code, m, k // taps, taps, cout)
+    if ws < 0:
+        return None
+    _b.require_device(fn, cols, dout)
+    _b.require_contiguous(fn, cols=cols, dout=dout)
+    _b.require_dtype(fn, cols, dout=dout)
+    _b.require_numel(fn, "cols", cols, m * (k // taps) * taps)
+    _b.require_numel(fn, "dout", dout, m * cout)
+    work = torch.empty(ws, dtype=torch.uint8, device=cols.device)
+    grad = torch.empty(cout, k // taps, kernel_h, kernel_w, device=cols.device,
+                       dtype=cols.dtype if out_dtype is None else out_dtype)
+    _b.call("bevk_dcn_weight_grad", code, _b.ptr(cols), _b.ptr(dout), m, k // taps, taps, cout,
+            _b.ptr(work), ws, _b.dtype_code(grad), _b.ptr(grad), _b.stream_of(cols))
+    return grad
 
 
 def _offset_conv_checks(fn, data_im, w_off_packed, b_off, batch_size, channels, height_im,

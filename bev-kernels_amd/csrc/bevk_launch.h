@@ -118,6 +118,14 @@ hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, co
                             const void *off, int geo, const void *msk, const void *w_split,
                             const float *bias, float *out, hipStream_t stream, bool relu);
 
+// Weight gradient [Cout][C][T] (out_dtype) = sum over the M pixels of dout [M][Cout] times cols
+// [M][T*C] (both dtype). Cout and C multiples of 16 bytes' worth of elements, T <= 25; the
+// workspace holds weight_grad_workspace_bytes.
+int64_t weight_grad_workspace_bytes(int dtype, int64_t M, int C, int T, int cout);
+hipError_t launch_weight_grad(int dtype, const void *cols, const void *dout, int64_t M, int C, int T,
+                              int cout, void *workspace, int out_dtype, void *grad_w,
+                              hipStream_t stream);
+
 // dst[b][c][r] = src[b][r][c] for 2- or 4-byte elements (NCHW <-> NHWC).
 hipError_t launch_transpose(int elem_bytes, const void *src, void *dst, int batch, int rows,
                             int cols, hipStream_t stream);

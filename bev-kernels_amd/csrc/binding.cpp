@@ -632,6 +632,46 @@ int bevk_gemm_f32(const void *a, const void *weight_split, int m, int k, int n, 
                     fn);
 }
 
+static int weight_grad_check(const char *fn, int dtype, long long m, int channels, int taps,
+                             int channels_out) {
+  if (dtype != BEVK_F32 && dtype != BEVK_F16 && dtype != BEVK_BF16)
+    return fail(BEVK_ERR_UNSUPPORTED, "\"%s\" not implemented for '%s'", fn, dtype_name(dtype));
+  const int vec = 16 / dtype_size(dtype);
+  if (m <= 0 || m >= (1LL << 30) || channels <= 0 || channels_out <= 0 || channels % vec != 0 ||
+      channels_out % vec != 0 || taps <= 0 || taps > 25)
+    return fail(BEVK_ERR_UNSUPPORTED,
+                "%s: channels must be positive multiples of %d for '%s', at most 25 taps", fn, vec,
+                dtype_name(dtype));
+  if ((long long)channels * taps * dtype_size(dtype) * 64 > (1 << 28) ||
+      (long long)channels_out * dtype_size(dtype) * 64 > (1 << 28))
+    return fail(BEVK_ERR_INVALID, "%s: rows too long for 32-bit buffer offsets", fn);
+  return 0;
+}
+
+int64_t bevk_dcn_weight_grad_workspace_bytes(int dtype, int64_t m, int channels, int taps,
+                                             int channels_out) {
+  if (weight_grad_check("dcn_weight_grad", dtype, m, channels, taps, channels_out)) return -1;
+  return bevk::weight_grad_workspace_bytes(dtype, m, channels, taps, channels_out);
+}
+
+int bevk_dcn_weight_grad(int dtype, const void *cols, const void *dout, int64_t m, int channels,
+                         int taps, int channels_out, void *workspace, int64_t workspace_bytes,
+                         int out_dtype, void *grad_weight, void *stream) {
+  const char *fn = "dcn_weight_grad";
+  g_last_error.clear();
+  if (int rc = weight_grad_check(fn, dtype, m, channels, taps, channels_out)) return rc;
+  if (out_dtype != BEVK_F32 && out_dtype != BEVK_F16 && out_dtype != BEVK_BF16)
+    return fail(BEVK_ERR_UNSUPPORTED, "\"%s\" not implemented for '%s'", fn, dtype_name(out_dtype));
+  if (workspace_bytes < bevk::weight_grad_workspace_bytes(dtype, m, channels, taps, channels_out))
+    return fail(BEVK_ERR_INVALID, "%s: workspace too small", fn);
+  if (!cols || !dout || !workspace || !grad_weight)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(bevk::launch_weight_grad(dtype, cols, dout, m, channels, taps, channels_out,
+                                             workspace, out_dtype, grad_weight,
+                                             (hipStream_t)stream),
+                    fn);
+}
+
 // Shared checks of the offset-conv entry points (dg == 1, fused-kernel dtypes, channel
 // vectors, 32-bit buffer offsets). Returns 0 or the failure code.
 static int check_offset_conv(const char *fn, int dtype, const bevk::DcnGeom &g) {

@@ -60,3 +60,16 @@ def columns_grad_f32(dout, weight):
         ext.gemm_f32(dout, ext.dcn_split_weight(weight.contiguous(), True), kh * kw * c, dcol)
         return dcol
     return torch.mm(dout, weight.permute(0, 2, 3, 1).reshape(cout, kh * kw * c))
+
+
+def weight_grad(cols, dout, weight, out_dtype):
+    """The weight's gradient [Cout, C, kh, kw] from the columns [M, T*C] and dout [M, Cout],
+    summed in fp32 and rounded once to out_dtype."""
+    cout, c, kh, kw = weight.shape
+    if out_dtype != torch.float64:
+        grad = _ext().dcn_weight_grad(cols, dout, kh, kw, out_dtype)
+        if grad is not None:
+            return grad
+    acc = cols.dtype if cols.dtype == torch.float64 else torch.float32
+    grad = torch.mm(dout.t().to(acc), cols.to(acc)).view(cout, kh, kw, c)
+    return grad.permute(0, 3, 1, 2).contiguous().to(out_dtype)

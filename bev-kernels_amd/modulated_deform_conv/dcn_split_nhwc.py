@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from ._packing import fused_conv, pack_weight, split_applies
+from ._packing import fused_conv, pack_weight, split_applies, weight_grad
 
 
 def out_size(H, pad, dil, k, stride):
@@ -220,8 +220,7 @@ def split_backward(grad_out, x, y, w_off, weight, stride, padding, dilation, wit
 
     cols = gather_cols_nhwc(x, y, None, kH, kW, st, pd, dl)
     dCol = torch.mm(dO, w_flat.t())
-    grad_weight = torch.mm(cols.t().float(), dO.float()) \
-        .view(kH, kW, Cin, Cout).permute(3, 2, 0, 1).contiguous().to(weight.dtype)
+    grad_weight = weight_grad(cols, dO, weight, weight.dtype)
     grad_bias = dO.float().sum(0).to(dt) if with_bias else None
 
     gX_samp, gOff, gmask_raw = col2im_nhwc(dCol, x, y, None, kH, kW, st, pd, dl)

@@ -16,7 +16,7 @@ import torch.nn as nn
 from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _pair, _single
-from ._packing import columns_grad_f32, fused_conv
+from ._packing import columns_grad_f32, fused_conv, weight_grad
 
 _ext = None
 
@@ -343,18 +343,16 @@ def _layer_backward_nhwc(ext, grad_output, input, offset, mask, weight, args):
     for name, t in (("data_im", input), ("data_offset", offset), ("data_mask", mask)):
         if not t.is_contiguous():  # as the NCHW column kernels
             raise RuntimeError(f"{name} must be contiguous")
-    taps, channels_out = kernel_h * kernel_w, weight.size(0)
     m = batch * height_out * width_out
     x, off, msk, dout = (ext.nchw_to_nhwc(t) for t in (input, offset, mask, grad_output))
-    dout = dout.view(m, channels_out)
+    dout = dout.view(m, weight.size(0))
     cols = columns_grad_f32(dout, weight)
     grad_x = torch.zeros_like(x)
     grad_off, grad_msk = torch.empty_like(off), torch.empty_like(msk)
     ext.dcn_layer_col2im_nhwc(cols, x, off, msk, *args, grad_x, grad_off, grad_msk)
     ext.dcn_layer_im2col_nhwc(x, off, msk, *args, cols)
-    grad_w = torch.mm(dout.t(), cols).view(channels_out, kernel_h, kernel_w, channels)
     return (ext.nhwc_to_nchw(grad_x), ext.nhwc_to_nchw(grad_off), ext.nhwc_to_nchw(grad_msk),
-            grad_w.permute(0, 3, 1, 2).contiguous())
+            weight_grad(cols, dout, weight, weight.dtype))
 
 
 def _modulated_deform_conv2d_forward(input, offset, mask, weight, bias, stride, padding,

@@ -182,6 +182,16 @@ int bevk_dcn_fused_fwd_nhwc_f32(const void *data_im, const void *data_offset, in
 int bevk_gemm_f32(const void *a, const void *weight_split, int m, int k, int n, void *out,
                   void *stream);
 
+/* Weight gradient of the NHWC column path: grad_weight [Cout, C, T] (out_dtype) = sum over the
+ * m pixels of dout [m, Cout] times cols [m, T*C] (dtype), fp32 sums (fp32 inputs: as
+ * bevk_gemm_f32), the same result on every run. C and Cout multiples of 16 bytes' worth of
+ * elements, T <= 25. The workspace query returns -1 for shapes that are not taken. */
+int64_t bevk_dcn_weight_grad_workspace_bytes(int dtype, int64_t m, int channels, int taps,
+                                             int channels_out);
+int bevk_dcn_weight_grad(int dtype, const void *cols, const void *dout, int64_t m, int channels,
+                         int taps, int channels_out, void *workspace, int64_t workspace_bytes,
+                         int out_dtype, void *grad_weight, void *stream);
+
 /* Workspace bytes bevk_modulated_deformable_fused_im2col_nhwc needs (-1 on bad
  * arguments): the packed offset-conv weight and the fp32 offset-conv output [M][3T]. */
 int64_t bevk_dcn_fused_im2col_nhwc_workspace_bytes(int dtype, int batch_size, int channels,
