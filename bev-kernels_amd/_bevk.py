@@ -55,6 +55,12 @@ _SIGNATURES = {
     "bevk_dcn_weight_grad_workspace_bytes": [_i, ctypes.c_int64] + [_i] * 3,
     "bevk_dcn_weight_grad": [_i, _vp, _vp, ctypes.c_int64] + [_i] * 3 + [_vp, ctypes.c_int64, _i,
                                                                          _vp, _vp],
+    "bevk_dcn_split_col2im_nhwc": [_i, _vp, _vp, _vp] + [_i] * 14 + [_vp, _vp, _vp],
+    "bevk_dcn_offset_conv_backward_workspace_bytes": [_i] * 6,
+    "bevk_dcn_offset_conv_backward": [_i, _vp, _vp, _vp, _vp] + [_i] * 14
+    + [_vp, ctypes.c_int64, _vp, _i, _vp, _vp, _vp],
+    "bevk_column_sums_workspace_bytes": [_i],
+    "bevk_column_sums": [_i, _vp, ctypes.c_int64, _i, _vp, ctypes.c_int64, _i, _vp, _vp],
     "bevk_transpose": [_i, _vp, _vp, _i, _i, _i, _vp],
     "bevk_dcn_offset_conv_nhwc": [_i, _vp, _vp, _vp] + [_i] * 14 + [_vp, _vp],
     "bevk_dcn_mega_fwd_nhwc": [_i, _vp, _vp, _vp, _vp, _vp] + [_i] * 16 + [_vp, _vp, _vp],
@@ -68,6 +74,8 @@ _SIGNATURES = {
 _RESTYPES = {"bevk_dcn_packed_weight_bytes": ctypes.c_int64,
              "bevk_f32_split_weight_bytes": ctypes.c_int64,
              "bevk_dcn_weight_grad_workspace_bytes": ctypes.c_int64,
+             "bevk_dcn_offset_conv_backward_workspace_bytes": ctypes.c_int64,
+             "bevk_column_sums_workspace_bytes": ctypes.c_int64,
              "bevk_dcn_fused_im2col_nhwc_workspace_bytes": ctypes.c_int64,
              "bevk_msda_backward_workspace_bytes": ctypes.c_int64}
 

@@ -49,6 +49,8 @@ __all__ = [
     "dcn_fused_fwd_nhwc_f32",
     "gemm_f32",
     "dcn_weight_grad",
+    "column_sums",
+    "dcn_split_backward_nhwc",
     "dcn_offset_conv_nhwc",
     "dcn_mega_fwd_nhwc",
     "transpose",
@@ -309,13 +311,14 @@ def gemm_f32(a, weight_split, n, out):
 def dcn_weight_grad(cols, dout, kernel_h, kernel_w, out_dtype=None):
     """grad_weight [Cout, C, kh, kw] (out_dtype, default cols') = sum over the rows of dout
     [M, Cout] times cols [M, kh*kw*C], fp32 sums; None where the kernel does not take the
-    shape (channel counts that are not multiples of 16 bytes, more than 25 taps, float64)."""
+    tensors (channel counts that are not multiples of 16 bytes, more than 25 taps, float64, not
+    16-byte aligned)."""
     fn = "dcn_weight_grad"
     m, k = cols.shape
     cout, taps = dout.shape[1], kernel_h * kernel_w
     code = _b._DTYPE_CODES.get(cols.dtype, -1)
     ws = _b.lib().bevk_dcn_weight_grad_workspace_bytes(code, m, k // taps, taps, cout)
-    if ws < 0:
+    if ws < 0 or cols.data_ptr() % 16 or dout.data_ptr() % 16:
         return None
     _b.require_device(fn, cols, dout)
     _b.require_contiguous(fn, cols=cols, dout=dout)
@@ -328,6 +331,58 @@ def dcn_weight_grad(cols, dout, kernel_h, kernel_w, out_dtype=None):
     _b.call("bevk_dcn_weight_grad", code, _b.ptr(cols), _b.ptr(dout), m, k // taps, taps, cout,
             _b.ptr(work), ws, _b.dtype_code(grad), _b.ptr(grad), _b.stream_of(cols))
     return grad
+
+
+def column_sums(src, out_dtype=None):
+    """fp32 sums over the rows of src [rows, n], rounded to out_dtype (default src's); None where
+    the kernel does not take the matrix (float64, rows that are not 16-byte vectors)."""
+    rows, n = src.shape
+    code = _b._DTYPE_CODES.get(src.dtype, -1)
+    if (code not in (_b.BEVK_F32, _b.BEVK_F16, _b.BEVK_BF16) or rows == 0 or n == 0
+            or n * src.element_size() % 16 or src.data_ptr() % 16):
+        return None
+    _b.require_device("column_sums", src)
+    _b.require_contiguous("column_sums", src=src)
+    ws = _b.lib().bevk_column_sums_workspace_bytes(n)
+    work = torch.empty(ws, dtype=torch.uint8, device=src.device)
+    out = src.new_empty(n, dtype=src.dtype if out_dtype is None else out_dtype)
+    _b.call("bevk_column_sums", code, _b.ptr(src), rows, n, _b.ptr(work), ws, _b.dtype_code(out),
+            _b.ptr(out), _b.stream_of(src))
+    return out
+
+
+def dcn_split_backward_nhwc(dcol, data_im, y, w_off, *sizes):
+    """The input side of the NHWC split layer's backward: dcol [M, T*C] and y [M, 3T] in the type
+    of data_im [B, H, W, C], w_off [3T, C, kh, kw]; sizes = (B, C, H, W, Ho, Wo, kh, kw, ph, pw,
+    sh, sw, dh, dw). Returns (grad_im in the input type, grad_w_off and grad_b_off in w_off's):
+    the column-to-image step, then the offset conv's backward with its input gradient added
+    before the one rounding. At most 9 taps, C a multiple of 8."""
+    fn = "dcn_split_backward_nhwc"
+    batch, channels, height, width, height_col, width_col, kernel_h, kernel_w = sizes[:8]
+    _b.require_device(fn, dcol, data_im, y, w_off)
+    _b.require_contiguous(fn, dcol=dcol, data_im=data_im, y=y)
+    _b.require_dtype(fn, data_im, dcol=dcol, y=y)
+    taps, m = kernel_h * kernel_w, batch * height_col * width_col
+    _b.require_numel(fn, "dcol", dcol, m * taps * channels)
+    _b.require_numel(fn, "data_im", data_im, batch * height * width * channels)
+    _b.require_numel(fn, "y", y, m * 3 * taps)
+    _b.require_numel(fn, "w_off", w_off, 3 * taps * channels * taps)
+    dev, code, stream = data_im.device, _b.dtype_code(data_im), _b.stream_of(data_im)
+    gx = torch.zeros(data_im.shape, dtype=torch.float32, device=dev)
+    gy = torch.zeros(m, 32, dtype=torch.float32, device=dev)
+    _b.call("bevk_dcn_split_col2im_nhwc", code, _b.ptr(dcol), _b.ptr(data_im), _b.ptr(y), *sizes,
+            _b.ptr(gx), _b.ptr(gy), stream)
+    ws = _b.lib().bevk_dcn_offset_conv_backward_workspace_bytes(batch, channels, height_col,
+                                                                width_col, kernel_h, kernel_w)
+    work = torch.empty(max(ws, 0), dtype=torch.uint8, device=dev)
+    w32 = w_off.float().contiguous()
+    grad_im = torch.empty_like(data_im)
+    grad_w = torch.empty(w_off.shape, dtype=w_off.dtype, device=dev)
+    grad_b = torch.empty(3 * taps, dtype=w_off.dtype, device=dev)
+    _b.call("bevk_dcn_offset_conv_backward", code, _b.ptr(data_im), _b.ptr(w32), _b.ptr(gy),
+            _b.ptr(gx), *sizes, _b.ptr(work), ws, _b.ptr(grad_im), _b.dtype_code(grad_w),
+            _b.ptr(grad_w), _b.ptr(grad_b), stream)
+    return grad_im, grad_w, grad_b
 
 
 def _offset_conv_checks(fn, data_im, w_off_packed, b_off, batch_size, channels, height_im,

@@ -54,6 +54,7 @@ struct DcnGeom {
   int deformable_group;
   int gate = 0;  // NHWC column-to-image: whole samples with h <= -1, w <= -1, h >= H or w >= W
                  // contribute nothing (the NCHW layer's rule)
+  int grad_ld = 0; // NHWC column-to-image: row length of grad_offset and grad_mask (0: 2T and T)
 };
 
 // NCHW modulated im2col; `tiled` picks the geometry-reuse kernel (im2col_opt).
@@ -118,6 +119,15 @@ hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, co
                             const void *off, int geo, const void *msk, const void *w_split,
                             const float *bias, float *out, hipStream_t stream, bool relu);
 
+// Input gradient of a plain convolution with n3 <= 32 outputs: out [B*H*W][C] (out_dtype) =
+// addend (fp32, or null) + the transposed convolution of y32 [B*Ho*Wo][32] (columns past n3 zero)
+// with w_off [n3][C][T], split by launch_f32_split_offset_weight into
+// f32_split_weight_bytes(C, 32 T) bytes.
+hipError_t launch_f32_split_offset_weight(const float *w_off, int n3, int C, int T, void *packed,
+                                          hipStream_t stream);
+hipError_t launch_f32_tconv(const DcnGeom &g, const float *y32, const void *w_split,
+                            const float *addend, int out_dtype, void *out, hipStream_t stream);
+
 // Weight gradient [Cout][C][T] (out_dtype) = sum over the M pixels of dout [M][Cout] times cols
 // [M][T*C] (both dtype). Cout and C multiples of 16 bytes' worth of elements, T <= 25; the
 // workspace holds weight_grad_workspace_bytes.
@@ -125,6 +135,19 @@ int64_t weight_grad_workspace_bytes(int dtype, int64_t M, int C, int T, int cout
 hipError_t launch_weight_grad(int dtype, const void *cols, const void *dout, int64_t M, int C, int T,
                               int cout, void *workspace, int out_dtype, void *grad_w,
                               hipStream_t stream);
+
+// The offset conv's weight gradient [n3][C][T] (out_dtype) from its input x [B, H, W, C] and fp32
+// output gradient y32 [M][32] (n3 <= 32 columns used; C % 4 == 0).
+int64_t offset_weight_grad_workspace_bytes(const DcnGeom &g, int n3);
+hipError_t launch_offset_weight_grad(int x_dtype, const DcnGeom &g, int n3, const void *x,
+                                     const float *y32, void *workspace, int out_dtype, void *grad_w,
+                                     hipStream_t stream);
+
+// out[c] (out_dtype) = fp32 sum over the rows of src [rows][ld], c < n; ld a multiple of 16 bytes'
+// worth of elements, src 16-byte aligned.
+int64_t column_sums_workspace_bytes(int n);
+hipError_t launch_column_sums(int dtype, const void *src, int64_t rows, int ld, int n, void *workspace,
+                              int out_dtype, void *out, hipStream_t stream);
 
 // dst[b][c][r] = src[b][r][c] for 2- or 4-byte elements (NCHW <-> NHWC).
 hipError_t launch_transpose(int elem_bytes, const void *src, void *dst, int batch, int rows,

@@ -672,6 +672,118 @@ int bevk_dcn_weight_grad(int dtype, const void *cols, const void *dout, int64_t 
                     fn);
 }
 
+// The NHWC split layer's backward steps: checks shared by the two entry points below.
+static int layer_backward_check(const char *fn, int dtype, const bevk::DcnGeom &g) {
+  if (dtype != BEVK_F32 && dtype != BEVK_F16 && dtype != BEVK_BF16)
+    return fail(BEVK_ERR_UNSUPPORTED, "\"%s\" not implemented for '%s'", fn, dtype_name(dtype));
+  if (int rc = check_geom(fn, g)) return rc;
+  const long long taps = (long long)g.kernel_h * g.kernel_w;
+  const long long m = (long long)g.batch * g.height_col * g.width_col;
+  if (taps > 9 || g.channels <= 0 || g.channels % 8 != 0)
+    return fail(BEVK_ERR_UNSUPPORTED, "%s: at most 9 taps and channels a multiple of 8", fn);
+  if (m * taps * g.channels >= 2147483647LL || m * 32 * 4 > kMaxBufferBytes ||
+      (long long)g.batch * g.height * g.width * g.channels * 4 > kMaxBufferBytes)
+    return fail(BEVK_ERR_INVALID, "%s: problem too large for 32-bit buffer offsets", fn);
+  return 0;
+}
+
+int bevk_dcn_split_col2im_nhwc(int dtype, const void *dcol, const void *data_im, const void *y,
+                               int batch_size, int channels, int height_im, int width_im,
+                               int height_col, int width_col, int kernel_h, int kernel_w, int pad_h,
+                               int pad_w, int stride_h, int stride_w, int dilation_h,
+                               int dilation_w, float *grad_im, float *grad_y, void *stream) {
+  const char *fn = "dcn_split_col2im_nhwc";
+  g_last_error.clear();
+  bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w, 1);
+  if (int rc = layer_backward_check(fn, dtype, g)) return rc;
+  if ((long long)batch_size * height_col * width_col == 0) return ok();
+  if (!dcol || !data_im || !y || !grad_im || !grad_y)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  g.grad_ld = 32;
+  return hip_status(bevk::launch_col2im_nhwc(dtype, g, dcol, data_im, y, true, nullptr, grad_im,
+                                             grad_y, grad_y + 2 * kernel_h * kernel_w,
+                                             (hipStream_t)stream),
+                    fn);
+}
+
+// Workspace of the offset conv's backward: the split weight, then the larger of the weight
+// gradient's parts and the column sums' (run one after the other).
+static long long offset_backward_split_bytes(const bevk::DcnGeom &g) {
+  return (bevk::f32_split_weight_bytes(g.channels, 32LL * g.kernel_h * g.kernel_w) + 255) / 256 * 256;
+}
+static long long offset_backward_ws(const bevk::DcnGeom &g) {
+  const int n3 = 3 * g.kernel_h * g.kernel_w;
+  const long long a = bevk::offset_weight_grad_workspace_bytes(g, n3);
+  const long long b = bevk::column_sums_workspace_bytes(n3);
+  return offset_backward_split_bytes(g) + (a > b ? a : b);
+}
+
+int64_t bevk_dcn_offset_conv_backward_workspace_bytes(int batch_size, int channels, int height_col,
+                                                      int width_col, int kernel_h, int kernel_w) {
+  bevk::DcnGeom g{};
+  g.batch = batch_size; g.channels = channels; g.height_col = height_col; g.width_col = width_col;
+  g.kernel_h = kernel_h; g.kernel_w = kernel_w;
+  if (batch_size <= 0 || channels <= 0 || height_col <= 0 || width_col <= 0 || kernel_h <= 0 ||
+      kernel_w <= 0 || kernel_h * kernel_w > 9)
+    return -1;
+  return offset_backward_ws(g);
+}
+
+int bevk_dcn_offset_conv_backward(int dtype, const void *data_im, const float *w_off,
+                                  const float *grad_y, const float *addend, int batch_size,
+                                  int channels, int height_im, int width_im, int height_col,
+                                  int width_col, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                                  int stride_h, int stride_w, int dilation_h, int dilation_w,
+                                  void *workspace, int64_t workspace_bytes, void *grad_im,
+                                  int weight_dtype, void *grad_w, void *grad_b, void *stream) {
+  const char *fn = "dcn_offset_conv_backward";
+  g_last_error.clear();
+  const bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w, 1);
+  if (int rc = layer_backward_check(fn, dtype, g)) return rc;
+  if (weight_dtype != BEVK_F32 && weight_dtype != BEVK_F16 && weight_dtype != BEVK_BF16)
+    return fail(BEVK_ERR_UNSUPPORTED, "\"%s\" not implemented for '%s'", fn,
+                dtype_name(weight_dtype));
+  const long long m = (long long)batch_size * height_col * width_col;
+  if (m == 0) return fail(BEVK_ERR_INVALID, "%s: empty batch", fn);
+  if (!data_im || !w_off || !grad_y || !workspace || !grad_im || !grad_w || !grad_b)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  if (workspace_bytes < offset_backward_ws(g))
+    return fail(BEVK_ERR_INVALID, "%s: workspace too small", fn);
+  const hipStream_t st = (hipStream_t)stream;
+  const int taps = kernel_h * kernel_w, n3 = 3 * taps;
+  void *parts = static_cast<char *>(workspace) + offset_backward_split_bytes(g);
+  hipError_t e = bevk::launch_f32_split_offset_weight(w_off, n3, channels, taps, workspace, st);
+  if (e == hipSuccess) e = bevk::launch_f32_tconv(g, grad_y, workspace, addend, dtype, grad_im, st);
+  if (e == hipSuccess)
+    e = bevk::launch_offset_weight_grad(dtype, g, n3, data_im, grad_y, parts, weight_dtype, grad_w, st);
+  if (e == hipSuccess)
+    e = bevk::launch_column_sums(BEVK_F32, grad_y, m, 32, n3, parts, weight_dtype, grad_b, st);
+  return hip_status(e, fn);
+}
+
+int64_t bevk_column_sums_workspace_bytes(int n) { return n < 0 ? -1 : bevk::column_sums_workspace_bytes(n); }
+
+int bevk_column_sums(int dtype, const void *src, int64_t rows, int n, void *workspace,
+                     int64_t workspace_bytes, int out_dtype, void *out, void *stream) {
+  const char *fn = "column_sums";
+  g_last_error.clear();
+  if (dtype < BEVK_F32 || dtype > BEVK_BF16 || out_dtype < BEVK_F32 || out_dtype > BEVK_BF16)
+    return fail(BEVK_ERR_UNSUPPORTED, "%s: fp32, fp16 and bf16 only", fn);
+  if (rows <= 0 || n <= 0 || n % (16 / dtype_size(dtype)) != 0 ||
+      reinterpret_cast<uintptr_t>(src) % 16 != 0)
+    return fail(BEVK_ERR_INVALID, "%s: rows must be 16-byte vectors of a 16-byte aligned matrix", fn);
+  if (workspace_bytes < bevk::column_sums_workspace_bytes(n))
+    return fail(BEVK_ERR_INVALID, "%s: workspace too small", fn);
+  if (!src || !workspace || !out) return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(bevk::launch_column_sums(dtype, src, rows, n, n, workspace, out_dtype, out,
+                                             (hipStream_t)stream),
+                    fn);
+}
+
 // Shared checks of the offset-conv entry points (dg == 1, fused-kernel dtypes, channel
 // vectors, 32-bit buffer offsets). Returns 0 or the failure code.
 static int check_offset_conv(const char *fn, int dtype, const bevk::DcnGeom &g) {

@@ -28,6 +28,7 @@
 #include "bevk_launch.h"
 
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
+#include <algorithm>
 #include <type_traits>
 
 namespace bevk {
@@ -131,9 +132,10 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
   }
   if (live && li == 0 && goff != nullptr) {
     if (g.gate && !fin) ah = aw = am = 0.f;  // also where the column gradient is not finite
-    goff[mg * 2 * T_ + 2 * t] = ah;
-    goff[mg * 2 * T_ + 2 * t + 1] = aw;
-    gmask[mg * T_ + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
+    const int lo = g.grad_ld ? g.grad_ld : 2 * T_, lm = g.grad_ld ? g.grad_ld : T_;
+    goff[mg * lo + 2 * t] = ah;
+    goff[mg * lo + 2 * t + 1] = aw;
+    gmask[mg * lm + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
   }
 }
 
@@ -401,9 +403,10 @@ __global__ void __launch_bounds__(kBlock) col2im_coord_nhwc_vec_kernel(
     float gx = mk * (hh * (s2 - s1) + lh * (s4 - s3));
     float am = w1 * s1 + w2 * s2 + w3 * s3 + w4 * s4;
     if (g.gate && !fin) gy = gx = am = 0.f;  // also where the column gradient is not finite
-    goff[mg * 2 * T_ + 2 * t] = gy;
-    goff[mg * 2 * T_ + 2 * t + 1] = gx;
-    gmask[mg * T_ + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
+    const int lo = g.grad_ld ? g.grad_ld : 2 * T_, lm = g.grad_ld ? g.grad_ld : T_;
+    goff[mg * lo + 2 * t] = gy;
+    goff[mg * lo + 2 * t + 1] = gx;
+    gmask[mg * lm + t] = FUSED_Y ? am * mk * (1.f - mk) : am;
   }
 }
 
@@ -752,7 +755,7 @@ hipError_t launch_t(const DcnGeom &g, const void *dcol, const void *im, const vo
                             g.kernel_h * g.kernel_w * g.channels;
   const bool vec = goff != nullptr && (sizeof(T) == 2 || sizeof(T) == 4) && cpg % VEC == 0 &&
                    im_bytes < ((int64_t)1 << 31) && col_elems < ((int64_t)1 << 31) &&
-                   (int64_t)g.batch * g.height_col * g.width_col * 3 * g.kernel_h * g.kernel_w * dg <
+                   (int64_t)g.batch * g.height_col * g.width_col * std::max(3 * g.kernel_h * g.kernel_w * dg, g.grad_ld) <
                        ((int64_t)1 << 31) &&
                    pairs / (g.kernel_h * g.kernel_w) < ((int64_t)1 << 22) &&
                    reinterpret_cast<uintptr_t>(dcol) % 16 == 0 &&

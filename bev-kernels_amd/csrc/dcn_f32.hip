@@ -46,6 +46,9 @@ constexpr int kMaxTaps = 9;
 constexpr int kThreads = 512;   // 8 waves
 constexpr int kBK = 32;         // K step: 128 bytes of an fp32 row
 constexpr int kRows = -1;       // GEO: A is a matrix, not deformable columns
+constexpr int kTConv = -2;      // GEO: transposed plain convolution of y [B, Ho, Wo, 32]: output
+                                // rows are input pixels, 32 terms per tap
+constexpr bool deform(int geo) { return geo >= 0; }
 constexpr int kBlkBytes = 3072; // split weight block: 16 columns x 32 k, three planes
 
 struct TapGeo {
@@ -59,7 +62,9 @@ struct Params {
   const void *w;              // split weight, then its flags
   const uint32_t *flags;
   const float *bias;
-  float *out;
+  const float *addend;        // kTConv: added to the sum before the rounding
+  void *out;
+  int out_kind;               // 0 fp32, 1 fp16, 2 bf16 (16 bits: kTConv only)
   int relu;
   int C, H, W, Ho, Wo, Cout, kw, ph, pw, sh, sw, dh, dw, M, taps;
   int nb_total, kb_total;     // 16-column blocks, 32-k blocks
@@ -124,6 +129,29 @@ __device__ __forceinline__ TapGeo tap_geo(const Params &p, int m, int t) {
   return G;
 }
 
+// kTConv: the output pixel of y whose tap t reads input pixel m, or out of range.
+__device__ __forceinline__ uint32_t tconv_offset(const Params &p, int m, int t) {
+  const int HW = p.H * p.W;
+  const int b = m / HW, r = m - b * HW, ih = r / p.W, iw = r - ih * p.W;
+  const int ki = t / p.kw, kj = t - ki * p.kw;
+  const int nh = ih + p.ph - ki * p.dh, nw = iw + p.pw - kj * p.dw;
+  const int oh = nh / p.sh, ow = nw / p.sw;
+  const bool ok = nh >= 0 && nw >= 0 && oh * p.sh == nh && ow * p.sw == nw && oh < p.Ho && ow < p.Wo;
+  return ok ? (uint32_t)((b * p.Ho + oh) * p.Wo + ow) * (kBK * 4u) : p.x_bytes;
+}
+
+// One output value: bias, addend, ReLU and the rounding of 16-bit outputs.
+__device__ __forceinline__ void emit(const Params &p, int m, int n, float v, float bias) {
+  const int64_t at = (int64_t)m * p.Cout + n;
+  v += bias;
+  if (p.addend != nullptr) v = p.addend[at] + v;
+  if (p.relu) v = v < 0.f ? 0.f : v;  // NaN stays NaN, as torch.relu
+  if (p.kparts > 1) unsafeAtomicAdd(static_cast<float *>(p.out) + at, v);
+  else if (p.out_kind == 0) static_cast<float *>(p.out)[at] = v;
+  else if (p.out_kind == 1) static_cast<f16 *>(p.out)[at] = static_cast<f16>(v);
+  else static_cast<bf16 *>(p.out)[at] = static_cast<bf16>(v);
+}
+
 // LDS address (bytes) of the A tile's 16-byte fragment piece (row, chunk of 8 k) inside one
 // plane: rows in 16-row blocks of 1 KB, stored in the order the MFMA fragments are read, so a
 // fragment read is 1 KB of consecutive addresses. The row is rotated by 4 per chunk: the
@@ -139,7 +167,7 @@ struct Shape {
   static constexpr int kSlots = kRowsN * (kBK / 4);      // (row, 4 channels) slots per step
   static constexpr int kNS = (kSlots + kThreads - 1) / kThreads;
   static constexpr int kFullWaves = (kSlots - (kNS - 1) * kThreads) / kWave;
-  static constexpr int kNQ = GEO == kRows ? 1 : 4;       // loads per slot
+  static constexpr int kNQ = deform(GEO) ? 4 : 1;       // loads per slot
 };
 
 // The K loop of one wave. Per step: the MFMAs of A buffer `buf`; meanwhile the next step's
@@ -158,7 +186,7 @@ __device__ __forceinline__ float k_loop(const Params &p, const TapGeo *geo, char
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = wave % WN, wm = wave / WN;
   const int kv = tid & 7;
-  const int spt = GEO == kRows ? p.kb_total : p.C / kBK;  // K steps per tap
+  const int spt = GEO == kRows ? p.kb_total : GEO == kTConv ? 1 : p.C / kBK;  // K steps per tap
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, p.x_bytes);
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(p.w, p.w_bytes);
 
@@ -198,7 +226,7 @@ __device__ __forceinline__ float k_loop(const Params &p, const TapGeo *geo, char
     }
   };
   auto load_w = [&](int i) __attribute__((always_inline)) {
-    if constexpr (GEO != kRows)
+    if constexpr (deform(GEO))
       w4 = *reinterpret_cast<const floatx4 *>(geo[slot_row(i) * p.taps + bt].w);
   };
   auto issue_slot = [&](int i) __attribute__((always_inline)) {
@@ -224,7 +252,7 @@ __device__ __forceinline__ float k_loop(const Params &p, const TapGeo *geo, char
   Pieces pc[4];
   auto blend_one = [&](int i, int e) __attribute__((always_inline)) {
     float v;
-    if constexpr (GEO == kRows) {
+    if constexpr (!deform(GEO)) {
       v = ra[i][0][e];
     } else {
       v = w4[0] * ra[i][0][e];
@@ -330,10 +358,10 @@ __device__ __forceinline__ float k_loop(const Params &p, const TapGeo *geo, char
 template <int NRB, int WN, int GEO>
 __device__ __forceinline__ void slow_tile(const Params &p, const TapGeo *geo, float *At, int n0, int m0,
                                        int rows, int k0, int nk, bool add_bias) {
-  constexpr int BN = WN * 32, RT = 16 * BN / kThreads;
+  constexpr int BN = WN * 32, RT = 16 * BN / kThreads, S4 = deform(GEO) ? 4 : 1;
   const int tid = threadIdx.x, n = n0 + tid % BN, r0 = (tid / BN) * RT;
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, p.x_bytes);
-  const int spt = GEO == kRows ? p.kb_total : p.C / kBK;
+  const int spt = GEO == kRows ? p.kb_total : GEO == kTConv ? 1 : p.C / kBK;
   const unsigned short *w = static_cast<const unsigned short *>(p.w);
   for (int rb = 0; rb * 16 < rows; ++rb) {
     float s[RT];
@@ -351,9 +379,9 @@ __device__ __forceinline__ void slow_tile(const Params &p, const TapGeo *geo, fl
           const int t = ks / spt;
           const TapGeo G = geo[(rb * 16 + row) * p.taps + t];
           const uint32_t cb = (uint32_t)((ks - t * spt) * kBK + c) * 4u;
-          for (int q = 0; q < 4; ++q) {
+          for (int q = 0; q < S4; ++q) {
             const float xv = G.o[q] == p.x_bytes ? 0.f : buffer_load_one<float>(xr, G.o[q] + cb);
-            v = q == 0 ? G.w[0] * xv : __builtin_fmaf(G.w[q], xv, v);
+            v = !deform(GEO) ? xv : q == 0 ? G.w[0] * xv : __builtin_fmaf(G.w[q], xv, v);
           }
         }
         At[row * kBK + c] = v;
@@ -375,12 +403,7 @@ __device__ __forceinline__ void slow_tile(const Params &p, const TapGeo *geo, fl
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
       const int m = m0 + rb * 16 + r0 + r;
-      float v = s[r] + bv;
-      if (p.relu) v = v < 0.f ? 0.f : v;
-      if (m < p.M && rb * 16 + r0 + r < rows && n < p.Cout) {
-        if (p.kparts > 1) unsafeAtomicAdd(p.out + (int64_t)m * p.Cout + n, v);
-        else p.out[(int64_t)m * p.Cout + n] = v;
-      }
+      if (m < p.M && rb * 16 + r0 + r < rows && n < p.Cout) emit(p, m, n, s[r], bv);
     }
   }
 }
@@ -413,7 +436,8 @@ __global__ void __launch_bounds__(kThreads) f32_gemm_kernel(const Params p) {
     for (int g = tid; g < S::kRowsN * p.taps; g += kThreads) {
       const int row = g / p.taps, t = g - row * p.taps, m = m0 + row;
       if (row < rows && m < p.M) {
-        geo[g] = tap_geo<GEO>(p, m, t);
+        if constexpr (GEO == kTConv) geo[g].o[0] = tconv_offset(p, m, t);
+        else geo[g] = tap_geo<GEO>(p, m, t);
       } else {
         TapGeo G;
         G.w[0] = G.w[1] = G.w[2] = G.w[3] = 0.f;
@@ -446,14 +470,34 @@ __global__ void __launch_bounds__(kThreads) f32_gemm_kernel(const Params p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = (wm * R + rb) * 16 + 4 * (lane >> 4) + e, m = m0 + row;
-        float v = acc[rb][cb][e] + bv;
-        if (p.relu) v = v < 0.f ? 0.f : v;  // NaN stays NaN, as torch.relu
-        if (row < rows && m < p.M && n < p.Cout) {
-          if (p.kparts > 1) unsafeAtomicAdd(p.out + (int64_t)m * p.Cout + n, v);
-          else p.out[(int64_t)m * p.Cout + n] = v;
-        }
+        if (row < rows && m < p.M && n < p.Cout) emit(p, m, n, acc[rb][cb][e], bv);
       }
   }
+}
+
+// The three pieces of a lane's 8 values of a split block; a non-finite value is kept whole in
+// the first piece. Returns whether there was one.
+__device__ __forceinline__ bool store_split(char *d, const float (&v)[8]) {
+  float h[8], m[8], l[8];
+  bool bad = false;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    Pieces p = cut(v[e]);
+    if (!(p.l == p.l)) {
+      bad = true;
+      p.h = v[e] == v[e] ? v[e] : __builtin_nanf("");
+      p.m = p.l = 0.f;
+    }
+    h[e] = p.h; m[e] = p.m; l[e] = p.l;
+  }
+  auto put = [](char *at, const float (&x)[8]) {
+    *reinterpret_cast<int4v *>(at) =
+        int4v{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
+  };
+  put(d, h);
+  put(d + 1024, m);
+  put(d + 2048, l);
+  return bad;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -491,27 +535,36 @@ __global__ void __launch_bounds__(256) split_weight_kernel(const float *__restri
   for (int t = threadIdx.x >> 6; t < T; t += 4) {  // a wave takes whole blocks (one per tap)
     const int64_t blk = TRANS ? (int64_t)((t * C + c0) >> 4) * kb_total + (int)blockIdx.x
                               : (int64_t)blockIdx.x * kb_total + ((t * C + c0) >> 5);
-    float h[8], m[8], l[8];
-    bool bad = false;
+    float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int n = lane & 15, k = (lane >> 4) * 8 + e;
-      const float v = TRANS ? s[k * pitch + n * T + t] : s[n * pitch + k * T + t];
-      Pieces p = cut(v);
-      if (!(p.l == p.l)) {  // non-finite: kept whole in h
-        bad = true;
-        p.h = v == v ? v : __builtin_nanf("");
-        p.m = p.l = 0.f;
-      }
-      h[e] = p.h; m[e] = p.m; l[e] = p.l;
+      v[e] = TRANS ? s[k * pitch + n * T + t] : s[n * pitch + k * T + t];
     }
-    char *d = packed + blk * kBlkBytes + lane * 16;
-    *reinterpret_cast<int4v *>(d) = int4v{pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
-    *reinterpret_cast<int4v *>(d + 1024) = int4v{pack2(m[0], m[1]), pack2(m[2], m[3]), pack2(m[4], m[5]), pack2(m[6], m[7])};
-    *reinterpret_cast<int4v *>(d + 2048) = int4v{pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7])};
+    const bool bad = store_split(packed + blk * kBlkBytes + lane * 16, v);
     const bool any = __any(bad);
     if (lane == 0) flags[blk] = any ? 1u : 0u;
   }
+}
+
+// Split offset-conv weight for kTConv: columns n = c, terms k = 32 t + j from w_off [n3][C][T]
+// (j < n3 <= 32, zero past it). One wave per block (n / 16, t).
+__global__ void __launch_bounds__(256) split_offset_weight_kernel(const float *__restrict__ w,
+                                                                  char *packed,
+                                                                  uint32_t *__restrict__ flags,
+                                                                  int n3, int C, int T, int blocks) {
+  const int blk = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (blk >= blocks) return;
+  const int nb = blk / T, t = blk - nb * T, c = nb * 16 + (lane & 15);
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int j = (lane >> 4) * 8 + e;
+    v[e] = j < n3 && c < C ? w[((int64_t)j * C + c) * T + t] : 0.f;
+  }
+  const bool bad = store_split(packed + (int64_t)blk * kBlkBytes + lane * 16, v);
+  const bool any = __any(bad);
+  if (lane == 0) flags[blk] = any ? 1u : 0u;
 }
 
 __global__ void __launch_bounds__(256) clear_f32x4(float *__restrict__ p, int64_t n4) {
@@ -566,9 +619,9 @@ template <int GEO>
 hipError_t launch_geo(Params p, hipStream_t stream) {
   p.rb_total = (p.M + 15) / 16;
   const int64_t n_out = (int64_t)p.M * p.Cout;
-  const bool can_split = GEO != kRows && !p.relu && p.kb_total >= 16 && n_out % 4 == 0 &&
+  const bool can_split = deform(GEO) && !p.relu && p.kb_total >= 16 && n_out % 4 == 0 &&
                          reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
-  const Plan pl = plan(p, p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64), GEO == kRows, can_split);
+  const Plan pl = plan(p, p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64), !deform(GEO), can_split);
   const int bn = pl.bn;
   p.nt = (p.Cout + bn - 1) / bn;
   p.mch = pl.mch;
@@ -580,7 +633,7 @@ hipError_t launch_geo(Params p, hipStream_t stream) {
   if (p.kparts == 2) {
     const int64_t n4 = n_out / 4;
     hipLaunchKernelGGL(clear_f32x4, dim3((unsigned)std::min<int64_t>((n4 + 255) / 256, 4096)),
-                       dim3(256), 0, stream, p.out, n4);
+                       dim3(256), 0, stream, static_cast<float *>(p.out), n4);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -655,6 +708,34 @@ hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, co
   if (g == nullptr) return launch_geo<kRows>(p, stream);
   if (geo == kGeoMask) return launch_geo<kGeoMask>(p, stream);
   return launch_geo<kGeoYF32>(p, stream);  // fp32 y: kGeoY and kGeoYF32 (no bias) are the same
+}
+
+hipError_t launch_f32_tconv(const DcnGeom &g, const float *y32, const void *w_split,
+                            const float *addend, int out_dtype, void *out, hipStream_t stream) {
+  Params p{};
+  p.x = y32; p.w = w_split; p.addend = addend; p.out = out; p.out_kind = out_dtype;
+  p.Cout = g.channels;
+  p.nb_total = (g.channels + 15) / 16;
+  p.M = g.batch * g.height * g.width;
+  p.taps = g.kernel_h * g.kernel_w;
+  p.kb_total = p.taps;
+  p.H = g.height; p.W = g.width; p.Ho = g.height_col; p.Wo = g.width_col;
+  p.kw = g.kernel_w; p.ph = g.pad_h; p.pw = g.pad_w; p.sh = g.stride_h; p.sw = g.stride_w;
+  p.dh = g.dil_h; p.dw = g.dil_w;
+  p.x_bytes = (uint32_t)((int64_t)g.batch * g.height_col * g.width_col * kBK * 4);
+  p.w_bytes = (uint32_t)((int64_t)p.nb_total * p.kb_total * kBlkBytes);
+  p.flags = reinterpret_cast<const uint32_t *>(static_cast<const char *>(w_split) + p.w_bytes);
+  return launch_geo<kTConv>(p, stream);
+}
+
+hipError_t launch_f32_split_offset_weight(const float *w_off, int n3, int C, int T, void *packed,
+                                          hipStream_t stream) {
+  char *d = static_cast<char *>(packed);
+  uint32_t *flags = reinterpret_cast<uint32_t *>(d + (int64_t)((C + 15) / 16) * T * kBlkBytes);
+  const int blocks = ((C + 15) / 16) * T;
+  hipLaunchKernelGGL(split_offset_weight_kernel, dim3((blocks + 3) / 4), dim3(256), 0, stream, w_off,
+                     d, flags, n3, C, T, blocks);
+  return hipGetLastError();
 }
 
 }  // namespace bevk

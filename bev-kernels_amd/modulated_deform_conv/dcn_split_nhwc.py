@@ -197,8 +197,9 @@ def split_backward(grad_out, x, y, w_off, weight, stride, padding, dilation, wit
     """Backward of the NHWC split forward (dcn_split_nhwc.py:230-291): the columns are
     re-gathered from x and y (the reference's default DCN_RECOMPUTE_COLS=1), dCol = dO @ W,
     grad_weight = cols^T @ dO in fp32, the column-to-image kernel gives grad_x (samples),
-    grad_offset and the pre-sigmoid grad_mask, and the offset conv's backward is the library
-    convolution backward. y is the offset-conv output with bias (float32 or the input
+    grad_offset and the pre-sigmoid grad_mask, and the offset conv's backward runs on the
+    matrix cores in fp32 (dcn_split_backward_nhwc; other shapes: the library convolution
+    backward). y is the offset-conv output with bias (float32 or the input
     dtype); the kernels read it in the input dtype. Returns (grad_x, grad_w_off,
     grad_b_off, grad_weight, grad_bias)."""
     st, pd, dl = stride, padding, dilation
@@ -221,8 +222,12 @@ def split_backward(grad_out, x, y, w_off, weight, stride, padding, dilation, wit
     cols = gather_cols_nhwc(x, y, None, kH, kW, st, pd, dl)
     dCol = torch.mm(dO, w_flat.t())
     grad_weight = weight_grad(cols, dO, weight, weight.dtype)
-    grad_bias = dO.float().sum(0).to(dt) if with_bias else None
+    grad_bias = _bias_grad(dO) if with_bias else None
 
+    if _native_backward(x, dCol, y, w_off, M, K):
+        return (*_ext().dcn_split_backward_nhwc(
+            dCol, x.contiguous(), y, w_off, B, Cin, H, W, Ho, Wo, kH, kW, pd, pd, st, st, dl, dl),
+            grad_weight, grad_bias)
     gX_samp, gOff, gmask_raw = col2im_nhwc(dCol, x, y, None, kH, kW, st, pd, dl)
 
     dY = torch.cat([gOff, gmask_raw], dim=-1).permute(0, 3, 1, 2).contiguous()
@@ -235,6 +240,24 @@ def split_backward(grad_out, x, y, w_off, weight, stride, padding, dilation, wit
     grad_x = (gX_samp + grad_x_off.permute(0, 2, 3, 1)).to(dt)
     return (grad_x, grad_w_off.to(w_off.dtype), grad_b_off.to(w_off.dtype), grad_weight,
             grad_bias)
+
+
+def _bias_grad(dO):
+    """Column sums of dO [M, Cout] in fp32, rounded once to its type."""
+    sums = _ext().column_sums(dO)
+    return dO.float().sum(0).to(dO.dtype) if sums is None else sums
+
+
+def _native_backward(x, dcol, y, w_off, m, k):
+    """True where dcn_split_backward_nhwc takes the layer: at most 9 taps, channels a multiple
+    of 8, sizes within its 32-bit offsets, 16-byte aligned tensors."""
+    n3, cin, kH, kW = w_off.shape
+    lim = 2 ** 31 - 256
+    return (x.dtype in (torch.float32, torch.float16, torch.bfloat16) and kH * kW <= 9
+            and n3 == 3 * kH * kW and cin == x.shape[-1] and cin % 8 == 0 and m > 0
+            and w_off.dtype in (torch.float32, torch.float16, torch.bfloat16)
+            and m * k < 2 ** 31 - 1 and 128 * m <= lim and 4 * x.numel() <= lim
+            and not any(t.data_ptr() % 16 for t in (x, dcol, y)))
 
 
 def dcn_split_forward_nhwc(x_nhwc, w_off, b_off, weight, bias=None, stride=1, padding=1,

@@ -253,7 +253,7 @@ def dcn_col2im_nhwc(dCol, X, offset, mask, kH, kW, stride=1, padding=0, dilation
 class _DCNSplitFunction(torch.autograd.Function):
     """Differentiable full DCNv2 (NHWC; fused_tl.py:866-943): forward = the one-kernel
     forward, backward = the NHWC split composition (re-gathered columns, dCol = dO @ W,
-    column-to-image kernel, library offset-conv backward)."""
+    column-to-image kernel, offset-conv backward on the matrix cores)."""
 
     @staticmethod
     def forward(ctx, x_nhwc, w_off, b_off, weight, bias, stride, padding, dilation):

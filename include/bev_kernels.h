@@ -192,6 +192,35 @@ int bevk_dcn_weight_grad(int dtype, const void *cols, const void *dout, int64_t 
                          int taps, int channels_out, void *workspace, int64_t workspace_bytes,
                          int out_dtype, void *grad_weight, void *stream);
 
+/* Backward of the NHWC layer with its offset conv inside (x [B, H, W, C] and y [B*Ho*Wo, 3T] in
+ * dtype; at most 9 taps, C a multiple of 8):
+ *   bevk_dcn_split_col2im_nhwc     bevk_modulated_deformable_col2im_nhwc (3T form) with the
+ *                                  gradient of y as rows of 32 floats grad_y [B*Ho*Wo, 32]:
+ *                                  offsets, then the pre-sigmoid mask; columns past 3T are not
+ *                                  written (zero them first)
+ *   bevk_dcn_offset_conv_backward  from grad_y and w_off [3T, C, kh, kw] (fp32):
+ *                                  grad_im [B, H, W, C] (dtype) = addend (fp32, or NULL) + the
+ *                                  input gradient; grad_w [3T, C, kh, kw] and grad_b [3T]
+ *                                  (weight_dtype). All sums in fp32 (as bevk_gemm_f32)
+ *   bevk_column_sums               out [n] (out_dtype) = fp32 sums over the rows of src [rows, n] */
+int bevk_dcn_split_col2im_nhwc(int dtype, const void *dcol, const void *data_im, const void *y,
+                               int batch_size, int channels, int height_im, int width_im,
+                               int height_col, int width_col, int kernel_h, int kernel_w, int pad_h,
+                               int pad_w, int stride_h, int stride_w, int dilation_h,
+                               int dilation_w, float *grad_im, float *grad_y, void *stream);
+int64_t bevk_dcn_offset_conv_backward_workspace_bytes(int batch_size, int channels, int height_col,
+                                                      int width_col, int kernel_h, int kernel_w);
+int bevk_dcn_offset_conv_backward(int dtype, const void *data_im, const float *w_off,
+                                  const float *grad_y, const float *addend, int batch_size,
+                                  int channels, int height_im, int width_im, int height_col,
+                                  int width_col, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                                  int stride_h, int stride_w, int dilation_h, int dilation_w,
+                                  void *workspace, int64_t workspace_bytes, void *grad_im,
+                                  int weight_dtype, void *grad_w, void *grad_b, void *stream);
+int64_t bevk_column_sums_workspace_bytes(int n);
+int bevk_column_sums(int dtype, const void *src, int64_t rows, int n, void *workspace,
+                     int64_t workspace_bytes, int out_dtype, void *out, void *stream);
+
 /* Workspace bytes bevk_modulated_deformable_fused_im2col_nhwc needs (-1 on bad
  * arguments): the packed offset-conv weight and the fp32 offset-conv output [M][3T]. */
 int64_t bevk_dcn_fused_im2col_nhwc_workspace_bytes(int dtype, int batch_size, int channels,
