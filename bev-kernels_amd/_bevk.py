@@ -61,6 +61,13 @@ _SIGNATURES = {
     + [_vp, ctypes.c_int64, _vp, _i, _vp, _vp, _vp],
     "bevk_column_sums_workspace_bytes": [_i],
     "bevk_column_sums": [_i, _vp, ctypes.c_int64, _i, _vp, ctypes.c_int64, _i, _vp, _vp],
+    "bevk_dcn_layer_nchw_f32_workspace_bytes": [_i] * 10,
+    "bevk_dcn_layer_nchw_f32": [_vp] * 5 + [_i] * 16 + [_vp, ctypes.c_int64, _vp, _vp],
+    "bevk_dcn_nhwc_workspace_bytes": [_i] * 11,
+    "bevk_dcn_conv_nhwc": [_i, _vp, _vp, _i, _vp, _vp, _vp] + [_i] * 15
+    + [_vp, ctypes.c_int64, _vp, _vp],
+    "bevk_dcn_layer_nhwc": [_i, _vp, _vp, _vp, _i, _vp, _vp] + [_i] * 16
+    + [_vp, ctypes.c_int64, _vp, _vp, _vp],
     "bevk_transpose": [_i, _vp, _vp, _i, _i, _i, _vp],
     "bevk_dcn_offset_conv_nhwc": [_i, _vp, _vp, _vp] + [_i] * 14 + [_vp, _vp],
     "bevk_dcn_mega_fwd_nhwc": [_i, _vp, _vp, _vp, _vp, _vp] + [_i] * 16 + [_vp, _vp, _vp],
@@ -76,6 +83,8 @@ _RESTYPES = {"bevk_dcn_packed_weight_bytes": ctypes.c_int64,
              "bevk_dcn_weight_grad_workspace_bytes": ctypes.c_int64,
              "bevk_dcn_offset_conv_backward_workspace_bytes": ctypes.c_int64,
              "bevk_column_sums_workspace_bytes": ctypes.c_int64,
+             "bevk_dcn_layer_nchw_f32_workspace_bytes": ctypes.c_int64,
+             "bevk_dcn_nhwc_workspace_bytes": ctypes.c_int64,
              "bevk_dcn_fused_im2col_nhwc_workspace_bytes": ctypes.c_int64,
              "bevk_msda_backward_workspace_bytes": ctypes.c_int64}
 

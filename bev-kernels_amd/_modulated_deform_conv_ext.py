@@ -49,6 +49,9 @@ __all__ = [
     "dcn_fused_fwd_nhwc_f32",
     "gemm_f32",
     "dcn_weight_grad",
+    "dcn_layer_nchw_f32",
+    "dcn_conv_nhwc",
+    "dcn_layer_nhwc",
     "column_sums",
     "dcn_split_backward_nhwc",
     "dcn_offset_conv_nhwc",
@@ -331,6 +334,104 @@ def dcn_weight_grad(cols, dout, kernel_h, kernel_w, out_dtype=None):
     _b.call("bevk_dcn_weight_grad", code, _b.ptr(cols), _b.ptr(dout), m, k // taps, taps, cout,
             _b.ptr(work), ws, _b.dtype_code(grad), _b.ptr(grad), _b.stream_of(cols))
     return grad
+
+
+def dcn_layer_nchw_f32(data_im, data_offset, data_mask, weight, bias, *sizes):
+    """The whole float32 NCHW layer (groups == 1) -> out [B, Cout, Ho, Wo], or None where the
+    kernels do not take the shape (C % 32, more than 9 taps, 2 GiB buffers). sizes = (B, C, H, W,
+    Ho, Wo, Cout, kh, kw, ph, pw, sh, sw, dh, dw, dg)."""
+    fn = "dcn_layer_nchw_f32"
+    b, c, h, w, ho, wo, cout, kh, kw = sizes[:9]
+    dg = sizes[15]
+    ws = _b.lib().bevk_dcn_layer_nchw_f32_workspace_bytes(b, c, h, w, ho, wo, cout, kh, kw, dg)
+    if ws < 0:
+        return None
+    _b.require_device(fn, data_im, data_offset, data_mask, weight, bias)
+    _b.require_contiguous(fn, data_im=data_im, data_offset=data_offset, data_mask=data_mask,
+                          weight=weight, bias=bias)
+    if data_im.dtype != torch.float32:
+        raise RuntimeError(f"{fn}: data_im must be float32, got {data_im.dtype}")
+    _b.require_dtype(fn, data_im, data_offset=data_offset, data_mask=data_mask, weight=weight,
+                     bias=bias)
+    taps, plane = kh * kw, ho * wo
+    _b.require_numel(fn, "data_im", data_im, b * c * h * w)
+    _b.require_numel(fn, "data_offset", data_offset, b * dg * 2 * taps * plane)
+    _b.require_numel(fn, "data_mask", data_mask, b * dg * taps * plane)
+    _b.require_numel(fn, "weight", weight, cout * c * taps)
+    if bias is not None:
+        _b.require_numel(fn, "bias", bias, cout)
+    work = torch.empty(ws, dtype=torch.uint8, device=data_im.device)
+    out = data_im.new_empty(b, cout, ho, wo)
+    _b.call("bevk_dcn_layer_nchw_f32", _b.ptr(data_im), _b.ptr(data_offset), _b.ptr(data_mask),
+            _b.ptr(weight), _b.ptr(bias), *sizes, _b.ptr(work), ws, _b.ptr(out),
+            _b.stream_of(data_im))
+    return out
+
+
+def dcn_conv_nhwc(data_im, data_offset, data_mask, weight, bias, *sizes):
+    """Fused NHWC deformable conv from the module weight [Cout, C, kh, kw] -> out [B, Ho, Wo, Cout];
+    data_offset 2T with data_mask, or the raw 3T offset-conv output, in the type of data_im. The
+    weight is packed on every call, into the call's workspace. sizes = (B, C, H, W, Ho, Wo, Cout,
+    kh, kw, ph, pw, sh, sw, dh, dw). Channels a multiple of 16 bytes, not float64."""
+    fn = "dcn_conv_nhwc"
+    b, c, h, w, ho, wo, cout, kh, kw = sizes[:9]
+    _b.require_device(fn, data_im, data_offset, data_mask, weight, bias)
+    _b.require_contiguous(fn, data_im=data_im, data_offset=data_offset, data_mask=data_mask,
+                          weight=weight, bias=bias)
+    taps, last, m = kh * kw, data_offset.size(-1), b * ho * wo
+    fused_y = last == 3 * taps
+    _b.require_dtype(fn, data_im, data_offset=data_offset, weight=weight, bias=bias,
+                     data_mask=None if fused_y else data_mask)
+    _b.require_numel(fn, "data_im", data_im, b * h * w * c)
+    _b.require_numel(fn, "data_offset", data_offset, m * last)
+    if not fused_y:
+        _b.require_numel(fn, "data_mask", data_mask, m * taps)
+    _b.require_numel(fn, "weight", weight, cout * c * taps)
+    if bias is not None:
+        _b.require_numel(fn, "bias", bias, cout)
+    code = _b.dtype_code(data_im)
+    ws = _b.lib().bevk_dcn_nhwc_workspace_bytes(code, 0, b, c, h, w, ho, wo, cout, kh, kw)
+    out = data_im.new_empty(b, ho, wo, cout)
+    if ws < 0:  # the packed entry point names what it does not take
+        dcn_fused_fwd_nhwc(data_im, data_offset, data_mask, dcn_pack_weight(weight), bias, *sizes,
+                           out)
+        return out
+    work = torch.empty(ws, dtype=torch.uint8, device=data_im.device)
+    _b.call("bevk_dcn_conv_nhwc", code, _b.ptr(data_im), _b.ptr(data_offset), last,
+            _b.ptr(data_mask), _b.ptr(weight), _b.ptr(bias), *sizes, _b.ptr(work), ws, _b.ptr(out),
+            _b.stream_of(data_im))
+    return out
+
+
+def dcn_layer_nhwc(data_im, w_off, b_off, weight, bias, *sizes, act_relu=False):
+    """The NHWC layer with its offset conv from the module's weights: (out [B, Ho, Wo, Cout] in
+    the type of data_im, y [B, Ho, Wo, 3T] float32). w_off and weight in the type of data_im, b_off
+    float32 or that type (or None); sizes as dcn_conv_nhwc. None where the kernels do not take the
+    shape."""
+    fn = "dcn_layer_nhwc"
+    b, c, h, w, ho, wo, cout, kh, kw = sizes[:9]
+    code = _b.dtype_code(data_im)
+    ws = _b.lib().bevk_dcn_nhwc_workspace_bytes(code, 1, b, c, h, w, ho, wo, cout, kh, kw)
+    if ws < 0:
+        return None
+    _b.require_device(fn, data_im, w_off, b_off, weight, bias)
+    _b.require_contiguous(fn, data_im=data_im, w_off=w_off, b_off=b_off, weight=weight, bias=bias)
+    _b.require_dtype(fn, data_im, w_off=w_off, weight=weight, bias=bias)
+    taps = kh * kw
+    _b.require_numel(fn, "data_im", data_im, b * h * w * c)
+    _b.require_numel(fn, "w_off", w_off, 3 * taps * c * taps)
+    _b.require_numel(fn, "weight", weight, cout * c * taps)
+    if b_off is not None:
+        _b.require_numel(fn, "b_off", b_off, 3 * taps)
+    if bias is not None:
+        _b.require_numel(fn, "bias", bias, cout)
+    out = data_im.new_empty(b, ho, wo, cout)
+    y = torch.empty(b, ho, wo, 3 * taps, dtype=torch.float32, device=data_im.device)
+    work = torch.empty(ws, dtype=torch.uint8, device=data_im.device)
+    _b.call("bevk_dcn_layer_nhwc", code, _b.ptr(data_im), _b.ptr(w_off), _b.ptr(b_off),
+            0 if b_off is None else _b.dtype_code(b_off), _b.ptr(weight), _b.ptr(bias), *sizes,
+            int(act_relu), _b.ptr(work), ws, _b.ptr(y), _b.ptr(out), _b.stream_of(data_im))
+    return out, y
 
 
 def column_sums(src, out_dtype=None):

@@ -84,7 +84,10 @@ hipError_t launch_dcn_fused_h(int dtype, const DcnGeom &g, int channels_out, con
                               const void *off, int geo, const void *msk,
                               const void *w_packed, const void *bias, void *out,
                               hipStream_t stream, const float *y_bias = nullptr,
-                              bool relu = false);
+                              bool relu = false, float *part = nullptr);
+// Bytes of the scratch `part` (16-byte aligned) with which this shape runs K in parts (geo
+// kGeoMask / kGeoYF32, 16-byte aligned output); 0 where it runs whole.
+int64_t dcn_fused_h_parts_bytes(int dtype, const DcnGeom &g, int channels_out);
 
 // One-launch DCNv2 forward with the offset conv inside (fp16 / bf16 on the persistent
 // kernel): y = conv(x, w_off) + b_off (fp32, kept in LDS and written to y_out), offsets
@@ -105,6 +108,12 @@ int64_t dcn_packed_weight_elems(int dtype, int cout, int K);
 hipError_t launch_dcn_pack_weight(int dtype, const void *weight, int cout, int C, int T,
                                   void *packed, hipStream_t stream, bool src_tc = false);
 
+// 16-bit layer preparation: weight [cout][C][T] and w_off [n3][C][T] packed, b_off [n3] (b_dtype, or
+// null; n3 <= 64) as fp32.
+hipError_t launch_dcn_prep16(int dtype, const void *weight, int cout, const void *w_off, int n3, int C,
+                             int T, const void *b_off, int b_dtype, void *packed, void *packed_off,
+                             float *b_out, hipStream_t stream);
+
 // fp32 products on the bf16 matrix cores (three exact bf16 pieces per operand, dcn_f32.hip).
 // Split weight of n columns and k reduction elements (with its flags), from the module weight
 // [Cout][C][T]: n = Cout, k = t*C + c (C % 32 == 0), or transposed n = t*C + c, k = Cout
@@ -118,6 +127,14 @@ hipError_t launch_f32_split_weight(const float *weight, int cout, int C, int T, 
 hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, const void *x,
                             const void *off, int geo, const void *msk, const void *w_split,
                             const float *bias, float *out, hipStream_t stream, bool relu);
+
+// The whole NCHW fp32 layer (groups == 1, any deformable_group): x [B, C, H, W], off [B, dg*2T, Ho,
+// Wo], msk [B, dg*T, Ho, Wo], weight [Cout, C, kh, kw] -> out [B, Cout, Ho, Wo]. C % 32 == 0, at
+// most 9 taps; with deformable groups a 16-byte aligned output and columns under 2 GiB.
+int64_t dcn_layer_f32_workspace_bytes(const DcnGeom &g, int channels_out);
+hipError_t launch_dcn_layer_f32(const DcnGeom &g, int cout, const float *x, const float *off,
+                                const float *msk, const float *weight, const float *bias,
+                                void *workspace, float *out, hipStream_t stream);
 
 // Input gradient of a plain convolution with n3 <= 32 outputs: out [B*H*W][C] (out_dtype) =
 // addend (fp32, or null) + the transposed convolution of y32 [B*Ho*Wo][32] (columns past n3 zero)

@@ -868,6 +868,220 @@ int bevk_dcn_mega_fwd_nhwc(int dtype, const void *data_im, const void *w_off_pac
                     fn);
 }
 
+// ---------------------------------------------------------------------------------------
+// Whole layers from the module's own weights: packing, offset conv, deformable product and layout
+// changes behind one call and one caller-owned workspace.
+// ---------------------------------------------------------------------------------------
+
+static long long up256(long long b) { return (b + 255) / 256 * 256; }
+
+// fp32 shapes of the split product (dcn_f32.hip).
+static bool split_takes(const bevk::DcnGeom &g, int channels_out) {
+  const long long taps = (long long)g.kernel_h * g.kernel_w;
+  return taps <= 9 && g.channels > 0 && g.channels % 32 == 0 &&
+         (long long)g.batch * g.height * g.width * g.channels * 4 <= kMaxBufferBytes &&
+         bevk::f32_split_weight_bytes(channels_out, taps * g.channels) <= kMaxBufferBytes &&
+         (long long)g.batch * g.height_col * g.width_col < (1LL << 30);
+}
+
+static bevk::DcnGeom ws_geom(int batch_size, int channels, int height_im, int width_im, int height_col,
+                             int width_col, int kernel_h, int kernel_w, int dg) {
+  return make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h, kernel_w,
+                   0, 0, 1, 1, 1, 1, dg);
+}
+
+static bool ws_sizes_ok(const bevk::DcnGeom &g, int channels_out) {
+  return g.batch > 0 && g.channels > 0 && g.height > 0 && g.width > 0 && g.height_col > 0 &&
+         g.width_col > 0 && g.kernel_h > 0 && g.kernel_w > 0 && channels_out > 0 &&
+         g.deformable_group > 0 && g.channels % g.deformable_group == 0;
+}
+
+int64_t bevk_dcn_layer_nchw_f32_workspace_bytes(int batch_size, int channels, int height_im,
+                                                int width_im, int height_col, int width_col,
+                                                int channels_out, int kernel_h, int kernel_w,
+                                                int deformable_group) {
+  const bevk::DcnGeom g = ws_geom(batch_size, channels, height_im, width_im, height_col, width_col,
+                                  kernel_h, kernel_w, deformable_group);
+  if (!ws_sizes_ok(g, channels_out) || !split_takes(g, channels_out) || batch_size > 65535) return -1;
+  const long long k = (long long)kernel_h * kernel_w * channels;
+  if (deformable_group > 1 &&
+      ((long long)batch_size * height_col * width_col * k * 4 > kMaxBufferBytes ||
+       channels / deformable_group % 4 != 0))
+    return -1;
+  return bevk::dcn_layer_f32_workspace_bytes(g, channels_out);
+}
+
+int bevk_dcn_layer_nchw_f32(const float *data_im, const float *data_offset, const float *data_mask,
+                            const float *weight, const float *bias, int batch_size, int channels,
+                            int height_im, int width_im, int height_col, int width_col,
+                            int channels_out, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                            int stride_h, int stride_w, int dilation_h, int dilation_w,
+                            int deformable_group, void *workspace, int64_t workspace_bytes,
+                            float *out, void *stream) {
+  const char *fn = "dcn_layer_nchw_f32";
+  g_last_error.clear();
+  const bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w,
+                deformable_group);
+  if (int rc = check_geom(fn, g)) return rc;
+  const int64_t need = bevk_dcn_layer_nchw_f32_workspace_bytes(
+      batch_size, channels, height_im, width_im, height_col, width_col, channels_out, kernel_h,
+      kernel_w, deformable_group);
+  if (need < 0) return fail(BEVK_ERR_UNSUPPORTED, "%s: shape not taken", fn);
+  if (workspace_bytes < need) return fail(BEVK_ERR_INVALID, "%s: workspace too small", fn);
+  if (!data_im || !data_offset || !data_mask || !weight || !workspace || !out)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  if (deformable_group > 1 && reinterpret_cast<uintptr_t>(out) % 16 != 0)
+    return fail(BEVK_ERR_INVALID, "%s: out must be 16-byte aligned", fn);
+  return hip_status(bevk::launch_dcn_layer_f32(g, channels_out, data_im, data_offset, data_mask, weight,
+                                               bias, workspace, out, (hipStream_t)stream),
+                    fn);
+}
+
+// Workspace of the NHWC layers: the main weight's packed or split form, and with the offset conv
+// its packed weight and fp32 bias; then the K parts' sums.
+struct NhwcWs {
+  long long w_off, b_off, part, total;
+  bool split;
+  long long parts;
+};
+static bool nhwc_ws(int dtype, const bevk::DcnGeom &g, int cout, bool layer, NhwcWs *out) {
+  if (dtype != BEVK_F32 && dtype != BEVK_F16 && dtype != BEVK_BF16) return false;
+  if (!ws_sizes_ok(g, cout) || g.channels % (16 / dtype_size(dtype)) != 0) return false;
+  const int T = g.kernel_h * g.kernel_w, K = T * g.channels, es = dtype_size(dtype);
+  if ((long long)g.batch * g.height * g.width * g.channels * es > kMaxBufferBytes ||
+      (long long)g.batch * g.height_col * g.width_col >= (1LL << 30) ||
+      (long long)K * (cout + 32) * es > kMaxBufferBytes)
+    return false;
+  if (layer && dtype != BEVK_F32 && T > 9) return false;
+  if (layer && 3 * T > 64) return false;
+  NhwcWs w;
+  w.split = dtype == BEVK_F32 && split_takes(g, cout);
+  w.parts = dtype == BEVK_F32 ? 0 : bevk::dcn_fused_h_parts_bytes(dtype, g, cout);
+  long long at = up256(w.split ? bevk::f32_split_weight_bytes(cout, K)
+                               : bevk::dcn_packed_weight_elems(dtype, cout, K) * es);
+  w.w_off = at;
+  if (layer) at += up256(bevk::dcn_packed_weight_elems(dtype, 3 * T, K) * es);
+  w.b_off = at;
+  if (layer) at += 256;
+  w.part = at;
+  w.total = at + w.parts;
+  *out = w;
+  return true;
+}
+
+int64_t bevk_dcn_nhwc_workspace_bytes(int dtype, int with_offset_conv, int batch_size, int channels,
+                                      int height_im, int width_im, int height_col, int width_col,
+                                      int channels_out, int kernel_h, int kernel_w) {
+  NhwcWs w;
+  const bevk::DcnGeom g = ws_geom(batch_size, channels, height_im, width_im, height_col, width_col,
+                                  kernel_h, kernel_w, 1);
+  return nhwc_ws(dtype, g, channels_out, with_offset_conv != 0, &w) ? w.total : -1;
+}
+
+// The deformable product from a packed / split weight in the workspace; y_f32: offsets are the
+// fp32 y.
+static hipError_t nhwc_product(int dtype, const bevk::DcnGeom &g, int cout, const NhwcWs &w, char *ws,
+                               const void *x, const void *off, int geo, const void *mask,
+                               const void *bias, bool relu, void *out, hipStream_t st) {
+  if (w.split)
+    return bevk::launch_f32_split(&g, cout, g.batch * g.height_col * g.width_col,
+                                  g.kernel_h * g.kernel_w * g.channels, x, off, geo, mask, ws,
+                                  static_cast<const float *>(bias), static_cast<float *>(out), st, relu);
+  if (w.parts > 0 && (geo == bevk::kGeoMask || geo == bevk::kGeoYF32) &&
+      reinterpret_cast<uintptr_t>(out) % 16 == 0)
+    return bevk::launch_dcn_fused_h(dtype, g, cout, x, off, geo, mask, ws, bias, out, st, nullptr, relu,
+                                    reinterpret_cast<float *>(ws + w.part));
+  return bevk::launch_dcn_fused_nhwc(dtype, g, cout, x, off, geo, mask, ws, bias, out, st, nullptr, relu);
+}
+
+int bevk_dcn_conv_nhwc(int dtype, const void *data_im, const void *data_offset, int offset_last_dim,
+                       const void *data_mask, const void *weight, const void *bias, int batch_size,
+                       int channels, int height_im, int width_im, int height_col, int width_col,
+                       int channels_out, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                       int stride_h, int stride_w, int dilation_h, int dilation_w, void *workspace,
+                       int64_t workspace_bytes, void *out, void *stream) {
+  const char *fn = "dcn_conv_nhwc";
+  g_last_error.clear();
+  const bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w, 1);
+  if (int rc = check_geom(fn, g)) return rc;
+  const int taps = kernel_h * kernel_w;
+  if (offset_last_dim != 2 * taps && offset_last_dim != 3 * taps)
+    return fail(BEVK_ERR_INVALID, "%s: offset last dim must be 2T (%d) or 3T (%d), got %d", fn,
+                2 * taps, 3 * taps, offset_last_dim);
+  const bool y = offset_last_dim == 3 * taps;
+  NhwcWs w;
+  if (!nhwc_ws(dtype, g, channels_out, false, &w))
+    return fail(BEVK_ERR_UNSUPPORTED, "%s: shape not taken", fn);
+  if (workspace_bytes < w.total) return fail(BEVK_ERR_INVALID, "%s: workspace too small", fn);
+  if (!data_im || !data_offset || (!y && !data_mask) || !weight || !workspace || !out)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  const hipStream_t st = (hipStream_t)stream;
+  char *ws = static_cast<char *>(workspace);
+  hipError_t e = w.split ? bevk::launch_f32_split_weight(static_cast<const float *>(weight), channels_out,
+                                                         channels, taps, false, ws, st)
+                         : bevk::launch_dcn_pack_weight(dtype, weight, channels_out, channels, taps, ws, st);
+  if (e == hipSuccess)
+    e = nhwc_product(dtype, g, channels_out, w, ws, data_im, data_offset,
+                     y ? bevk::kGeoY : bevk::kGeoMask, data_mask, bias, false, out, st);
+  return hip_status(e, fn);
+}
+
+int bevk_dcn_layer_nhwc(int dtype, const void *data_im, const void *w_off, const void *b_off,
+                        int b_off_dtype, const void *weight, const void *bias, int batch_size,
+                        int channels, int height_im, int width_im, int height_col, int width_col,
+                        int channels_out, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                        int stride_h, int stride_w, int dilation_h, int dilation_w, int act_relu,
+                        void *workspace, int64_t workspace_bytes, float *y, void *out, void *stream) {
+  const char *fn = "dcn_layer_nhwc";
+  g_last_error.clear();
+  const bevk::DcnGeom g =
+      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
+                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w, 1);
+  if (int rc = check_geom(fn, g)) return rc;
+  NhwcWs w;
+  if (!nhwc_ws(dtype, g, channels_out, true, &w))
+    return fail(BEVK_ERR_UNSUPPORTED, "%s: shape not taken", fn);
+  if (workspace_bytes < w.total) return fail(BEVK_ERR_INVALID, "%s: workspace too small", fn);
+  if (b_off != nullptr && (b_off_dtype < BEVK_F32 || b_off_dtype > BEVK_BF16 ||
+                           (dtype == BEVK_F32 && b_off_dtype != BEVK_F32)))
+    return fail(BEVK_ERR_UNSUPPORTED, "%s: b_off must be float32 or a 16-bit layer's type", fn);
+  if (!data_im || !w_off || !weight || !workspace || !y || !out)
+    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
+  const hipStream_t st = (hipStream_t)stream;
+  const int taps = kernel_h * kernel_w, n3 = 3 * taps;
+  char *ws = static_cast<char *>(workspace);
+  void *packed_off = ws + w.w_off;
+  const float *bo = static_cast<const float *>(b_off);
+  hipError_t e;
+  if (dtype == BEVK_F32) {
+    e = bevk::launch_dcn_pack_weight(dtype, w_off, n3, channels, taps, packed_off, st);
+    if (e == hipSuccess)
+      e = w.split ? bevk::launch_f32_split_weight(static_cast<const float *>(weight), channels_out,
+                                                  channels, taps, false, ws, st)
+                  : bevk::launch_dcn_pack_weight(dtype, weight, channels_out, channels, taps, ws, st);
+  } else {
+    float *b32 = reinterpret_cast<float *>(ws + w.b_off);
+    e = bevk::launch_dcn_prep16(dtype, weight, channels_out, w_off, n3, channels, taps, b_off,
+                                b_off_dtype, ws, packed_off, b32, st);
+    if (b_off != nullptr) bo = b32;
+  }
+  if (e != hipSuccess) return hip_status(e, fn);
+  if (w.parts == 0 && bevk::dcn_mega_supported(dtype, g, channels_out, out))
+    return hip_status(bevk::launch_dcn_mega(dtype, g, channels_out, data_im, packed_off, bo, ws, bias,
+                                            act_relu != 0, y, out, st),
+                      fn);
+  e = bevk::launch_dcn_fused_nhwc(dtype, g, n3, data_im, nullptr, bevk::kGeoRegular, nullptr, packed_off,
+                                  bo, y, st);
+  if (e == hipSuccess)
+    e = nhwc_product(dtype, g, channels_out, w, ws, data_im, y, bevk::kGeoYF32, nullptr, bias,
+                     act_relu != 0, out, st);
+  return hip_status(e, fn);
+}
+
 int bevk_msda_forward(int dtype, const void *value, const int64_t *spatial_shapes,
                       const int64_t *level_start_index, const void *sampling_loc,
                       const void *attn_weight, int batch, int spatial_size, int num_heads,

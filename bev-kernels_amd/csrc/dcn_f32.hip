@@ -65,6 +65,7 @@ struct Params {
   const float *addend;        // kTConv: added to the sum before the rounding
   void *out;
   int out_kind;               // 0 fp32, 1 fp16, 2 bf16 (16 bits: kTConv only)
+  int plane;                  // > 0: out is [B, Cout, plane] with m = (b, position), fp32
   int relu;
   int C, H, W, Ho, Wo, Cout, kw, ph, pw, sh, sw, dh, dw, M, taps;
   int nb_total, kb_total;     // 16-column blocks, 32-k blocks
@@ -142,7 +143,11 @@ __device__ __forceinline__ uint32_t tconv_offset(const Params &p, int m, int t) 
 
 // One output value: bias, addend, ReLU and the rounding of 16-bit outputs.
 __device__ __forceinline__ void emit(const Params &p, int m, int n, float v, float bias) {
-  const int64_t at = (int64_t)m * p.Cout + n;
+  int64_t at = (int64_t)m * p.Cout + n;
+  if (p.plane > 0) {
+    const int b = m / p.plane;
+    at = ((int64_t)b * p.Cout + n) * p.plane + (m - b * p.plane);
+  }
   v += bias;
   if (p.addend != nullptr) v = p.addend[at] + v;
   if (p.relu) v = v < 0.f ? 0.f : v;  // NaN stays NaN, as torch.relu
@@ -461,6 +466,34 @@ __global__ void __launch_bounds__(kThreads) f32_gemm_kernel(const Params p) {
     return;
   }
   const int wn = wave % WN, wm = wave / WN;
+  if (p.plane > 0 && (p.plane & 1) == 0) {
+    // NCHW: a lane's four rows are consecutive positions of its channel's plane
+    float *outf = static_cast<float *>(p.out);
+    const bool quad = (p.plane & 3) == 0;
+#pragma unroll
+    for (int rb = 0; rb < R; ++rb) {
+      const int row = (wm * R + rb) * 16 + 4 * (lane >> 4);
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const int m = m0 + row + 2 * hf;
+        if (row >= rows || m >= p.M || (quad && hf)) continue;
+        const int b = m / p.plane;
+        const int64_t at = (int64_t)b * p.Cout * p.plane + (m - b * p.plane);
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+          const int n = n0 + wn * 32 + cb * 16 + (lane & 15);
+          if (n >= p.Cout) continue;
+          const float bv = p.bias != nullptr ? p.bias[n] : 0.f;
+          const floatx4 v = acc[rb][cb] + floatx4{bv, bv, bv, bv};
+          typedef float floatx2 __attribute__((ext_vector_type(2)));
+          float *d = outf + at + (int64_t)n * p.plane;
+          if (quad) *reinterpret_cast<floatx4 *>(d) = v;
+          else *reinterpret_cast<floatx2 *>(d) = hf ? floatx2{v[2], v[3]} : floatx2{v[0], v[1]};
+        }
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int cb = 0; cb < 2; ++cb) {
     const int n = n0 + wn * 32 + cb * 16 + (lane & 15);
@@ -509,13 +542,14 @@ __device__ __forceinline__ bool store_split(char *d, const float (&v)[8]) {
 // A workgroup stages a 16 x 32 (n x c, or c x Cout) group of all taps through LDS, where each
 // source row's span is contiguous.
 // ---------------------------------------------------------------------------------------
+constexpr int kSplitLds = 16 * (32 * kMaxTaps + 1);  // floats; 32 x (16 * 9 + 1) is fewer + 16
 template <bool TRANS>
-__global__ void __launch_bounds__(256) split_weight_kernel(const float *__restrict__ w, char *packed,
-                                                           uint32_t *__restrict__ flags, int cout,
-                                                           int C, int T, int kb_total) {
+__device__ __forceinline__ void split_weight_block(const float *__restrict__ w, char *packed,
+                                                   uint32_t *__restrict__ flags, int cout, int C, int T,
+                                                   int kb_total, int bx, int by, float *s) {
   constexpr int RO = TRANS ? 32 : 16, CO = TRANS ? 16 : 32;  // source rows (Cout), channels
-  __shared__ float s[RO * (CO * kMaxTaps + 1)];
-  const int r0 = (int)blockIdx.x * RO, c0 = (int)blockIdx.y * CO;
+  static_assert(RO * (CO * kMaxTaps + 1) <= kSplitLds + 16, "LDS of a block");
+  const int r0 = bx * RO, c0 = by * CO;
   const int span = CO * T, pitch = span + 1;
   const int vspan = span / 4;  // CO is a multiple of 16
   const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0;
@@ -533,8 +567,8 @@ __global__ void __launch_bounds__(256) split_weight_kernel(const float *__restri
   __syncthreads();
   const int lane = threadIdx.x & 63;
   for (int t = threadIdx.x >> 6; t < T; t += 4) {  // a wave takes whole blocks (one per tap)
-    const int64_t blk = TRANS ? (int64_t)((t * C + c0) >> 4) * kb_total + (int)blockIdx.x
-                              : (int64_t)blockIdx.x * kb_total + ((t * C + c0) >> 5);
+    const int64_t blk = TRANS ? (int64_t)((t * C + c0) >> 4) * kb_total + bx
+                              : (int64_t)bx * kb_total + ((t * C + c0) >> 5);
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -544,6 +578,89 @@ __global__ void __launch_bounds__(256) split_weight_kernel(const float *__restri
     const bool bad = store_split(packed + blk * kBlkBytes + lane * 16, v);
     const bool any = __any(bad);
     if (lane == 0) flags[blk] = any ? 1u : 0u;
+  }
+}
+template <bool TRANS>
+__global__ void __launch_bounds__(256) split_weight_kernel(const float *__restrict__ w, char *packed,
+                                                           uint32_t *__restrict__ flags, int cout,
+                                                           int C, int T, int kb_total) {
+  __shared__ float s[kSplitLds + 16];
+  split_weight_block<TRANS>(w, packed, flags, cout, C, T, kb_total, (int)blockIdx.x, (int)blockIdx.y, s);
+}
+
+// Everything the NCHW layer's forward needs before its product, in one launch (five short ones
+// cost more than a small layer itself: a call with 64 channels of 32 x 32 took 70 us with seven
+// launches and takes 28 with three): the input,
+// offsets and mask as NHWC copies (64 x 64 tiles through LDS), the split weight, and the cleared
+// output where K runs in two parts. Workgroups are dealt to the jobs in that order.
+struct PrepJob {
+  const float *src;
+  float *dst;
+  int rows, cols, tr, tc, first;  // [batch][rows][cols] -> [batch][cols][rows], tiles, first block
+};
+struct PrepParams {
+  PrepJob t[3];
+  const float *w;
+  char *packed;
+  uint32_t *flags;
+  int cout, C, T, kb_total, nbo, first_w, first_clear, nblocks;
+  float *clear;
+  int64_t clear4;
+};
+__global__ void __launch_bounds__(256) f32_prep_kernel(const PrepParams p) {
+  __shared__ float s[kSplitLds + 16];
+  const int blk = (int)blockIdx.x;
+  if (blk >= p.first_clear) {
+    const int64_t step = (int64_t)(p.nblocks - p.first_clear) * 256;
+    for (int64_t i = (int64_t)(blk - p.first_clear) * 256 + threadIdx.x; i < p.clear4; i += step)
+      reinterpret_cast<floatx4 *>(p.clear)[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    return;
+  }
+  if (blk >= p.first_w) {
+    const int i = blk - p.first_w;
+    split_weight_block<false>(p.w, p.packed, p.flags, p.cout, p.C, p.T, p.kb_total, i % p.nbo, i / p.nbo, s);
+    return;
+  }
+  const PrepJob &j = blk >= p.t[2].first ? p.t[2] : blk >= p.t[1].first ? p.t[1] : p.t[0];
+  const int R = j.rows, C = j.cols;
+  int i = blk - j.first;
+  const int tc = i % j.tc;
+  i /= j.tc;
+  const int r0 = (i % j.tr) * 64, c0 = tc * 64;
+  const float *src = j.src + (int64_t)(i / j.tr) * R * C;
+  float *dst = j.dst + (int64_t)(i / j.tr) * R * C;
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  const bool vin = (C & 3) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+  const bool vout = (R & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int r = r0 + ty + 16 * q, c = c0 + 4 * tx;
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    if (vin && r < R && c < C) {
+      v = *reinterpret_cast<const floatx4 *>(src + (int64_t)r * C + c);
+    } else if (r < R) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < C) v[e] = src[(int64_t)r * C + c + e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[(ty + 16 * q) * 65 + 4 * tx + e] = v[e];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c = c0 + ty + 16 * q, r = r0 + 4 * tx;
+    floatx4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = s[(4 * tx + e) * 65 + ty + 16 * q];
+    if (c >= C) continue;
+    if (vout && r < R) {
+      *reinterpret_cast<floatx4 *>(dst + (int64_t)c * R + r) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (r + e < R) dst[(int64_t)c * R + r + e] = v[e];
+    }
   }
 }
 
@@ -584,7 +701,7 @@ __global__ void __launch_bounds__(256) clear_f32x4(float *__restrict__ p, int64_
 struct Plan {
   int nrb, kparts, mch, bn;
 };
-Plan plan(const Params &p, int bn_max, bool rows_mode, bool can_split) {
+Plan plan(const Params &p, int bn_max, bool rows_mode, bool can_split, bool nchw) {
   const int cus = std::max(1, device_cus());
   Plan best{0, 1, 0, bn_max};
   double best_t = 0;
@@ -602,6 +719,7 @@ Plan plan(const Params &p, int bn_max, bool rows_mode, bool can_split) {
                        : steps * (std::max(38.0 * kb, mm) + 250.0) + 6000.0;
         t *= (double)rounds;
         if (kparts == 2) t += 8000.0 + (double)p.M * p.Cout * 8.0 / 1600.0;  // clear and add
+        if (kparts == 2 && nchw) t += 8000.0 + (double)p.M * p.Cout * 8.0 / 1600.0;  // layout change
         if (best.nrb == 0 || t < best_t) {
           best_t = t;
           best = Plan{nrb, kparts, (int)mch, bn};
@@ -615,22 +733,29 @@ void launch_one(const Params &p, hipStream_t stream) {
   hipLaunchKernelGGL((f32_gemm_kernel<NRB, WN, GEO>), dim3(8 * p.per_xcd), dim3(kThreads), 0, stream, p);
 }
 
+// Fills in the tiling; returns the tile height and width. nchw: the caller changes the layout of
+// a two-part output afterwards.
 template <int GEO>
-hipError_t launch_geo(Params p, hipStream_t stream) {
+Plan make_plan(Params &p, bool nchw) {
   p.rb_total = (p.M + 15) / 16;
-  const int64_t n_out = (int64_t)p.M * p.Cout;
-  const bool can_split = deform(GEO) && !p.relu && p.kb_total >= 16 && n_out % 4 == 0 &&
+  const bool can_split = deform(GEO) && !p.relu && p.kb_total >= 16 && (int64_t)p.M * p.Cout % 4 == 0 &&
                          reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
-  const Plan pl = plan(p, p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64), !deform(GEO), can_split);
-  const int bn = pl.bn;
-  p.nt = (p.Cout + bn - 1) / bn;
+  const Plan pl = plan(p, p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64), !deform(GEO), can_split, nchw);
+  p.nt = (p.Cout + pl.bn - 1) / pl.bn;
   p.mch = pl.mch;
   p.kparts = pl.kparts;
   p.ksteps = (p.kb_total + pl.kparts - 1) / pl.kparts;
+  return pl;
+}
+
+template <int GEO>
+hipError_t launch_geo(Params p, const Plan &pl, bool cleared, hipStream_t stream) {
+  const int bn = pl.bn;
+  const int64_t n_out = (int64_t)p.M * p.Cout;
   const int64_t wgs = (int64_t)p.mch * p.nt * p.kparts;
   if (wgs > (1 << 28)) return hipErrorInvalidValue;
   p.per_xcd = (int)((wgs + 7) / 8);
-  if (p.kparts == 2) {
+  if (p.kparts == 2 && !cleared) {
     const int64_t n4 = n_out / 4;
     hipLaunchKernelGGL(clear_f32x4, dim3((unsigned)std::min<int64_t>((n4 + 255) / 256, 4096)),
                        dim3(256), 0, stream, static_cast<float *>(p.out), n4);
@@ -683,9 +808,9 @@ hipError_t launch_f32_split_weight(const float *w, int cout, int C, int T, bool 
   return hipGetLastError();
 }
 
-hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, const void *x,
-                            const void *off, int geo, const void *msk, const void *w_split,
-                            const float *bias, float *out, hipStream_t stream, bool relu) {
+namespace {
+Params make_params(const DcnGeom *g, int channels_out, int M, int K, const void *x, const void *off,
+                   const void *msk, const void *w_split, const float *bias, float *out, bool relu) {
   Params p{};
   p.x = x; p.off = off; p.msk = msk; p.w = w_split; p.bias = bias; p.out = out;
   p.relu = relu ? 1 : 0;
@@ -705,9 +830,108 @@ hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, co
   }
   p.w_bytes = (uint32_t)((int64_t)p.nb_total * p.kb_total * kBlkBytes);
   p.flags = reinterpret_cast<const uint32_t *>(static_cast<const char *>(w_split) + p.w_bytes);
-  if (g == nullptr) return launch_geo<kRows>(p, stream);
-  if (geo == kGeoMask) return launch_geo<kGeoMask>(p, stream);
-  return launch_geo<kGeoYF32>(p, stream);  // fp32 y: kGeoY and kGeoYF32 (no bias) are the same
+  return p;
+}
+}  // namespace
+
+hipError_t launch_f32_split(const DcnGeom *g, int channels_out, int M, int K, const void *x,
+                            const void *off, int geo, const void *msk, const void *w_split,
+                            const float *bias, float *out, hipStream_t stream, bool relu) {
+  Params p = make_params(g, channels_out, M, K, x, off, msk, w_split, bias, out, relu);
+  if (g == nullptr) {
+    const Plan pl = make_plan<kRows>(p, false);
+    return launch_geo<kRows>(p, pl, false, stream);
+  }
+  const Plan pl = make_plan<kGeoMask>(p, false);
+  if (geo == kGeoMask) return launch_geo<kGeoMask>(p, pl, false, stream);
+  return launch_geo<kGeoYF32>(p, pl, false, stream);  // fp32 y: kGeoY and kGeoYF32 (no bias) are the same
+}
+
+// Workspace of the NCHW layer's forward, 256-byte pieces: NHWC input, offsets and mask, split
+// weight, then columns (deformable groups) or the NHWC output (room for a two-part product).
+namespace {
+struct LayerWs {
+  int64_t off, msk, w, last, total;
+};
+LayerWs layer_ws(const DcnGeom &g, int cout) {
+  auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+  const int64_t T = g.kernel_h * g.kernel_w, M = (int64_t)g.batch * g.height_col * g.width_col;
+  LayerWs l;
+  l.off = up((int64_t)g.batch * g.height * g.width * g.channels * 4);
+  l.msk = l.off + up(M * g.deformable_group * 2 * T * 4);
+  l.w = l.msk + up(M * g.deformable_group * T * 4);
+  l.last = l.w + up(f32_split_weight_bytes(cout, T * g.channels));
+  l.total = l.last + up(g.deformable_group > 1 ? M * T * g.channels * 4 : M * cout * 4);
+  return l;
+}
+}  // namespace
+
+int64_t dcn_layer_f32_workspace_bytes(const DcnGeom &g, int channels_out) {
+  return layer_ws(g, channels_out).total;
+}
+
+hipError_t launch_dcn_layer_f32(const DcnGeom &g, int cout, const float *x, const float *off,
+                                const float *msk, const float *weight, const float *bias,
+                                void *workspace, float *out, hipStream_t stream) {
+  const int T = g.kernel_h * g.kernel_w, dg = g.deformable_group, HoWo = g.height_col * g.width_col;
+  const int M = g.batch * HoWo, K = T * g.channels;
+  const LayerWs l = layer_ws(g, cout);
+  char *ws = static_cast<char *>(workspace);
+  float *xn = reinterpret_cast<float *>(ws), *on = reinterpret_cast<float *>(ws + l.off);
+  float *mn = reinterpret_cast<float *>(ws + l.msk), *last = reinterpret_cast<float *>(ws + l.last);
+  Params p = make_params(dg > 1 ? nullptr : &g, cout, M, K, dg > 1 ? last : xn, on, mn, ws + l.w, bias,
+                         out, false);
+  p.plane = HoWo;
+  // 16-byte stores of four positions need an aligned output
+  const bool nchw = reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  if (!nchw) p.plane = 0;
+  Plan pl = dg > 1 ? make_plan<kRows>(p, true) : make_plan<kGeoMask>(p, true);
+  const bool two = p.kparts == 2 || !nchw;  // NHWC output first
+  if (two && dg > 1) return hipErrorInvalidValue;  // checked by the caller: out is aligned
+  if (two) {
+    p.plane = 0;
+    p.out = last;
+  }
+  PrepParams q{};
+  int blocks = 0;
+  const float *src[3] = {x, off, msk};
+  float *dst[3] = {xn, on, mn};
+  const int rows[3] = {g.channels, dg * 2 * T, dg * T};
+  const int cols[3] = {g.height * g.width, HoWo, HoWo};
+  for (int i = 0; i < 3; ++i) {
+    PrepJob &j = q.t[i];
+    j.src = src[i]; j.dst = dst[i]; j.rows = rows[i]; j.cols = cols[i];
+    j.tr = (rows[i] + 63) / 64;
+    j.tc = (cols[i] + 63) / 64;
+    j.first = blocks;
+    const int64_t n = (int64_t)g.batch * j.tr * j.tc;
+    if (blocks + n > (1 << 30)) return hipErrorInvalidValue;
+    blocks += (int)n;
+  }
+  q.w = weight;
+  q.packed = ws + l.w;
+  q.flags = const_cast<uint32_t *>(p.flags);
+  q.cout = cout; q.C = g.channels; q.T = T; q.kb_total = p.kb_total;
+  q.nbo = p.nb_total;
+  q.first_w = blocks;
+  blocks += q.nbo * (g.channels / 32);
+  q.first_clear = blocks;
+  if (p.kparts == 2) {
+    q.clear = last;
+    q.clear4 = (int64_t)M * cout / 4;
+    blocks += (int)std::min<int64_t>((q.clear4 + 1023) / 1024, 2048);
+  }
+  q.nblocks = blocks;
+  hipLaunchKernelGGL(f32_prep_kernel, dim3(blocks), dim3(256), 0, stream, q);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (dg > 1) {
+    e = launch_im2col_nhwc(0, g, xn, on, false, mn, last, stream);
+    return e != hipSuccess ? e : launch_geo<kRows>(p, pl, false, stream);
+  }
+  e = launch_geo<kGeoMask>(p, pl, true, stream);
+  if (e != hipSuccess || !two) return e;
+  return launch_transpose(4, last, out, g.batch, HoWo, cout, stream);
 }
 
 hipError_t launch_f32_tconv(const DcnGeom &g, const float *y32, const void *w_split,
@@ -725,7 +949,8 @@ hipError_t launch_f32_tconv(const DcnGeom &g, const float *y32, const void *w_sp
   p.x_bytes = (uint32_t)((int64_t)g.batch * g.height_col * g.width_col * kBK * 4);
   p.w_bytes = (uint32_t)((int64_t)p.nb_total * p.kb_total * kBlkBytes);
   p.flags = reinterpret_cast<const uint32_t *>(static_cast<const char *>(w_split) + p.w_bytes);
-  return launch_geo<kTConv>(p, stream);
+  const Plan pl = make_plan<kTConv>(p, false);
+  return launch_geo<kTConv>(p, pl, false, stream);
 }
 
 hipError_t launch_f32_split_offset_weight(const float *w_off, int n3, int C, int T, void *packed,

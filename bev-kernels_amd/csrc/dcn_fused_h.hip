@@ -440,12 +440,10 @@ __global__ void __launch_bounds__(256) pack_weight_frag_tc_kernel(const uint16_t
 // loads), and the group's T K blocks (one per tap) are written from LDS as whole 16-byte
 // chunks. The per-element form reads 8 values 2 T bytes apart for every chunk (res5: 14 us).
 constexpr int kPackMaxT = 25;
-__global__ void __launch_bounds__(256) pack_weight_frag_lds_kernel(const uint16_t *__restrict__ w,
-                                                                   uint16_t *__restrict__ packed,
-                                                                   int cout, int C, int T,
-                                                                   int KB) {
-  __shared__ __attribute__((aligned(16))) uint16_t s[32 * (16 * kPackMaxT + 8)];
-  const int nb = (int)blockIdx.x, c0 = (int)blockIdx.y * 16;
+constexpr int kPackLds = 32 * (16 * kPackMaxT + 8);
+__device__ __forceinline__ void pack_frag_block(const uint16_t *__restrict__ w,
+                                                uint16_t *__restrict__ packed, int cout, int C,
+                                                int T, int KB, int nb, int c0, uint16_t *s) {
   const int pitch = 16 * T + 8;  // elements per LDS row (16-byte multiple)
   const int vrow = 2 * T;        // 16-byte vectors per row span (16 T elements)
   for (int i = threadIdx.x; i < 32 * vrow; i += 256) {
@@ -469,6 +467,44 @@ __global__ void __launch_bounds__(256) pack_weight_frag_lds_kernel(const uint16_
     for (int e = 0; e < 8; ++e) o.v[e] = s[r * pitch + (cl + e) * T + t];
     store_vec<uint16_t, 8>(packed + (((int64_t)nb * KB + kb) * 64 + l) * 8, o);
   }
+}
+__global__ void __launch_bounds__(256) pack_weight_frag_lds_kernel(const uint16_t *__restrict__ w,
+                                                                   uint16_t *__restrict__ packed,
+                                                                   int cout, int C, int T,
+                                                                   int KB) {
+  __shared__ __attribute__((aligned(16))) uint16_t s[kPackLds];
+  pack_frag_block(w, packed, cout, C, T, KB, (int)blockIdx.x, (int)blockIdx.y * 16, s);
+}
+
+// Both weights of a layer (main and offset conv, same C and T) and the offset conv's bias in fp32,
+// in one launch: the offset weight's few workgroups (27 rows: one block column) run beside the
+// main weight's instead of after them (512 x 512: two launches of 6 us and the bias cast 2 us;
+// 5.6 us together).
+struct Prep16 {
+  const uint16_t *w, *w2;
+  uint16_t *packed, *packed2;
+  const void *b_off;
+  float *b_out;
+  int b_dtype, n3, cout, C, T, KB, groups, blocks1;
+};
+__device__ __forceinline__ float as_f32(const void *p, int dtype, int i) {
+  return dtype == 0 ? static_cast<const float *>(p)[i]
+         : dtype == 1 ? (float)static_cast<const f16 *>(p)[i] : (float)static_cast<const bf16 *>(p)[i];
+}
+__global__ void __launch_bounds__(256) prep16_kernel(const Prep16 p) {
+  __shared__ __attribute__((aligned(16))) uint16_t s[kPackLds];
+  int b = (int)blockIdx.x;
+  if (b == 0 && p.b_off != nullptr && (int)threadIdx.x < p.n3)
+    p.b_out[threadIdx.x] = as_f32(p.b_off, p.b_dtype, threadIdx.x);
+  if (b < p.blocks1) {
+    pack_frag_block(p.w, p.packed, p.cout, p.C, p.T, p.KB, b / p.groups, b % p.groups * 16, s);
+  } else {
+    b -= p.blocks1;
+    pack_frag_block(p.w2, p.packed2, p.n3, p.C, p.T, p.KB, b / p.groups, b % p.groups * 16, s);
+  }
+}
+__global__ void __launch_bounds__(64) bias_f32_kernel(const void *b, int dtype, int n, float *out) {
+  if ((int)threadIdx.x < n) out[threadIdx.x] = as_f32(b, dtype, threadIdx.x);
 }
 
 // Weight [Cout][C][T] (or [Cout][T][C] with src_tc) -> [Cout][T][C] (fp32), one thread
@@ -814,6 +850,10 @@ struct PParams {
   int rounds;    // the grid is nblocks * rounds workgroups, one row chunk each: each
                  // half's blocks are cut into rounds * nblocks / halves balanced chunks of
                  // at most NRB blocks
+  // K in parts (few rows): chunks row chunks x halves x kparts workgroups, each over ksteps K
+  // steps, fp32 sums to part [kparts][M][Cout]
+  int chunks, kparts, ksteps, per_xcd;
+  float *part;
 };
 
 // B fragment of v_mfma_f32_16x16x32 read from the 32x32x16 fragment packing: lane l takes
@@ -832,10 +872,12 @@ __device__ __forceinline__ uint32_t b_frag_offset(int n, int kh, int lane, int n
 // which the whole workgroup stores afterwards as full 16-byte pieces of output rows.
 // Always NRB row blocks (compile-time, so the MFMA loop and the accumulators carry no
 // run-time conditions).
+// ks0: the first K step (parts of K); with a part, its fp32 sums go to part [M][Cout] instead.
 template <typename T, int NRB, int CD>
 __device__ __forceinline__ void dcn_p_consumer(const HParams &p, T (*As)[NRB * 16 * kPLDA],
                                                T *stage, int n0, int nk, int lane, int wave,
-                                               const int4v (&b0)[kPKH][4], bool b0_loaded) {
+                                               const int4v (&b0)[kPKH][4], bool b0_loaded,
+                                               int ks0, float *part, int m0, int nrows) {
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(p.w, p.w_bytes);
   uint32_t bo[kPKH][4];
 #pragma unroll
@@ -850,7 +892,7 @@ __device__ __forceinline__ void dcn_p_consumer(const HParams &p, T (*As)[NRB * 1
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb)
         br[kh][cb] = __builtin_amdgcn_raw_buffer_load_b128(
-            wr, bo[kh][cb], (uint32_t)ks * (uint32_t)(kPBK / 16) * 1024u, 0);
+            wr, bo[kh][cb], (uint32_t)(ks + ks0) * (uint32_t)(kPBK / 16) * 1024u, 0);
   };
   floatx4 acc[NRB][4];
 #pragma unroll
@@ -899,6 +941,21 @@ __device__ __forceinline__ void dcn_p_consumer(const HParams &p, T (*As)[NRB * 1
     if (ks + d < nk) step(ks + d, br[d]);
 
   // Epilogue: lane holds column 64 wave + 16 cb + (lane & 15), rows 4 (lane >> 4) + e.
+  if (part != nullptr) {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      const int n = n0 + wave * 64 + cb * 16 + (lane & 15);
+#pragma unroll
+      for (int rbi = 0; rbi < NRB; ++rbi)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = rbi * 16 + 4 * (lane >> 4) + e;
+          if (row < nrows && m0 + row < p.M && n < p.Cout)
+            part[(int64_t)(m0 + row) * p.Cout + n] = acc[rbi][cb][e];
+        }
+    }
+    return;
+  }
   const T *bias = static_cast<const T *>(p.bias);
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
@@ -998,9 +1055,11 @@ __device__ __forceinline__ void dcn_p_offset_consumer(const HParams &p,
 // (k+1) % PD into buffer (k+1) % 2. Every load is issued unconditionally (steps past the
 // end read out of range), so the compiler's wait counts stay exact and the gathers of the
 // next steps stay in flight. REG: plain convolution taps (one pixel per slot, no blend).
+// ks0: the first K step (parts of K).
 template <typename T, int NS, int NRB, bool REG, int PD>
 __device__ __forceinline__ void dcn_p_producer(const HParams &p, const TapGeo *geo,
-                                               T (*As)[NRB * 16 * kPLDA], int nk, int ptid) {
+                                               T (*As)[NRB * 16 * kPLDA], int nk, int ptid,
+                                               int ks0 = 0) {
   using V = Vec<T, 8>;
   constexpr int KV = kPBK / 8;
   constexpr int NQ = REG ? 1 : 4;
@@ -1025,8 +1084,8 @@ __device__ __forceinline__ void dcn_p_producer(const HParams &p, const TapGeo *g
     }
   };
   auto issue_gather = [&](int ks, V (&ra)[NS][NQ]) __attribute__((always_inline)) {
-    const int t = ks / spt, cs = ks - t * spt;
-    if (cs == 0) load_geo(t);
+    const int t = (ks + ks0) / spt, cs = ks + ks0 - t * spt;
+    if (cs == 0 || (ks0 != 0 && ks == 0)) load_geo(t);
     const uint32_t so = (uint32_t)(cs * kPBK * sizeof(T));
 #pragma unroll
     for (int i = 0; i < NS; ++i)
@@ -1037,7 +1096,7 @@ __device__ __forceinline__ void dcn_p_producer(const HParams &p, const TapGeo *g
   auto blend = [&](int ks, const V (&ra)[NS][NQ], int buf) __attribute__((always_inline)) {
     // Past the last step the gathered corners are zero (out-of-range offsets); the tap is
     // clamped so the weight read stays inside the table.
-    const int t = min(ks / spt, TT - 1);
+    const int t = min((ks + ks0) / spt, TT - 1);
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
       const int row = (ptid + i * kPProd) / KV;
@@ -1077,14 +1136,15 @@ __device__ __forceinline__ void dcn_p_producer(const HParams &p, const TapGeo *g
 // matrix cores (dcn_p_offset_consumer + plain-convolution producers), its fp32 output
 // with bias is kept in LDS (aliasing the A ring) and the deformable geometry is built from
 // it, as the reference's single-kernel forward does (fused_tl.py:565-688).
-template <typename T, int GEO, int NRB, bool MEGA>
+// KPARTS: a part of K per workgroup, fp32 sums to pp.part (reduced by kparts_total_kernel).
+template <typename T, int GEO, int NRB, bool MEGA, bool KPARTS>
 __global__ void __launch_bounds__(kPThreads) dcn_fused_p_kernel(const PParams pp) {
   using SH = PShape<NRB>;
   constexpr int kPRows = SH::kRows;
   const HParams &p = pp.h;
   __shared__ __attribute__((aligned(16))) TapGeo geo[kPRows * kMaxTaps];
   __shared__ __attribute__((aligned(16))) T As[2][kPRows * kPLDA];
-  __shared__ __attribute__((aligned(16))) T stage[kPRows * kPStage];  // the output tile
+  __shared__ __attribute__((aligned(16))) T stage[KPARTS ? 8 : kPRows * kPStage];  // the output tile
   static_assert(!MEGA || sizeof(As) >= sizeof(float) * kPRows * 3 * kMaxTaps,
                 "the offset-conv output must fit in the A ring");
 
@@ -1096,13 +1156,23 @@ __global__ void __launch_bounds__(kPThreads) dcn_fused_p_kernel(const PParams pp
   const int bpx = (int)(gridDim.x >> 3);               // workgroups per XCD
   const int xcd = (int)(blockIdx.x & 7);
   const int xph = 8 / pp.halves;                       // XCDs per half
-  const int half = xcd / xph;
-  const int nch = (int)gridDim.x / pp.halves;          // row chunks per half
-  const int j = (xcd - half * xph) * bpx + (int)(blockIdx.x >> 3);
+  int half = xcd / xph;
+  int nch = (int)gridDim.x / pp.halves;                // row chunks per half
+  int j = (xcd - half * xph) * bpx + (int)(blockIdx.x >> 3);
+  int kz = 0;
+  if constexpr (KPARTS) {  // XCD-contiguous (half, K part, chunk), chunks fastest
+    nch = pp.chunks;
+    const int L = xcd * pp.per_xcd + (int)(blockIdx.x >> 3);
+    if (L >= nch * pp.kparts * pp.halves) return;
+    j = L % nch;
+    kz = L / nch % pp.kparts;
+    half = L / nch / pp.kparts;
+  }
   const int n0 = half * kPCols;
   const int TT = p.taps;
   const uint32_t xoob = p.x_bytes;
-  const int nk = TT * (p.C / kPBK);
+  const int ks0 = KPARTS ? kz * pp.ksteps : 0;
+  const int nk = KPARTS ? min(pp.ksteps, TT * (p.C / kPBK) - ks0) : TT * (p.C / kPBK);
   float *ys = reinterpret_cast<float *>(&As[0][0]);
   const int rb0 = (int)((int64_t)pp.rb_total * j / nch);
   const int nrb = (int)((int64_t)pp.rb_total * (j + 1) / nch) - rb0;  // at most NRB
@@ -1165,11 +1235,14 @@ __global__ void __launch_bounds__(kPThreads) dcn_fused_p_kernel(const PParams pp
   // 67.8 us; the consumers raised instead, 70.2 us).
   if (wave >= 4) __builtin_amdgcn_s_setprio(2);
   if (wave < 4)
-    dcn_p_consumer<T, NRB, SH::kCD>(p, As, stage, n0, nk, lane, wave, b0, kB0Early);
+    dcn_p_consumer<T, NRB, SH::kCD>(
+        p, As, stage, n0, nk, lane, wave, b0, kB0Early, ks0,
+        KPARTS ? pp.part + (int64_t)kz * p.M * p.Cout : nullptr, m0, nrows);
   else if (wave - 4 < SH::kLastWaves)
-    dcn_p_producer<T, SH::kSPT, NRB, false, SH::kPD>(p, geo, As, nk, tid - kPProd);
+    dcn_p_producer<T, SH::kSPT, NRB, false, SH::kPD>(p, geo, As, nk, tid - kPProd, ks0);
   else if constexpr (SH::kLastWaves < 4)
-    dcn_p_producer<T, SH::kSPT - 1, NRB, false, SH::kPD>(p, geo, As, nk, tid - kPProd);
+    dcn_p_producer<T, SH::kSPT - 1, NRB, false, SH::kPD>(p, geo, As, nk, tid - kPProd, ks0);
+  if constexpr (KPARTS) return;
   // The output tile: full 16-byte pieces of the workgroup's rows (Cout % 8 == 0 and a
   // 16-byte aligned output, checked on the host: a piece is wholly inside or outside),
   // streaming stores (written once; the input rows stay in L2).
@@ -1504,19 +1577,112 @@ template <typename T, int GEO, bool MEGA>
 hipError_t launch_p_geo(const PParams &pp, int nrb, hipStream_t stream) {
   const dim3 g(pp.nblocks * pp.rounds), b(kPThreads);
   switch (nrb) {
-    case 2: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 2, MEGA>), g, b, 0, stream, pp); break;
-    case 3: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 3, MEGA>), g, b, 0, stream, pp); break;
-    case 4: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 4, MEGA>), g, b, 0, stream, pp); break;
-    case 5: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 5, MEGA>), g, b, 0, stream, pp); break;
+    case 2: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 2, MEGA, false>), g, b, 0, stream, pp); break;
+    case 3: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 3, MEGA, false>), g, b, 0, stream, pp); break;
+    case 4: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 4, MEGA, false>), g, b, 0, stream, pp); break;
+    case 5: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 5, MEGA, false>), g, b, 0, stream, pp); break;
     default: return hipErrorInvalidValue;  // 6-9 blocks run dcn_fused_s_kernel
   }
+  return hipGetLastError();
+}
+
+// out = round(sum of the K parts + bias), ReLU: 8 outputs per thread.
+template <typename T>
+__global__ void __launch_bounds__(256) kparts_total_kernel(const float *__restrict__ part, int kparts,
+                                                           int64_t n8, int cout,
+                                                           const T *__restrict__ bias, int relu,
+                                                           T *__restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  float s[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) s[e] = 0.f;
+#pragma unroll 4
+  for (int q = 0; q < kparts; ++q) {
+    const float *src = part + ((int64_t)q * n8 + i) * 8;
+    const Vec<float, 4> a = load_vec<float, 4>(src), b = load_vec<float, 4>(src + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[e] += a.v[e];
+      s[4 + e] += b.v[e];
+    }
+  }
+  const int n = (int)(i * 8 % cout);
+  Vec<T, 8> o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float v = s[e] + (bias != nullptr ? (float)bias[n + e] : 0.f);
+    if (relu) v = v < 0.f ? 0.f : v;  // NaN stays NaN, as torch.relu
+    o.v[e] = static_cast<T>(v);
+  }
+  store_vec<T, 8>(out + i * 8, o);
+}
+
+// Few rows leave the persistent kernel one or two row blocks per CU for the whole K (its time
+// is then K steps x their latency) or CUs without work. K in parts over more workgroups shortens
+// that chain for the price of the parts' fp32 sums. A K step of NRB row blocks takes about
+// 0.1 + 0.155 NRB us (measured at 2, 5 and 9), a launch 6 us, the sums 8 bytes each at 4.5 TB/s
+// and their reduction 3 us; parts run where that is under 0.9 of the whole-K time: 512 channels
+// of 29 x 50, one image, 512 outputs: 35 us whole (2 row blocks x 72 steps), 25 us (20.5 + 4.3) in 4
+// parts; 256 channels of 58 x 100, one image: whole.
+struct KConfig {
+  int nrb = 0, kparts = 1, chunks = 0;
+};
+KConfig kparts_for(const HParams &p, const PConfig &c) {
+  KConfig best;
+  if (c.nblocks == 0 || c.rounds != 1) return best;
+  auto step_us = [](int nrb) { return 0.1 + 0.155 * nrb; };
+  const int steps = p.taps * (p.C / 64), rb = (p.M + 15) / 16;
+  double best_t = 0.9 * (steps * step_us(c.nrb) + 6.0);
+  for (int nrb = 2; nrb <= 5; ++nrb) {
+    const int chunks = (rb + nrb - 1) / nrb;
+    const int kparts = std::min(steps / 2, c.nblocks / (chunks * c.halves));
+    if (kparts < 2) continue;
+    const int per = (steps + kparts - 1) / kparts, used = (steps + per - 1) / per;
+    const double t = per * step_us(nrb) + 9.0 + (double)used * p.M * p.Cout * 8e-6 / 4.5;
+    if (t < best_t) {
+      best_t = t;
+      best.nrb = nrb;
+      best.kparts = used;
+      best.chunks = chunks;
+    }
+  }
+  return best;
+}
+
+template <typename T, int GEO>
+hipError_t launch_kparts(const HParams &h, const PConfig &c, const KConfig &k, float *part,
+                         hipStream_t stream) {
+  PParams pp{};
+  pp.h = h;
+  pp.rb_total = (h.M + 15) / 16;
+  pp.halves = c.halves;
+  pp.chunks = k.chunks;
+  pp.kparts = k.kparts;
+  const int steps = h.taps * (h.C / kPBK);
+  pp.ksteps = (steps + k.kparts - 1) / k.kparts;
+  pp.per_xcd = (k.chunks * k.kparts * c.halves + 7) / 8;
+  pp.part = part;
+  const dim3 g(8 * pp.per_xcd), b(kPThreads);
+  switch (k.nrb) {
+    case 2: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 2, false, true>), g, b, 0, stream, pp); break;
+    case 3: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 3, false, true>), g, b, 0, stream, pp); break;
+    case 4: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 4, false, true>), g, b, 0, stream, pp); break;
+    default: hipLaunchKernelGGL((dcn_fused_p_kernel<T, GEO, 5, false, true>), g, b, 0, stream, pp); break;
+  }
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int64_t n8 = (int64_t)h.M * h.Cout / 8;  // Cout % 8 == 0 (p_config_for)
+  hipLaunchKernelGGL((kparts_total_kernel<T>), dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, stream,
+                     part, k.kparts, n8, h.Cout, static_cast<const T *>(h.bias), h.relu,
+                     static_cast<T *>(h.out));
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_p(const HParams &h, int geo, const PConfig &c, bool mega,
                     hipStream_t stream) {
-  PParams pp;
+  PParams pp{};
   pp.h = h;
   pp.rb_total = (h.M + 15) / 16;
   pp.nblocks = c.nblocks;
@@ -1539,8 +1705,14 @@ hipError_t launch_p(const HParams &h, int geo, const PConfig &c, bool mega,
 }
 
 template <typename T>
-hipError_t launch_t(const HParams &p, int geo, hipStream_t stream) {
+hipError_t launch_t(const HParams &p, int geo, float *part, hipStream_t stream) {
   const PConfig c = p_config_for(p, geo);
+  if (c.nblocks && part != nullptr && (geo == kGeoMask || geo == kGeoYF32)) {
+    const KConfig k = kparts_for(p, c);
+    if (k.kparts > 1)
+      return geo == kGeoMask ? launch_kparts<T, kGeoMask>(p, c, k, part, stream)
+                             : launch_kparts<T, kGeoYF32>(p, c, k, part, stream);
+  }
   if (c.nblocks) return launch_p<T>(p, geo, c, false, stream);
   return p.C % 64 == 0 ? launch_tt<T, true>(p, geo, stream) : launch_tt<T, false>(p, geo, stream);
 }
@@ -1587,6 +1759,33 @@ hipError_t launch_dcn_pack_weight(int dtype, const void *weight, int cout, int C
   return hipGetLastError();
 }
 
+hipError_t launch_dcn_prep16(int dtype, const void *weight, int cout, const void *w_off, int n3, int C,
+                             int T, const void *b_off, int b_dtype, void *packed, void *packed_off,
+                             float *b_out, hipStream_t stream) {
+  const bool aligned = ((reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(w_off) |
+                         reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(packed_off)) &
+                        15) == 0;
+  if (aligned && C % 16 == 0 && T <= kPackMaxT && n3 <= 256) {
+    Prep16 p;
+    p.w = static_cast<const uint16_t *>(weight); p.w2 = static_cast<const uint16_t *>(w_off);
+    p.packed = static_cast<uint16_t *>(packed); p.packed2 = static_cast<uint16_t *>(packed_off);
+    p.b_off = b_off; p.b_out = b_out; p.b_dtype = b_dtype;
+    p.n3 = n3; p.cout = cout; p.C = C; p.T = T; p.KB = (C * T + 15) / 16;
+    p.groups = C / 16;
+    p.blocks1 = (cout + 31) / 32 * p.groups;
+    const int blocks = p.blocks1 + (n3 + 31) / 32 * p.groups;
+    hipLaunchKernelGGL(prep16_kernel, dim3(blocks), dim3(256), 0, stream, p);
+    return hipGetLastError();
+  }
+  hipError_t e = launch_dcn_pack_weight(dtype, weight, cout, C, T, packed, stream);
+  if (e == hipSuccess) e = launch_dcn_pack_weight(dtype, w_off, n3, C, T, packed_off, stream);
+  if (e == hipSuccess && b_off != nullptr) {
+    hipLaunchKernelGGL(bias_f32_kernel, dim3(1), dim3(64), 0, stream, b_off, b_dtype, n3, b_out);
+    e = hipGetLastError();
+  }
+  return e;
+}
+
 bool dcn_fused_h_supported(const DcnGeom &g) { return g.kernel_h * g.kernel_w <= kMaxTaps; }
 
 namespace {
@@ -1614,14 +1813,22 @@ HParams make_hparams(int dtype, const DcnGeom &g, int channels_out, const void *
 hipError_t launch_dcn_fused_h(int dtype, const DcnGeom &g, int channels_out, const void *x,
                               const void *off, int geo, const void *msk,
                               const void *w_packed, const void *bias, void *out,
-                              hipStream_t stream, const float *y_bias, bool relu) {
+                              hipStream_t stream, const float *y_bias, bool relu, float *part) {
   const HParams p =
       make_hparams(dtype, g, channels_out, x, off, msk, w_packed, bias, out, y_bias, relu);
   switch (dtype) {
-    case 1: return launch_t<f16>(p, geo, stream);
-    case 2: return launch_t<bf16>(p, geo, stream);
+    case 1: return launch_t<f16>(p, geo, part, stream);
+    case 2: return launch_t<bf16>(p, geo, part, stream);
     default: return hipErrorInvalidValue;
   }
+}
+
+int64_t dcn_fused_h_parts_bytes(int dtype, const DcnGeom &g, int channels_out) {
+  if ((dtype != 1 && dtype != 2) || !dcn_fused_h_supported(g)) return 0;
+  const HParams p = make_hparams(dtype, g, channels_out, nullptr, nullptr, nullptr, nullptr,
+                                 nullptr, nullptr, nullptr, false);
+  const KConfig k = kparts_for(p, p_config_for(p, kGeoMask));
+  return k.kparts > 1 ? (int64_t)k.kparts * p.M * p.Cout * 4 : 0;
 }
 
 // The one-launch form runs where Cout fits one 256-column half. With two halves every

@@ -1,4 +1,5 @@
-"""Packed main weight for the fused NHWC kernel.
+"""Weights and gradients of the layers: packing for the fused NHWC kernel, and the gradient
+products of the backward passes.
 
 The fused kernel reads the weight in the layout dcn_pack_weight produces (MFMA-fragment
 blocks for fp16 / bf16, [Cout][kh][kw][C] for fp32). The weight is packed on every call,
@@ -20,32 +21,6 @@ def _ext():
 def pack_weight(weight: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """Pack weight [Cout, C, kh, kw] converted to `dtype`."""
     return _ext().dcn_pack_weight(weight.detach().to(dtype).contiguous())
-
-
-def split_applies(x, channels, channels_out, taps):
-    """fp32 shapes of the split kernel: whole 32-channel K steps, at most 9 taps, and buffers
-    under 2 GiB."""
-    lim = 2 ** 31 - 256
-    return (x.dtype == torch.float32 and channels % 32 == 0 and taps <= 9
-            and 4 * x.numel() <= lim
-            and 6.5 * (channels_out + 15) * channels * taps <= lim)
-
-
-def fused_conv(x, offset, mask, weight, bias, sizes, out, relu=False):
-    """The fused deformable forward into out, with the weight packed for the kernel that takes
-    the shape. sizes = (B, C, H, W, Ho, Wo, Cout, kh, kw, ph, pw, sh, sw, dh, dw); offset 2T
-    with a mask, or the 3T y (then mask is ignored). relu: fp32 shapes of the split kernel only
-    (returns whether it was applied).
-
-    fp32: C % 32 == 0 runs on the bf16 matrix cores (dcn_fused_fwd_nhwc_f32), other channel
-    counts on the fp32 ones."""
-    ext = _ext()
-    if split_applies(x, sizes[1], sizes[6], sizes[7] * sizes[8]):
-        split = ext.dcn_split_weight(weight.detach().to(x.dtype).contiguous())
-        ext.dcn_fused_fwd_nhwc_f32(x, offset, mask, split, bias, *sizes, out, relu)
-        return relu
-    ext.dcn_fused_fwd_nhwc(x, offset, mask, pack_weight(weight, x.dtype), bias, *sizes, out)
-    return False
 
 
 def columns_grad_f32(dout, weight):

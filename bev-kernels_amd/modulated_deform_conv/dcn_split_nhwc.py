@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from ._packing import fused_conv, pack_weight, split_applies, weight_grad
+from ._packing import pack_weight, weight_grad
 
 
 def out_size(H, pad, dil, k, stride):
@@ -98,16 +98,16 @@ def _fused_forward(x_nhwc, offset, mask, weight, bias, stride, padding, dilation
     dt = x_nhwc.dtype
     w, b = _fold_bn(weight, bias, bn_scale, bn_shift)
     b = b.to(dt).contiguous() if b is not None else None
-    out = torch.empty(B, Ho, Wo, Cout, device=x_nhwc.device, dtype=dt)
     vec = 16 // x_nhwc.element_size()
     if Cin % vec == 0 and dt != torch.float64:
-        fused_conv(x_nhwc.contiguous(), offset.contiguous(),
-                   (mask if mask is not None else offset).contiguous(), w, b,
-                   (B, Cin, H, W, Ho, Wo, Cout, kH, kW, padding, padding, stride, stride,
-                    dilation, dilation), out)
+        out = _ext().dcn_conv_nhwc(
+            x_nhwc.contiguous(), offset.contiguous(),
+            (mask if mask is not None else offset).contiguous(), w.detach().to(dt).contiguous(), b,
+            B, Cin, H, W, Ho, Wo, Cout, kH, kW, padding, padding, stride, stride, dilation, dilation)
     else:
         col = gather_cols_nhwc(x_nhwc, offset, mask, kH, kW, stride, padding, dilation)
         w_flat = w.permute(0, 2, 3, 1).to(dt).contiguous().view(Cout, kH * kW * Cin).t()
+        out = torch.empty(B, Ho, Wo, Cout, device=x_nhwc.device, dtype=dt)
         torch.mm(col, w_flat, out=out.view(-1, Cout))
         if b is not None:
             out += b.view(1, 1, 1, -1)
@@ -160,20 +160,20 @@ def mega_forward(x_nhwc, w_off, b_off, weight, bias=None, stride=1, padding=1, d
     Cout, _, kH, kW = weight.shape
     Ho, Wo = out_size(H, ph, dh, kH, sh), out_size(W, pw, dw, kW, sw)
     dt = x_nhwc.dtype
+    x = x_nhwc.contiguous()
+    bias = bias.to(dt).contiguous() if bias is not None else None
+    w_off, weight = (t.detach().to(dt).contiguous() for t in (w_off, weight))
+    if b_off is not None:
+        b_off = (b_off if b_off.dtype == dt else b_off.float()).contiguous()
+    sizes = (B, Cin, H, W, Ho, Wo, Cout, kH, kW, ph, pw, sh, sw, dh, dw)
+    done = _ext().dcn_layer_nhwc(x, w_off, b_off, weight, bias, *sizes, act_relu=act_relu)
+    if done is not None:
+        return done
     out = torch.empty(B, Ho, Wo, Cout, device=x_nhwc.device, dtype=dt)
-    if split_applies(x_nhwc, Cin, Cout, kH * kW):
-        # two launches either way in fp32: the offset conv, then the split kernel reading y
-        x = x_nhwc.contiguous()
-        y = offset_conv_y(x, w_off, b_off, stride, padding, dilation)
-        fused_conv(x, y, None, weight, bias.to(dt).contiguous() if bias is not None else None,
-                   (B, Cin, H, W, Ho, Wo, Cout, kH, kW, ph, pw, sh, sw, dh, dw), out, act_relu)
-        return out, y
     y = torch.empty(B, Ho, Wo, 3 * kH * kW, device=x_nhwc.device, dtype=torch.float32)
     _ext().dcn_mega_fwd_nhwc(
-        x_nhwc.contiguous(), pack_weight(w_off, dt),
-        b_off.float().contiguous() if b_off is not None else None, pack_weight(weight, dt),
-        bias.to(dt).contiguous() if bias is not None else None, B, Cin, H, W, Ho, Wo, Cout,
-        kH, kW, ph, pw, sh, sw, dh, dw, act_relu, y, out)
+        x, pack_weight(w_off, dt), b_off.float() if b_off is not None else None,
+        pack_weight(weight, dt), bias, *sizes, act_relu, y, out)
     return out, y
 
 

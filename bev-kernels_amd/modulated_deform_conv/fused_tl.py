@@ -22,7 +22,6 @@ import torch
 import torch.nn.functional as F
 
 from . import dcn_split_nhwc as _split
-from ._packing import fused_conv
 
 
 def out_size(H, pad, dil, k, stride):
@@ -136,15 +135,16 @@ def fused_dcn_forward_nhwc(data_im, offset, mask, weight, bias=None, stride=1, p
     Ho = out_size(H, ph, dh, kH, sh)
     Wo = out_size(W, pw, dw, kW, sw)
     dt = data_im.dtype
-    out = torch.empty(B, Ho, Wo, Cout, device=data_im.device, dtype=dt)
     b = bias.to(dt).contiguous() if bias is not None else None
     vec = 16 // data_im.element_size()
     if Cin % vec == 0 and dt != torch.float64:
-        fused_conv(data_im.contiguous(), offset.contiguous(), mask.contiguous(), weight, b,
-                   (B, Cin, H, W, Ho, Wo, Cout, kH, kW, ph, pw, sh, sw, dh, dw), out)
+        out = _ext().dcn_conv_nhwc(data_im.contiguous(), offset.contiguous(), mask.contiguous(),
+                                   weight.detach().to(dt).contiguous(), b, B, Cin, H, W, Ho, Wo,
+                                   Cout, kH, kW, ph, pw, sh, sw, dh, dw)
     else:
         cols = dcn_gather_cols_nhwc(data_im, offset, mask, kH, kW, (sh, sw), (ph, pw), (dh, dw))
         w_kc = weight.permute(0, 2, 3, 1).to(dt).contiguous()
+        out = torch.empty(B, Ho, Wo, Cout, device=data_im.device, dtype=dt)
         torch.mm(cols, w_kc.view(Cout, -1).t(), out=out.view(-1, Cout))
         if b is not None:
             out += b.view(1, 1, 1, -1)

@@ -16,7 +16,7 @@ import torch.nn as nn
 from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _pair, _single
-from ._packing import columns_grad_f32, fused_conv, weight_grad
+from ._packing import columns_grad_f32, weight_grad
 
 _ext = None
 
@@ -366,6 +366,15 @@ def _modulated_deform_conv2d_forward(input, offset, mask, weight, bias, stride, 
     dil_h, dil_w = dilation
     ho = _out_size(height, pad_h, dil_h, kernel_h, stride_h)
     wo = _out_size(width, pad_w, dil_w, kernel_w, stride_w)
+    sizes = (batch, channels, height, width, ho, wo, channels_out, kernel_h, kernel_w, pad_h, pad_w,
+             stride_h, stride_w, dil_h, dil_w)
+    if groups == 1 and input.dtype == torch.float32:
+        # Layout changes and product behind one call; the output is written NCHW.
+        out = ext.dcn_layer_nchw_f32(
+            input.contiguous(), offset.contiguous(), mask.contiguous(), weight.contiguous(),
+            bias.to(input.dtype).contiguous() if bias is not None else None, *sizes, deform_groups)
+        if out is not None:
+            return out
     vec = 16 // input.element_size()
     if (groups == 1 and deform_groups == 1 and input.dtype != torch.float64
             and channels % vec == 0):
@@ -374,11 +383,8 @@ def _modulated_deform_conv2d_forward(input, offset, mask, weight, bias, stride, 
         off_nhwc = ext.nchw_to_nhwc(offset)
         msk_nhwc = ext.nchw_to_nhwc(mask)
         b = bias.to(input.dtype).contiguous() if bias is not None else None
-        out = input.new_empty(batch, ho, wo, channels_out)
-        fused_conv(x_nhwc, off_nhwc, msk_nhwc, weight, b,
-                   (batch, channels, height, width, ho, wo, channels_out, kernel_h, kernel_w,
-                    pad_h, pad_w, stride_h, stride_w, dil_h, dil_w), out)
-        return ext.nhwc_to_nchw(out)
+        return ext.nhwc_to_nchw(ext.dcn_conv_nhwc(x_nhwc, off_nhwc, msk_nhwc, weight.contiguous(),
+                                                  b, *sizes))
     # Columns [C*kh*kw, B*Ho*Wo] then one GEMM per group (modulated_deform_conv.py:369-401).
     bhw = batch * ho * wo
     columns = input.new_empty(channels * kernel_h * kernel_w, bhw)

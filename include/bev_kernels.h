@@ -221,6 +221,42 @@ int64_t bevk_column_sums_workspace_bytes(int n);
 int bevk_column_sums(int dtype, const void *src, int64_t rows, int n, void *workspace,
                      int64_t workspace_bytes, int out_dtype, void *out, void *stream);
 
+/* Whole layers from the module's own weights ([Cout, C, kh, kw], [3T, C, kh, kw]): packing, layout
+ * changes, offset conv and deformable product behind one call; the queries give the workspace bytes
+ * (-1: shape not taken).
+ *   bevk_dcn_layer_nchw_f32  fp32 NCHW layer with given offsets [B, dg*2T, Ho, Wo] and mask
+ *                            [B, dg*T, Ho, Wo] (C % 32 == 0, at most 9 taps; dg > 1: out 16-byte
+ *                            aligned, columns under 2 GiB)
+ *   bevk_dcn_conv_nhwc       NHWC deformable conv, offsets as bevk_dcn_fused_fwd_nhwc
+ *   bevk_dcn_layer_nhwc      NHWC layer with its offset conv: y [B, Ho, Wo, 3T] fp32 (written) and
+ *                            out; b_off (may be NULL) fp32, or 16-bit for a 16-bit layer */
+int64_t bevk_dcn_layer_nchw_f32_workspace_bytes(int batch_size, int channels, int height_im,
+                                                int width_im, int height_col, int width_col,
+                                                int channels_out, int kernel_h, int kernel_w,
+                                                int deformable_group);
+int bevk_dcn_layer_nchw_f32(const float *data_im, const float *data_offset, const float *data_mask,
+                            const float *weight, const float *bias, int batch_size, int channels,
+                            int height_im, int width_im, int height_col, int width_col,
+                            int channels_out, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                            int stride_h, int stride_w, int dilation_h, int dilation_w,
+                            int deformable_group, void *workspace, int64_t workspace_bytes,
+                            float *out, void *stream);
+int64_t bevk_dcn_nhwc_workspace_bytes(int dtype, int with_offset_conv, int batch_size, int channels,
+                                      int height_im, int width_im, int height_col, int width_col,
+                                      int channels_out, int kernel_h, int kernel_w);
+int bevk_dcn_conv_nhwc(int dtype, const void *data_im, const void *data_offset, int offset_last_dim,
+                       const void *data_mask, const void *weight, const void *bias, int batch_size,
+                       int channels, int height_im, int width_im, int height_col, int width_col,
+                       int channels_out, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                       int stride_h, int stride_w, int dilation_h, int dilation_w, void *workspace,
+                       int64_t workspace_bytes, void *out, void *stream);
+int bevk_dcn_layer_nhwc(int dtype, const void *data_im, const void *w_off, const void *b_off,
+                        int b_off_dtype, const void *weight, const void *bias, int batch_size,
+                        int channels, int height_im, int width_im, int height_col, int width_col,
+                        int channels_out, int kernel_h, int kernel_w, int pad_h, int pad_w,
+                        int stride_h, int stride_w, int dilation_h, int dilation_w, int act_relu,
+                        void *workspace, int64_t workspace_bytes, float *y, void *out, void *stream);
+
 /* Workspace bytes bevk_modulated_deformable_fused_im2col_nhwc needs (-1 on bad
  * arguments): the packed offset-conv weight and the fp32 offset-conv output [M][3T]. */
 int64_t bevk_dcn_fused_im2col_nhwc_workspace_bytes(int dtype, int batch_size, int channels,

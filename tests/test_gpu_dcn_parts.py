@@ -1,0 +1,71 @@
+"""16-bit fused forward with the reduction in parts (few pixels) against the float64 oracle with
+columns rounded once to the type, and against the whole-K kernel (both round one fp32 sum of the
+same products, so they differ by fp32 sums in another order and at most one rounding step)."""
+import pytest
+import torch
+
+from _tol import check
+from oracle import dcn as od
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("cin,cout,h,w,relu", [(128, 256, 3, 5, False), (512, 512, 29, 50, True),
+                                               (256, 136, 17, 23, False), (320, 264, 9, 41, True)])
+def test_fused_parts(dtype, cin, cout, h, w, relu):
+    import _modulated_deform_conv_ext as ext
+    g = torch.Generator().manual_seed(cin + h)
+    sizes = (1, cin, h, w, h, w, cout, 3, 3, 1, 1, 1, 1, 1, 1)
+    import _bevk
+    code = _bevk._DTYPE_CODES[dtype]
+    # the workspace holds the parts beside the packed weight: this shape runs in parts
+    assert (_bevk.lib().bevk_dcn_nhwc_workspace_bytes(code, 0, *sizes[:9])
+            > 2 * ext.dcn_packed_weight_numel(dtype, cout, 3, 3, cin) + 256)
+    x = torch.randn(1, h, w, cin, generator=g).to(dtype).to(DEV)
+    off = (2.0 * torch.randn(1, h, w, 18, generator=g)).to(dtype).to(DEV)
+    mask = torch.rand(1, h, w, 9, generator=g).to(dtype).to(DEV)
+    weight = (0.05 * torch.randn(cout, cin, 3, 3, generator=g)).to(dtype).to(DEV)
+    bias = torch.randn(cout, generator=g).to(dtype).to(DEV)
+    out = ext.dcn_conv_nhwc(x, off, mask, weight, bias, *sizes)
+
+    def oracle(o, m):
+        return od.forward_nhwc(x.double().cpu(), o.double().cpu(), m.double().cpu(),
+                               weight.double().cpu(), bias.double().cpu(), 1, 1, 1, col_dtype=dtype)
+    check(out.cpu(), oracle(off, mask), dtype, "parts")
+    whole = torch.empty_like(out)
+    ext.dcn_fused_fwd_nhwc(x, off, mask, ext.dcn_pack_weight(weight), bias, *sizes, whole)
+    ulp = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    d = (out.double() - whole.double()).abs()
+    assert (d <= ulp * whole.double().abs() + 1e-4).all()
+
+    w_off = (0.02 * torch.randn(27, cin, 3, 3, generator=g)).to(dtype).to(DEV)
+    b_off = torch.randn(27, generator=g).to(dtype).to(DEV)
+    out, y = ext.dcn_layer_nhwc(x, w_off, b_off, weight, bias, *sizes, act_relu=relu)
+    yref = od.offset_conv_nhwc(x.double().cpu(), w_off.double().cpu(), b_off.double().cpu(), 1, 1, 1)
+    check(y.cpu(), yref, torch.float32, "y")
+    ref = oracle(y[..., :18], torch.sigmoid(y[..., 18:].double()))
+    check(out.cpu(), ref.clamp(min=0) if relu else ref, dtype, "layer in parts")
+
+
+@pytest.mark.parametrize("b,c,cout,h,w,stride,dg", [
+    (1, 32, 16, 1, 1, 1, 1), (2, 64, 72, 9, 7, 1, 1), (1, 64, 64, 32, 32, 1, 1),
+    (3, 96, 160, 13, 10, 2, 1), (2, 64, 100, 11, 14, 1, 4), (1, 128, 264, 8, 9, 2, 2),
+    (2, 256, 256, 20, 33, 1, 1)])
+def test_layer_nchw_f32(b, c, cout, h, w, stride, dg):
+    """The NCHW fp32 layer behind one call: planes of 4k, 2k and odd positions (the three widths of
+    the NCHW stores), two K parts, deformable groups; against the float64 oracle."""
+    import _modulated_deform_conv_ext as ext
+    g = torch.Generator().manual_seed(c + h)
+    ho, wo = (h - 1) // stride + 1, (w - 1) // stride + 1
+    x = torch.randn(b, c, h, w, generator=g)
+    off = 2.0 * torch.randn(b, dg * 18, ho, wo, generator=g)
+    mask = torch.rand(b, dg * 9, ho, wo, generator=g)
+    weight = 0.1 * torch.randn(cout, c, 3, 3, generator=g)
+    bias = torch.randn(cout, generator=g)
+    out = ext.dcn_layer_nchw_f32(*(t.to(DEV) for t in (x, off, mask, weight, bias)), b, c, h, w, ho,
+                                 wo, cout, 3, 3, 1, 1, stride, stride, 1, 1, dg)
+    ref = od.forward_nchw(x.double(), off.double(), mask.double(), weight.double(), bias.double(),
+                          (stride, stride), (1, 1), (1, 1), 1, dg)
+    check(out.cpu(), ref, torch.float32, "nchw layer")
