@@ -805,8 +805,9 @@ def modulated_deformable_fused_im2col_nhwc_cuda(data_im, w_off, b_off, batch_siz
 
 def _msda_check(fn, value, spatial_shapes, level_start_index, sampling_loc, attn_weight):
     """Checks of binding_musa.mu:292-298 / :420-427 plus shape agreement; returns
-    (batch, spatial, heads, channels, num_levels, num_query, num_point)."""
-    if value.device.type != "cuda":
+    (batch, spatial, heads, channels, num_levels, num_query, num_point). Kept to plain attribute
+    tests: a decoder's call is as long as its host side."""
+    if not value.is_cuda:
         raise RuntimeError("value must be a HIP device tensor")
     if not value.is_contiguous():
         raise RuntimeError("value must be contiguous")
@@ -819,26 +820,26 @@ def _msda_check(fn, value, spatial_shapes, level_start_index, sampling_loc, attn
     if not attn_weight.is_contiguous():
         raise RuntimeError("attn_weight must be contiguous")
     _b.require_device(fn, value, spatial_shapes, level_start_index, sampling_loc, attn_weight)
-    _b.require_dtype(fn, value, sampling_loc=sampling_loc, attn_weight=attn_weight)
+    dtype = value.dtype
+    if sampling_loc.dtype != dtype or attn_weight.dtype != dtype:
+        _b.require_dtype(fn, value, sampling_loc=sampling_loc, attn_weight=attn_weight)
     if spatial_shapes.dtype != torch.int64 or level_start_index.dtype != torch.int64:
         raise RuntimeError(f"{fn}: spatial_shapes and level_start_index must be int64")
-    if value.dim() != 4 or sampling_loc.dim() != 6 or attn_weight.dim() != 5:
+    v_shape, loc_shape, a_shape = value.shape, sampling_loc.shape, attn_weight.shape
+    if len(v_shape) != 4 or len(loc_shape) != 6 or len(a_shape) != 5:
         raise RuntimeError(
             f"{fn}: expected value [B,S,heads,D], sampling_loc [B,Lq,heads,L,P,2] and "
             "attn_weight [B,Lq,heads,L,P]")
-    batch, spatial, heads, channels = value.shape
-    num_levels = spatial_shapes.size(0)
-    num_query = sampling_loc.size(1)
-    num_point = sampling_loc.size(4)
-    if tuple(spatial_shapes.shape) != (num_levels, 2) or \
-            tuple(level_start_index.shape) != (num_levels,):
+    batch, spatial, heads, channels = v_shape
+    num_levels, num_query, num_point = spatial_shapes.size(0), loc_shape[1], loc_shape[4]
+    if spatial_shapes.shape != (num_levels, 2) or level_start_index.shape != (num_levels,):
         raise RuntimeError(f"{fn}: spatial_shapes must be [L, 2] and level_start_index [L]")
-    if tuple(sampling_loc.shape) != (batch, num_query, heads, num_levels, num_point, 2):
-        raise RuntimeError(f"{fn}: sampling_loc shape {tuple(sampling_loc.shape)} does not match "
-                           f"value {tuple(value.shape)} and {num_levels} levels")
-    if tuple(attn_weight.shape) != (batch, num_query, heads, num_levels, num_point):
-        raise RuntimeError(f"{fn}: attn_weight shape {tuple(attn_weight.shape)} does not match "
-                           f"sampling_loc {tuple(sampling_loc.shape)}")
+    if loc_shape != (batch, num_query, heads, num_levels, num_point, 2):
+        raise RuntimeError(f"{fn}: sampling_loc shape {tuple(loc_shape)} does not match "
+                           f"value {tuple(v_shape)} and {num_levels} levels")
+    if a_shape != (batch, num_query, heads, num_levels, num_point):
+        raise RuntimeError(f"{fn}: attn_weight shape {tuple(a_shape)} does not match "
+                           f"sampling_loc {tuple(loc_shape)}")
     return batch, spatial, heads, channels, num_levels, num_query, num_point
 
 
@@ -849,8 +850,7 @@ def forward(value, spatial_shapes, level_start_index, sampling_loc, attn_weight,
     attn_weight [B, Lq, heads, L, P] -> output [B, Lq, heads * D]."""
     batch, spatial, heads, channels, num_levels, num_query, num_point = _msda_check(
         "msda_forward", value, spatial_shapes, level_start_index, sampling_loc, attn_weight)
-    output = torch.empty(batch, num_query, heads * channels, dtype=value.dtype,
-                         device=value.device)
+    output = value.new_empty((batch, num_query, heads * channels))
     _b.call("bevk_msda_forward", _b.dtype_code(value), _b.ptr(value), _b.ptr(spatial_shapes),
             _b.ptr(level_start_index), _b.ptr(sampling_loc), _b.ptr(attn_weight), batch, spatial,
             heads, channels, num_levels, num_query, num_point, int(im2col_step),

@@ -7,10 +7,15 @@ from typing import Optional, Tuple
 
 import torch
 
+_loaded = None
+
 
 def _ext():
-    import _modulated_deform_conv_ext
-    return _modulated_deform_conv_ext
+    global _loaded
+    if _loaded is None:
+        import _modulated_deform_conv_ext
+        _loaded = _modulated_deform_conv_ext
+    return _loaded
 
 
 def ms_deform_attn_forward(
@@ -26,7 +31,7 @@ def ms_deform_attn_forward(
     """value [B, S, heads, D], spatial_shapes [L, 2] int64, level_start_index [L] int64,
     sampling_loc [B, Lq, heads, L, P, 2] in [0, 1], attn_weight [B, Lq, heads, L, P]
     -> [B, Lq, heads * D]. fp32 / fp16 / bf16 (fp32 accumulation) / fp64."""
-    if not torch.cuda.is_available():
+    if not value.is_cuda and not torch.cuda.is_available():
         raise RuntimeError("ms_deform_attn_forward requires a HIP device (torch.cuda)")
     return _ext().forward(value, spatial_shapes, level_start_index, sampling_loc, attn_weight,
                           im2col_step=im2col_step, force_generic=force_generic)
@@ -50,7 +55,7 @@ def ms_deform_attn_backward(
     reference) caps the scratch: above it the atomic kernels run with the reference's
     memory use (default: the BEVK_MSDA_BACKWARD_MAX_WORKSPACE environment variable,
     unset = no cap)."""
-    if not torch.cuda.is_available():
+    if not value.is_cuda and not torch.cuda.is_available():
         raise RuntimeError("ms_deform_attn_backward requires a HIP device (torch.cuda)")
     grad_value = torch.zeros_like(value)
     grad_sampling_loc = torch.zeros_like(sampling_loc)
