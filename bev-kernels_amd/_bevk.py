@@ -75,6 +75,8 @@ _SIGNATURES = {
     "bevk_msda_backward_workspace_bytes": [_i] * 8,
     "bevk_msda_backward": [_i, _vp, _vp, _vp, _vp, _vp, _vp] + [ctypes.c_int64] * 4
     + [_i] * 9 + [_vp, _vp, _vp, _vp, ctypes.c_int64, _vp],
+    "bevk_msda_gradients": [_i, _vp, _vp, _vp, _vp, _vp, _vp] + [ctypes.c_int64] * 4
+    + [_i] * 9 + [_vp, _vp, _vp, _vp, ctypes.c_int64, _vp],
 }
 
 # entry points that return a value instead of a bevk_status

@@ -61,6 +61,7 @@ __all__ = [
     "nhwc_to_nchw",
     "forward",
     "backward",
+    "gradients",
 ]
 
 
@@ -925,6 +926,36 @@ def backward(value, spatial_shapes, level_start_index, sampling_loc, attn_weight
             tuple(grad_attn_weight.shape) != tuple(attn_weight.shape):
         raise RuntimeError(f"{fn}: gradient tensors must have the shapes of value, "
                            "sampling_loc and attn_weight")
+    _backward_call("bevk_msda_backward", value, spatial_shapes, level_start_index, sampling_loc,
+                   attn_weight, grad_output, grad_value, grad_sampling_loc, grad_attn_weight,
+                   im2col_step, force_generic_col2im, max_workspace_bytes)
+
+
+def gradients(value, spatial_shapes, level_start_index, sampling_loc, attn_weight, grad_output,
+              im2col_step=64, force_generic_col2im=False, max_workspace_bytes=None):
+    """(grad_value, grad_sampling_loc, grad_attn_weight) in new tensors: ``backward`` without its
+    accumulation into the caller's grad_value, so that no tensor is zeroed on its own first."""
+    fn = "msda_backward"
+    _msda_check(fn, value, spatial_shapes, level_start_index, sampling_loc, attn_weight)
+    if not grad_output.is_cuda:
+        raise RuntimeError("grad_output must be a HIP device tensor")
+    _b.require_device(fn, value, grad_output)
+    _b.require_dtype(fn, value, grad_output=grad_output)
+    # (without queries or points no kernel writes the empty or untouched tensors)
+    new = torch.empty_like if sampling_loc.numel() > 0 and value.numel() > 0 else torch.zeros_like
+    grads = new(value), new(sampling_loc), new(attn_weight)
+    _backward_call("bevk_msda_gradients", value, spatial_shapes, level_start_index, sampling_loc,
+                   attn_weight, grad_output, *grads, im2col_step, force_generic_col2im,
+                   max_workspace_bytes)
+    return grads
+
+
+def _backward_call(entry, value, spatial_shapes, level_start_index, sampling_loc, attn_weight,
+                   grad_output, grad_value, grad_sampling_loc, grad_attn_weight, im2col_step,
+                   force_generic_col2im, max_workspace_bytes):
+    batch, spatial, heads, channels = value.shape
+    num_levels, num_query, num_point = (spatial_shapes.size(0), sampling_loc.size(1),
+                                        sampling_loc.size(4))
     # binding_musa.mu:446-447 views grad_output per (batch, query, head, channel)
     g4 = grad_output.view(batch, num_query, heads, channels)
     sb, sq, sh, sc = g4.stride()
@@ -938,7 +969,7 @@ def backward(value, spatial_shapes, level_start_index, sampling_loc, attn_weight
             raise
         nbytes = least
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=value.device)
-    _b.call("bevk_msda_backward", code, _b.ptr(value), _b.ptr(spatial_shapes),
+    _b.call(entry, code, _b.ptr(value), _b.ptr(spatial_shapes),
             _b.ptr(level_start_index), _b.ptr(sampling_loc), _b.ptr(attn_weight), _b.ptr(g4),
             sb, sq, sh, sc, batch, spatial, heads, channels, num_levels, num_query, num_point,
             int(im2col_step), 1 if force_generic_col2im else 0, _b.ptr(grad_value),

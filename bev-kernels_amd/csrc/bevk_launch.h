@@ -34,6 +34,7 @@ struct MsdaBwdArgs {
   void *grad_value, *grad_loc, *grad_attn;
   void *workspace;       // fp32 accumulator for 16-bit dtypes, then the sorted path's buffers
   int64_t workspace_bytes;
+  bool fresh = false;    // fp32 / fp64 grad_value is written, not added to
 };
 
 // Bytes of fp32 accumulator the 16-bit backward needs at least (0 for f32 / f64).

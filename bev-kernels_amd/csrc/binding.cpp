@@ -1123,16 +1123,15 @@ int64_t bevk_msda_backward_workspace_bytes(int dtype, int batch, int spatial_siz
                                              num_levels, num_query, num_point);
 }
 
-int bevk_msda_backward(int dtype, const void *value, const int64_t *spatial_shapes,
-                       const int64_t *level_start_index, const void *sampling_loc,
-                       const void *attn_weight, const void *grad_output, int64_t go_stride_b,
-                       int64_t go_stride_q, int64_t go_stride_h, int64_t go_stride_c,
-                       int batch, int spatial_size, int num_heads, int channels,
-                       int num_levels, int num_query, int num_point, int im2col_step,
-                       int force_generic_col2im, void *grad_value, void *grad_sampling_loc,
-                       void *grad_attn_weight, void *workspace, int64_t workspace_bytes,
-                       void *stream) {
-  const char *fn = "msda_backward";
+static int msda_backward_run(const char *fn, bool fresh, int dtype, const void *value, const int64_t *spatial_shapes,
+                             const int64_t *level_start_index, const void *sampling_loc,
+                             const void *attn_weight, const void *grad_output, int64_t go_stride_b,
+                             int64_t go_stride_q, int64_t go_stride_h, int64_t go_stride_c,
+                             int batch, int spatial_size, int num_heads, int channels,
+                             int num_levels, int num_query, int num_point, int im2col_step,
+                             int force_generic_col2im, void *grad_value, void *grad_sampling_loc,
+                             void *grad_attn_weight, void *workspace, int64_t workspace_bytes,
+                             void *stream) {
   g_last_error.clear();
   if (!valid_dtype(dtype)) return fail(BEVK_ERR_INVALID, "%s: unknown dtype code %d", fn, dtype);
   if (batch < 0 || spatial_size < 0 || num_heads < 0 || channels < 0 || num_levels < 0 ||
@@ -1151,7 +1150,7 @@ int bevk_msda_backward(int dtype, const void *value, const int64_t *spatial_shap
   const long long units = (long long)batch * num_query * num_heads;
   // 16-bit grad_value is fully written (narrowed from the cleared accumulator) even when
   // there are no queries; with no values there is nothing to write at all
-  if (value_elems == 0 || (units == 0 && need == 0)) return ok();
+  if (value_elems == 0 || (units == 0 && need == 0 && !fresh)) return ok();
   if (channels == 0) return ok();
   if (!value || !spatial_shapes || !level_start_index || !grad_value ||
       (units > 0 && (!sampling_loc || !attn_weight || !grad_output || !grad_sampling_loc ||
@@ -1173,8 +1172,41 @@ int bevk_msda_backward(int dtype, const void *value, const int64_t *spatial_shap
   a.grad_value = grad_value; a.grad_loc = grad_sampling_loc; a.grad_attn = grad_attn_weight;
   a.workspace = workspace;
   a.workspace_bytes = workspace_bytes;
+  a.fresh = fresh;
   return hip_status(
       bevk::launch_msda_backward(dtype, a, force_generic_col2im != 0, (hipStream_t)stream), fn);
+}
+
+int bevk_msda_backward(int dtype, const void *value, const int64_t *spatial_shapes,
+                       const int64_t *level_start_index, const void *sampling_loc,
+                       const void *attn_weight, const void *grad_output, int64_t go_stride_b,
+                       int64_t go_stride_q, int64_t go_stride_h, int64_t go_stride_c,
+                       int batch, int spatial_size, int num_heads, int channels,
+                       int num_levels, int num_query, int num_point, int im2col_step,
+                       int force_generic_col2im, void *grad_value, void *grad_sampling_loc,
+                       void *grad_attn_weight, void *workspace, int64_t workspace_bytes,
+                       void *stream) {
+  return msda_backward_run("msda_backward", false, dtype, value, spatial_shapes, level_start_index, sampling_loc, attn_weight, grad_output,
+                           go_stride_b, go_stride_q, go_stride_h, go_stride_c, batch, spatial_size,
+                           num_heads, channels, num_levels, num_query, num_point, im2col_step,
+                           force_generic_col2im, grad_value, grad_sampling_loc, grad_attn_weight,
+                           workspace, workspace_bytes, stream);
+}
+
+int bevk_msda_gradients(int dtype, const void *value, const int64_t *spatial_shapes,
+                        const int64_t *level_start_index, const void *sampling_loc,
+                        const void *attn_weight, const void *grad_output, int64_t go_stride_b,
+                        int64_t go_stride_q, int64_t go_stride_h, int64_t go_stride_c,
+                        int batch, int spatial_size, int num_heads, int channels,
+                        int num_levels, int num_query, int num_point, int im2col_step,
+                        int force_generic_col2im, void *grad_value, void *grad_sampling_loc,
+                        void *grad_attn_weight, void *workspace, int64_t workspace_bytes,
+                        void *stream) {
+  return msda_backward_run("msda_gradients", true, dtype, value, spatial_shapes, level_start_index, sampling_loc, attn_weight, grad_output,
+                           go_stride_b, go_stride_q, go_stride_h, go_stride_c, batch, spatial_size,
+                           num_heads, channels, num_levels, num_query, num_point, im2col_step,
+                           force_generic_col2im, grad_value, grad_sampling_loc, grad_attn_weight,
+                           workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -1915,12 +1915,12 @@ bool sorted_path(const MsdaBwdArgs &a, int dtype, BktLayout &L) {
 
 // grad_value (fp32, added to gv) by the four bucket kernels, then the coordinate kernel.
 // fused_n: 16-bit types with a 16-byte aligned fp32 workspace gv and an 8-byte aligned
-// grad_value: the workspace's element count; the count kernel clears gv and the coordinate
-// kernel narrows it into grad_value. 0: gv is the caller's fp32 grad_value, or the
-// caller clears and narrows.
+// grad_value: the workspace's element count; the coordinate kernel narrows it into grad_value.
+// 0: gv is the caller's fp32 grad_value, or the caller narrows. clear_n: elements of gv that the
+// count kernel clears first (0: gv holds what is added to).
 template <typename T>
 hipError_t launch_sorted(const MsdaBwdArgs &a, const BktLayout &L, char *ws, float *gv,
-                         int64_t fused_n, hipStream_t stream) {
+                         int64_t fused_n, int64_t clear_n, hipStream_t stream) {
   BktParams p;
   p.loc = a.f.sampling_loc;
   p.attn = a.f.attn_weight;
@@ -1957,8 +1957,8 @@ hipError_t launch_sorted(const MsdaBwdArgs &a, const BktLayout &L, char *ws, flo
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   p.pblk = count_pblk;
-  p.zero = fused_n > 0 ? gv : nullptr;
-  p.nzero4 = fused_n / 4;
+  p.zero = clear_n > 0 ? gv : nullptr;
+  p.nzero4 = clear_n / 4;
   hipLaunchKernelGGL((msda_bkt_count_kernel<T>), dim3(8u * (unsigned)count_pblk), dim3(kBkThreads), 0,
                      stream, p);
   if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -2133,11 +2133,21 @@ hipError_t launch_grid_coord(const MsdaBwdArgs &a, float *gv, hipStream_t stream
 template <typename T>
 hipError_t launch_f32(const MsdaBwdArgs &a, bool generic, hipStream_t stream) {
   float *gv = static_cast<float *>(a.grad_value);
+  const int64_t n = (int64_t)a.f.batch * a.f.spatial_size * a.f.num_heads * a.f.channels;
   BktLayout L;
+  // a fresh gradient is cleared by the count kernel beside its own work (sorted_path has checked
+  // the 16-byte alignment; n is a multiple of 32 there) instead of a fill of its own before it
   if (!generic && sorted_path<T>(a, 0, L))
-    return launch_sorted<T>(a, L, static_cast<char *>(a.workspace), gv, 0, stream);
-  if (generic || !owner_path<T>(a)) return launch_t<T, float>(a, gv, generic, stream);
-  hipError_t e = launch_owner<T>(a, gv, true, stream);
+    return launch_sorted<T>(a, L, static_cast<char *>(a.workspace), gv, 0, a.fresh ? n : 0, stream);
+  hipError_t e;
+  if (generic || !owner_path<T>(a)) {
+    if (a.fresh) {
+      hipLaunchKernelGGL(fill_zero_f32, dim3(stream_grid(n)), dim3(kBlock), 0, stream, gv, n);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    return launch_t<T, float>(a, gv, generic, stream);
+  }
+  e = launch_owner<T>(a, gv, !a.fresh, stream);  // the owner pass writes or adds to every element
   if (e != hipSuccess) return e;
   return launch_grid_coord<T>(a, gv, stream);
 }
@@ -2160,7 +2170,7 @@ hipError_t launch_half(const MsdaBwdArgs &a, bool generic, hipStream_t stream) {
       if (e != hipSuccess) return e;
     }
     e = launch_sorted<T>(a, L, static_cast<char *>(a.workspace) + half_acc_bytes(dtype, n), acc,
-                         fuse ? n : 0, stream);
+                         fuse ? n : 0, fuse ? n : 0, stream);
     if (e != hipSuccess || fuse) return e;
   } else if (!generic && owner_path<T>(a)) {  // the owner pass writes every element of the workspace
     e = launch_owner<T>(a, acc, false, stream);
@@ -2201,6 +2211,13 @@ hipError_t launch_msda_backward(int dtype, const MsdaBwdArgs &a, bool force_gene
     case 1: return launch_half<f16>(a, force_generic, stream);
     case 2: return launch_half<bf16>(a, force_generic, stream);
     case 3:
+      if (a.fresh) {  // two zero words per element
+        const int64_t n = (int64_t)a.f.batch * a.f.spatial_size * a.f.num_heads * a.f.channels * 2;
+        hipLaunchKernelGGL(fill_zero_f32, dim3(stream_grid(n)), dim3(kBlock), 0, stream,
+                           static_cast<float *>(a.grad_value), n);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+      }
       return launch_t<double, double>(a, static_cast<double *>(a.grad_value), true, stream);
     default: return hipErrorInvalidValue;
   }

@@ -57,11 +57,7 @@ def ms_deform_attn_backward(
     unset = no cap)."""
     if not value.is_cuda and not torch.cuda.is_available():
         raise RuntimeError("ms_deform_attn_backward requires a HIP device (torch.cuda)")
-    grad_value = torch.zeros_like(value)
-    grad_sampling_loc = torch.zeros_like(sampling_loc)
-    grad_attn_weight = torch.zeros_like(attn_weight)
-    _ext().backward(value, spatial_shapes, level_start_index, sampling_loc, attn_weight,
-                    grad_output, grad_value, grad_sampling_loc, grad_attn_weight,
-                    im2col_step=im2col_step, force_generic_col2im=force_generic_col2im,
-                    max_workspace_bytes=max_workspace_bytes)
-    return grad_value, grad_sampling_loc, grad_attn_weight
+    return _ext().gradients(value, spatial_shapes, level_start_index, sampling_loc, attn_weight,
+                            grad_output, im2col_step=im2col_step,
+                            force_generic_col2im=force_generic_col2im,
+                            max_workspace_bytes=max_workspace_bytes)

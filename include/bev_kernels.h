@@ -447,6 +447,17 @@ int bevk_msda_backward(
     void *grad_value, void *grad_sampling_loc, void *grad_attn_weight, void *workspace,
     int64_t workspace_bytes, void *stream);
 
+/* bevk_msda_backward with every gradient written: grad_value of F32 / F64 is not added to what the
+ * tensor holds (the clear runs beside other work), so nothing needs zeroing beforehand. */
+int bevk_msda_gradients(int dtype, const void *value, const int64_t *spatial_shapes,
+                        const int64_t *level_start_index, const void *sampling_loc,
+                        const void *attn_weight, const void *grad_output, int64_t go_stride_b,
+                        int64_t go_stride_q, int64_t go_stride_h, int64_t go_stride_c, int batch,
+                        int spatial_size, int num_heads, int channels, int num_levels,
+                        int num_query, int num_point, int im2col_step, int force_generic_col2im,
+                        void *grad_value, void *grad_sampling_loc, void *grad_attn_weight,
+                        void *workspace, int64_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -772,3 +772,35 @@ def test_sorted_path_query_limit(nq):
     for name, x, r in zip(("grad_value", "grad_sampling_loc", "grad_attn_weight"), api,
                           (gv, gl, ga)):
         check(x.cpu(), r.cpu(), dt, f"{nq} queries {name}: API vs atomic kernels")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.float64],
+                         ids=["fp32", "fp16", "fp64"])
+@pytest.mark.parametrize("case", ["sorted", "atomic", "owner", "generic", "d64", "few_queries",
+                                  "uncovered"])
+def test_gradients_need_no_zeroing(case, dtype):
+    """gradients() writes every element of its new tensors (which come from memory full of NaN
+    here) on each backward path: the same as backward() into zeros, up to the order of the sums."""
+    import _modulated_deform_conv_ext as ext
+    shapes = [(11, 13)] if case == "owner" else [(12, 17), (6, 9), (3, 5)]
+    nq = 143 if case == "owner" else 2 if case == "few_queries" else 60
+    d = inputs.msda_random(2, shapes, nq, 4, 64 if case == "d64" else 32, 4, seed=7)
+    if case == "uncovered":  # positions that no level covers, and samples outside the maps
+        d["value"] = torch.cat([d["value"], d["value"][:, :40]], 1)
+        d["sampling_loc"] = d["sampling_loc"] * 3 - 1
+    t = [d[k].to(DEV) for k in ("value", "spatial_shapes", "level_start_index", "sampling_loc",
+                                "attn_weight")]
+    t = [v.to(dtype) if v.is_floating_point() else v for v in t]
+    go = torch.randn(2, nq, t[0].shape[2] * t[0].shape[3], device=DEV).to(dtype)
+    kw = dict(force_generic_col2im=case == "generic",
+              max_workspace_bytes=0 if case in ("atomic", "owner") else None)
+    want = [torch.zeros_like(t[i]) for i in (0, 3, 4)]
+    ext.backward(*t, go, *want, **kw)
+    torch.cuda.synchronize()
+    # the blocks that the allocator hands out next
+    poison = [torch.full_like(t[i], float("nan")) for i in (0, 3, 4)]
+    torch.cuda.synchronize()
+    del poison
+    got = ext.gradients(*t, go, **kw)
+    for a, b, what in zip(got, want, ("grad_value", "grad_loc", "grad_attn")):
+        check(a.cpu(), b.double().cpu(), dtype, f"{case} {what}")
