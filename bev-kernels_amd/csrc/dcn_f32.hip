@@ -508,6 +508,170 @@ __global__ void __launch_bounds__(kThreads) f32_gemm_kernel(const Params p) {
   }
 }
 
+// Small problems: a workgroup takes one 16-row block x 64 columns and its eight waves take every
+// eighth K step each, without barriers: a lane builds its MFMA A fragment (one row, 8 channels)
+// straight from the corners, the next step's loads are in flight while a step multiplies, and the
+// waves' sums meet in LDS at the end. The tiled kernel needs about 1.4 us per K step when few
+// workgroups are on the chip (each step waits for its loads and a barrier); here eight steps wait
+// together. A whole layer of 64 channels of 32 x 32 to 64: 23.5 -> 16 us.
+constexpr int kSmallCols = 64;
+template <int GEO>
+__global__ void __launch_bounds__(kThreads) f32_small_kernel(const Params p) {
+  constexpr int NQ = deform(GEO) ? 4 : 1, NB = kSmallCols / 16, kPitch = kSmallCols + 1;
+  __shared__ __attribute__((aligned(16))) TapGeo geo[deform(GEO) ? 16 * kMaxTaps : 1];
+  __shared__ float red[8][16 * kPitch];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int L = (int)(blockIdx.x & 7) * p.per_xcd + (int)(blockIdx.x >> 3);
+  if (L >= p.mch * p.nt) return;  // uniform
+  const int m0 = L % p.mch * 16, n0 = L / p.mch * kSmallCols;
+  const int spt = GEO == kRows ? p.kb_total : p.C / kBK;
+  bool bad = false;
+  for (int i = tid; i < NB * p.kb_total; i += kThreads) {
+    const int nb = (n0 >> 4) + i / p.kb_total;
+    bad |= nb < p.nb_total && p.flags[(int64_t)nb * p.kb_total + i % p.kb_total] != 0;
+  }
+  if constexpr (deform(GEO)) {
+    for (int g = tid; g < 16 * p.taps; g += kThreads) {
+      const int row = g / p.taps, t = g - row * p.taps, m = m0 + row;
+      TapGeo G;
+      G.w[0] = G.w[1] = G.w[2] = G.w[3] = 0.f;
+      G.o[0] = G.o[1] = G.o[2] = G.o[3] = p.x_bytes;
+      if (m < p.M) G = tap_geo<GEO>(p, m, t);
+      geo[g] = G;
+    }
+    __syncthreads();
+  }
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, p.x_bytes);
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(p.w, p.w_bytes);
+  const int row = lane & 15, oct = lane >> 4;
+  uint32_t bo[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int nb = (n0 >> 4) + j;
+    bo[j] = nb < p.nb_total ? (uint32_t)nb * (uint32_t)p.kb_total * kBlkBytes + (uint32_t)lane * 16u
+                            : p.w_bytes;
+  }
+  struct Step {
+    floatx4 a[NQ][2], w;
+    int4v b[NB][3];
+  };
+  auto load = [&](int ks, Step &st) __attribute__((always_inline)) {
+    uint32_t o[NQ];
+    if constexpr (GEO == kRows) {
+      const int m = m0 + row;
+      o[0] = m < p.M ? ((uint32_t)m * (uint32_t)p.kb_total + (uint32_t)ks) * (kBK * 4u) + (uint32_t)oct * 32u
+                     : p.x_bytes;
+    } else {
+      const int t = ks / spt;
+      const TapGeo &G = geo[row * p.taps + t];
+      const uint32_t cb = (uint32_t)(ks - t * spt) * (kBK * 4u) + (uint32_t)oct * 32u;
+      st.w = *reinterpret_cast<const floatx4 *>(G.w);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) o[q] = G.o[q] == p.x_bytes ? p.x_bytes : G.o[q] + cb;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+        st.a[q][hf] = __builtin_bit_cast(
+            floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                         xr, o[q] == p.x_bytes ? p.x_bytes : o[q] + hf * 16u, 0, 0));
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        st.b[j][q] = __builtin_amdgcn_raw_buffer_load_b128(wr, bo[j] + q * 1024, (uint32_t)ks * kBlkBytes, 0);
+  };
+  floatx4 hi[NB], lo[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) hi[j] = lo[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float nf = 0.f;
+  auto multiply = [&](const Step &st) __attribute__((always_inline)) {
+    Pieces pc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float v = st.a[0][e >> 2][e & 3];
+      if constexpr (deform(GEO)) {
+        v *= st.w[0];
+#pragma unroll
+        for (int q = 1; q < NQ; ++q) v = __builtin_fmaf(st.w[q], st.a[q][e >> 2][e & 3], v);
+      }
+      pc[e] = cut(v);
+      nf += pc[e].l;
+    }
+    const int4v a[3] = {
+        int4v{pack2(pc[0].h, pc[1].h), pack2(pc[2].h, pc[3].h), pack2(pc[4].h, pc[5].h), pack2(pc[6].h, pc[7].h)},
+        int4v{pack2(pc[0].m, pc[1].m), pack2(pc[2].m, pc[3].m), pack2(pc[4].m, pc[5].m), pack2(pc[6].m, pc[7].m)},
+        int4v{pack2(pc[0].l, pc[1].l), pack2(pc[2].l, pc[3].l), pack2(pc[4].l, pc[5].l), pack2(pc[6].l, pc[7].l)}};
+    constexpr int kTa[5] = {2, 0, 1, 1, 0}, kTb[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+    for (int q = 0; q < 5; ++q)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) lo[j] = mfma(a[kTa[q]], st.b[j][kTb[q]], lo[j]);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) hi[j] = mfma(a[0], st.b[j][0], hi[j]);
+  };
+  const int kb = p.kb_total;
+  if (wave < kb) {
+    Step s0, s1;
+    load(wave, s0);
+    for (int ks = wave;;) {  // a step past the end repeats the last one, not used
+      load(min(ks + 8, kb - 1), s1);
+      multiply(s0);
+      if ((ks += 8) >= kb) break;
+      load(min(ks + 8, kb - 1), s0);
+      multiply(s1);
+      if ((ks += 8) >= kb) break;
+    }
+  }
+  bad |= !(nf == nf);
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      red[wave][(4 * (lane >> 4) + e) * kPitch + 16 * j + (lane & 15)] = hi[j][e] + lo[j][e];
+  const bool slow = __syncthreads_or(bad);
+  // Two outputs per thread: consecutive rows of a column (NCHW: a channel's positions), or
+  // consecutive columns of a row.
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int i = 2 * tid + u;
+    const int r = p.plane > 0 ? i & 15 : i / kSmallCols, c = p.plane > 0 ? i >> 4 : i % kSmallCols;
+    const int m = m0 + r, n = n0 + c;
+    if (m >= p.M || n >= p.Cout) continue;
+    float v = 0.f;
+    if (!slow) {
+#pragma unroll
+      for (int w = 0; w < 8; ++w) v += red[w][r * kPitch + c];
+    } else {  // plain fp32
+      for (int k = 0; k < kb * kBK; ++k) {
+        const int ks = k / kBK, kk = k % kBK;
+        float x = 0.f;
+        if constexpr (GEO == kRows) {
+          x = static_cast<const float *>(p.x)[(int64_t)m * kb * kBK + k];
+        } else {
+          const int t = ks / spt;
+          const TapGeo &G = geo[r * p.taps + t];
+          for (int q = 0; q < 4; ++q) {
+            const float xv = G.o[q] == p.x_bytes
+                                 ? 0.f
+                                 : buffer_load_one<float>(xr, G.o[q] + (uint32_t)(k - t * spt * kBK) * 4u);
+            x = q == 0 ? G.w[0] * xv : __builtin_fmaf(G.w[q], xv, x);
+          }
+        }
+        const unsigned short *blk = static_cast<const unsigned short *>(p.w) +
+                                    ((int64_t)(n >> 4) * kb + ks) * (kBlkBytes / 2);
+        const int e = ((n & 15) + 16 * (kk >> 3)) * 8 + (kk & 7);
+        float wv = 0.f;
+        for (int q = 2; q >= 0; --q) wv += __builtin_bit_cast(float, (uint32_t)blk[q * 512 + e] << 16);
+        v = __builtin_fmaf(x, wv, v);
+      }
+    }
+    emit(p, m, n, v, p.bias != nullptr ? p.bias[n] : 0.f);
+  }
+}
+
 // The three pieces of a lane's 8 values of a split block; a non-finite value is kept whole in
 // the first piece. Returns whether there was one.
 __device__ __forceinline__ bool store_split(char *d, const float (&v)[8]) {
@@ -698,10 +862,15 @@ __global__ void __launch_bounds__(256) clear_f32x4(float *__restrict__ p, int64_
 // 2,304: 281 and 297). Two K parts add into a cleared output (two addends: the same result in
 // any order). Swept over 8 layers and 6 products from 9 to 300 us, the choice was the fastest
 // or within 7% of it, one layer 10% off.
+// The small kernel: a set of eight K steps moves 160 KB (112 from a matrix) through a CU's vector
+// memory path, 2.3 us (1.7), a launch and the final sums take 3 us. Measured against the tiled
+// kernel, whole layers: 256 channels of 15 x 25 to 256 33 / 41 us, 512 to 512 62 / 66, 128 of
+// 30 x 40 23 / 29; 64 of 58 x 100 26 / 25, 96 to 160 of 4 x 20 x 30 32 / 30: the rule picks the
+// faster of each.
 struct Plan {
-  int nrb, kparts, mch, bn;
+  int nrb, kparts, mch, bn;  // nrb 0: the small kernel
 };
-Plan plan(const Params &p, int bn_max, bool rows_mode, bool can_split, bool nchw) {
+Plan plan(const Params &p, int bn_max, bool rows_mode, bool can_split, bool nchw, bool small) {
   const int cus = std::max(1, device_cus());
   Plan best{0, 1, 0, bn_max};
   double best_t = 0;
@@ -725,6 +894,10 @@ Plan plan(const Params &p, int bn_max, bool rows_mode, bool can_split, bool nchw
           best = Plan{nrb, kparts, (int)mch, bn};
         }
       }
+  const int64_t wgs = (int64_t)p.rb_total * ((p.Cout + kSmallCols - 1) / kSmallCols);
+  const double t = (double)((wgs + cus - 1) / cus) *
+                   ((p.kb_total + 7) / 8 * (rows_mode ? 4000.0 : 5600.0) + 7000.0);
+  if (t < best_t && small) best = Plan{0, 1, p.rb_total, kSmallCols};
   return best;
 }
 
@@ -740,7 +913,8 @@ Plan make_plan(Params &p, bool nchw) {
   p.rb_total = (p.M + 15) / 16;
   const bool can_split = deform(GEO) && !p.relu && p.kb_total >= 16 && (int64_t)p.M * p.Cout % 4 == 0 &&
                          reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
-  const Plan pl = plan(p, p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64), !deform(GEO), can_split, nchw);
+  const Plan pl = plan(p, p.Cout > 128 ? 256 : (p.Cout > 64 ? 128 : 64), !deform(GEO), can_split, nchw,
+                       GEO != kTConv);
   p.nt = (p.Cout + pl.bn - 1) / pl.bn;
   p.mch = pl.mch;
   p.kparts = pl.kparts;
@@ -755,6 +929,12 @@ hipError_t launch_geo(Params p, const Plan &pl, bool cleared, hipStream_t stream
   const int64_t wgs = (int64_t)p.mch * p.nt * p.kparts;
   if (wgs > (1 << 28)) return hipErrorInvalidValue;
   p.per_xcd = (int)((wgs + 7) / 8);
+  if constexpr (GEO != kTConv) {
+    if (pl.nrb == 0) {
+      hipLaunchKernelGGL((f32_small_kernel<GEO>), dim3(8 * p.per_xcd), dim3(kThreads), 0, stream, p);
+      return hipGetLastError();
+    }
+  }
   if (p.kparts == 2 && !cleared) {
     const int64_t n4 = n_out / 4;
     hipLaunchKernelGGL(clear_f32x4, dim3((unsigned)std::min<int64_t>((n4 + 255) / 256, 4096)),

@@ -69,3 +69,29 @@ def test_layer_nchw_f32(b, c, cout, h, w, stride, dg):
     ref = od.forward_nchw(x.double(), off.double(), mask.double(), weight.double(), bias.double(),
                           (stride, stride), (1, 1), (1, 1), 1, dg)
     check(out.cpu(), ref, torch.float32, "nchw layer")
+
+
+def test_small_layer_nonfinite_f32():
+    """The small-problem kernel's plain fp32 path: NaN / Inf in the input and in the weight reach
+    exactly the outputs they reach in float64."""
+    import _modulated_deform_conv_ext as ext
+    g = torch.Generator().manual_seed(9)
+    b, c, cout, h, w = 1, 64, 72, 12, 11
+    x = torch.randn(b, c, h, w, generator=g)
+    x[0, 7, 2, 3] = float("inf")
+    x[0, 9, 8, 8] = float("nan")
+    x[0, :, 5] = 0.0
+    off, mask = torch.zeros(b, 18, h, w), torch.ones(b, 9, h, w)
+    weight = 0.5 * torch.randint(1, 3, (cout, c, 3, 3), generator=g).float()
+    weight[3, 5, 1, 1] = float("-inf")
+    args = (b, c, h, w, h, w, cout, 3, 3, 1, 1, 1, 1, 1, 1, 1)
+    out = ext.dcn_layer_nchw_f32(*(t.to(DEV) for t in (x, off, mask, weight)), None, *args)
+    out = out.double().cpu()
+    ref = od.forward_nchw(x.double(), off.double(), mask.double(), weight.double(), None, (1, 1),
+                          (1, 1), (1, 1), 1, 1)
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert inf.any() and torch.equal(out[inf], ref[inf])
+    fin = torch.isfinite(ref)
+    assert 0.5 < fin.double().mean() < 1
+    check(out[fin], ref[fin], torch.float32, "finite outputs")
