@@ -10,14 +10,14 @@
 //   * msda_wave_kernel / msda_wave_lds_kernel: one wavefront owns UPW (b, q, head)
 //     units. G = D/VEC lanes cover the head_dim channels of one sample with 16-byte
 //     loads; the other lane groups take other (level, point) samples at the same time
-//     and the partial sums meet in a butterfly over the lane groups (lane_group_sum). All
-//     corner loads of a unit are issued before the first use. Corner loads are buffer
-//     loads: an invalid corner gets an out-of-range offset and reads 0 without a memory
-//     request, so the zero padding is branch-free.
-//     The _lds variant (many samples per unit) computes each sample's geometry once,
-//     in one lane, with the attention weight folded into the four corner weights, and
-//     shares it with the sample's lane group through LDS; the plain variant (few
-//     samples, or L/P known only at run time) lets every lane of the group compute it.
+//     and the partial sums meet in a butterfly over the lane groups (lane_group_sum).
+//     Corner loads are buffer loads: an invalid corner gets an out-of-range offset and
+//     reads 0 without a memory request, so the zero padding is branch-free.
+//     The _lds variant (level and point counts known at compile time) computes each
+//     sample's geometry once, in one lane, with the attention weight folded into the four
+//     corner weights, and shares it with the sample's lane group through LDS, two samples
+//     in flight per lane; the plain variant (few units, or L/P known only at run time)
+//     lets every lane of the group compute it.
 //   * Work order: units are enumerated per (batch, head-group) slice, queries in order,
 //     slices one after the other. The _lds variant lets XCD x take the x-th contiguous
 //     eighth of that order: each XCD works through its own slices (a whole slice at a
@@ -368,12 +368,19 @@ __device__ __forceinline__ void stream_slice_records(const WaveParams &p, int b,
 }
 
 // Compile-time L/P with UPW * L * P <= 64: lane i of the wave computes sample i of the
-// wave's UPW units, then every lane group gathers its samples' corners.
+// wave's UPW units, then every lane group gathers its samples' corners, NB samples (4 * NB
+// loads) at a time. What bounds it is the number of 128-byte lines the vector-memory path
+// serves, which needs many waves and few instructions per line: with two samples in flight
+// per lane a wave takes 34 to 63 registers (8 waves per SIMD) at any sample count. All of
+// a unit's samples in flight took 74 to 254 registers, 2 to 6 waves: 4 levels x 4 points
+// fp32, 2 x 10,000 queries, 8 heads of 32: 68.3 us, 2 at a time 57.5; 4 heads of 64: 86 us
+// and 60; 3 levels x 8 points, 4 x 5,000 queries: 117 us and 93. Four at a time: 59.4, 63,
+// 99 us; one: 58.1, 57.3, 95 us. A second launch bound instead spills (194 us and more).
 template <typename T, int D, int VEC, int NL, int NP, int UPW>
 __global__ void __launch_bounds__(kBlock) msda_wave_lds_kernel(const WaveParams p) {
   using V = Vec<T, VEC>;
   constexpr int G = D / VEC, LPU = kWave / UPW, SPU = LPU / G, NS = NL * NP;
-  constexpr int NITER = (NS + SPU - 1) / SPU;
+  constexpr int NITER = (NS + SPU - 1) / SPU, NB = NITER % 2 == 0 ? 2 : 1;
   static_assert(UPW * NS <= kWave && G >= 1 && (kWave % (G * UPW)) == 0, "bad lane split");
   __shared__ SampleGeo geo[kWavesPerBlock][UPW * NS];
 
@@ -435,35 +442,31 @@ __global__ void __launch_bounds__(kBlock) msda_wave_lds_kernel(const WaveParams 
   const T *vbase = static_cast<const T *>(p.value) + (int64_t)b * p.S * p.NH * D;
   const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(vbase, p.batch_bytes);
   const uint32_t cb = (uint32_t)(c0 * sizeof(T));
-  V v[NITER][4];
-  float w[NITER][4];
-#pragma unroll
-  for (int it = 0; it < NITER; ++it) {
-    const int s = it * SPU + gi;
-    if (NS % SPU == 0 || s < NS) {
-      const SampleGeo sg = geo[wave][u * NS + s];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        w[it][c] = sg.w[c];
-        v[it][c] = buffer_load_vec<T, VEC>(rsrc, sg.o[c] == kOOB ? kOOB : sg.o[c] + cb);
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        w[it][c] = 0.f;
-        v[it][c] = buffer_load_vec<T, VEC>(rsrc, kOOB);
-      }
-    }
-  }
   float acc[VEC];
 #pragma unroll
   for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
+#pragma unroll 1
+  for (int i0 = 0; i0 < NITER; i0 += NB) {
+    V v[NB][4];
+    float w[NB][4];
 #pragma unroll
-  for (int it = 0; it < NITER; ++it)
+    for (int j = 0; j < NB; ++j) {
+      const int s = (i0 + j) * SPU + gi;
+      const bool live = NS % (SPU * NB) == 0 || s < NS;
+      const SampleGeo sg = geo[wave][u * NS + (live ? s : 0)];
 #pragma unroll
-    for (int k = 0; k < VEC; ++k)
-      acc[k] += w[it][0] * (float)v[it][0].v[k] + w[it][1] * (float)v[it][1].v[k] +
-                w[it][2] * (float)v[it][2].v[k] + w[it][3] * (float)v[it][3].v[k];
+      for (int c = 0; c < 4; ++c) {
+        w[j][c] = live ? sg.w[c] : 0.f;
+        v[j][c] = buffer_load_vec<T, VEC>(rsrc, !live || sg.o[c] == kOOB ? kOOB : sg.o[c] + cb);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int k = 0; k < VEC; ++k)
+        acc[k] += w[j][0] * (float)v[j][0].v[k] + w[j][1] * (float)v[j][1].v[k] +
+                  w[j][2] * (float)v[j][2].v[k] + w[j][3] * (float)v[j][3].v[k];
+  }
   lane_group_sum<G, LPU>(acc);
   if (q < p.NQ && gi == 0) {
     V o;
@@ -881,17 +884,13 @@ constexpr int upw_for(int G, int ns) {
   return upw;
 }
 
-template <typename T, int D, int NL, int NP>
+// LDS = 0: the plain kernel (per-lane geometry; with NL = NP = 0 any level and point
+// counts). Else the shared-geometry kernel with LDS units per wave.
+template <typename T, int D, int NL, int NP, int LDS>
 hipError_t launch_wave_t(const MsdaArgs &a, hipStream_t stream) {
   constexpr int VEC = 16 / sizeof(T) < D ? 16 / sizeof(T) : D;
   constexpr int G = D / VEC;
-  constexpr bool kStatic = NL > 0 && NP > 0;
-  // Many samples per unit: shared geometry through LDS, two units per wave when their
-  // samples fit one geometry pass. Few samples: per-lane geometry, units packed so the
-  // wave's lanes are all busy.
-  constexpr bool kLds = kStatic && NL * NP >= 16 && NL * NP <= kWave;
-  constexpr int UPW = kLds ? (2 * NL * NP <= kWave && kWave % (2 * G) == 0 ? 2 : 1)
-                           : (kStatic ? upw_for(G, NL * NP) : 1);
+  constexpr int UPW = LDS > 0 ? LDS : NL > 0 ? upw_for(G, NL * NP) : 1;
   WaveParams p;
   p.value = a.value;
   p.shapes = a.spatial_shapes;
@@ -919,7 +918,7 @@ hipError_t launch_wave_t(const MsdaArgs &a, hipStream_t stream) {
   p.batch_bytes = (uint32_t)((int64_t)a.spatial_size * a.num_heads * D * sizeof(T));
   const int64_t blocks = slices * p.blocks_per_slice;
   if (blocks == 0) return hipSuccess;
-  if constexpr (kLds)
+  if constexpr (LDS > 0)
     hipLaunchKernelGGL((msda_wave_lds_kernel<T, D, VEC, NL, NP, UPW>), dim3((unsigned)blocks),
                        dim3(kBlock), 0, stream, p);
   else
@@ -1288,6 +1287,32 @@ hipError_t launch_tile_t(const MsdaArgs &a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Level and point counts known at compile time: the shared-geometry kernel with as many
+// units per wave as its 64 geometry lanes hold (back to back, 8 heads of 32 fp32, 2 x 10,000
+// queries, 4 x 4: 1 / 2 / 4 units per wave 79.5 / 64.4 / 57.5 us; 4 heads of 64, 16-bit:
+// 50.4 / 41.2 / 31.4 us, where the kernel for any counts takes 102 and 57 us; one level of
+// 8 points, 4 x 10,000 queries, 1 / 2 / 4 / 8: 134 / 91 / 72 / 67 us, any counts 130 us).
+// Few units leave most SIMDs with a wave or none, and then the serial chain of one wave
+// counts (GPU time of one call):
+//   * 16 to 31 samples, fewer than 2,048 units: one unit per wave (4 x 4, 100 queries, 8
+//     heads of 32, fp32: 3.3 us against 3.6; 300 queries, 4 heads of 64: 4.3 against 4.9;
+//     300 queries, 8 heads of 32: 3.9 and 3.9; 900 queries: 6.1 against 5.1).
+//   * fewer than 16 samples, fewer than 4,096 units: the kernel for any counts (3 x 4, 300
+//     queries, 8 heads: 4.0 us against 4.9; 900 queries: 7.7 against 5.8).
+template <typename T, int D, int NL, int NP>
+hipError_t launch_counts(const MsdaArgs &a, hipStream_t stream) {
+  constexpr int G = D * (int)sizeof(T) / 16, NS = NL * NP;
+  constexpr int MAXU = (kWave / G < kWave / NS ? kWave / G : kWave / NS);
+  constexpr int UPW = MAXU >= 8 ? 8 : MAXU >= 4 ? 4 : MAXU >= 2 ? 2 : 1;
+  const int64_t units = (int64_t)a.batch * a.num_query * a.num_heads;
+  if constexpr (NS < 16) {
+    if (units < 4096) return launch_wave_t<T, D, 0, 0, 0>(a, stream);
+  } else if constexpr (UPW > 2) {
+    if (units < 2048) return launch_wave_t<T, D, NL, NP, 1>(a, stream);
+  }
+  return launch_wave_t<T, D, NL, NP, UPW>(a, stream);
+}
+
 template <typename T>
 hipError_t launch_wave(const MsdaArgs &a, hipStream_t stream) {
   const int L = a.num_levels, P = a.num_point;
@@ -1298,7 +1323,7 @@ hipError_t launch_wave(const MsdaArgs &a, hipStream_t stream) {
         // cached kernel (whose partly cached level still costs a load per corner).
         if constexpr (sizeof(T) == 2)
           if (cached_worthwhile<T, 32, 4, 8>(a)) return launch_cached_t<T, 32, 4, 8, 12, 2>(a, stream);
-        return launch_wave_t<T, 32, 4, 8>(a, stream);
+        return launch_counts<T, 32, 4, 8>(a, stream);
       }
       if (L == 1 && P == 4) {  // BEVFormer TSA
         // the tiled kernel (neighbourhood in LDS) measured faster than the per-sample
@@ -1309,7 +1334,13 @@ hipError_t launch_wave(const MsdaArgs &a, hipStream_t stream) {
           else
             return launch_tile_t<T, 4, 16, 6, 8, 1, false>(a, stream);
         }
-        return launch_wave_t<T, 32, 1, 4>(a, stream);
+        // four samples: every lane's own geometry is cheap and its chain the shortest, so
+        // up to more units than elsewhere (7,200 units 3.3 us against 4.3 fp32, 3.3 / 3.8
+        // fp16; 16,000 units 5.3 / 4.8 and 4.5 / 4.2; 320,000 units 64.7 / 60.1 and
+        // 42.6 / 37.0)
+        if ((int64_t)a.batch * a.num_query * a.num_heads < 12288)
+          return launch_wave_t<T, 32, 1, 4, 0>(a, stream);
+        return launch_counts<T, 32, 1, 4>(a, stream);
       }
       if (L == 4 && P == 4) {  // Deformable DETR
         // 16-bit types: the LDS-cached kernel. fp32: the per-sample kernel, whose slice
@@ -1317,12 +1348,30 @@ hipError_t launch_wave(const MsdaArgs &a, hipStream_t stream) {
         // warm 138.6 -> 132.2 us against the cached kernel (fp16: 119.6 against 87.7 us).
         if constexpr (sizeof(T) == 2)
           if (cached_worthwhile<T, 32, 4, 4>(a)) return launch_cached_t<T, 32, 4, 4, 12, 2>(a, stream);
-        return launch_wave_t<T, 32, 4, 4>(a, stream);
+        return launch_counts<T, 32, 4, 4>(a, stream);
       }
-      return launch_wave_t<T, 32, 0, 0>(a, stream);
-    case 16: return launch_wave_t<T, 16, 0, 0>(a, stream);
-    case 64: return launch_wave_t<T, 64, 0, 0>(a, stream);
-    case 128: return launch_wave_t<T, 128, 0, 0>(a, stream);
+      if (L == 3 && P == 4) {
+        // as with four levels (2 x 10,000 queries fp16: 34.7 us against 43.8; 5,000 queries
+        // 15.3 against 13.4)
+        if constexpr (sizeof(T) == 2)
+          if (cached_worthwhile<T, 32, 3, 4>(a)) return launch_cached_t<T, 32, 3, 4, 12, 2>(a, stream);
+        return launch_counts<T, 32, 3, 4>(a, stream);
+      }
+      // (3 x 8 in 16 bits: 70.6 us, the cached kernel 69.2, the same within the noise)
+      if (L == 3 && P == 8) return launch_counts<T, 32, 3, 8>(a, stream);
+      if (L == 1 && P == 8) return launch_counts<T, 32, 1, 8>(a, stream);
+      return launch_wave_t<T, 32, 0, 0, 0>(a, stream);
+    case 16: return launch_wave_t<T, 16, 0, 0, 0>(a, stream);
+    case 64:
+      // 16-bit cached kernel: 35.4 us for 4 x 4 (here 31.4), 203 us for 4 x 8 (51)
+      if (L == 4 && P == 4) return launch_counts<T, 64, 4, 4>(a, stream);
+      if (L == 4 && P == 8) return launch_counts<T, 64, 4, 8>(a, stream);
+      if (L == 3 && P == 4) return launch_counts<T, 64, 3, 4>(a, stream);
+      if (L == 3 && P == 8) return launch_counts<T, 64, 3, 8>(a, stream);
+      if (L == 1 && P == 4) return launch_counts<T, 64, 1, 4>(a, stream);
+      if (L == 1 && P == 8) return launch_counts<T, 64, 1, 8>(a, stream);
+      return launch_wave_t<T, 64, 0, 0, 0>(a, stream);
+    case 128: return launch_wave_t<T, 128, 0, 0, 0>(a, stream);
     default: return launch_generic<T>(a, stream);
   }
 }

@@ -201,6 +201,35 @@ def test_geometries(geom, dtype):
     check(out, _ref(d, dtype), dtype, f"geom {geom}")
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("geom", [
+    # heads, head_dim, levels, points, queries on both sides of each unit-count line of the
+    # dispatch (4,096 units below 16 samples, 12,288 for one level of 4 points, 2,048 from
+    # 16 samples on), off the units of a workgroup; the last sizes stream their slices
+    (8, 32, 1, 4, (5, 1535, 1537)), (8, 32, 1, 8, (511, 513)), (8, 32, 3, 4, (511, 8195)),
+    (8, 32, 3, 8, (1, 259)), (8, 32, 4, 4, (255, 257, 4099)), (7, 32, 3, 4, (587,)),
+    (4, 64, 1, 4, (1023, 1025)), (4, 64, 1, 8, (1023, 1031)), (4, 64, 3, 4, (1023, 1033)),
+    (4, 64, 3, 8, (3, 261)), (4, 64, 4, 4, (511, 513)), (3, 64, 4, 8, (85, 2051)),
+])
+def test_level_and_point_counts(geom, dtype):
+    """Every kernel with compile-time level and point counts against the one-thread-per-
+    element kernel on the whole output and the oracle on some queries."""
+    nh, hd, nl, npnt, counts = geom
+    shapes = [(19, 26), (10, 13), (5, 7), (1, 4)][:nl]
+    for nq in counts:
+        d = inputs.msda_random(1, shapes, nq, nh, hd, npnt, seed=43, loc_lo=-0.2, loc_hi=1.2)
+        out = _run(d, dtype)
+        gen = _run(d, dtype, force_generic=True)
+        if dtype == torch.float32:
+            # at most 32 samples x 4 corners of N(0, 1) values times weights that sum to 1:
+            # a sum in another order differs by at most 128 rounding steps of its size
+            torch.testing.assert_close(out, gen, rtol=1e-5, atol=1e-5)
+        else:
+            check(out.double(), gen.double(), dtype, f"counts vs generic {geom} {nq}")
+        q_idx = torch.arange(0, nq, max(1, nq // 50))
+        check(out[:, q_idx], _ref(d, dtype, q_idx), dtype, f"counts {geom} {nq}")
+
+
 def test_edge_locations():
     """Pixel centres return the pixel, loc 0/1 give half-weight edges, far-out samples
     are zero, loc exactly at the -1 / H gates."""
