@@ -39,8 +39,8 @@ struct MsdaBwdArgs {
 
 // Bytes of fp32 accumulator the 16-bit backward needs at least (0 for f32 / f64).
 int64_t msda_backward_workspace_min(int dtype, int64_t value_elems);
-// Bytes that also hold the buffers of the sorted grad_value path (D = 32), which runs when
-// the workspace is at least this large.
+// Bytes that also hold the buffers of the sorted grad_value path (D = 32; 64 with many
+// samples), which runs when the workspace is at least this large.
 int64_t msda_backward_workspace_bytes(int dtype, int64_t batch, int64_t spatial_size,
                                       int64_t num_heads, int64_t channels, int64_t num_levels,
                                       int64_t num_query, int64_t num_point);

@@ -21,7 +21,7 @@
 // fp32 workspace that is cleared here, accumulated, and narrowed into grad_value at the
 // end (binding_musa.mu:456-510 does the same for fp16).
 //
-// D = 32 with fp32 accumulation (every BEVFormer and DETR shape) and a workspace of
+// D = 32 (every BEVFormer and DETR shape) or 64 with fp32 accumulation and a workspace of
 // msda_backward_workspace_bytes takes the sorted path (the msda_bkt_* kernels and
 // msda_coord_kernel below): the corner adds are bucketed by position and each bucket is
 // summed by the workgroup that owns its grad_value rows, so no corner takes an atomic.
@@ -908,12 +908,15 @@ struct BktParams {
   int *count;       // [nbk] records per bucket
   int *cursor;      // [nbk] next free slot (offsets after the scan)
   int *offset;      // [nbk + 1]
-  int *nitems;      // [8] pieces per XCD list, then [8] work-queue counters
+  int *nitems;      // [8] pieces per XCD list, then [8] work-queue counters per accumulate launch
   int4 *items;      // [8][item_cap] (bucket, first record, records, 1 if the bucket is one piece)
   float2 *rw;       // [capacity] record weights: (position, next position)
   uint32_t *rq;     // [capacity] query << kBkShift | position in bucket
   int64_t go_sb, go_sq, go_sh, go_sc;
   uint32_t go_rows_bytes;  // bytes from row (b, 0, h, 0) past row (b, NQ - 1, h, 31)
+  int row, dim;     // the accumulate kernel: grad_value position length NH * dim, channels of
+                    // a head (grad_out and gv point at the first of the launch's 32 channels)
+  int queue;        //   and its work-queue counters: nitems[queue + XCD]
   int B, NH, NQ, NL, NP, S, NBS, nbk, item_cap, qpb;
   int by_bucket;    // fewer than 8 slices: buckets go to XCD bucket % 8, else slice % 8
   int blocks_per_xcd;
@@ -1157,7 +1160,7 @@ __global__ void __launch_bounds__(1024) msda_bkt_scan_kernel(const BktParams p) 
   if (tid == 0) {
     if (x == 0) p.offset[p.nbk] = total[0];
     p.nitems[x] = min(total[1] + total[2], p.item_cap);
-    p.nitems[8 + x] = 0;  // the accumulate kernel's queue
+    p.nitems[8 + x] = p.nitems[16 + x] = 0;  // the accumulate launches' queues
   }
 }
 
@@ -1290,7 +1293,7 @@ __global__ void __launch_bounds__(kAccThreads, 4) msda_bkt_acc_kernel(const BktP
   const int cl = tid % LPC, gi = tid / LPC;
   const int xcd = blockIdx.x & 7;
   const int n_items = p.nitems[xcd];
-  int *queue = p.nitems + 8 + xcd;
+  int *queue = p.nitems + p.queue + xcd;
   const int4 *items = p.items + (int64_t)xcd * p.item_cap;
   const T *gout = static_cast<const T *>(p.grad_out);
   // the records of a chunk, kAccPerThread per thread (streamed once: non-temporal loads
@@ -1509,7 +1512,7 @@ __global__ void __launch_bounds__(kAccThreads, 4) msda_bkt_acc_kernel(const BktP
     // rows no record reached are skipped): 4 channels per thread for the plain
     // read-modify-write; atomics on consecutive floats across the lanes (the L2 works per
     // line of each atomic instruction)
-    float *gvb = p.gv + ((int64_t)b * p.S + (int64_t)kb * kBkPos) * (p.NH * D) + h * D;
+    float *gvb = p.gv + ((int64_t)b * p.S + (int64_t)kb * kBkPos) * p.row + h * p.dim;
     const int npos = min(kBkPos + 1, p.S - kb * kBkPos);
     __syncthreads();
     auto used = [&](int pp) __attribute__((always_inline)) {
@@ -1520,7 +1523,7 @@ __global__ void __launch_bounds__(kAccThreads, 4) msda_bkt_acc_kernel(const BktP
         const int pp = i / (D / 4), c = (i - pp * (D / 4)) * 4;
         if (used(pp)) {
           const float4 v = *reinterpret_cast<const float4 *>(&accs[pp * D + c]);
-          float *dst = gvb + (int64_t)pp * (p.NH * D) + c;
+          float *dst = gvb + (int64_t)pp * p.row + c;
           if (pp == 0 || pp == kBkPos) {
             unsafeAtomicAdd(dst, v.x);
             unsafeAtomicAdd(dst + 1, v.y);
@@ -1536,14 +1539,14 @@ __global__ void __launch_bounds__(kAccThreads, 4) msda_bkt_acc_kernel(const BktP
     } else {
       for (int i = tid; i < npos * D; i += kAccThreads) {
         const int pp = i / D, c = i - pp * D;
-        if (used(pp)) unsafeAtomicAdd(gvb + (int64_t)pp * (p.NH * D) + c, accs[i]);
+        if (used(pp)) unsafeAtomicAdd(gvb + (int64_t)pp * p.row + c, accs[i]);
       }
     }
     m = __builtin_amdgcn_readfirstlane(s_next);
   }
 }
 
-// grad_sampling_loc / grad_attn_weight for D = 32 without grad_value. A wave takes a tile
+// grad_sampling_loc / grad_attn_weight for D = 32 or 64 without grad_value. A wave takes a tile
 // of queries of one (batch, head) slice, `upi` units at a time (upi * L * P <= 64 samples,
 // one per lane; more samples than 64 go in chunks of 64 with upi = 1):
 //   1. lane i takes sample i: loads its location and attention weight, and writes the four
@@ -1575,16 +1578,18 @@ struct CoordParams {
   int64_t nn4;
 };
 
-// Sum over each LPS-lane group (4 or 8) with DPP moves, no LDS traffic: xor 1 and xor 2
+// Sum over each LPS-lane group (4, 8 or 16) with DPP moves, no LDS traffic: xor 1 and xor 2
 // inside each quad (quad_perm [1,0,3,2] and [2,3,0,1]); for 8 lanes, row_shr:4 then adds
 // the lower quad's sum to the upper quad (lanes whose source is outside the 16-lane row
-// read 0). Lane LPS - 1 of the group ends with the group's total.
+// read 0); for 16 lanes, row_shr:8 then adds lane 7's sum to lane 15's. Lane LPS - 1 of the group ends with the group's total.
 template <int LPS>
 __device__ __forceinline__ float group_sum(float v) {
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));
-  if constexpr (LPS == 8)
+  if constexpr (LPS >= 8)
     v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x114, 0xF, 0xF, true));
+  if constexpr (LPS == 16)
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x118, 0xF, 0xF, true));
   return v;
 }
 
@@ -1625,9 +1630,9 @@ __device__ __forceinline__ void wave_lds_handover() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <typename T>
+template <typename T, int D>
 __global__ void __launch_bounds__(kCoWaves * kWave) msda_coord_kernel(const CoordParams p) {
-  constexpr int D = 32, VEC = 16 / (int)sizeof(T), LPS = D / VEC, G = kWave / LPS;
+  constexpr int VEC = 16 / (int)sizeof(T), LPS = D / VEC, G = kWave / LPS;
   constexpr uint32_t kPast = 0x80000000u;
   __shared__ uint4 s_off[kCoWaves][kWave];   // corner byte offsets
   __shared__ float4 s_par[kCoWaves][kWave];  // lh, lw, a * H, a * W
@@ -1875,14 +1880,26 @@ int64_t half_acc_bytes(int dtype, int64_t value_elems) {
   return (dtype == 1 || dtype == 2) ? (value_elems * (int64_t)sizeof(float) + 255) / 256 * 256 : 0;
 }
 
-// The sorted path: D = 32, fp32 accumulation (f32 / f16 / bf16 inputs), one batch of value
+// Head dimensions of the sorted path. 64 channels take it from 128 Ki samples on: its seven
+// launches against the atomic kernel's one or two cost a small call more than the atomics do
+// (training step, 4 heads of 64, 4 x 4, fp32: 900 queries, 58 K samples, atomics 125 us and
+// sorted 143; 2,000 queries, 128 K samples, 140 / 138; 2 x 10,000 queries 1,081 / 289; 3 x 8,
+// 4 x 5,000 queries 1,379 / 356, fp16 1,386 / 300; one level, 15,000 grid cells, 222 / 139).
+bool sorted_dim(int64_t channels, int64_t samples) {
+  return channels == 32 || (channels == 64 && samples >= ((int64_t)1 << 17));
+}
+
+// The sorted path: D = 32 or 64, fp32 accumulation (f32 / f16 / bf16 inputs), one batch of value
 // under 2 GiB (32-bit buffer offsets), and a workspace that holds its buffers.
 template <typename T>
 bool sorted_path(const MsdaBwdArgs &a, int dtype, BktLayout &L) {
-  if (a.f.channels != 32 || a.f.batch <= 0 || a.f.num_heads <= 0 || a.f.num_query <= 0 ||
+  const int64_t D = a.f.channels;
+  if (!sorted_dim(D, (int64_t)a.f.batch * a.f.num_query * a.f.num_heads * a.f.num_levels *
+                         a.f.num_point) ||
+      a.f.batch <= 0 || a.f.num_heads <= 0 || a.f.num_query <= 0 ||
       a.f.num_levels <= 0 || a.f.num_point <= 0 || device_cus() < 8)
     return false;
-  if ((int64_t)a.f.spatial_size * a.f.num_heads * 32 * (int64_t)sizeof(T) >= ((int64_t)1 << 31))
+  if ((int64_t)a.f.spatial_size * a.f.num_heads * D * (int64_t)sizeof(T) >= ((int64_t)1 << 31))
     return false;
   if ((int64_t)a.f.batch * a.f.num_query * a.f.num_heads >= ((int64_t)1 << 31) / 64) return false;
   // sample indices of loc / grad_loc in 32 bits
@@ -1902,13 +1919,13 @@ bool sorted_path(const MsdaBwdArgs &a, int dtype, BktLayout &L) {
       (a.go_stride[2] * (int64_t)sizeof(T)) % 16 != 0)
     return false;
   if (a.go_stride[1] < 0 || a.go_stride[3] != 1 || (a.go_stride[1] * (int64_t)sizeof(T)) % 16 != 0 ||
-      ((int64_t)(a.f.num_query - 1) * a.go_stride[1] + 31 * a.go_stride[3] + 1) * (int64_t)sizeof(T) >=
+      ((int64_t)(a.f.num_query - 1) * a.go_stride[1] + D) * (int64_t)sizeof(T) >=
           ((int64_t)1 << 31))
     return false;
   L = bkt_layout(a.f.batch, a.f.spatial_size, a.f.num_heads, a.f.num_levels, a.f.num_query,
                  a.f.num_point);
   if (L.bytes == 0) return false;
-  const int64_t value_elems = (int64_t)a.f.batch * a.f.spatial_size * a.f.num_heads * 32;
+  const int64_t value_elems = (int64_t)a.f.batch * a.f.spatial_size * a.f.num_heads * D;
   return a.workspace != nullptr &&
          a.workspace_bytes >= half_acc_bytes(dtype, value_elems) + L.bytes;
 }
@@ -1968,8 +1985,16 @@ hipError_t launch_sorted(const MsdaBwdArgs &a, const BktLayout &L, char *ws, flo
   hipLaunchKernelGGL((msda_bkt_place_kernel<T>), dim3(8u * (unsigned)place_pblk), dim3(kBkThreads), 0,
                      stream, p);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL((msda_bkt_acc_kernel<T>), dim3(blocks), dim3(kAccThreads), 0, stream, p);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  // 32 channels of every head per launch: the records, sorted once, serve each
+  p.dim = a.f.channels;
+  p.row = a.f.num_heads * a.f.channels;
+  p.queue = 8;
+  for (int ch0 = 0; ch0 < p.dim; ch0 += 32, p.queue += 8) {
+    p.grad_out = static_cast<const T *>(a.grad_output) + ch0;
+    p.gv = gv + ch0;
+    hipLaunchKernelGGL((msda_bkt_acc_kernel<T>), dim3(blocks), dim3(kAccThreads), 0, stream, p);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
   CoordParams c;
   c.value = a.f.value;
   c.loc = a.f.sampling_loc;
@@ -1992,7 +2017,10 @@ hipError_t launch_sorted(const MsdaBwdArgs &a, const BktLayout &L, char *ws, flo
   c.ndst = a.grad_value;
   c.nn4 = fused_n / 4;
   const unsigned cgrid = 8u * (unsigned)((c.nt8 + kCoWaves - 1) / kCoWaves);
-  hipLaunchKernelGGL((msda_coord_kernel<T>), dim3(cgrid), dim3(kCoWaves * kWave), 0, stream, c);
+  if (a.f.channels == 64)
+    hipLaunchKernelGGL((msda_coord_kernel<T, 64>), dim3(cgrid), dim3(kCoWaves * kWave), 0, stream, c);
+  else
+    hipLaunchKernelGGL((msda_coord_kernel<T, 32>), dim3(cgrid), dim3(kCoWaves * kWave), 0, stream, c);
   return hipGetLastError();
 }
 
@@ -2198,7 +2226,8 @@ int64_t msda_backward_workspace_bytes(int dtype, int64_t batch, int64_t spatial_
                                       int64_t num_heads, int64_t channels, int64_t num_levels,
                                       int64_t num_query, int64_t num_point) {
   const int64_t value_elems = batch * spatial_size * num_heads * channels;
-  if (dtype == 3 || channels != 32) return msda_backward_workspace_min(dtype, value_elems);
+  if (dtype == 3 || !sorted_dim(channels, batch * num_query * num_heads * num_levels * num_point))
+    return msda_backward_workspace_min(dtype, value_elems);
   const BktLayout L = bkt_layout(batch, spatial_size, num_heads, num_levels, num_query, num_point);
   if (L.bytes == 0) return msda_backward_workspace_min(dtype, value_elems);
   return half_acc_bytes(dtype, value_elems) + L.bytes;

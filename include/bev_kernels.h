@@ -406,7 +406,8 @@ int bevk_msda_forward(
 /* Bytes of workspace for bevk_msda_backward, -1 for an unknown dtype or a negative size.
  * F16/BF16 need at least an fp32 accumulator of batch*spatial_size*num_heads*channels
  * elements (the reference allocates it inside its fp16 backward, binding_musa.mu:456-463;
- * here the caller owns it); F32/F64 need none. With channels == 32 the value returned
+ * here the caller owns it); F32/F64 need none. With channels == 32, or 64 and at least
+ * 131,072 samples (batch * num_query * num_heads * num_levels * num_point), the value returned
  * also holds the buffers of the sorted grad_value path (for every sample, up to two
  * 12-byte records, one per image row of its valid corners, bucketed by position), which
  * bevk_msda_backward takes whenever
@@ -432,7 +433,7 @@ int64_t bevk_msda_backward_workspace_bytes(int dtype, int batch, int spatial_siz
  * im2col_step keeps the reference's contract. force_generic_col2im != 0 runs the
  * per-(batch, query, head) kernel alone, adding every level's grad_value with atomics
  * (the reference's generic col2im, binding_musa.mu:459); otherwise the sorted grad_value
- * path (D = 32, full workspace), then the grid-query owner pass or the D = 32 kernel with
+ * path (D = 32 or 64, full workspace), then the grid-query owner pass or the D = 32 kernel with
  * the coarse-level sort (smaller workspaces) are used where they apply.
  * spatial_shapes / level_start_index must describe value (lsi[l] + H_l * W_l <=
  * spatial_size), as in the reference; they are read on the device only.

@@ -181,6 +181,9 @@ def test_msda_backward_workspace_bytes():
     assert f(1, 2, 10, 8, 32, 1, 4, 4) == acc(2 * 10 * 8 * 32) + _sorted_bytes(2, 10, 8, 1, 4, 4)
     assert f(2, 6, 30825, 8, 32, 4, 10000, 8) == (acc(6 * 30825 * 8 * 32)
                                                  + _sorted_bytes(6, 30825, 8, 4, 10000, 8))
+    # D == 64: from 128 Ki samples on
+    assert f(0, 2, 1000, 8, 64, 4, 511, 4) == 0
+    assert f(0, 2, 1000, 8, 64, 4, 512, 4) == _sorted_bytes(2, 1000, 8, 4, 512, 4)
     assert f(4, 2, 10, 8, 32, 1, 4, 4) == -1
     assert f(1, -1, 10, 8, 32, 1, 4, 4) == -1
     assert f(1, 2, 10, 8, 32, 1, -4, 4) == -1

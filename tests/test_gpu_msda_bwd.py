@@ -390,6 +390,27 @@ def test_sorted_ragged(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("geom", [
+    # batch, shapes, queries, heads, channels, points
+    (3, [(20, 30), (10, 15), (5, 8)], 1217, 3, 64, 4),  # 9 slices, ragged buckets and tiles
+    (1, [(16, 16), (8, 8), (4, 4), (2, 2)], 1025, 4, 64, 8),
+    (2, [(25, 41)], 16387, 1, 64, 4),                   # 2 slices: buckets spread over XCDs
+    (1, [(7, 5), (3, 3)], 937, 2, 64, 35),              # 70 samples: two coordinate passes
+    (1, [(25, 41)], 32767, 1, 64, 4),                   # 4 samples below the line: atomics
+])
+def test_sorted_two_halves(geom, dtype):
+    """Heads of 64 channels: the records are sorted once and summed in two launches of 32
+    channels each; concentrated locations too, whose buckets fill several pieces."""
+    d = inputs.msda_random(*geom, seed=19, loc_lo=-0.2, loc_hi=1.2)
+    go = _grad_output(d, seed=8)
+    _check3(_run(d, go, dtype), _ref(d, go, dtype), dtype, f"halves {geom} {dtype}")
+    if len(geom[1]) == 3:
+        g = torch.Generator().manual_seed(3)
+        d["sampling_loc"] = 0.5 + 0.02 * torch.randn(d["sampling_loc"].shape, generator=g)
+        _check3(_run(d, go, dtype), _ref(d, go, dtype), dtype, f"halves, one place {dtype}")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 @pytest.mark.parametrize("num_query", [60, 2500], ids=["one_chunk", "pieces"])
 def test_sorted_bucket_edges(num_query, dtype):
     """Sorted path, records at the edges of the 256-position buckets of a 6 x 100 map
