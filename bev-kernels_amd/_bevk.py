@@ -50,7 +50,6 @@ _SIGNATURES = {
     "bevk_dcn_fused_fwd_nhwc": [_i, _vp, _vp, _i, _vp, _vp, _vp] + [_i] * 15 + [_vp, _vp],
     "bevk_f32_split_weight_bytes": [_i] * 2,
     "bevk_dcn_split_weight": [_vp] + [_i] * 5 + [_vp, _vp],
-    "bevk_dcn_fused_fwd_nhwc_f32": [_vp, _vp, _i, _vp, _vp, _vp] + [_i] * 16 + [_vp, _vp],
     "bevk_gemm_f32": [_vp, _vp] + [_i] * 3 + [_vp, _vp],
     "bevk_dcn_weight_grad_workspace_bytes": [_i, ctypes.c_int64] + [_i] * 3,
     "bevk_dcn_weight_grad": [_i, _vp, _vp, ctypes.c_int64] + [_i] * 3 + [_vp, ctypes.c_int64, _i,

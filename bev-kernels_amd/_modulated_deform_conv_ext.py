@@ -46,7 +46,6 @@ __all__ = [
     "dcn_pack_weight",
     "dcn_fused_fwd_nhwc",
     "dcn_split_weight",
-    "dcn_fused_fwd_nhwc_f32",
     "gemm_f32",
     "dcn_weight_grad",
     "dcn_layer_nchw_f32",
@@ -243,8 +242,8 @@ def dcn_fused_fwd_nhwc(data_im, data_offset, data_mask, weight_packed, bias, bat
 
 
 def dcn_split_weight(weight, transposed=False):
-    """fp32 module weight [Cout, C, kh, kw] -> its split form (uint8) for dcn_fused_fwd_nhwc_f32
-    or, transposed, for gemm_f32 with columns (tap, C) and terms Cout."""
+    """fp32 module weight [Cout, C, kh, kw] -> its split form (uint8) for gemm_f32: columns
+    Cout, terms (tap, C) or, transposed, columns (tap, C) and terms Cout."""
     fn = "dcn_split_weight"
     _b.require_device(fn, weight)
     _b.require_contiguous(fn, weight=weight)
@@ -263,39 +262,6 @@ def _require_split(fn, split, n, k):
     if split.dtype != torch.uint8:
         raise RuntimeError(f"{fn}: weight_split must come from dcn_split_weight")
     _b.require_numel(fn, "weight_split", split, _b.lib().bevk_f32_split_weight_bytes(n, k))
-
-
-def dcn_fused_fwd_nhwc_f32(data_im, data_offset, data_mask, weight_split, bias, batch_size,
-                           channels, height_im, width_im, height_col, width_col, channels_out,
-                           kernel_h, kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h,
-                           dilation_w, out, act_relu=False):
-    """dcn_fused_fwd_nhwc for float32 on the bf16 matrix cores (weight_split from
-    dcn_split_weight; C % 32 == 0, at most 9 taps), with an optional ReLU."""
-    fn = "dcn_fused_fwd_nhwc_f32"
-    _b.require_device(fn, data_im, data_offset, data_mask, weight_split, bias, out)
-    _b.require_contiguous(fn, data_im=data_im, data_offset=data_offset, data_mask=data_mask,
-                          weight_split=weight_split, bias=bias, out=out)
-    taps = kernel_h * kernel_w
-    last = data_offset.size(-1)
-    fused_y = last == 3 * taps
-    if data_im.dtype != torch.float32:
-        raise RuntimeError(f"{fn}: data_im must be float32, got {data_im.dtype}")
-    _b.require_dtype(fn, data_im, data_offset=data_offset, bias=bias, out=out,
-                     data_mask=None if fused_y else data_mask)
-    m = batch_size * height_col * width_col
-    _b.require_numel(fn, "data_im", data_im, batch_size * height_im * width_im * channels)
-    _b.require_numel(fn, "data_offset", data_offset, m * last)
-    if not fused_y:
-        _b.require_numel(fn, "data_mask", data_mask, m * taps)
-    _require_split(fn, weight_split, channels_out, taps * channels)
-    if bias is not None:
-        _b.require_numel(fn, "bias", bias, channels_out)
-    _b.require_numel(fn, "out", out, m * channels_out)
-    _b.call("bevk_dcn_fused_fwd_nhwc_f32", _b.ptr(data_im), _b.ptr(data_offset), last,
-            _b.ptr(data_mask), _b.ptr(weight_split), _b.ptr(bias), batch_size, channels,
-            height_im, width_im, height_col, width_col, channels_out, kernel_h, kernel_w, pad_h,
-            pad_w, stride_h, stride_w, dilation_h, dilation_w, int(act_relu), _b.ptr(out),
-            _b.stream_of(data_im))
 
 
 def gemm_f32(a, weight_split, n, out):

@@ -577,44 +577,6 @@ int bevk_dcn_split_weight(const void *weight, int channels_out, int kernel_h, in
                     fn);
 }
 
-int bevk_dcn_fused_fwd_nhwc_f32(const void *data_im, const void *data_offset, int offset_last_dim,
-                                const void *data_mask, const void *weight_split, const void *bias,
-                                int batch_size, int channels, int height_im, int width_im,
-                                int height_col, int width_col, int channels_out, int kernel_h,
-                                int kernel_w, int pad_h, int pad_w, int stride_h, int stride_w,
-                                int dilation_h, int dilation_w, int act_relu, void *out,
-                                void *stream) {
-  const char *fn = "dcn_fused_fwd_nhwc_f32";
-  g_last_error.clear();
-  const bevk::DcnGeom g =
-      make_geom(batch_size, channels, height_im, width_im, height_col, width_col, kernel_h,
-                kernel_w, pad_h, pad_w, stride_h, stride_w, dilation_h, dilation_w, 1);
-  if (int rc = check_geom(fn, g)) return rc;
-  if (channels_out < 0) return fail(BEVK_ERR_INVALID, "%s: negative channels_out", fn);
-  const int taps = kernel_h * kernel_w;
-  if (offset_last_dim != 2 * taps && offset_last_dim != 3 * taps)
-    return fail(BEVK_ERR_INVALID, "%s: offset last dim must be 2T (%d) or 3T (%d), got %d", fn,
-                2 * taps, 3 * taps, offset_last_dim);
-  const bool fused_y = offset_last_dim == 3 * taps;
-  const long long m = (long long)batch_size * height_col * width_col;
-  if (m * channels_out == 0) return ok();
-  if (channels <= 0 || channels % 32 != 0 || taps > 9)
-    return fail(BEVK_ERR_UNSUPPORTED, "%s: channels (%d) must be a multiple of 32, at most 9 taps",
-                fn, channels);
-  if ((long long)batch_size * height_im * width_im * channels * 4 > kMaxBufferBytes ||
-      bevk::f32_split_weight_bytes(channels_out, (long long)taps * channels) > kMaxBufferBytes ||
-      m >= (1LL << 30))
-    return fail(BEVK_ERR_INVALID, "%s: problem too large for 32-bit buffer offsets", fn);
-  if (!data_im || !data_offset || (!fused_y && !data_mask) || !weight_split || !out)
-    return fail(BEVK_ERR_INVALID, "%s: null tensor pointer", fn);
-  return hip_status(
-      bevk::launch_f32_split(&g, channels_out, (int)m, taps * channels, data_im, data_offset,
-                             fused_y ? bevk::kGeoY : bevk::kGeoMask, data_mask, weight_split,
-                             static_cast<const float *>(bias), static_cast<float *>(out),
-                             (hipStream_t)stream, act_relu != 0),
-      fn);
-}
-
 int bevk_gemm_f32(const void *a, const void *weight_split, int m, int k, int n, void *out,
                   void *stream) {
   const char *fn = "gemm_f32";

@@ -166,19 +166,10 @@ int bevk_dcn_layer_col2im_nhwc(
  *                                columns Cout, terms (tap, C) with C % 32 == 0; transposed:
  *                                columns (tap, C), terms Cout with C % 16 == 0, Cout % 32 == 0;
  *                                at most 9 taps
- *   bevk_dcn_fused_fwd_nhwc_f32  bevk_dcn_fused_fwd_nhwc for F32 with the split weight
- *                                (C % 32 == 0, at most 9 taps) and an optional ReLU
  *   bevk_gemm_f32                out [m, n] = a [m, k] times the split weight's columns */
 int64_t bevk_f32_split_weight_bytes(int n, int k);
 int bevk_dcn_split_weight(const void *weight, int channels_out, int kernel_h, int kernel_w,
                           int channels, int transposed, void *split, void *stream);
-int bevk_dcn_fused_fwd_nhwc_f32(const void *data_im, const void *data_offset, int offset_last_dim,
-                                const void *data_mask, const void *weight_split, const void *bias,
-                                int batch_size, int channels, int height_im, int width_im,
-                                int height_col, int width_col, int channels_out, int kernel_h,
-                                int kernel_w, int pad_h, int pad_w, int stride_h, int stride_w,
-                                int dilation_h, int dilation_w, int act_relu, void *out,
-                                void *stream);
 int bevk_gemm_f32(const void *a, const void *weight_split, int m, int k, int n, void *out,
                   void *stream);
 
