@@ -1008,8 +1008,11 @@ __device__ __forceinline__ void sample_corners(const BktParams &p, int l, const 
 
 // The two records of a sample (r = 0: corners 0 and 1, image row y0; r = 1: corners 2 and
 // 3, row y0 + 1). Both corners valid: position of the left one, weights (left, right);
-// one valid: its position, weights (its weight, 0); none: position -1. The right corner of
-// a row is the position after the left one.
+// one valid: its position, weights (its weight, kNoCorner); none: position -1. The right
+// corner of a row is the position after the left one. A valid right corner's weight is never
+// the bits of kNoCorner (-0): 0 is added to it.
+constexpr uint32_t kNoCorner = 0x80000000u;
+
 template <typename T>
 __device__ __forceinline__ void sample_records(const BktParams &p, int l, const Vec<T, 2> &xy,
                                                T at, int (&rp)[2], float2 (&rw)[2]) {
@@ -1020,8 +1023,9 @@ __device__ __forceinline__ void sample_records(const BktParams &p, int l, const 
   for (int r = 0; r < 2; ++r) {
     const int a = pos[2 * r], b = pos[2 * r + 1];
     rp[r] = a >= 0 ? a : b;
-    rw[r] = a >= 0 ? make_float2(wt[2 * r], b >= 0 ? wt[2 * r + 1] : 0.f)
-                   : make_float2(wt[2 * r + 1], 0.f);
+    const float none = __builtin_bit_cast(float, kNoCorner);
+    rw[r] = a >= 0 ? make_float2(wt[2 * r], b >= 0 ? wt[2 * r + 1] + 0.f : none)
+                   : make_float2(wt[2 * r + 1], none);
   }
 }
 
@@ -1273,7 +1277,10 @@ __global__ void __launch_bounds__(kBkThreads) msda_bkt_place_kernel(const BktPar
 // workgroup writes those rows), else with atomics. The bucket's first row and the row
 // after the bucket are also reached by the neighbouring buckets' records (and the pieces
 // that sum them), so they always take atomics.
-template <typename T>
+// EXACT: a record of one corner adds nothing to the position after it, whatever grad_output
+// holds (the select per channel keeps NaN / Inf where the per-corner kernels put them, which is
+// what heads of 64 ran before); else it adds 0 * grad_output there.
+template <typename T, bool EXACT>
 __global__ void __launch_bounds__(kAccThreads, 4) msda_bkt_acc_kernel(const BktParams p) {
   // a group of LPC lanes reads one 128-byte (fp32) or 64-byte (16-bit) grad_output row,
   // 16 bytes per lane
@@ -1470,11 +1477,12 @@ __global__ void __launch_bounds__(kAccThreads, 4) msda_bkt_acc_kernel(const BktP
                 }
                 pos = np;
               }
+              const bool one = EXACT && __builtin_bit_cast(uint32_t, w[u].y) == kNoCorner;
 #pragma unroll
               for (int c = 0; c < VEC; ++c) {
                 const float g = (float)v[u].v[c];
                 accl[c] += w[u].x * g;
-                accr[c] += w[u].y * g;
+                accr[c] += w[u].y * (one ? 0.f : g);
               }
             }
           }
@@ -1992,7 +2000,10 @@ hipError_t launch_sorted(const MsdaBwdArgs &a, const BktLayout &L, char *ws, flo
   for (int ch0 = 0; ch0 < p.dim; ch0 += 32, p.queue += 8) {
     p.grad_out = static_cast<const T *>(a.grad_output) + ch0;
     p.gv = gv + ch0;
-    hipLaunchKernelGGL((msda_bkt_acc_kernel<T>), dim3(blocks), dim3(kAccThreads), 0, stream, p);
+    if (p.dim == 32)
+      hipLaunchKernelGGL((msda_bkt_acc_kernel<T, false>), dim3(blocks), dim3(kAccThreads), 0, stream, p);
+    else
+      hipLaunchKernelGGL((msda_bkt_acc_kernel<T, true>), dim3(blocks), dim3(kAccThreads), 0, stream, p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   CoordParams c;

@@ -762,6 +762,26 @@ def test_nonfinite_backward(kind, dtype):
     assert 0.05 < fin < 0.999, f"{what}: degenerate poison pattern"
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+def test_nonfinite_border_two_halves(dtype):
+    """Heads of 64 on the sorted path: a NaN grad_output of samples with one valid corner in a
+    row (left and right border) reaches the valid corners only, not the positions after them."""
+    H, W, nq = 25, 41, 32771
+    d = inputs.msda_random(1, [(H, W)], nq, 1, 64, 4, seed=29, loc_lo=-0.2, loc_hi=1.2)
+    go = _grad_output(d, seed=8)
+    for q, (px, py) in enumerate([(-0.5, 3.25), (W - 0.5, 7.5), (-0.25, H - 0.75),
+                                  (W - 0.75, -0.5)]):
+        d["sampling_loc"][0, q, :, :, :, 0] = (px + 0.5) / W
+        d["sampling_loc"][0, q, :, :, :, 1] = (py + 0.5) / H
+        go[0, q] = float("nan") if q % 2 else float("inf")
+    got, ref = _run(d, go, dtype)[0].double(), _ref(d, go, dtype)[0].double()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isinf(got), torch.isinf(ref))
+    fin = torch.isfinite(ref)
+    assert 0 < (~fin).sum() <= 10 * 64  # at most 2 + 2 + 1 + 1 corners, and none after them
+    check(got[fin], ref[fin], dtype, f"border {dtype}")
+
+
 @pytest.mark.parametrize("nq", [(1 << 22) - 4, (1 << 22) + 4], ids=["below", "above"])
 def test_sorted_path_query_limit(nq):
     """fp16, one head, one 512 x 512 level, one point, about 2^22 queries: the API (the
