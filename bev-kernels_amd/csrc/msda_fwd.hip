@@ -460,12 +460,18 @@ __global__ void __launch_bounds__(kBlock) msda_wave_lds_kernel(const WaveParams 
         v[j][c] = buffer_load_vec<T, VEC>(rsrc, !live || sg.o[c] == kOOB ? kOOB : sg.o[c] + cb);
       }
     }
+    // the batch's terms first, then the sum so far: shorter chains of roundings
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+    for (int k = 0; k < VEC; ++k) {
+      float t = 0.f;
 #pragma unroll
-      for (int k = 0; k < VEC; ++k)
-        acc[k] += w[j][0] * (float)v[j][0].v[k] + w[j][1] * (float)v[j][1].v[k] +
-                  w[j][2] * (float)v[j][2].v[k] + w[j][3] * (float)v[j][3].v[k];
+      for (int j = 0; j < NB; ++j) {
+        const float tj = w[j][0] * (float)v[j][0].v[k] + w[j][1] * (float)v[j][1].v[k] +
+                         w[j][2] * (float)v[j][2].v[k] + w[j][3] * (float)v[j][3].v[k];
+        t = j == 0 ? tj : t + tj;
+      }
+      acc[k] += t;
+    }
   }
   lane_group_sum<G, LPU>(acc);
   if (q < p.NQ && gi == 0) {
