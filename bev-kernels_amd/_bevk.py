@@ -63,6 +63,7 @@ _SIGNATURES = {
     "bevk_dcn_layer_nchw_f32_workspace_bytes": [_i] * 10,
     "bevk_dcn_layer_nchw_f32": [_vp] * 5 + [_i] * 16 + [_vp, ctypes.c_int64, _vp, _vp],
     "bevk_dcn_nhwc_workspace_bytes": [_i] * 11,
+    "bevk_dcn_nhwc_parts": [_i] * 10 + [_vp],
     "bevk_dcn_conv_nhwc": [_i, _vp, _vp, _i, _vp, _vp, _vp] + [_i] * 15
     + [_vp, ctypes.c_int64, _vp, _vp],
     "bevk_dcn_layer_nhwc": [_i, _vp, _vp, _vp, _i, _vp, _vp] + [_i] * 16

@@ -89,6 +89,8 @@ hipError_t launch_dcn_fused_h(int dtype, const DcnGeom &g, int channels_out, con
 // Bytes of the scratch `part` (16-byte aligned) with which this shape runs K in parts (geo
 // kGeoMask / kGeoYF32, 16-byte aligned output); 0 where it runs whole.
 int64_t dcn_fused_h_parts_bytes(int dtype, const DcnGeom &g, int channels_out);
+// K parts of that shape (1: whole) and the 16-row blocks of a workgroup (0: whole).
+int dcn_fused_h_parts(int dtype, const DcnGeom &g, int channels_out, int *row_blocks);
 
 // One-launch DCNv2 forward with the offset conv inside (fp16 / bf16 on the persistent
 // kernel): y = conv(x, w_off) + b_off (fp32, kept in LDS and written to y_out), offsets

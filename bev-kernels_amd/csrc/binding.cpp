@@ -942,6 +942,20 @@ int64_t bevk_dcn_nhwc_workspace_bytes(int dtype, int with_offset_conv, int batch
   return nhwc_ws(dtype, g, channels_out, with_offset_conv != 0, &w) ? w.total : -1;
 }
 
+int bevk_dcn_nhwc_parts(int dtype, int batch_size, int channels, int height_im, int width_im,
+                        int height_col, int width_col, int channels_out, int kernel_h, int kernel_w,
+                        int *row_blocks) {
+  NhwcWs w;
+  const bevk::DcnGeom g = ws_geom(batch_size, channels, height_im, width_im, height_col, width_col,
+                                  kernel_h, kernel_w, 1);
+  int rows = 0;
+  const int parts = nhwc_ws(dtype, g, channels_out, false, &w) && dtype != BEVK_F32
+                        ? bevk::dcn_fused_h_parts(dtype, g, channels_out, &rows)
+                        : 1;
+  if (row_blocks) *row_blocks = rows;
+  return parts;
+}
+
 // The deformable product from a packed / split weight in the workspace; y_f32: offsets are the
 // fp32 y.
 static hipError_t nhwc_product(int dtype, const bevk::DcnGeom &g, int cout, const NhwcWs &w, char *ws,

@@ -1197,8 +1197,8 @@ __global__ void __launch_bounds__(kPThreads) dcn_fused_p_kernel(const PParams pp
     __syncthreads();  // y of every row in ys
   }
 
-  // The consumers' B fragments of K step 0, loaded before the geometry table (they do not
-  // need it) where the consumers keep two B sets (4-5 row blocks): res5 fp16 74.1 -> 71.7 us,
+  // The consumers' B fragments of their first K step, loaded before the geometry table (they do
+  // not need it) where the consumers keep two B sets (4-5 row blocks): res5 fp16 74.1 -> 71.7 us,
   // bf16 74.4 -> 74.1 us, res5 one-launch fp16 84.6 -> 83.0 us. Loading both sets early
   // measured res5 bf16 74.2 -> 75.0 us, and with four sets (2-3 row blocks) it spills.
   constexpr bool kB0Early = SH::kCD == 2;
@@ -1211,7 +1211,7 @@ __global__ void __launch_bounds__(kPThreads) dcn_fused_p_kernel(const PParams pp
       for (int cb = 0; cb < 4; ++cb)
         b0[kh][cb] = __builtin_amdgcn_raw_buffer_load_b128(
             wr, b_frag_offset(n0 + wave * 64 + cb * 16 + (lane & 15), kh, lane, p.nb_total,
-                              p.kb_total, p.w_bytes), 0u, 0);
+                              p.kb_total, p.w_bytes), (uint32_t)ks0 * (uint32_t)(kPBK / 16) * 1024u, 0);
   }
   // Geometry table for all NRB * 16 rows (rows outside the range or past M: zero weights,
   // out-of-range offsets).
@@ -1823,12 +1823,20 @@ hipError_t launch_dcn_fused_h(int dtype, const DcnGeom &g, int channels_out, con
   }
 }
 
-int64_t dcn_fused_h_parts_bytes(int dtype, const DcnGeom &g, int channels_out) {
-  if ((dtype != 1 && dtype != 2) || !dcn_fused_h_supported(g)) return 0;
+int dcn_fused_h_parts(int dtype, const DcnGeom &g, int channels_out, int *row_blocks) {
+  *row_blocks = 0;
+  if ((dtype != 1 && dtype != 2) || !dcn_fused_h_supported(g)) return 1;
   const HParams p = make_hparams(dtype, g, channels_out, nullptr, nullptr, nullptr, nullptr,
                                  nullptr, nullptr, nullptr, false);
   const KConfig k = kparts_for(p, p_config_for(p, kGeoMask));
-  return k.kparts > 1 ? (int64_t)k.kparts * p.M * p.Cout * 4 : 0;
+  *row_blocks = k.nrb;
+  return k.kparts;
+}
+
+int64_t dcn_fused_h_parts_bytes(int dtype, const DcnGeom &g, int channels_out) {
+  int row_blocks = 0;
+  const int64_t parts = dcn_fused_h_parts(dtype, g, channels_out, &row_blocks);
+  return parts > 1 ? parts * g.batch * g.height_col * g.width_col * channels_out * 4 : 0;
 }
 
 // The one-launch form runs where Cout fits one 256-column half. With two halves every

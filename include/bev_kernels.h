@@ -235,6 +235,12 @@ int bevk_dcn_layer_nchw_f32(const float *data_im, const float *data_offset, cons
 int64_t bevk_dcn_nhwc_workspace_bytes(int dtype, int with_offset_conv, int batch_size, int channels,
                                       int height_im, int width_im, int height_col, int width_col,
                                       int channels_out, int kernel_h, int kernel_w);
+/* Reduction parts of the 16-bit NHWC layers' product on the current device (1: whole, also where the
+ * shape is not taken); *row_blocks (may be NULL): 16-pixel blocks of a workgroup, 0 where it is
+ * whole. */
+int bevk_dcn_nhwc_parts(int dtype, int batch_size, int channels, int height_im, int width_im,
+                        int height_col, int width_col, int channels_out, int kernel_h, int kernel_w,
+                        int *row_blocks);
 int bevk_dcn_conv_nhwc(int dtype, const void *data_im, const void *data_offset, int offset_last_dim,
                        const void *data_mask, const void *weight, const void *bias, int batch_size,
                        int channels, int height_im, int width_im, int height_col, int width_col,

@@ -11,21 +11,29 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+# (batch, cin, cout, h, w, relu) and the 16-row blocks of a workgroup that the shape takes on a
+# 256-CU device: each height is a kernel of its own, and 4 and 5 keep other prefetch depths.
+SHAPES = [(1, 128, 256, 3, 5, False, 2), (1, 512, 512, 29, 50, True, 3), (1, 256, 136, 17, 23, False, 2),
+          (1, 320, 264, 9, 41, True, 2), (1, 512, 256, 58, 71, True, 4), (6, 512, 160, 15, 35, False, 4),
+          (1, 1024, 512, 40, 40, False, 4), (3, 512, 160, 29, 50, True, 5), (1, 2048, 256, 50, 50, False, 5)]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
-@pytest.mark.parametrize("cin,cout,h,w,relu", [(128, 256, 3, 5, False), (512, 512, 29, 50, True),
-                                               (256, 136, 17, 23, False), (320, 264, 9, 41, True)])
-def test_fused_parts(dtype, cin, cout, h, w, relu):
+@pytest.mark.parametrize("b,cin,cout,h,w,relu,rows", SHAPES)
+def test_fused_parts(dtype, b, cin, cout, h, w, relu, rows):
+    import ctypes
+    import _bevk
     import _modulated_deform_conv_ext as ext
     g = torch.Generator().manual_seed(cin + h)
-    sizes = (1, cin, h, w, h, w, cout, 3, 3, 1, 1, 1, 1, 1, 1)
-    import _bevk
-    code = _bevk._DTYPE_CODES[dtype]
-    # the workspace holds the parts beside the packed weight: this shape runs in parts
-    assert (_bevk.lib().bevk_dcn_nhwc_workspace_bytes(code, 0, *sizes[:9])
-            > 2 * ext.dcn_packed_weight_numel(dtype, cout, 3, 3, cin) + 256)
-    x = torch.randn(1, h, w, cin, generator=g).to(dtype).to(DEV)
-    off = (2.0 * torch.randn(1, h, w, 18, generator=g)).to(dtype).to(DEV)
-    mask = torch.rand(1, h, w, 9, generator=g).to(dtype).to(DEV)
+    sizes = (b, cin, h, w, h, w, cout, 3, 3, 1, 1, 1, 1, 1, 1)
+    blocks = ctypes.c_int(-1)
+    parts = _bevk.lib().bevk_dcn_nhwc_parts(_bevk._DTYPE_CODES[dtype], *sizes[:9], ctypes.addressof(blocks))
+    assert parts > 1
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert blocks.value == rows
+    x = torch.randn(b, h, w, cin, generator=g).to(dtype).to(DEV)
+    off = (2.0 * torch.randn(b, h, w, 18, generator=g)).to(dtype).to(DEV)
+    mask = torch.rand(b, h, w, 9, generator=g).to(dtype).to(DEV)
     weight = (0.05 * torch.randn(cout, cin, 3, 3, generator=g)).to(dtype).to(DEV)
     bias = torch.randn(cout, generator=g).to(dtype).to(DEV)
     out = ext.dcn_conv_nhwc(x, off, mask, weight, bias, *sizes)
