@@ -56,6 +56,7 @@ __all__ = [
     "dcn_offset_conv_nhwc",
     "dcn_mega_fwd_nhwc",
     "transpose",
+    "transpose_takes",
     "nchw_to_nhwc",
     "nhwc_to_nchw",
     "forward",
@@ -189,6 +190,11 @@ def transpose(src, dst, batch, rows, cols):
     _b.call("bevk_transpose", _b.dtype_code(src), _b.ptr(src), _b.ptr(dst), batch, rows, cols,
             _b.stream_of(src))
     return dst
+
+
+def transpose_takes(batch, rows, cols):
+    """Whether ``transpose`` takes these sizes (its launch grid: one block row per 64 rows)."""
+    return batch <= 65535 and (rows + 63) // 64 <= 65535 and (cols + 63) // 64 <= 2 ** 30
 
 
 def nchw_to_nhwc(x):

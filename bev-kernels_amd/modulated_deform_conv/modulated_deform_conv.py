@@ -277,7 +277,7 @@ class ModulatedDeformConv2dFunction(Function):
         """modulated_deform_conv.py:405-500: columns = W^T @ dO per group; grad_offset /
         grad_mask and grad_input from the column-to-image kernel; the columns of the input
         again for grad_weight = dO @ columns^T; grad_bias = sum of dO. groups == 1 runs these
-        steps on NHWC copies (_layer_backward_nhwc)."""
+        steps on NHWC copies (_layer_backward_nhwc) where those take the sizes."""
         input, offset, mask, weight, bias = ctx.saved_tensors
         ext = _load_ext()
         # 16-bit inputs: the gradients are accumulated in fp32 and rounded once (the
@@ -303,7 +303,8 @@ class ModulatedDeformConv2dFunction(Function):
         args = (batch, channels, height, width, height_out, width_out, kernel_h, kernel_w,
                 pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, deform_groups)
         if (groups == 1 and input.dtype != torch.float64
-                and bhw * c_in_g_kkw < 2 ** 31 - 1):  # the NHWC column kernels' index range
+                and _nhwc_backward_takes(ext, batch, channels, height * width,
+                                         height_out * width_out, kernel_h * kernel_w)):
             grads = _layer_backward_nhwc(ext, grad_output, input, offset, mask, weight, args)
             return _round_grads(out_dtype, *grads, grad_bias) + (None,) * 5
 
@@ -331,6 +332,15 @@ class ModulatedDeformConv2dFunction(Function):
 
 def _round_grads(dtype, *grads):
     return tuple(g if g is None else g.to(dtype) for g in grads)
+
+
+def _nhwc_backward_takes(ext, batch, channels, plane_in, plane_out, taps):
+    """Sizes of _layer_backward_nhwc: the NHWC column kernels' index range, and maps whose
+    gradients the layout change takes back to NCHW (up to 4,194,240 positions). Others run on
+    the NCHW kernels."""
+    return (batch * plane_out * channels * taps < 2 ** 31 - 1
+            and ext.transpose_takes(batch, plane_in, channels)
+            and ext.transpose_takes(batch, plane_out, channels))
 
 
 def _layer_backward_nhwc(ext, grad_output, input, offset, mask, weight, args):

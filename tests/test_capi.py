@@ -250,3 +250,21 @@ def test_noalloc_front_end_rejects_oversize_before_device_work():
     rc = f(1, p(0x10000), p(0x20000), p(0x30000), 1, 16, 400, 400, 400, 400, 3, 3, 1, 1, 1, 1,
            1, 1, 1, p(0x40000), NULL)
     assert rc == INVALID and "static scratch" in _err()
+
+
+def test_nhwc_backward_size_rule_matches_transpose():
+    """The NCHW layer's backward runs on NHWC copies only where bevk_transpose takes the way back
+    (a larger map stays on the NCHW kernels): the rule against the entry's own answer, which
+    checks the sizes before the pointers."""
+    import _modulated_deform_conv_ext as ext
+    from modulated_deform_conv.modulated_deform_conv import _nhwc_backward_takes
+    lib = _bevk.lib()
+    for batch, plane in ((1, 2047 * 2047), (1, 65535 * 64), (1, 65535 * 64 + 1), (1, 2048 * 2048),
+                         (65535, 64), (65536, 64), (1, 1)):
+        rc = lib.bevk_transpose(0, None, None, batch, plane, 8, None)
+        assert rc != 0
+        taken = b"launch grid" not in lib.bevk_last_error()
+        assert ext.transpose_takes(batch, plane, 8) == taken, (batch, plane)
+        assert _nhwc_backward_takes(ext, batch, 8, plane, 16, 9) == taken
+        assert _nhwc_backward_takes(ext, batch, 8, 16, plane, 1) == taken
+    assert not _nhwc_backward_takes(ext, 1, 512, 4000, 2 ** 22 // 9 + 1, 9)  # columns past int32

@@ -51,3 +51,29 @@ def test_dcn_input_over_2gib_rejected():
     weight = torch.zeros(Cout, C, 3, 3, dtype=torch.float16, device=DEV)
     with pytest.raises(RuntimeError, match="too large for 32-bit buffer offsets"):
         fused_tl.fused_dcn_forward_nhwc(x, off, mask, weight, None, 1, 1, 1)
+
+
+def test_dcn_backward_on_a_map_past_the_layout_change():
+    """The NCHW module's backward on a 2048 x 2048 map at stride 2, one position block more than
+    the NHWC route's layout change takes. With zero offsets and a mask of ones the layer is the
+    plain convolution: gradients of input, weight and bias against float64 (sums of 9, of 2^20
+    and of 2^20 products; values near 1)."""
+    import torch.nn.functional as F
+    from modulated_deform_conv import ModulatedDeformConv2d
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(1, 4, 2048, 2048, generator=g)
+    go = torch.randn(1, 2, 1024, 1024, generator=g)
+    mod = ModulatedDeformConv2d(4, 2, 3, stride=2, padding=1).to(DEV)
+    xd = x.to(DEV).requires_grad_()
+    off = torch.zeros(1, 18, 1024, 1024, device=DEV, requires_grad=True)
+    mask = torch.ones(1, 9, 1024, 1024, device=DEV)
+    mod(xd, off, mask).backward(go.to(DEV))
+    xr = x.double().requires_grad_()
+    w = mod.weight.detach().cpu().double().requires_grad_()
+    F.conv2d(xr, w, None, 2, 1).backward(go.double())
+    check(xd.grad.cpu(), xr.grad, torch.float32, "grad_input")
+    assert torch.isfinite(off.grad).all()
+    # 2^20 products per sum: fp32 sums of magnitudes up to about 2^20
+    for a, r in ((mod.weight.grad.cpu().double(), w.grad), (mod.bias.grad.cpu().double(),
+                                                            go.double().sum((0, 2, 3)))):
+        assert ((a - r).abs() <= 2.0 ** -24 * 2 ** 20).all()
