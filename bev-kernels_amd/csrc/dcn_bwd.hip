@@ -50,9 +50,12 @@ __global__ void __launch_bounds__(kBlock) col2im_nhwc_kernel(
   // Lanes past the last pair still take part in the butterfly below; they do no work.
   const bool live = pair < HoWo * T_ * dg;  // (pixel, tap, group)
   const int pc = live ? pair : 0;
-  // Quotients by the runtime sizes from a float reciprocal, corrected by one step (the
-  // launch keeps every quotient below 2^22, where the estimate is off by at most one).
-  auto qdiv = [](int a, int d) {
+  // Quotients by the runtime sizes from a float reciprocal, corrected by one step: below 2^22
+  // the estimate is off by at most one. Larger maps (from 2^23 on it was off by two, and the
+  // gradients of those samples went to another position) divide.
+  const bool wide = HoWo >= (1 << 22);
+  auto qdiv = [wide](int a, int d) {
+    if (wide) return a / d;
     int q = (int)((float)a * __builtin_amdgcn_rcpf((float)d));
     const int r = a - q * d;
     return q + (r >= d) - (r < 0);

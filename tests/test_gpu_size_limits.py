@@ -77,3 +77,30 @@ def test_dcn_backward_on_a_map_past_the_layout_change():
     for a, r in ((mod.weight.grad.cpu().double(), w.grad), (mod.bias.grad.cpu().double(),
                                                             go.double().sum((0, 2, 3)))):
         assert ((a - r).abs() <= 2.0 ** -24 * 2 ** 20).all()
+
+
+def test_dcn_col2im_nhwc_on_a_map_of_9m_positions():
+    """The per-sample column-to-image kernel past 2^23 output positions, where its float estimate of
+    pair / taps is off by more than the one step it corrects. With zero offsets and a mask of ones
+    a tap's gradient goes to one pixel: grad_x is the sum of 5 shifted columns, grad_mask a
+    sum of 2 products (fp32)."""
+    import _modulated_deform_conv_ext as ext
+    import torch.nn.functional as F
+    h = w = 3000
+    c, t = 2, 5
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(1, h, w, c, generator=g, device=DEV)
+    dcol = torch.randn(h * w, t * c, generator=g, device=DEV)
+    off, mask = torch.zeros(1, h, w, 2 * t, device=DEV), torch.ones(1, h, w, t, device=DEV)
+    gx = torch.zeros_like(x)
+    goff, gmask = torch.empty_like(off), torch.empty_like(mask)
+    ext.modulated_deformable_col2im_nhwc_cuda(dcol, x, off, mask, 1, c, h, w, h, w, 1, t, 0, 2, 1, 1, 1,
+                                              1, 1, gx, goff, gmask)
+    d = dcol.view(h, w, t, c)
+    wide = torch.zeros(h, w + 4, c, device=DEV)
+    xp = F.pad(x[0], (0, 0, 2, 2))
+    for k in range(t):
+        wide[:, k:k + w] += d[:, :, k]
+        assert torch.allclose(gmask[0, :, :, k], (d[:, :, k] * xp[:, k:k + w]).sum(-1), rtol=0, atol=1e-5)
+    # values up to about 6: ten roundings of 2^-24 of sums below 32
+    assert torch.allclose(gx[0], wide[:, 2:-2], rtol=0, atol=2e-5)
