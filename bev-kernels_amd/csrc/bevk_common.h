@@ -21,6 +21,39 @@ template <typename A, typename T> __device__ __forceinline__ A cvt(T x) { return
 template <typename T> __device__ __forceinline__ T from_acc(float x) { return static_cast<T>(x); }
 template <> __device__ __forceinline__ double from_acc<double>(float x) { return x; }
 
+// fp32 operands of the bf16 matrix cores: a value is cut into three bf16 pieces, each the
+// nearest bf16 of what the pieces before it leave, x = h + m + l exactly (8 + 8 + 8 significant
+// bits; values of 2^-110 and more, below that l runs out of bf16's exponents and up to 2^-134 is
+// lost). |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, of either sign, so the products that six of the
+// nine leave out (m l' + l m' + l l') stay below 2^-23 of x x' and average out over a sum. (Pieces
+// cut off instead of rounded have m and l of x's sign and up to twice and four times that size:
+// a sum of equal operands 1 + 2^-7 - 2^-23 was off by 3.9 * 2^-23.)
+// Two values at a time: words of two pieces, a's in the low half, and what is NaN if a or b is
+// not finite or rounds to Inf (the residues' sum).
+struct Cut2 {
+  int h, m, l;
+  float nf;
+};
+__device__ __forceinline__ Cut2 cut2(float a, float b) {
+  typedef float float2v __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  auto word = [](float x, float y) __attribute__((always_inline)) {
+    return __builtin_bit_cast(int, __builtin_convertvector(float2v{x, y}, bf16x2));
+  };
+  auto low = [](int w) __attribute__((always_inline)) { return __builtin_bit_cast(float, w << 16); };
+  auto high = [](int w) __attribute__((always_inline)) {
+    return __builtin_bit_cast(float, (int)(w & 0xffff0000u));
+  };
+  Cut2 c;
+  c.h = word(a, b);
+  const float ra = a - low(c.h), rb = b - high(c.h);
+  c.m = word(ra, rb);
+  const float la = ra - low(c.m), lb = rb - high(c.m);
+  c.l = word(la, lb);
+  c.nf = la + lb;
+  return c;
+}
+
 // Plain vector of N elements of T, loaded/stored as one memory instruction.
 template <typename T, int N> struct alignas(sizeof(T) * N) Vec { T v[N]; };
 

@@ -117,7 +117,7 @@ hipError_t launch_dcn_prep16(int dtype, const void *weight, int cout, const void
                              int T, const void *b_off, int b_dtype, void *packed, void *packed_off,
                              float *b_out, hipStream_t stream);
 
-// fp32 products on the bf16 matrix cores (three exact bf16 pieces per operand, dcn_f32.hip).
+// fp32 products on the bf16 matrix cores (three bf16 pieces per operand, dcn_f32.hip).
 // Split weight of n columns and k reduction elements (with its flags), from the module weight
 // [Cout][C][T]: n = Cout, k = t*C + c (C % 32 == 0), or transposed n = t*C + c, k = Cout
 // (C % 16 == 0, Cout % 32 == 0); T <= 9, 16-byte aligned buffers.

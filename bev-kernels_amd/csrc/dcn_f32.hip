@@ -4,17 +4,17 @@
 //   out[m, n] = sum_k A[m, k] * W[n, k] (+ bias[n])
 //
 // with A either the deformable columns of an NHWC input, built on the fly (m = (b, oh, ow),
-// k = t*C + c), or the rows of a matrix. Every fp32 operand is cut into three bf16 pieces that
-// add up to it exactly (8 + 8 + 8 significant bits, each piece the next 16 high bits of what
-// is left), x = h + m + l, and a product is taken as
+// k = t*C + c), or the rows of a matrix. Every fp32 operand is cut into three bf16 pieces
+// (cut2 in bevk_common.h: exact from 2^-110 up), x = h + m + l, and a product is taken as
 //   h*h' + (h*m' + m*h') + (m*m' + h*l' + l*h'),
 // six v_mfma_f32_16x16x32_bf16 with fp32 accumulation. What is left out (m*l' + l*m' + l*l')
-// is below 2^-23 of the product and 4e-8 of it on average, and the large sum is rounded twice
+// is below 2^-23 of the product and of either sign, and the large sum is rounded twice
 // per 32 terms instead of once per two terms as with v_mfma_f32_32x32x2_f32, so the sums come
 // out closer to the exact ones: 2-norm errors against 64 bits at 64 / 512 / 2,304 / 4,608 terms
-// 0.8e-7 / 1.6e-7 / 3.3e-7 / 4.8e-7, where a library fp32 product has 1.4e-7 / 4.0e-7 / 8.6e-7
+// 0.5e-7 / 1.5e-7 / 3.3e-7 / 4.7e-7, where a library fp32 product has 1.4e-7 / 4.1e-7 / 8.6e-7
 // / 12e-7 and this layer's fp32 matrix kernel had 5.9e-7 at 2,304 (all six products in one
-// accumulator: 7.3e-7).
+// accumulator: 7.3e-7). Operands below 2^-110 lose low bits (all nonzero operands of one side at
+// 2^-115: 1.1e-6, at 2^-120: 3.5e-5; the library product 2.8e-7).
 //
 // Bound: the matrix cores. Six cameras at 256 channels of 58 x 100 to 256 (41 GFLOP): 500 us
 // on the fp32 matrix cores (82 TFLOP/s of 157), 220-245 us here (1.0-1.1 PFLOP/s of bf16
@@ -24,9 +24,10 @@
 // Pairs of row blocks with four independent MFMA chains, or two chains for the small products,
 // measured the same or slower: their dependent chain is not what limits.
 //
-// Non-finite operands do not survive the cut (inf - inf, 0 * inf): a workgroup that meets one
-// (in its columns, or flagged when the weight was split) computes its tile again in plain
-// fp32 (slow_tile), which has the reference's NaN / Inf behaviour.
+// Non-finite operands do not survive the cut (inf - inf, 0 * inf), nor do those that round to
+// Inf as a bf16 (from 3.396e38 up): a workgroup that meets one (in its columns, or flagged when the
+// weight was split) computes its tile again in plain fp32 (slow_tile), which has the reference's
+// NaN / Inf behaviour.
 #include "bevk_common.h"
 #include "bevk_launch.h"
 
@@ -73,27 +74,6 @@ struct Params {
   int per_xcd;
   uint32_t x_bytes, w_bytes;
 };
-
-// The three pieces as fp32 values (the low 16 bits of each are zero).
-struct Pieces {
-  float h, m, l;
-};
-__device__ __forceinline__ float high_part(float v) {
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xffff0000u);
-}
-__device__ __forceinline__ Pieces cut(float v) {
-  Pieces p;
-  p.h = high_part(v);
-  const float r = v - p.h;
-  p.m = high_part(r);
-  p.l = r - p.m;
-  return p;
-}
-// Two pieces' high halves in one word (the first in the low half).
-__device__ __forceinline__ int pack2(float a, float b) {
-  return (int)__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a),
-                                    0x07060302u);
-}
 
 __device__ __forceinline__ floatx4 mfma(int4v a, int4v b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
@@ -254,7 +234,8 @@ __device__ __forceinline__ float k_loop(const Params &p, const TapGeo *geo, char
     }
   };
   float nf = 0.f;  // NaN once a non-finite value was cut
-  Pieces pc[4];
+  float pv = 0.f;  // the even element of a pair
+  Cut2 pc[2];
   auto blend_one = [&](int i, int e) __attribute__((always_inline)) {
     float v;
     if constexpr (!deform(GEO)) {
@@ -265,14 +246,18 @@ __device__ __forceinline__ float k_loop(const Params &p, const TapGeo *geo, char
       v = __builtin_fmaf(w4[2], ra[i][2][e], v);
       v = __builtin_fmaf(w4[3], ra[i][3][e], v);
     }
-    pc[e] = cut(v);
-    nf += pc[e].l;
+    if (e % 2 == 0) {
+      pv = v;
+    } else {
+      pc[e / 2] = cut2(pv, v);
+      nf += pc[e / 2].nf;
+    }
   };
   auto store_slot = [&](int i, char *buf) __attribute__((always_inline)) {
     char *d = buf + a_off(slot_row(i), kv >> 1) + (kv & 1) * 8;
-    *reinterpret_cast<int2v *>(d) = int2v{pack2(pc[0].h, pc[1].h), pack2(pc[2].h, pc[3].h)};
-    *reinterpret_cast<int2v *>(d + S::kPlane) = int2v{pack2(pc[0].m, pc[1].m), pack2(pc[2].m, pc[3].m)};
-    *reinterpret_cast<int2v *>(d + 2 * S::kPlane) = int2v{pack2(pc[0].l, pc[1].l), pack2(pc[2].l, pc[3].l)};
+    *reinterpret_cast<int2v *>(d) = int2v{pc[0].h, pc[1].h};
+    *reinterpret_cast<int2v *>(d + S::kPlane) = int2v{pc[0].m, pc[1].m};
+    *reinterpret_cast<int2v *>(d + 2 * S::kPlane) = int2v{pc[0].l, pc[1].l};
   };
 
   const int fa = a_off(lane & 15, lane >> 4) + wm * R * 1024;  // the wave's first fragment
@@ -588,22 +573,23 @@ __global__ void __launch_bounds__(kThreads) f32_small_kernel(const Params p) {
   for (int j = 0; j < NB; ++j) hi[j] = lo[j] = floatx4{0.f, 0.f, 0.f, 0.f};
   float nf = 0.f;
   auto multiply = [&](const Step &st) __attribute__((always_inline)) {
-    Pieces pc[8];
+    float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      float v = st.a[0][e >> 2][e & 3];
+      v[e] = st.a[0][e >> 2][e & 3];
       if constexpr (deform(GEO)) {
-        v *= st.w[0];
+        v[e] *= st.w[0];
 #pragma unroll
-        for (int q = 1; q < NQ; ++q) v = __builtin_fmaf(st.w[q], st.a[q][e >> 2][e & 3], v);
+        for (int q = 1; q < NQ; ++q) v[e] = __builtin_fmaf(st.w[q], st.a[q][e >> 2][e & 3], v[e]);
       }
-      pc[e] = cut(v);
-      nf += pc[e].l;
     }
-    const int4v a[3] = {
-        int4v{pack2(pc[0].h, pc[1].h), pack2(pc[2].h, pc[3].h), pack2(pc[4].h, pc[5].h), pack2(pc[6].h, pc[7].h)},
-        int4v{pack2(pc[0].m, pc[1].m), pack2(pc[2].m, pc[3].m), pack2(pc[4].m, pc[5].m), pack2(pc[6].m, pc[7].m)},
-        int4v{pack2(pc[0].l, pc[1].l), pack2(pc[2].l, pc[3].l), pack2(pc[4].l, pc[5].l), pack2(pc[6].l, pc[7].l)}};
+    int4v a[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const Cut2 c = cut2(v[2 * e], v[2 * e + 1]);
+      a[0][e] = c.h; a[1][e] = c.m; a[2][e] = c.l;
+      nf += c.nf;
+    }
     constexpr int kTa[5] = {2, 0, 1, 1, 0}, kTb[5] = {0, 2, 1, 0, 1};
 #pragma unroll
     for (int q = 0; q < 5; ++q)
@@ -672,28 +658,38 @@ __global__ void __launch_bounds__(kThreads) f32_small_kernel(const Params p) {
   }
 }
 
-// The three pieces of a lane's 8 values of a split block; a non-finite value is kept whole in
-// the first piece. Returns whether there was one.
+// The three pieces of a lane's 8 values of a split block. A pair with a value that is not finite
+// or rounds to Inf is cut off instead (the pieces of a finite value still add up to it; Inf and NaN
+// are kept whole in the first piece), for slow_tile. Returns whether there was one.
 __device__ __forceinline__ bool store_split(char *d, const float (&v)[8]) {
-  float h[8], m[8], l[8];
+  int4v h, m, l;
   bool bad = false;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    Pieces p = cut(v[e]);
-    if (!(p.l == p.l)) {
+  for (int e = 0; e < 4; ++e) {
+    Cut2 c = cut2(v[2 * e], v[2 * e + 1]);
+    if (!(c.nf == c.nf)) {
       bad = true;
-      p.h = v[e] == v[e] ? v[e] : __builtin_nanf("");
-      p.m = p.l = 0.f;
+      uint32_t p[2][3];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        float x = v[2 * e + q];
+        if (!(x == x)) x = __builtin_nanf("");
+        const bool fin = __builtin_fabsf(x) <= 3.402823466e38f;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          p[q][i] = i == 0 || fin ? __builtin_bit_cast(uint32_t, x) & 0xffff0000u : 0u;
+          x -= __builtin_bit_cast(float, p[q][i]);
+        }
+      }
+      c.h = (int)(p[0][0] >> 16 | p[1][0]);
+      c.m = (int)(p[0][1] >> 16 | p[1][1]);
+      c.l = (int)(p[0][2] >> 16 | p[1][2]);
     }
-    h[e] = p.h; m[e] = p.m; l[e] = p.l;
+    h[e] = c.h; m[e] = c.m; l[e] = c.l;
   }
-  auto put = [](char *at, const float (&x)[8]) {
-    *reinterpret_cast<int4v *>(at) =
-        int4v{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
-  };
-  put(d, h);
-  put(d + 1024, m);
-  put(d + 2048, l);
+  *reinterpret_cast<int4v *>(d) = h;
+  *reinterpret_cast<int4v *>(d + 1024) = m;
+  *reinterpret_cast<int4v *>(d + 2048) = l;
   return bad;
 }
 

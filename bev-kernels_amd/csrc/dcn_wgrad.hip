@@ -8,7 +8,7 @@
 // (one instruction per two elements), so no transposed copy exists anywhere and every global
 // load is a run of 512 or 256 bytes. LDS holds the fragments in the order they are read.
 //   16-bit types: products exact, fp32 sums; 64 pixels per step.
-//   fp32: three exact bf16 pieces per element and six products, the small ones summed apart
+//   fp32: three bf16 pieces per element (cut2) and six products, the small ones summed apart
 //         (dcn_f32.hip has the arithmetic and its errors); 32 pixels per step. A tile that
 //         meets NaN or Inf is computed again in plain fp32.
 // The parts' fp32 sums [parts][n][k] go to a workspace and weight_grad_reduce adds them in part
@@ -17,8 +17,8 @@
 // Measured: 34,800 pixels x 2,304 columns x 256 channels (41 GFLOP) bf16 72 us (library fp32
 // product of converted operands 648 us and the conversions 80), fp32 302 us (648), the same work
 // at 8,700 x 4,608 x 512 bf16 80, fp32 281 us (357): the matrix cores in fp32 (six products, 205
-// us at the rate of a large library product), loads and LDS in 16 bits. Errors against 64 bits
-// 3e-7 (library fp32 1.8e-6).
+// us at the rate of a large library product), loads and LDS in 16 bits. Errors against 64 bits at 2,304 / 8,700 / 34,800
+// pixels 1.3e-7 / 1.8e-7 / 3.5e-7 (library fp32 0.9e-6 / 1.7e-6 / 1.8e-6).
 // The offset conv's weight gradient (CONV) runs the same tiles with plain-convolution columns
 // read from the input itself (16-bit inputs are exact in one or two of the pieces, so fewer
 // products) and the 3T <= 32 columns of its fp32 output gradient.
@@ -76,9 +76,6 @@ template <typename T> __device__ __forceinline__ floatx4 mfma(int4v a, int4v b, 
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ float high_part(float v) {
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xffff0000u);
 }
 // High halves of two words (first in the low half), or low halves.
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
@@ -203,20 +200,18 @@ __global__ void __launch_bounds__(kThreads, 2) weight_grad_kernel(const WParams 
       int4v o[3];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        uint32_t x[2], y[2], z[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          x[q] = elem(2 * j + q, e, tag);
-          const float f = __builtin_bit_cast(float, x[q]);
-          const float r = f - high_part(f);
-          y[q] = __builtin_bit_cast(uint32_t, r);
-          const float t = r - high_part(r);
-          z[q] = __builtin_bit_cast(uint32_t, t);
-          nf += t;
+        const float x = __builtin_bit_cast(float, elem(2 * j, e, tag));
+        const float y = __builtin_bit_cast(float, elem(2 * j + 1, e, tag));
+        if constexpr (NP == 1) {
+          o[0][j] = (int)pack_hi(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, y));
+          nf += (x - x) + (y - y);
+        } else {
+          const Cut2 c = cut2(x, y);
+          o[0][j] = c.h;
+          o[1][j] = c.m;
+          o[2][j] = c.l;
+          nf += c.nf;
         }
-        o[0][j] = (int)pack_hi(x[0], x[1]);
-        o[1][j] = (int)pack_hi(y[0], y[1]);
-        o[2][j] = (int)pack_hi(z[0], z[1]);
       }
       char *d = base + frag_at<COLS>(uc + e, uo);
 #pragma unroll

@@ -159,8 +159,9 @@ int bevk_dcn_layer_col2im_nhwc(
     float *grad_offset, float *grad_mask, void *stream);
 
 /* fp32 on the bf16 matrix cores: operands cut into three bf16 pieces that add up to them
- * exactly, six products of pieces per product, fp32 sums (errors no larger than fp32 matrix
- * instructions'; NaN / Inf as in plain fp32).
+ * (exactly from 2^-110 up, to 2^-134 below), six products of pieces per product (what is left
+ * out is below 2^-23 of the product), fp32 sums: two roundings per 32 terms, where fp32 matrix
+ * instructions round every second. NaN / Inf as in plain fp32.
  *   bevk_f32_split_weight_bytes  bytes of the split weight of n columns x k terms
  *   bevk_dcn_split_weight        weight [Cout, C, kh, kw] fp32 -> split (16-byte aligned):
  *                                columns Cout, terms (tap, C) with C % 32 == 0; transposed:

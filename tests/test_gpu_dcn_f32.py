@@ -35,6 +35,59 @@ def test_gemm_f32(m, k, c):
     _bounded(out, a.double() @ wf, a.double().abs() @ wf.abs(), k, f"gemm {m}x{k}x{9 * c}")
 
 
+# Operands whose pieces left out are large: cut off instead of rounded the first two leave 2^-21 of
+# the product; rounded, the second leaves the most that can be, 2^-24.
+EQUAL = [1 + 2.0 ** -7 - 2.0 ** -23, 1 + 2.0 ** -8 - 2.0 ** -17, 2 - 2.0 ** -23,
+         -1 - 2.0 ** -7 + 2.0 ** -23]
+
+
+@pytest.mark.parametrize("v", EQUAL)
+@pytest.mark.parametrize("m,k", [(16, 32), (400, 32), (16, 64), (5000, 64)])
+def test_gemm_equal_operands(m, k, v):
+    """All products alike, so that what they leave out adds up: 2^-24 of the sum, and at most three
+    fp32 roundings per 32 terms (two sums, one addition)."""
+    import _modulated_deform_conv_ext as ext
+    out = torch.empty(m, 144, device=DEV)
+    w = torch.full((k, 16, 3, 3), v, device=DEV)
+    ext.gemm_f32(torch.full((m, k), v, device=DEV), ext.dcn_split_weight(w, True), 144, out)
+    ref = k * w[0, 0, 0, 0].double().item() ** 2
+    assert (out.double() - ref).abs().max().item() <= (3 * k / 32 + 1) * 2.0 ** -24 * ref
+
+
+@pytest.mark.parametrize("exp", [-90, -110])
+def test_gemm_small_operands(exp):
+    """Operands of 2^exp .. 2^(exp + 2) keep their 24 bits (the lowest of 2^-110 is bf16's smallest
+    subnormal, 2^-133); the bound of every other product."""
+    import _modulated_deform_conv_ext as ext
+    g = torch.Generator().manual_seed(-exp)
+    m, k = 200, 256
+    mant = (1 + 3 * torch.rand(m, k, generator=g)) * (torch.randint(0, 2, (m, k), generator=g) * 2 - 1)
+    a = mant * 2.0 ** (exp // 2) * 2.0 ** (exp - exp // 2)
+    w = torch.randn(k, 16, 3, 3, generator=g) * 2.0 ** 40
+    out = torch.empty(m, 144, device=DEV)
+    ext.gemm_f32(a.to(DEV), ext.dcn_split_weight(w.to(DEV), True), 144, out)
+    wf = w.permute(0, 2, 3, 1).reshape(k, 144).double()
+    scale = 2.0 ** (-exp - 40)  # the bound's 1e-30 is for results near 1
+    _bounded(out.double() * scale, (a.double() @ wf) * scale, (a.double().abs() @ wf.abs()) * scale, k,
+             f"2^{exp}")
+
+
+def test_gemm_weight_near_the_largest_float():
+    """A finite weight that rounds to Inf as a bf16: the tile runs in plain fp32 and keeps it."""
+    import _modulated_deform_conv_ext as ext
+    g = torch.Generator().manual_seed(2)
+    a = torch.randn(40, 64, generator=g) * 2.0 ** -100
+    w = torch.randn(64, 16, 3, 3, generator=g)
+    w[7, 3, 1, 1] = 3.4028234e38
+    w[9, 4, 0, 2] = -3.3961776e38
+    out = torch.empty(40, 144, device=DEV)
+    ext.gemm_f32(a.to(DEV), ext.dcn_split_weight(w.to(DEV), True), 144, out)
+    wf = w.permute(0, 2, 3, 1).reshape(64, 144).double()
+    # 64 fused multiply-adds, each rounded once
+    bound = 64 * 2.0 ** -24 * (a.double().abs() @ wf.abs()) + 1e-37
+    assert ((out.double().cpu() - a.double() @ wf).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("b,cin,cout,h,w,stride", [
     (1, 32, 16, 5, 7, 1), (1, 64, 64, 32, 32, 1), (2, 32, 100, 23, 31, 2),
     (1, 96, 160, 20, 30, 1), (1, 64, 264, 41, 37, 1), (3, 32, 320, 60, 61, 1)])

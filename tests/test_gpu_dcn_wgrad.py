@@ -40,6 +40,18 @@ def test_weight_grad(dtype, m, c, cout, k):
     assert torch.equal(got, again), "not the same on every run"
 
 
+@pytest.mark.parametrize("v", [1 + 2.0 ** -7 - 2.0 ** -23, 1 + 2.0 ** -8 - 2.0 ** -17])
+@pytest.mark.parametrize("m", [32, 64])
+def test_weight_grad_equal_operands(m, v):
+    """All products alike, so that the pieces left out add up: 2^-24 of the sum, and at most three
+    fp32 roundings per 32 pixels."""
+    import _modulated_deform_conv_ext as ext
+    t = torch.full((m, 72), v, device=DEV)
+    got = ext.dcn_weight_grad(t, t, 3, 3).double()
+    ref = m * t[0, 0].double().item() ** 2
+    assert (got - ref).abs().max().item() <= (3 * m / 32 + 1) * 2.0 ** -24 * ref
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_weight_grad_nonfinite(dtype):
     """Inf and NaN reach exactly the sums they reach in float64 (a zero times Inf is NaN, Inf
