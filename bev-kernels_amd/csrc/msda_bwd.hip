@@ -900,6 +900,10 @@ constexpr int kAccThreads = 512;
 constexpr int kAccChunk = 3584;            // records per accumulate chunk (79 KB LDS; 2 blocks per CU)
 constexpr int kAccPerThread = kAccChunk / kAccThreads;
 constexpr int kAccPiece = 2;               // chunks of one bucket a workgroup sums in turn
+constexpr int kAccCh = 32;                 // channels of a head per accumulate launch
+constexpr int kSortedMaxD = 64;            // largest head dimension of the sorted path
+constexpr int kAccLaunches = kSortedMaxD / kAccCh;
+constexpr int kItemInts = 8 * (1 + kAccLaunches);  // list lengths, then a queue set per launch
 
 struct BktParams {
   const void *loc, *attn, *grad_out;
@@ -908,7 +912,8 @@ struct BktParams {
   int *count;       // [nbk] records per bucket
   int *cursor;      // [nbk] next free slot (offsets after the scan)
   int *offset;      // [nbk + 1]
-  int *nitems;      // [8] pieces per XCD list, then [8] work-queue counters per accumulate launch
+  int *nitems;      // [kItemInts] pieces per XCD list, then [8] work-queue counters per
+                    // accumulate launch
   int4 *items;      // [8][item_cap] (bucket, first record, records, 1 if the bucket is one piece)
   float2 *rw;       // [capacity] record weights: (position, next position)
   uint32_t *rq;     // [capacity] query << kBkShift | position in bucket
@@ -1164,7 +1169,7 @@ __global__ void __launch_bounds__(1024) msda_bkt_scan_kernel(const BktParams p) 
   if (tid == 0) {
     if (x == 0) p.offset[p.nbk] = total[0];
     p.nitems[x] = min(total[1] + total[2], p.item_cap);
-    p.nitems[8 + x] = p.nitems[16 + x] = 0;  // the accumulate launches' queues
+    for (int q = 1; q <= kAccLaunches; ++q) p.nitems[8 * q + x] = 0;  // the accumulate launches' queues
   }
 }
 
@@ -1285,7 +1290,7 @@ template <typename T, bool EXACT>
 __global__ void __launch_bounds__(kAccThreads, 4) msda_bkt_acc_kernel(const BktParams p) {
   // a group of LPC lanes reads one 128-byte (fp32) or 64-byte (16-bit) grad_output row,
   // 16 bytes per lane
-  constexpr int D = 32, VEC = 16 / (int)sizeof(T), LPC = D / VEC;
+  constexpr int D = kAccCh, VEC = 16 / (int)sizeof(T), LPC = D / VEC;
   constexpr int NGR = kAccThreads / LPC;
   constexpr int BT = VEC == 4 ? 4 : 3;      // records per batch of a group (no spills)
   __shared__ float accs[(kBkPos + 1) * D];  // the piece's sums per position (+ the next bucket's first)
@@ -1877,7 +1882,7 @@ BktLayout bkt_layout(int64_t B, int64_t S, int64_t NH, int64_t NL, int64_t NQ, i
   L.off_count = o;  o += up(nbk * 4);
   L.off_cursor = o; o += up(nbk * 4);
   L.off_offset = o; o += up((nbk + 1) * 4);
-  L.off_nitems = o; o += up(8 * 4);
+  L.off_nitems = o; o += up(kItemInts * 4);
   L.off_items = o;  o += up(8 * item_cap * 16);
   L.off_rw = o;     o += up(cap * 8);
   L.off_rq = o;     o += up(cap * 4);
@@ -1895,7 +1900,7 @@ int64_t half_acc_bytes(int dtype, int64_t value_elems) {
 // sorted 143; 2,000 queries, 128 K samples, 140 / 138; 2 x 10,000 queries 1,081 / 299; 3 x 8,
 // 4 x 5,000 queries 1,381 / 359, fp16 1,389 / 311; one level, 15,000 grid cells, 223 / 136).
 bool sorted_dim(int64_t channels, int64_t samples) {
-  return channels == 32 || (channels == 64 && samples >= ((int64_t)1 << 17));
+  return channels == kAccCh || (channels == kSortedMaxD && samples >= ((int64_t)1 << 17));
 }
 
 // The sorted path: D = 32 or 64, fp32 accumulation (f32 / f16 / bf16 inputs), one batch of value
@@ -1998,7 +2003,7 @@ hipError_t launch_sorted(const MsdaBwdArgs &a, const BktLayout &L, char *ws, flo
   p.dim = a.f.channels;
   p.row = a.f.num_heads * a.f.channels;
   p.queue = 8;
-  for (int ch0 = 0; ch0 < p.dim; ch0 += 32, p.queue += 8) {
+  for (int ch0 = 0; ch0 < p.dim; ch0 += kAccCh, p.queue += 8) {
     p.grad_out = static_cast<const T *>(a.grad_output) + ch0;
     p.gv = gv + ch0;
     if (p.dim == 32)
