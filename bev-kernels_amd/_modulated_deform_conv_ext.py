@@ -874,8 +874,8 @@ def backward(value, spatial_shapes, level_start_index, sampling_loc, attn_weight
     (accumulated in an fp32 buffer, then narrowed); grad_sampling_loc and
     grad_attn_weight are written. grad_output [B, Lq, heads*D] may be strided.
 
-    Scratch: with head_dim 32 (64 from 128 Ki samples on) the fastest kernels (grad_value by a bucket sort of the
-    samples, no per-corner atomics) take bevk_msda_backward_workspace_bytes of device
+    Scratch: with head_dim 32 (64 with many samples) the fastest kernels (grad_value by a bucket sort
+    of the samples, no per-corner atomics) take bevk_msda_backward_workspace_bytes of device
     memory, about 12 bytes per (sample, corner row) on top of the fp32 accumulator 16-bit
     types need (SCA, 6 cameras: 370 MB fp32, 560 MB fp16). When that exceeds
     max_workspace_bytes (default: the BEVK_MSDA_BACKWARD_MAX_WORKSPACE environment

@@ -1894,13 +1894,23 @@ int64_t half_acc_bytes(int dtype, int64_t value_elems) {
   return (dtype == 1 || dtype == 2) ? (value_elems * (int64_t)sizeof(float) + 255) / 256 * 256 : 0;
 }
 
-// Head dimensions of the sorted path. 64 channels take it from 128 Ki samples on: its seven
-// launches against the atomic kernel's one or two cost a small call more than the atomics do
-// (training step, 4 heads of 64, 4 x 4, fp32: 900 queries, 58 K samples, atomics 125 us and
-// sorted 143; 2,000 queries, 128 K samples, 140 / 138; 2 x 10,000 queries 1,081 / 299; 3 x 8,
-// 4 x 5,000 queries 1,381 / 359, fp16 1,389 / 311; one level, 15,000 grid cells, 223 / 136).
+// Head dimensions of the sorted path. Heads of 64 take it from a number of samples on: its seven
+// launches against the atomic kernel's one or two cost a small call more than the atomics do, and
+// with more levels a larger share of the records meets in the few buckets of the coarsest one,
+// which then last longest. Calls with 4 heads, atomics / sorted, us:
+//   1 level   128 Ki samples fp32  98 / 77, fp16 106 / 83
+//   2 levels  128 Ki        104 / 97, 106 / 101
+//   3 levels  128 Ki        102 / 120, 108 / 123; 160 Ki 121 / 119, 135 / 124
+//   4 levels  160 Ki        131 / 137, 137 / 175; 192 Ki 151 / 135, 157 / 181; 224 Ki 175 / 137,
+//             186 / 178; 320 Ki 245 / 144, 257 / 187
+// (training step of 2 x 10,000 queries, 4 x 4, 1,081 / 299; 3 x 8, 4 x 5,000 queries 1,381 / 359.)
+// The workspace holds the path's buffers from the lowest line on.
 bool sorted_dim(int64_t channels, int64_t samples) {
-  return channels == kAccCh || (channels == kSortedMaxD && samples >= ((int64_t)1 << 17));
+  return channels == kAccCh || (channels == kSortedMaxD && samples >= (128 << 10));
+}
+bool sorted_pays(int64_t channels, int64_t levels, int64_t samples, bool fp32) {
+  if (channels != kSortedMaxD || levels <= 2) return true;
+  return samples >= ((levels == 3 ? 160 : fp32 ? 192 : 224) << 10);
 }
 
 // The sorted path: D = 32 or 64, fp32 accumulation (f32 / f16 / bf16 inputs), one batch of value
@@ -1908,8 +1918,9 @@ bool sorted_dim(int64_t channels, int64_t samples) {
 template <typename T>
 bool sorted_path(const MsdaBwdArgs &a, int dtype, BktLayout &L) {
   const int64_t D = a.f.channels;
-  if (!sorted_dim(D, (int64_t)a.f.batch * a.f.num_query * a.f.num_heads * a.f.num_levels *
-                         a.f.num_point) ||
+  const int64_t samples = (int64_t)a.f.batch * a.f.num_query * a.f.num_heads * a.f.num_levels *
+                          a.f.num_point;
+  if (!sorted_dim(D, samples) || !sorted_pays(D, a.f.num_levels, samples, sizeof(T) == 4) ||
       a.f.batch <= 0 || a.f.num_heads <= 0 || a.f.num_query <= 0 ||
       a.f.num_levels <= 0 || a.f.num_point <= 0 || device_cus() < 8)
     return false;

@@ -408,9 +408,10 @@ int bevk_msda_forward(
  * 131,072 samples (batch * num_query * num_heads * num_levels * num_point), the value returned
  * also holds the buffers of the sorted grad_value path (for every sample, up to two
  * 12-byte records, one per image row of its valid corners, bucketed by position), which
- * bevk_msda_backward takes whenever
- * the workspace it is given is at least this large; a smaller workspace (at least the
- * accumulator) runs the atomic kernels instead. */
+ * bevk_msda_backward takes whenever the workspace it is given is at least this large (heads of
+ * 64: from 131,072 samples on with one or two levels, 163,840 with three, 196,608 (F32) or
+ * 229,376 (F16/BF16) with more); a smaller workspace (at least the accumulator) runs the atomic
+ * kernels instead. */
 int64_t bevk_msda_backward_workspace_bytes(int dtype, int batch, int spatial_size,
                                            int num_heads, int channels, int num_levels,
                                            int num_query, int num_point);

@@ -411,6 +411,19 @@ def test_sorted_two_halves(geom, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("geom", [
+    (3, [(20, 30), (10, 15), (5, 8)], 1517, 3, 64, 4),         # 163,836 samples: atomics
+    (3, [(20, 30), (10, 15), (5, 8)], 1518, 3, 64, 4),         # 163,944: sorted
+    (1, [(16, 16), (8, 8), (4, 4), (2, 2)], 1791, 4, 64, 8),   # 229,248: sorted in fp32 only
+    (1, [(16, 16), (8, 8), (4, 4), (2, 2)], 1792, 4, 64, 8),   # 229,376: sorted
+])
+def test_sorted_two_halves_line(geom, dtype):
+    """Heads of 64 with three and four levels around the numbers of samples from which the sorted
+    path pays; the three-level geometry with concentrated locations too."""
+    test_sorted_two_halves(geom, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 @pytest.mark.parametrize("num_query", [60, 2500], ids=["one_chunk", "pieces"])
 def test_sorted_bucket_edges(num_query, dtype):
     """Sorted path, records at the edges of the 256-position buckets of a 6 x 100 map
