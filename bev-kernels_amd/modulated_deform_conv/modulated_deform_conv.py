@@ -302,9 +302,11 @@ class ModulatedDeformConv2dFunction(Function):
         grad_bias = grad_output.sum(dim=(0, 2, 3)) if ctx.with_bias else None
         args = (batch, channels, height, width, height_out, width_out, kernel_h, kernel_w,
                 pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, deform_groups)
+        plane_out, taps = height_out * width_out, kernel_h * kernel_w
         if (groups == 1 and input.dtype != torch.float64
-                and _nhwc_backward_takes(ext, batch, channels, height * width,
-                                         height_out * width_out, kernel_h * kernel_w)):
+                and _nhwc_backward_takes(ext, batch, channels, height * width, plane_out, taps)
+                and _nhwc_backward_pays(batch, channels, channels_out, plane_out, taps,
+                                        deform_groups)):
             grads = _layer_backward_nhwc(ext, grad_output, input, offset, mask, weight, args)
             return _round_grads(out_dtype, *grads, grad_bias) + (None,) * 5
 
@@ -343,12 +345,27 @@ def _nhwc_backward_takes(ext, batch, channels, plane_in, plane_out, taps):
             and ext.transpose_takes(batch, plane_out, channels))
 
 
+def _nhwc_backward_pays(batch, channels, channels_out, plane_out, taps, deform_groups):
+    """False for the small layers that the NCHW kernels' fewer launches finish earlier: a step of
+    few columns is as long as its host side, about 135 us there and 170 to 190 us on NHWC copies
+    where the column gradient is a library product with its own layout change (fp32; 45 us more in
+    16 bits on both). Up to 512 Ki columns of at most 32 channels a group (NCHW / NHWC: 16 to 16
+    channels, 3 x 3, 441 Ki columns 133 / 171 us, 1,764 Ki 238 / 171; 24 to 40, 7 x 7, 459 Ki
+    135 / 192, 1,837 Ki 280 / 194). A thread of their coordinate kernel adds up a group's channels
+    in turn, so wider groups lose at any size (64 channels, 36 Ki columns 194 / 141). Shapes of
+    gemm_f32 stay on NHWC copies, whose products are closer to the exact ones (32 to 32, 450 Ki
+    136 / 151)."""
+    return (channels // deform_groups > 32
+            or batch * plane_out * channels * taps > 512 * 1024
+            or (channels % 16 == 0 and channels_out % 32 == 0 and taps <= 9))
+
+
 def _layer_backward_nhwc(ext, grad_output, input, offset, mask, weight, args):
     """fp32 (grad_input, grad_offset, grad_mask, grad_weight) of the groups == 1 layer, any
     deform_groups, on NHWC copies: dCol = dO @ W [M, T*C], the binned column-to-image kernel,
     the columns again for grad_weight = dO^T @ cols. The NCHW kernel adds every corner of
     every channel with one scattered atomic: a training step of six cameras at 512 channels of
-    29 x 50 took 5,880 us with it (4.3 ms in its two calls) and takes 1,519 us here."""
+    29 x 50 took 5,880 us with it (4.3 ms in its two calls) and takes 980 us here."""
     batch, channels, height, width, height_out, width_out, kernel_h, kernel_w = args[:8]
     for name, t in (("data_im", input), ("data_offset", offset), ("data_mask", mask)):
         if not t.is_contiguous():  # as the NCHW column kernels

@@ -269,6 +269,36 @@ def test_modulated_deform_conv2d_backward(groups, dg, dtype):
         check(a.grad.cpu(), r.grad, tol, f"grad {name} g{groups} dg{dg}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("b,cin,cout,h,w,k,stride,dil,dg", [
+    (2, 16, 24, 9, 10, 3, 1, 1, 1), (1, 32, 32, 7, 11, 3, 2, 1, 1), (1, 3, 8, 13, 8, 3, 1, 2, 1),
+    (3, 36, 60, 6, 5, 3, 1, 1, 3), (1, 24, 40, 12, 9, 5, 2, 1, 1), (2, 48, 64, 5, 7, 1, 1, 1, 4)])
+def test_backward_routes_agree(monkeypatch, b, cin, cout, h, w, k, stride, dil, dg, dtype):
+    """Small layers' backward on the NCHW kernels and on NHWC copies (the rule between them is one of
+    speed): each against float64, with odd sizes, strides, dilations, deformable groups and sizes
+    that the NHWC route's own products do not take."""
+    import modulated_deform_conv.modulated_deform_conv as mdc
+    g = torch.Generator().manual_seed(cin + k)
+    pad = dil * (k // 2)
+    ho, wo = ((n + 2 * pad - dil * (k - 1) - 1) // stride + 1 for n in (h, w))
+    x = torch.randn(b, cin, h, w, generator=g)
+    off = 2.0 * torch.randn(b, dg * 2 * k * k, ho, wo, generator=g)
+    mask = torch.rand(b, dg * k * k, ho, wo, generator=g)
+    weight = 0.1 * torch.randn(cout, cin, k, k, generator=g)
+    bias = torch.randn(cout, generator=g)
+    go = torch.randn(b, cout, ho, wo, generator=g).to(dtype)
+    ref_leaves = [t.to(dtype).double().requires_grad_() for t in (x, off, mask, weight, bias)]
+    od.forward_nchw(*ref_leaves, (stride, stride), (pad, pad), (dil, dil), 1, dg).backward(go.double())
+    own = cin % 16 == 0 and cout % 32 == 0 and k <= 3
+    assert mdc._nhwc_backward_pays(b, cin, cout, ho * wo, k * k, dg) == own
+    for nhwc in (False, True):
+        monkeypatch.setattr(mdc, "_nhwc_backward_pays", lambda *a: nhwc)
+        leaves = [t.to(dtype).to(DEV).requires_grad_() for t in (x, off, mask, weight, bias)]
+        mdc.modulated_deform_conv2d(*leaves, stride, pad, dil, 1, dg).backward(go.to(DEV))
+        for name, a, r in zip(("x", "offset", "mask", "weight", "bias"), leaves, ref_leaves):
+            check(a.grad.cpu(), r.grad, dtype, f"grad {name}, {'NHWC' if nhwc else 'NCHW'}")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["fp32", "fp16"])
 @pytest.mark.parametrize("bn,relu", [(False, False), (True, False), (True, True)])
 def test_dcn_split_nhwc_backward(dtype, bn, relu):
