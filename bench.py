@@ -134,8 +134,10 @@ def msda_case(name, dtype, cache):
 
 
 def dcn_fused_case(name, dtype, cache, batch=None):
-    """Fused NHWC kernel call of one DCN configuration (weight packed once, untimed, as a
-    module does on its first call); batch overrides the configuration's image count."""
+    """Call of the packed-weight entry dcn_fused_fwd_nhwc at one DCN configuration (weight packed
+    once, untimed); batch overrides the configuration's image count. The package's layers pack
+    the weight on every call and run other kernels in fp32 (channels a multiple of 32) and with
+    few pixels."""
     import torch
     import _modulated_deform_conv_ext as ext
     from oracle import inputs
@@ -157,9 +159,9 @@ def dcn_fused_case(name, dtype, cache, batch=None):
 
 
 def dcn_mega_case(name, dtype, cache):
-    """One-launch full forward (offset conv + sigmoid + deformable gather + GEMM) of one DCN
-    configuration, weights packed once (untimed). Work: 2*M*K*(Cout + 3T) flops (the offset
-    conv and the deformable conv)."""
+    """Full forward (offset conv + sigmoid + deformable gather + GEMM) through the packed-weight
+    entry dcn_mega_fwd_nhwc at one DCN configuration, weights packed once (untimed). Work:
+    2*M*K*(Cout + 3T) flops (the offset conv and the deformable conv)."""
     import torch
     import _modulated_deform_conv_ext as ext
     from oracle import inputs

@@ -17,10 +17,10 @@
 // 2^-115: 1.1e-6, at 2^-120: 3.5e-5; the library product 2.8e-7).
 //
 // Bound: the matrix cores. Six cameras at 256 channels of 58 x 100 to 256 (41 GFLOP): 500 us
-// on the fp32 matrix cores (82 TFLOP/s of 157), 220-245 us here (1.0-1.1 PFLOP/s of bf16
+// on the fp32 matrix cores (82 TFLOP/s of 157), 205-220 us here (1.1-1.2 PFLOP/s of bf16
 // products, where a large bf16 library product reaches 1.2 on the same card); with the module's
-// layout changes 253 us, of which four of the six products take 100, the gathers 64, the
-// weight loads 12 and the blend and cut 10 (each left out in turn).
+// preparation launch 225-232 us a call. Left out in turn in an earlier form of 253 us a call: four of
+// the six products 100, the gathers 64, the weight loads 12, the blend and cut 10.
 // Pairs of row blocks with four independent MFMA chains, or two chains for the small products,
 // measured the same or slower: their dependent chain is not what limits.
 //

@@ -1624,7 +1624,9 @@ __global__ void __launch_bounds__(256) kparts_total_kernel(const float *__restri
 // 0.1 + 0.155 NRB us (measured at 2, 5 and 9), a launch 6 us, the sums 8 bytes each at 4.5 TB/s
 // and their reduction 3 us; parts run where that is under 0.9 of the whole-K time: 512 channels
 // of 29 x 50, one image, 512 outputs: 35 us whole (2 row blocks x 72 steps), 25 us (20.5 + 4.3) in 4
-// parts; 256 channels of 58 x 100, one image: whole.
+// parts; 256 channels of 58 x 100, one image: whole. Calls, parts against whole: 512 to 256 channels
+// of 58 x 71 (4 row blocks, 3 parts) 32 / 39 us, 1,024 to 512 of 40 x 40 (4, 5) 37 / 67, 512 to 160
+// of 3 x 29 x 50 (5, 4) 31 / 34, 2,048 to 256 of 50 x 50 (5, 8) 48 / 126.
 struct KConfig {
   int nrb = 0, kparts = 1, chunks = 0;
 };

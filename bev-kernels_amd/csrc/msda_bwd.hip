@@ -927,8 +927,8 @@ struct BktParams {
   int blocks_per_xcd;
   int cblk8;        // count / place chunks per XCD
   int pblk;         // count / place blocks per XCD (persistent)
-  float *zero;      // 16-bit types: the fp32 grad_value workspace, cleared by the count
-  int64_t nzero4;   //   kernel (float4 groups; 0: nothing to clear)
+  float *zero;      // the fp32 grad_value (16-bit types: its workspace) that the count kernel
+  int64_t nzero4;   //   clears (float4 groups; 0: it holds what is added to)
 };
 
 // a / d for 0 <= a < 2^24 and 0 < d: a reciprocal estimate and one correction step
@@ -1043,8 +1043,8 @@ __global__ void __launch_bounds__(kBkThreads) msda_bkt_count_kernel(const BktPar
   ChunkSamples<T> cs;
   int lb = lb0 + (int)(blockIdx.x >> 3);
   if (lb < lb1) load_chunk<T>(p, lb, cs);
-  // the fp32 workspace of 16-bit types, cleared here (the accumulate kernel adds to it
-  // after this kernel): the block's share in 16-byte stores, a few per thread and chunk
+  // a fresh fp32 grad_value or the fp32 workspace of 16-bit types, cleared here (the accumulate
+  // kernel adds to it after this kernel): the block's share in 16-byte stores, a few per thread and chunk
   // so that they stream out while the blocks compute, the rest after the last chunk
   const int64_t zper = (p.nzero4 + gridDim.x - 1) / gridDim.x;
   const int64_t z0 = (int64_t)blockIdx.x * zper, z1 = min(z0 + zper, p.nzero4);

@@ -4,8 +4,9 @@ naotic/bev-kernels modulated_deform_conv/dcn_split_nhwc.py.
 Layout: x [B,H,W,Cin], w_off [3T,Cin,kH,kW], b_off [3T], weight [Cout,Cin,kH,kW];
 output [B,Ho,Wo,Cout].
 
-The forward is one gfx950 kernel (_modulated_deform_conv_ext.dcn_mega_fwd_nhwc): the
-offset conv runs on the matrix cores with fp32 accumulation, its output y [B,Ho,Wo,3T]
+The forward is one call (_modulated_deform_conv_ext.dcn_layer_nhwc) that packs the weights and runs
+one gfx950 kernel where Cout fits it, else the offset conv and the deformable product one after the
+other: the offset conv runs on the matrix cores with fp32 accumulation, its output y [B,Ho,Wo,3T]
 (offsets, then the pre-sigmoid mask; kept in fp32) feeds the deformable taps, which are
 built in LDS and multiplied on the matrix cores, and the FrozenBN + ReLU epilogue is
 folded into the weight, the bias and the kernel's store. Neither the [M, T*Cin] column
@@ -130,7 +131,7 @@ def offset_conv_supported(x_nhwc, w_off):
 
 
 def mega_supported(x_nhwc, w_off, weight):
-    """True when the one-kernel forward (dcn_mega_fwd_nhwc) takes these tensors."""
+    """True when the one-call forward (dcn_layer_nhwc, dcn_mega_fwd_nhwc) takes these tensors."""
     return (offset_conv_supported(x_nhwc, w_off)
             and tuple(weight.shape[1:]) == tuple(w_off.shape[1:]))
 
