@@ -400,7 +400,8 @@ def test_sorted_ragged(dtype):
 ])
 def test_sorted_two_halves(geom, dtype):
     """Heads of 64 channels: the records are sorted once and summed in two launches of 32
-    channels each; concentrated locations too, whose buckets fill several pieces."""
+    channels each (three and four levels: from more samples on, test_sorted_two_halves_line; these
+    sizes run the atomic kernels); concentrated locations too, whose buckets fill several pieces."""
     d = inputs.msda_random(*geom, seed=19, loc_lo=-0.2, loc_hi=1.2)
     go = _grad_output(d, seed=8)
     _check3(_run(d, go, dtype), _ref(d, go, dtype), dtype, f"halves {geom} {dtype}")
